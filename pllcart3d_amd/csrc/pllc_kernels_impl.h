@@ -405,6 +405,7 @@ struct LineSet {
     const T* Nm1;
     int ghost_c;          // also fill c_new's y/z ghosts (700-712)
     int ghost_v;          // 0, or FU/FV/FW: also fill that component's ghosts (velo_ghost_point)
+    int jg, kg, inlet;    // which those are: y ghosts, z ghosts, inlet ghosts
     int F;                // the field (FC, FU, FV, FW): its constants in a batch's table
 };
 
@@ -2434,9 +2435,7 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     template __global__ void k_sweep_z_lds<T>(Dims, LineSets<T>, const double*, T, T);                         \
     template __global__ void k_sweep_part<T, 0>(Dims, LineSets<T>, const double*, int, T, T, Bt);             \
     template __global__ void k_sweep_part<T, 1>(Dims, LineSets<T>, const double*, int, T, T, Bt);             \
-    template __global__ void k_sweep_part_z<T>(Dims, LineSets<T>, const double*, T, T, int, int, int, int,     \
-                                               int);                                                            \
-    template __global__ void k_sweep_part_zt<T>(Dims, LineSets<T>, const double*, T, T, int, Bt);              \
+    template __global__ void k_sweep_wave_z<T>(Dims, LineSets<T>, const double*, T, T, int, int, int, int, Bt); \
     template __global__ void k_visc<T>(Dims, Phys, const T*, T*, T*, T*, T*, Bt);                              \
     template __global__ void k_velo_ghost<T>(Dims, T*, T*, T*);                                                \
     template __global__ void k_phi_ghost<T>(Dims, T*);                                                         \
@@ -2559,28 +2558,69 @@ __device__ __forceinline__ int2 xcd_block_xy()
 
 // ------------------------------------------------ partitioned line solve
 //
-// The same systems as k_sweep, cut into P chunks of at most PM rows per
-// line, one thread per chunk (the partition method for tridiagonal systems
-// used by hybrid batched solvers).  A thread eliminates its chunk down to
-// rows of the form A_t x_first + x_t + C_t x_last = D_t; its first and last
-// rows couple only to the neighbouring chunks' boundary unknowns and make a
-// reduced tridiagonal system of 2P rows per line, solved in LDS by one
-// thread per line; every row then follows from its chunk's two boundary
-// values.  Compared with one thread per line this gives P times the
-// threads, keeps the eliminated rows in registers (no Thomas factors in
-// HBM: S and mu are read once, the solution written once) and reads each
-// row with one coalesced access per wavefront.  (I - fac A) is strictly
+// The same systems as k_sweep, each line cut into P chunks of PM rows, one
+// thread per chunk (the partition method for tridiagonal systems used by
+// hybrid batched solvers).  A thread eliminates its chunk down to rows of the
+// form A_t x_first + x_t + C_t x_last = D_t; its first and last rows couple
+// only to the neighbouring chunks' boundary unknowns, a system solved by the
+// line's threads together (PcrRow); every row then follows from its chunk's
+// two boundary values.  Compared with one thread per line this gives P times
+// the threads, keeps the eliminated rows in registers (no Thomas factors in
+// HBM: S and mu are read once, the solution written once) and reads each row
+// with one coalesced access per wavefront.  (I - fac A) is strictly
 // diagonally dominant, so the result equals the Thomas solution to rounding.
+//
+// The kernels are bound by the latency of one chunk's instructions, so a
+// chunk is straight code: all chunks have PM rows, a line's last chunk filled
+// up with rows x = 0 that couple to nothing, and boundary rows differ by
+// numbers instead of branches.  (Chunks of varying length with their rows
+// under conditions took 711 branches and 1700 integer instructions for the
+// 650 FP64 operations of an x chunk, and one thread per line solving the
+// coupling from LDS 2P dependent steps.)
 constexpr int PM = 16;
+constexpr int PART_THREADS = 512;    // threads per block of k_sweep_part at most
+constexpr int POIS_THREADS = 1024;   // of k_pois_part
 
-// rows [x0, x0+m) of a line: forward elimination as rows arrive, then the
-// backward pass and the first row's fold; leaves the two reduced rows in
-// A/C/D[0] and A/C/D[m-1]
+// keeps the scheduler from moving a chunk's rows into each other, which
+// takes more registers than a wave has for them
+__device__ __forceinline__ void row_done() { __builtin_amdgcn_sched_barrier(0); }
+
+// the same offset with its origin hidden from the compiler, which otherwise
+// keeps the 16 addresses of a chunk's loads in registers (32 of them) for
+// the stores after the solve
+__device__ __forceinline__ long renew(long o)
+{
+    asm volatile("" : "+v"(o));
+    return o;
+}
+
+// a line's rows of one chunk: row t is -k_t x_{t-1} + (1 + k_t + k_{t+1}) x_t
+// - k_{t+1} x_{t+1} = sv[t], k_t = kf mv[t], kf = fac del / h, mv the
+// viscosity (1 for c).  The line's last row is row tl (PM or more: in a later
+// chunk), its upper coefficient k_{tl+1} counted e1 times in the diagonal and
+// dropped; first: row 0 is the line's first, its k_0 counted e0 times and
+// dropped.  Rows past tl hold anything finite: they read row tl, no row reads
+// them.
+template <typename T>
+struct PRows {
+    T sv[PM], mv[PM + 1], kf, e0, e1;
+    int tl;
+    bool first;
+};
+
+// the factor of a boundary row's outer coefficient in its diagonal: Neumann
+// b += off, Dirichlet b -= off (apply_bc) with off = -k
+template <typename T>
+__device__ __forceinline__ T bc_factor(int kind)
+{
+    return kind == BC_NEU ? T(0.0) : kind == BC_DIR ? T(2.0) : T(1.0);
+}
+
 template <typename T>
 struct PChunk {
     T A[PM], C[PM], D[PM];
 
-    // row t of the chunk (t is a constant once the callers' loops unroll)
+    // row t: a x_{t-1} + b x_t + c x_{t+1} = d (rows in order)
     __device__ __forceinline__ void fwd(int t, T a, T b, T c, T d)
     {
         if (t < 2) {
@@ -2594,15 +2634,16 @@ struct PChunk {
         }
     }
 
-    __device__ __forceinline__ void fold(int m)
+    // the backward pass and the first row's fold; leaves the chunk's outer
+    // rows in A/C/D[0] and A/C/D[PM - 1]
+    __device__ __forceinline__ void fold()
     {
 #pragma unroll
         for (int t = PM - 3; t >= 1; t--) {
-            if (t <= m - 3) {
-                D[t] = D[t] - C[t] * D[t + 1];
-                A[t] = A[t] - C[t] * A[t + 1];
-                C[t] = -C[t] * C[t + 1];
-            }
+            D[t] = D[t] - C[t] * D[t + 1];
+            A[t] = A[t] - C[t] * A[t + 1];
+            C[t] = -C[t] * C[t + 1];
+            row_done();
         }
         const T rb = prcp<T>(T(1.0) - C[0] * A[1]);
         D[0] = rb * (D[0] - C[0] * D[1]);
@@ -2610,570 +2651,545 @@ struct PChunk {
         C[0] = -rb * C[0] * C[1];
     }
 
-    // the chunk's last row (runtime m, static register indices)
-    __device__ __forceinline__ void last(int m, T& a, T& c, T& d) const
+    // the chunk's solution from its boundary values, in D
+    __device__ __forceinline__ void solve(T xf, T xl)
     {
+        D[0] = xf;
 #pragma unroll
-        for (int t = 2; t < PM; t++)
-            if (t == m - 1) { a = A[t]; c = C[t]; d = D[t]; }
+        for (int t = 1; t < PM - 1; t++) D[t] = D[t] - A[t] * xf - C[t] * xl;
+        D[PM - 1] = xl;
     }
 };
 
-// the reduced system of one line: rows e = 2s (first row of chunk s) and
-// e = 2s+1 (last row), unit diagonal; stored [3][E][LPB] with the line
-// index fastest.  Thomas in place: D ends as the boundary values.
 template <typename T>
-__device__ __forceinline__ void pchunk_reduced(T* __restrict__ red, int E, int LPB, int q)
+__device__ __forceinline__ void chunk_rows(PChunk<T>& ch, const PRows<T>& r)
 {
-    T* rA = red;
-    T* rC = red + E * LPB;
-    T* rD = red + 2 * E * LPB;
-    T cp = rC[q], dp = rD[q];
-    for (int e = 1; e < E; e++) {
-        const int o = e * LPB + q;
-        const T a = rA[o];
-        const T rb = prcp<T>(T(1.0) - a * cp);
-        cp = rC[o] * rb;
-        dp = (rD[o] - a * dp) * rb;
-        rC[o] = cp;
-        rD[o] = dp;
+    T k0 = r.kf * r.mv[0];
+#pragma unroll
+    for (int t = 0; t < PM; t++) {
+        const T k1 = r.kf * r.mv[t + 1];
+        const bool end = t == r.tl;
+        T a = -k0, kb = k0;
+        if (t == 0) {
+            kb = (r.first ? r.e0 : T(1.0)) * k0;
+            a = r.first ? T(0.0) : a;
+        }
+        const T b = T(1.0) + kb + (end ? r.e1 * k1 : k1);
+        ch.fwd(t, a, b, end ? T(0.0) : -k1, r.sv[t]);
+        k0 = k1;
+        row_done();
     }
-    T xn = dp;
-    for (int e = E - 2; e >= 0; e--) {
-        const int o = e * LPB + q;
-        xn = rD[o] - rC[o] * xn;
-        rD[o] = xn;
-    }
+    ch.fold();
 }
 
-// raw row of line set L at row x (x in [0, n)): coefficients from the
-// viscosity value of the row below (araw) and above (craw), boundary rows
-// closed as in k_sweep; a at row 0 and c at row n-1 are dropped after
-template <typename T, int DIR>
-__device__ __forceinline__ void prow(const LineSet<T>& L, int x, int n, T fac, T araw, T craw, T bcor, T& a, T& b,
-                                     T& c, T& rhs)
+// A chunk's share of its line's coupling.  The first row is A0 x_last(s-1) +
+// x_first + C0 x_last = D0, the last Al x_first + x_last + Cl x_first(s+1) =
+// Dl; with the first rows eliminated the P last unknowns form a tridiagonal
+// system of unit diagonal, a x_last(s-1) + x_last + c x_last(s+1) = d, solved
+// by parallel cyclic reduction: log2(P) rounds in which row s takes rows
+// s -/+ w, w = 1, 2, 4, ..., zero outside the line.
+template <typename T>
+struct PcrRow {
+    T a, c, d;
+    // An, Cn, Dn: the next chunk's first row (zero after the last chunk)
+    __device__ __forceinline__ void start(const PChunk<T>& ch, T An, T Cn, T Dn)
+    {
+        const T Al = ch.A[PM - 1], Cl = ch.C[PM - 1];
+        const T r = prcp<T>(T(1.0) - Al * ch.C[0] - Cl * An);
+        a = -(Al * ch.A[0]) * r;
+        c = -(Cl * Cn) * r;
+        d = (ch.D[PM - 1] - Al * ch.D[0] - Cl * Dn) * r;
+    }
+    __device__ __forceinline__ void round(T am, T cm, T dm, T ap, T cp, T dp)
+    {
+        const T r = prcp<T>(T(1.0) - a * cm - c * ap);
+        d = (d - a * dm - c * dp) * r;
+        a = -(a * am) * r;
+        c = -(c * cp) * r;
+    }
+};
+
+// the coupling through LDS, for lines whose chunks are threads s = 0 .. P-1
+// of a block at the same q: two sets of [3][P][LPB] values read and written
+// in turn, so a round needs one barrier.  Every thread of the block calls it
+// (dead threads, without a line, only keep the barriers).
+template <typename T>
+__device__ __forceinline__ void chunk_couple(T* __restrict__ buf, int P, int LPB, int q, int s, bool live,
+                                             PChunk<T>& ch)
 {
-    const bool cst = L.mu == nullptr;
-    const T braw = cst ? L.cb : -(araw + craw);
-    a = -fac * araw;
-    b = T(1.0) - fac * braw;
-    c = -fac * craw;
-    if (x == 0) { apply_bc(L.bc0, b, a, rhs); a = T(0.0); }
-    if (x == n - 1) {
-        if (DIR == 0) rhs -= c * bcor;
-        else apply_bc(L.bc1, b, c, rhs);
-        c = T(0.0);
+    const int PL = P * LPB, o = s * LPB + q;
+    T* cur = buf;
+    T* nxt = buf + 3 * PL;
+    if (live) {
+        cur[o] = ch.A[0];
+        cur[PL + o] = ch.C[0];
+        cur[2 * PL + o] = ch.D[0];
+    }
+    __syncthreads();
+    PcrRow<T> w;
+    if (live) {
+        const bool in = s + 1 < P;
+        const int e = in ? o + LPB : o;
+        const T An = cur[e], Cn = cur[PL + e], Dn = cur[2 * PL + e];
+        w.start(ch, in ? An : T(0.0), in ? Cn : T(0.0), in ? Dn : T(0.0));
+        nxt[o] = w.a;
+        nxt[PL + o] = w.c;
+        nxt[2 * PL + o] = w.d;
+    }
+    __syncthreads();
+    for (int k = 1; k < P; k <<= 1) {
+        T* t = cur;
+        cur = nxt;
+        nxt = t;
+        if (live) {
+            const bool lo = s >= k, hi = s + k < P;
+            const int el = lo ? o - k * LPB : o, eh = hi ? o + k * LPB : o;
+            const T am = cur[el], cm = cur[PL + el], dm = cur[2 * PL + el];
+            const T ap = cur[eh], cp = cur[PL + eh], dp = cur[2 * PL + eh];
+            w.round(lo ? am : T(0.0), lo ? cm : T(0.0), lo ? dm : T(0.0), hi ? ap : T(0.0), hi ? cp : T(0.0),
+                    hi ? dp : T(0.0));
+            nxt[o] = w.a;
+            nxt[PL + o] = w.c;
+            nxt[2 * PL + o] = w.d;
+        }
+        __syncthreads();
+    }
+    if (live) {
+        const T xp = s > 0 ? nxt[2 * PL + o - LPB] : T(0.0);
+        ch.solve(ch.D[0] - ch.C[0] * w.d - ch.A[0] * xp, w.d);
     }
 }
 
 // x- and y-lines (rows strided by sx / sy): block (LPB lines along k,
-// P chunks); a wavefront reads one row of consecutive k, coalesced
+// P chunks); a wavefront reads one row of consecutive k, coalesced.  At most
+// 128 registers (q_old is read after the coupling), so that in FP64 two
+// blocks of 512 threads share a CU.  Measured, u, v and w in one launch, with
+// branches and a serial coupling before: 256x128x128 x 117 -> 83 us FP64
+// (5.1 TB/s of S, mu, q_old, q_new), 59 -> 40 mixed, y 63 -> 57 and 35 -> 27;
+// 512x256x256 x 1110 -> 750 and 552 -> 422, y 475 -> 473 (5.3 TB/s) and 257 ->
+// 232; 64x32x32 (latency) x 11.6 -> 9.1, y 8.1 -> 5.3
 template <typename T, int DIR>
-__global__ __launch_bounds__(512) void k_sweep_part(Dims d, LineSets<T> sets, const double* __restrict__ scal,
-                                                    int slot, T g, T r, Bt bt)
+__global__ __launch_bounds__(PART_THREADS, 4) void k_sweep_part(Dims d, LineSets<T> sets, const double* __restrict__ scal,
+                                                       int slot, T g, T r, Bt bt)
 {
     extern __shared__ unsigned char pllc_smem[];
     T* red = reinterpret_cast<T*>(pllc_smem);
-    const int LPB = blockDim.x, P = blockDim.y, E = 2 * P;
-    const int q = threadIdx.x, s = threadIdx.y;
+    const int LPB = blockDim.x, q = threadIdx.x, s = threadIdx.y;
     // member: blockIdx.z
     const LineSet<T> L = bt_lines<T, DIR>(bt, sets.s[blockIdx.y], blockIdx.z);
     scal += blockIdx.z * S_SIZE;
     const Rng R = L.R;
-    const int n0 = R.ke - R.ks + 1;
-    const int n1 = DIR == 0 ? R.je - R.js + 1 : R.ie - R.is + 1;
+    // x-lines: the y and z ghosts of the new values (kg, jg) are lanes of
+    // their own that solve the line next to the wall again and store at
+    // their own place, so a ghost costs no store of its own
+    const int kg = DIR == 0 && L.kg, jg = DIR == 0 && L.jg;
+    const int n0 = R.ke - R.ks + 1 + 2 * kg;
+    const int n1 = DIR == 0 ? R.je - R.js + 1 + 2 * jg : R.ie - R.is + 1;
     // blocks of one line set: grid x is a multiple of 8 (XCD order within the set)
     const int bx = (gridDim.x & 7) == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const int l = bx * LPB + q;
-    const bool live = l < n0 * n1;
-    const int a0 = live ? l % n0 : 0, a1 = live ? l / n0 : 0;
-    int i, j, k, n;
+    const int n = DIR == 0 ? R.ie - R.is + 1 : R.je - R.js + 1;
+    const int x0 = s * PM;
+    // a set with shorter lines than the launch's longest may need fewer chunks
+    const bool live = l < n0 * n1 && x0 < n;
+    const int a1 = live ? l / n0 : 0, a0 = live ? l - a1 * n0 : 0;
+    const int kl = R.ks - kg + a0, jl = R.js - jg + a1;   // the lane's place (x-lines)
+    const int k = min(max(kl, R.ks), R.ke);
+    int i, j;
     long st;
-    if (DIR == 0) { k = R.ks + a0; j = R.js + a1; i = R.is; n = R.ie - R.is + 1; st = d.sx; }
-    else { k = R.ks + a0; i = R.is + a1; j = R.js; n = R.je - R.js + 1; st = d.sy; }
-    const int x0 = (s * n) / P;
-    const int m = ((s + 1) * n) / P - x0;
-    const long o0 = IX(d, i, j, k);
-    T* __restrict__ S = L.S + o0;
+    if (DIR == 0) { j = min(max(jl, R.js), R.je); i = R.is; st = d.sx; }
+    else { i = R.is + a1; j = R.js; st = d.sy; }
+    const bool own = k == kl && (DIR != 0 || j == jl);   // not a ghost lane
+    const bool last = x0 + PM >= n;
+    const int nv = min(PM, n - x0);
+    const long o0 = IX(d, i, j, k) + (long)(live ? x0 : 0) * st;
+    const T* __restrict__ S = L.S + o0;
     const bool cst = L.mu == nullptr;
-    const T* __restrict__ mu = cst ? nullptr : L.mu + o0 + L.mu_off;
-    const T del = L.del, h = L.h;
-    const double rh = L.rh;
     const T dt = T(scal[S_DT]);
     const T fac = T(0.5) * dt * (g + r);
 
     PChunk<T> ch;
-    T qo[PM];
     if (live) {
-        T bcor = T(0.0);
-        if (DIR == 0 && s == P - 1) {
-            // explicit outflow face iend+1 (677-683 and matching lines)
-            const long ob = o0 + (long)n * st;
-            const T vbulk = T(scal[S_RK + 4 * slot]);
-            const T nb = divh<T>(-vbulk * (L.qold[ob] - L.qold[ob - st]), T(d.dx), d.rdx);
-            L.N[ob] = nb;
-            bcor = dt * (g * nb + r * L.Nm1[ob]);
-            L.qnew[ob] = L.qold[ob] + bcor;
-        }
-        T sv[PM], mv[PM + 1];
+        PRows<T> w;
+        w.tl = nv - 1;
+        if (!last) w.tl = PM;
+        // past the line's end: its last row (and the mu above it) again
+        const T* __restrict__ mu = cst ? nullptr : L.mu + o0 + L.mu_off;
+        if (nv == PM) {
 #pragma unroll
-        for (int t = 0; t < PM; t++)
-            if (t < m) sv[t] = S[(long)(x0 + t) * st];
-        if (!cst) {
+            for (int t = 0; t < PM; t++) w.sv[t] = S[(long)t * st];
+            if (!cst) {
 #pragma unroll
-            for (int t = 0; t <= PM; t++)
-                if (t <= m) mv[t] = mu[(long)(x0 + t) * st];
-        }
-        T araw = cst ? L.ca : divh<T>(del * mv[0], h, rh);
+                for (int t = 0; t <= PM; t++) w.mv[t] = mu[(long)t * st];
+            }
+        } else {
+            const int si = (int)st;
+            const unsigned lim = (nv - 1) * si;
 #pragma unroll
-        for (int t = 0; t < PM; t++) {
-            if (t < m) {
-                const T craw = cst ? L.cc : divh<T>(del * mv[t + 1], h, rh);
-                T a, b, c, rhs = sv[t];
-                prow<T, DIR>(L, x0 + t, n, fac, araw, craw, bcor, a, b, c, rhs);
-                ch.fwd(t, a, b, c, rhs);
-                araw = craw;
+            for (int t = 0; t < PM; t++) w.sv[t] = S[min((unsigned)(t * si), lim)];
+            if (!cst) {
+#pragma unroll
+                for (int t = 0; t <= PM; t++) w.mv[t] = mu[min((unsigned)(t * si), lim + si)];
             }
         }
-        ch.fold(m);
-        T la, lc, ld;
-        ch.last(m, la, lc, ld);
-        const int e0 = 2 * s;
-        red[e0 * LPB + q] = ch.A[0];
-        red[(E + e0) * LPB + q] = ch.C[0];
-        red[(2 * E + e0) * LPB + q] = ch.D[0];
-        red[(e0 + 1) * LPB + q] = la;
-        red[(E + e0 + 1) * LPB + q] = lc;
-        red[(2 * E + e0 + 1) * LPB + q] = ld;
-        if (DIR == 0) {
-            // q_old for the update, in flight during the reduced solve (and
-            // all of it loaded before the first store of q_new)
+        if (cst) {
+#pragma unroll
+            for (int t = 0; t <= PM; t++) w.mv[t] = T(1.0);
+        }
+        w.kf = cst ? fac * L.ca : fac * L.del * T(L.rh);
+        w.first = s == 0;
+        w.e0 = bc_factor<T>(L.bc0);
+        w.e1 = DIR == 0 ? T(1.0) : bc_factor<T>(L.bc1);
+        if (DIR == 0 && last) {
+            // explicit outflow face iend+1 (677-683 and matching lines)
+            const long ob = o0 + (long)nv * st;
+            const T vbulk = T(scal[S_RK + 4 * slot]);
+            const T q1 = L.qold[ob], q0 = L.qold[ob - st], n1o = L.Nm1[ob];
+            const T mtop = cst ? T(1.0) : mu[(long)nv * st];
+            const T nb = divh<T>(-vbulk * (q1 - q0), T(d.dx), d.rdx);
+            const T bcor = dt * (g * nb + r * n1o);
+            if (own) {
+                L.N[ob] = nb;
+                L.qnew[ob] = q1 + bcor;
+            }
+            const T radd = w.kf * mtop * bcor;
+#pragma unroll
+            for (int t = 0; t < PM; t++) w.sv[t] += t == w.tl ? radd : T(0.0);
+        }
+        chunk_rows<T>(ch, w);
+    }
+    chunk_couple<T>(red, (n + PM - 1) / PM, LPB, q, s, live, ch);
+    if (!live) return;
+    const long on = renew(o0);
+    if (DIR == 1) {
+        T* so = L.S + on;
+        if (nv == PM) {
+#pragma unroll
+            for (int t = 0; t < PM; t++) so[(long)t * st] = ch.D[t];
+        } else {
 #pragma unroll
             for (int t = 0; t < PM; t++)
-                if (t < m) qo[t] = L.qold[o0 + (long)(x0 + t) * st];
+                if (t < nv) so[(long)t * st] = ch.D[t];
         }
+        return;
     }
-    __syncthreads();
-    if (live && s == 0) pchunk_reduced<T>(red, E, LPB, q);
-    __syncthreads();
-    if (!live) return;
-    const T X0 = red[(2 * E + 2 * s) * LPB + q], X1 = red[(2 * E + 2 * s + 1) * LPB + q];
+    // c's ghosts are copies (700-712; the y-ghost rows' z ghosts too), the
+    // velocities' z ghosts copies, their y ghosts negated, their corners
+    // never written (velo_ghost_point)
+    const bool vel = L.F != FC, jgh = j != jl;
+    if (vel && jgh && k != kl) return;
+    const T sg = vel && jgh ? T(-1.0) : T(1.0);
+    const T* qo = L.qold + on;
+    T* qn = L.qnew + on + (long)(jl - j) * d.sy + (kl - k);
+    if (nv == PM) {
+        T v[PM];
 #pragma unroll
-    for (int t = 0; t < PM; t++) {
-        if (t < m) {
-            const T sol = t == 0 ? X0 : t == m - 1 ? X1 : ch.D[t] - ch.A[t] * X0 - ch.C[t] * X1;
-            const long o = (long)(x0 + t) * st;
-            if (DIR == 0) {
-                const T val = qo[t] + sol;
-                T* qn = L.qnew;
-                qn[o0 + o] = val;
-                if (L.ghost_v) velo_ghost_point<T>(d, L.ghost_v, qn + o0 + o, R.is + x0 + t, j, k, val);
-                if (L.ghost_c) {
-                    // c_new's ghost copies of this value: y ghosts (701-704),
-                    // then z ghosts incl. the y-ghost rows (707-712)
-                    const int ii = R.is + x0 + t;
-                    if (j == R.js) qn[IX(d, ii, j - 1, k)] = val;
-                    if (j == R.je) qn[IX(d, ii, j + 1, k)] = val;
-                    if (k == R.ks) {
-                        qn[IX(d, ii, j, k - 1)] = val;
-                        if (j == R.js) qn[IX(d, ii, j - 1, k - 1)] = val;
-                        if (j == R.je) qn[IX(d, ii, j + 1, k - 1)] = val;
-                    }
-                    if (k == R.ke) {
-                        qn[IX(d, ii, j, k + 1)] = val;
-                        if (j == R.js) qn[IX(d, ii, j - 1, k + 1)] = val;
-                        if (j == R.je) qn[IX(d, ii, j + 1, k + 1)] = val;
-                    }
-                }
-            } else {
-                S[o] = sol;
-            }
+        for (int t = 0; t < PM; t++) v[t] = qo[(long)t * st];
+#pragma unroll
+        for (int t = 0; t < PM; t++) {
+            ch.D[t] = sg * (v[t] + ch.D[t]);
+            qn[(long)t * st] = ch.D[t];
         }
+    } else {
+#pragma unroll
+        for (int t = 0; t < PM; t++)
+            if (t < nv) {
+                ch.D[t] = sg * (qo[(long)t * st] + ch.D[t]);
+                qn[(long)t * st] = ch.D[t];
+            }
     }
+    // the inlet ghosts of v and w
+    if (s == 0 && own && L.inlet) qn[-d.sx] = -ch.D[0];
 }
 
-// z-lines, one tile per block (the FP32 path): the block's LPB lines (one
-// i, LPB consecutive j) are staged through LDS with consecutive threads on
-// consecutive k, solved by chunk from LDS, and written back the same way.
-// w is the LDS row pitch of a line (at least n + 1).
-template <typename T>
-__global__ __launch_bounds__(256) void k_sweep_part_zt(Dims d, LineSets<T> sets, const double* __restrict__ scal, T g,
-                                                      T r, int w, Bt bt)
+// value of x moved by W lanes within its row of 16 lanes (UP: from the lane
+// W below), by a DPP move; zero where that lies outside the row
+template <int W, bool UP>
+__device__ __forceinline__ int dpp_shift(int x)
 {
-    extern __shared__ unsigned char pllc_smem[];
-    const int LPB = blockDim.x, P = blockDim.y, E = 2 * P, NT = LPB * P;
-    const int q = threadIdx.x, s = threadIdx.y, tid = s * LPB + q;
-    // blockIdx.z: member * sets + set
-    int set;
-    const int mb = bt_member(bt, blockIdx.z, gridDim.z, set);
+    return __builtin_amdgcn_update_dpp(0, x, (UP ? 0x110 : 0x100) + W, 0xf, 0xf, true);
+}
+template <int W, bool UP>
+__device__ __forceinline__ float lane_shift(float x)
+{
+    return __int_as_float(dpp_shift<W, UP>(__float_as_int(x)));
+}
+template <int W, bool UP>
+__device__ __forceinline__ double lane_shift(double x)
+{
+    return __hiloint2double(dpp_shift<W, UP>(__double2hiint(x)), dpp_shift<W, UP>(__double2loint(x)));
+}
+
+// one round of the coupling between lanes W apart, lane g of a line's P.
+// ROW: the line's lanes lie in one row of 16 (DPP moves); else ds_bpermute.
+template <typename T, int W, bool ROW>
+__device__ __forceinline__ void lane_round(PcrRow<T>& w, int g, int P)
+{
+    const bool lo = g >= W, hi = g + W < P;
+    T am, cm, dm, ap, cp, dp;
+    if constexpr (ROW) {
+        am = lane_shift<W, true>(w.a); cm = lane_shift<W, true>(w.c); dm = lane_shift<W, true>(w.d);
+        ap = lane_shift<W, false>(w.a); cp = lane_shift<W, false>(w.c); dp = lane_shift<W, false>(w.d);
+    } else {
+        am = __shfl_up(w.a, W); cm = __shfl_up(w.c, W); dm = __shfl_up(w.d, W);
+        ap = __shfl_down(w.a, W); cp = __shfl_down(w.c, W); dp = __shfl_down(w.d, W);
+    }
+    w.round(lo ? am : T(0.0), lo ? cm : T(0.0), lo ? dm : T(0.0), hi ? ap : T(0.0), hi ? cp : T(0.0),
+            hi ? dp : T(0.0));
+}
+
+// z-lines (rows contiguous along k).  A wave owns 64 chunks: 64 / G lines of
+// one i-plane and one line set (consecutive j), G lanes per line, G the power
+// of two of at least the P chunks of a line.  The rows pass through the
+// wave's own LDS tile (coalesced in HBM, by chunk in registers; slot 17 g +
+// t holds row 16 g + t, so the lanes' chunk reads fall in distinct banks and
+// slot 17 g + 16 is free), S first, then mu in the same slots, then the
+// solution; the coupling runs between lanes.  Waves are independent of each
+// other: no block barriers, so the loads, eliminations and stores of a CU's
+// waves overlap.  Bound by HBM in both precisions: u, v and w at 256x128x128
+// 56 us FP64 (5.7 TB/s of S, mu, S) and 28 us mixed, where a tile per block
+// with the rows' loads, eliminations and stores between block barriers took
+// 90 and 51; at 512x256x256 480 and 229 us against 790 and 325; at 64x32x32
+// 7.1 against 12.  (FP64 at 4 waves per SIMD spills: 64 us.)  nbx: tiles per
+// plane; ntiles: tiles of all planes and sets
+// of a member.
+constexpr int ZW = 17;                    // LDS slots per chunk
+constexpr int Z_TILE = 64 * ZW;           // per wave
+constexpr int Z_WAVES = 4;                // waves per block at most
+
+template <typename T>
+__global__ __launch_bounds__(64 * Z_WAVES, sizeof(T) == 8 ? 3 : 4) void k_sweep_wave_z(Dims d, LineSets<T> sets,
+                                                                  const double* __restrict__ scal, T g, T r, int G,
+                                                                  int nbx, int ni, int ntiles, Bt bt)
+{
+    extern __shared__ __align__(16) unsigned char pllc_smem[];
+    const int lane = threadIdx.x & 63;
+    T* ls = reinterpret_cast<T*>(pllc_smem) + (threadIdx.x >> 6) * Z_TILE;
+    const int mb = blockIdx.y;   // member
+    // XCD x takes the x-th eighth of the blocks: neighbouring tiles share
+    // cache lines at their edges
+    const int bx = (gridDim.x & 7) == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int tile = __builtin_amdgcn_readfirstlane(bx * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    if (tile >= ntiles) return;
+    const int per_set = nbx * ni, set = tile / per_set, rem = tile - set * per_set;
+    const int ii = rem / nbx, jb = rem - ii * nbx;
     const LineSet<T> L = bt_lines<T, 2>(bt, sets.s[set], mb);
     scal += mb * S_SIZE;
     const Rng R = L.R;
-    const int nj = R.je - R.js + 1, n = R.ke - R.ks + 1;
-    const int2 tb = xcd_block_xy();   // (j block, plane)
-    const int i = R.is + tb.y;
-    const int nl = (i <= R.ie) ? min(LPB, nj - (int)(tb.x * LPB)) : 0;
-    if (nl <= 0) return;   // whole block
-    // tiles tS[LPB][w], tM[LPB][w] (w >= n + 1: rows and the mu row above
-    // the last), then the reduced rows
-    // constant-coefficient sets have no mu tile (the launch sizes the LDS
-    // for a mu tile when any of its sets has one)
+    const int n = R.ke - R.ks + 1, LW = 64 / G;
+    const int i = R.is + ii, j0 = R.js + jb * LW;
+    const int nl = min(LW, R.je - j0 + 1);
+    if (i > R.ie || nl <= 0) return;
+    const int P = (n + PM - 1) / PM;
+    const long base = IX(d, i, j0, R.ks);
     const bool cst = L.mu == nullptr;
-    T* tS = reinterpret_cast<T*>(pllc_smem);
-    T* tM = tS + LPB * w;
-    T* red = cst ? tM : tM + LPB * w;
-    const long base = IX(d, i, R.js + tb.x * LPB, R.ks);
-    const T* __restrict__ mu = cst ? nullptr : L.mu + L.mu_off;
-    const T del = L.del, h = L.h;
-    const double rh = L.rh;
-    const T fac = T(0.5) * T(scal[S_DT]) * (g + r);
-
-    // the mu row above the last (x = n) of each line, issued first; then
-    // rows x < n, the loads of 8 lines before their LDS stores
-    T mtop = T(0.0);
-    if (!cst && tid < nl) mtop = mu[base + (long)tid * d.sy + n];
-    for (int x = tid; x < n; x += NT) {
-        for (int l0 = 0; l0 < nl; l0 += 8) {
-            T vs[8], vm[8];
+    // element m of the lane: e = lane + 64 m of the tile's LW x 16 G slots,
+    // row e % (16 G) of line e / (16 G): a lane's part and a part of m alone
+    const int W = PM * G, lw = __builtin_ctz(W);
+    const int xl = lane & (W - 1), ll = lane >> lw;
+    const int ml = ll * G * ZW + xl + (xl >> 4);
+    auto xs = [&](int m) { return (64 * m) & (W - 1); };
+    auto rs = [&](int m) { return (64 * m) >> lw; };
+    auto slot = [&](int m) { return ml + rs(m) * G * ZW + xs(m) + (xs(m) >> 4); };
+    const bool exact = n == W && nl == LW;   // every slot is an element
+    // past the line's end (xe: its last element to be read) or the last
+    // line: its last element again
+    auto load = [&](const T* __restrict__ p, int xe, T (&v)[PM]) {
+        if (exact) {
+            const T* __restrict__ pl = p + (long)ll * d.sy + xl;
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int lq = l0 + u;
-                const long gb = base + (long)lq * d.sy + x;
-                if (lq < nl) vs[u] = L.S[gb];
-                if (lq < nl && !cst) vm[u] = mu[gb];
-            }
+            for (int m = 0; m < PM; m++) v[m] = pl[(long)rs(m) * d.sy + xs(m)];
+        } else {
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int lq = l0 + u;
-                if (lq < nl) tS[lq * w + x] = vs[u];
-                if (lq < nl && !cst) tM[lq * w + x] = vm[u];
-            }
+            for (int m = 0; m < PM; m++)
+                v[m] = p[min(ll + rs(m), nl - 1) * (unsigned)d.sy + min(xl + xs(m), xe)];
         }
+    };
+    T vs[PM], vm[PM], mt = T(1.0);
+    load(L.S + base, n - 1, vs);
+    const int q = lane / G, c = lane - q * G;   // the lane's line and chunk
+    if (!cst) {
+        const T* __restrict__ mu = L.mu + L.mu_off + base;
+        load(mu, n, vm);
+        // the value above the last row has no slot in a line of 16 G rows
+        mt = mu[(long)min(q, nl - 1) * d.sy + n];
     }
-    if (!cst && tid < nl) tM[tid * w + n] = mtop;
-    __syncthreads();
-
-    const bool live = q < nl;
-    const int x0 = (s * n) / P;
-    const int m = ((s + 1) * n) / P - x0;
+    T* mine = ls + lane * ZW;
+#pragma unroll
+    for (int m = 0; m < PM; m++) ls[slot(m)] = vs[m];
+    line_sync();
+    PRows<T> w;
+#pragma unroll
+    for (int t = 0; t < PM; t++) w.sv[t] = mine[t];
+    const T fac = T(0.5) * T(scal[S_DT]) * (g + r);
+    w.tl = n - c * PM - 1;
+    w.first = c == 0;
+    w.e0 = bc_factor<T>(L.bc0);
+    w.e1 = bc_factor<T>(L.bc1);
+    if (cst) {
+#pragma unroll
+        for (int t = 0; t <= PM; t++) w.mv[t] = T(1.0);
+    } else {
+        line_sync();
+#pragma unroll
+        for (int m = 0; m < PM; m++) ls[slot(m)] = vm[m];
+        line_sync();
+#pragma unroll
+        for (int t = 0; t < PM; t++) w.mv[t] = mine[t];
+        w.mv[PM] = mine[c == G - 1 ? PM - 1 : ZW];
+        if (c == G - 1) w.mv[PM] = mt;
+    }
+    w.kf = cst ? fac * L.ca : fac * L.del * T(L.rh);
     PChunk<T> ch;
-    if (live) {
-        const T* rs = tS + q * w + x0;
-        const T* rm = tM + q * w + x0;
-        T araw = cst ? L.ca : divh<T>(del * rm[0], h, rh);
-#pragma unroll
-        for (int t = 0; t < PM; t++) {
-            if (t < m) {
-                const T craw = cst ? L.cc : divh<T>(del * rm[t + 1], h, rh);
-                T a, b, c, rhs = rs[t];
-                prow<T, 2>(L, x0 + t, n, fac, araw, craw, T(0.0), a, b, c, rhs);
-                ch.fwd(t, a, b, c, rhs);
-                araw = craw;
-            }
-        }
-        ch.fold(m);
-        T la, lc, lD;
-        ch.last(m, la, lc, lD);
-        const int e0 = 2 * s;
-        red[e0 * LPB + q] = ch.A[0];
-        red[(E + e0) * LPB + q] = ch.C[0];
-        red[(2 * E + e0) * LPB + q] = ch.D[0];
-        red[(e0 + 1) * LPB + q] = la;
-        red[(E + e0 + 1) * LPB + q] = lc;
-        red[(2 * E + e0 + 1) * LPB + q] = lD;
+    chunk_rows<T>(ch, w);
+    PcrRow<T> p;
+    const bool nx = c + 1 < P;
+    const T An = __shfl_down(ch.A[0], 1), Cn = __shfl_down(ch.C[0], 1), Dn = __shfl_down(ch.D[0], 1);
+    p.start(ch, nx ? An : T(0.0), nx ? Cn : T(0.0), nx ? Dn : T(0.0));
+    if (G <= 16) {
+        if (P > 1) lane_round<T, 1, true>(p, c, P);
+        if (P > 2) lane_round<T, 2, true>(p, c, P);
+        if (P > 4) lane_round<T, 4, true>(p, c, P);
+        if (P > 8) lane_round<T, 8, true>(p, c, P);
+    } else {
+        lane_round<T, 1, false>(p, c, P);
+        lane_round<T, 2, false>(p, c, P);
+        lane_round<T, 4, false>(p, c, P);
+        lane_round<T, 8, false>(p, c, P);
+        lane_round<T, 16, false>(p, c, P);
+        if (P > 32) lane_round<T, 32, false>(p, c, P);
     }
-    __syncthreads();
-    if (live && s == 0) pchunk_reduced<T>(red, E, LPB, q);
-    __syncthreads();
-    if (live) {
-        const T X0 = red[(2 * E + 2 * s) * LPB + q], X1 = red[(2 * E + 2 * s + 1) * LPB + q];
-        T* ws = tS + q * w + x0;
+    const T xp = __shfl_up(p.d, 1);
+    ch.solve(ch.D[0] - ch.C[0] * p.d - ch.A[0] * (c > 0 ? xp : T(0.0)), p.d);
+    line_sync();
 #pragma unroll
-        for (int t = 0; t < PM; t++)
-            if (t < m) ws[t] = t == 0 ? X0 : t == m - 1 ? X1 : ch.D[t] - ch.A[t] * X0 - ch.C[t] * X1;
-    }
-    __syncthreads();
-    for (int x = tid; x < n; x += NT) {
-        for (int l0 = 0; l0 < nl; l0 += 8) {
-            T vs[8];
+    for (int t = 0; t < PM; t++) mine[t] = ch.D[t];
+    line_sync();
+    T* So = L.S + renew(base) + (long)ll * d.sy + xl;
+    if (exact) {
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (l0 + u < nl) vs[u] = tS[(l0 + u) * w + x];
+        for (int m = 0; m < PM; m++) vs[m] = ls[slot(m)];
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (l0 + u < nl) L.S[base + (long)(l0 + u) * d.sy + x] = vs[u];
-        }
-    }
-}
-
-// z-lines (rows contiguous along k), persistent (the FP64 path).  A tile is
-// LPB lines of one i-plane
-// (LPB consecutive j) of one line set; tiles are numbered (j block, plane,
-// set) and a persistent block takes tiles t = blockIdx.x, + gridDim.x, ...
-// A tile is staged through LDS with consecutive threads on consecutive k,
-// solved by chunk from LDS and written back the same way.  The next tile's
-// rows are loaded into registers while the current one is solved, so the
-// load latency overlaps the elimination.  w is the LDS row pitch of a line
-// (at least n + 1); mu_tiles says whether the launch's sets have a mu tile.
-constexpr int ZMAX = 16;   // staged values per thread and array: n <= 16 P
-
-template <typename T>
-struct ZTile {
-    int set, nl;   // line set; lines in the tile (0: nothing to do)
-    long base;     // first row of the first line
-};
-
-template <typename T>
-__device__ __forceinline__ ZTile<T> z_tile(const Dims& d, const LineSets<T>& sets, int t, int ntiles, int nbx,
-                                           int ni, int LPB)
-{
-    ZTile<T> z{0, 0, 0};
-    if (t >= ntiles) return z;
-    const int per_set = nbx * ni;
-    z.set = t / per_set;
-    const int rem = t - z.set * per_set;
-    const int ii = rem / nbx, bx = rem - ii * nbx;
-    const Rng R = sets.s[z.set].R;
-    const int i = R.is + ii, nj = R.je - R.js + 1;
-    z.nl = (i <= R.ie) ? max(0, min(LPB, nj - bx * LPB)) : 0;
-    z.base = IX(d, i, R.js + bx * LPB, R.ks);
-    return z;
-}
-
-// the tile's nl x n rows of S (and of mu, with the mu row above the last
-// of each line in mtop) into registers: element e = tid + NT m is row
-// e % n of line e / n
-template <typename T>
-__device__ __forceinline__ void z_load(const Dims& d, const LineSets<T>& sets, const ZTile<T>& z, int tid, int NT,
-                                       T (&vs)[ZMAX], T (&vm)[ZMAX], T& mtop)
-{
-    if (z.nl == 0) return;
-    const LineSet<T>& L = sets.s[z.set];
-    const int n = L.R.ke - L.R.ks + 1;
-    const T* __restrict__ S = L.S + z.base;
-    const T* __restrict__ mu = L.mu ? L.mu + L.mu_off + z.base : nullptr;
-    const int tot = z.nl * n, dl = NT / n, dx = NT - dl * n;
-    int lq = tid / n, x = tid - lq * n;
+        for (int m = 0; m < PM; m++) So[(long)rs(m) * d.sy + xs(m)] = vs[m];
+    } else {
 #pragma unroll
-    for (int m = 0; m < ZMAX; m++) {
-        if (tid + m * NT < tot) {
-            const long g = (long)lq * d.sy + x;
-            vs[m] = S[g];
-            if (mu) vm[m] = mu[g];
-        }
-        x += dx; lq += dl;
-        if (x >= n) { x -= n; lq++; }
-    }
-    if (mu && tid < z.nl) mtop = mu[(long)tid * d.sy + n];
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_sweep_part_z(Dims d, LineSets<T> sets, const double* __restrict__ scal, T g,
-                                                      T r, int w, int mu_tiles, int nbx, int ni, int ntiles)
-{
-    extern __shared__ unsigned char pllc_smem[];
-    const int LPB = blockDim.x, P = blockDim.y, E = 2 * P, NT = LPB * P;
-    const int q = threadIdx.x, s = threadIdx.y, tid = s * LPB + q;
-    // tiles tS[LPB][w] (and tM[LPB][w]: rows and the mu row above the
-    // last), then the reduced rows
-    T* tS = reinterpret_cast<T*>(pllc_smem);
-    T* tM = tS + LPB * w;
-    T* red = tS + (mu_tiles ? 2 : 1) * LPB * w;
-    const T fac = T(0.5) * T(scal[S_DT]) * (g + r);
-
-    T vs[ZMAX], vm[ZMAX], mtop = T(0.0);
-    int t = blockIdx.x;
-    ZTile<T> cur = z_tile<T>(d, sets, t, ntiles, nbx, ni, LPB);
-    z_load<T>(d, sets, cur, tid, NT, vs, vm, mtop);
-    while (t < ntiles) {
-        const LineSet<T>& L = sets.s[cur.set];
-        const bool cst = L.mu == nullptr;
-        const int nl = cur.nl;
-        const int n = L.R.ke - L.R.ks + 1;   // line length of this set
-        const int x0 = (s * n) / P;
-        const int m = ((s + 1) * n) / P - x0;
-        if (nl > 0) {
-            const int tot = nl * n, dl = NT / n, dx = NT - dl * n;
-            int lq = tid / n, x = tid - lq * n;
-#pragma unroll
-            for (int mm = 0; mm < ZMAX; mm++) {
-                if (tid + mm * NT < tot) {
-                    tS[lq * w + x] = vs[mm];
-                    if (!cst) tM[lq * w + x] = vm[mm];
-                }
-                x += dx; lq += dl;
-                if (x >= n) { x -= n; lq++; }
-            }
-            if (!cst && tid < nl) tM[tid * w + n] = mtop;
-        }
-        __syncthreads();
-        // the next tile's rows, in flight during this tile's solve
-        const int tn = t + gridDim.x;
-        const ZTile<T> nxt = z_tile<T>(d, sets, tn, ntiles, nbx, ni, LPB);
-        z_load<T>(d, sets, nxt, tid, NT, vs, vm, mtop);
-        if (nl > 0) {
-            const T del = L.del, h = L.h;
-            const double rh = L.rh;
-            const bool live = q < nl;
-            PChunk<T> ch;
-            if (live) {
-                const T* rs = tS + q * w + x0;
-                const T* rm = tM + q * w + x0;
-                T araw = cst ? L.ca : divh<T>(del * rm[0], h, rh);
-#pragma unroll
-                for (int tt = 0; tt < PM; tt++) {
-                    if (tt < m) {
-                        const T craw = cst ? L.cc : divh<T>(del * rm[tt + 1], h, rh);
-                        T a, b, c, rhs = rs[tt];
-                        prow<T, 2>(L, x0 + tt, n, fac, araw, craw, T(0.0), a, b, c, rhs);
-                        ch.fwd(tt, a, b, c, rhs);
-                        araw = craw;
-                    }
-                }
-                ch.fold(m);
-                T la, lc, lD;
-                ch.last(m, la, lc, lD);
-                const int e0 = 2 * s;
-                red[e0 * LPB + q] = ch.A[0];
-                red[(E + e0) * LPB + q] = ch.C[0];
-                red[(2 * E + e0) * LPB + q] = ch.D[0];
-                red[(e0 + 1) * LPB + q] = la;
-                red[(E + e0 + 1) * LPB + q] = lc;
-                red[(2 * E + e0 + 1) * LPB + q] = lD;
-            }
-            __syncthreads();
-            if (live && s == 0) pchunk_reduced<T>(red, E, LPB, q);
-            __syncthreads();
-            if (live) {
-                const T X0 = red[(2 * E + 2 * s) * LPB + q], X1 = red[(2 * E + 2 * s + 1) * LPB + q];
-                T* ws = tS + q * w + x0;
-#pragma unroll
-                for (int tt = 0; tt < PM; tt++)
-                    if (tt < m) ws[tt] = tt == 0 ? X0 : tt == m - 1 ? X1 : ch.D[tt] - ch.A[tt] * X0 - ch.C[tt] * X1;
-            }
-            __syncthreads();
-            T* __restrict__ S = L.S + cur.base;
-            const int tot = nl * n, dl = NT / n, dx = NT - dl * n;
-            int lq = tid / n, x = tid - lq * n;
-#pragma unroll
-            for (int mm = 0; mm < ZMAX; mm++) {
-                if (tid + mm * NT < tot) S[(long)lq * d.sy + x] = tS[lq * w + x];
-                x += dx; lq += dl;
-                if (x >= n) { x -= n; lq++; }
-            }
-        }
-        __syncthreads();   // tS is refilled by the next tile
-        cur = nxt;
-        t = tn;
+        for (int m = 0; m < PM; m++)
+            if (xl + xs(m) < n && ll + rs(m) < nl) So[(long)rs(m) * d.sy + xs(m)] = ls[slot(m)];
     }
 }
 
 // Poisson x-lines (phisolver_dct's pll_tridiag, 2055-2100) by the same
 // partition method: line l = (y mode, z mode) of the packed block, rows x
 // nm = ny nz apart, a = c = 1/dx^2, b = -2/dx^2 + lam_y + lam_z, Neumann
-// rows at the inlet and (all modes but the mean) at the outlet; the (0,0)
-// mode keeps its outlet ghost phi = 0.  The (0,0) line is eliminated in FP64
-// whatever the field type (its own LDS rows), as the gauge line of the
-// otherwise singular problem.
-template <typename U, typename T>
-__device__ __forceinline__ void pois_chunk(const T* __restrict__ p, long nm, int x0, int m, int n, U dx2i, U bmid,
-                                           bool mean_mode, PChunk<U>& ch)
+// rows at the inlet and (all modes but the mean) at the outlet.
+//
+// The mean mode (0,0), the gauge line of the otherwise singular problem, has
+// lam = 0, Neumann at the inlet and the ghost phi = 0 at the outlet: its
+// differences phi_{i+1} - phi_i are dx^2 times the sum of the sources up to
+// i, and phi_i minus the sum of those from i on.  A block of its own forms
+// the two sums in FP64 whatever the field type, each thread over consecutive
+// rows with a scan over the threads between, so that the FP32 kernel holds
+// no FP64 chunk (which cost it 166 registers).  Measured (FP64, mixed):
+// 256x128x128 28 -> 15 us and 25 -> 11.5; 512x256x256, whose 32 chunks per
+// line left 8 lines (64 or 32 bytes of a row) per block of 256 threads, 173
+// -> 86 and 179 -> 57; 64x32x32 14 -> 4.8.
+template <typename T>
+__device__ __forceinline__ void pois_mean(const Dims& d, T* __restrict__ p, long nm, double* __restrict__ sh, int t,
+                                          int NT)
 {
-    U v[PM];
-#pragma unroll
-    for (int t = 0; t < PM; t++)
-        if (t < m) v[t] = U(p[(long)(x0 + t) * nm]);
-#pragma unroll
-    for (int t = 0; t < PM; t++) {
-        if (t < m) {
-            const int x = x0 + t;
-            U a = dx2i, b = bmid, c = dx2i;
-            if (x == 0) { b += a; a = U(0.0); }
-            if (x == n - 1) {
-                if (!mean_mode) b += c;
-                c = U(0.0);
-            }
-            ch.fwd(t, a, b, c, v[t]);
+    const int n = d.nx;
+    const int x0 = (int)((long)t * n / NT), x1 = (int)((long)(t + 1) * n / NT);
+    const double h2 = d.dx * d.dx;
+    // inclusive scan of v over the block's threads (up: t ascending)
+    auto scan = [&](double v, bool up) {
+        double* cur = sh;
+        double* nxt = sh + NT;
+        cur[t] = v;
+        __syncthreads();
+        for (int w = 1; w < NT; w <<= 1) {
+            if (up) { if (t >= w) v += cur[t - w]; }
+            else { if (t + w < NT) v += cur[t + w]; }
+            nxt[t] = v;
+            __syncthreads();
+            double* q = cur;
+            cur = nxt;
+            nxt = q;
         }
+        __syncthreads();
+        return v;
+    };
+    double f = 0.0;
+    for (int x = x0; x < x1; x++) f += double(p[(long)x * nm]);
+    const double before = scan(f, true) - f;   // the sources of the rows before x0
+    double acc = before, g = 0.0;
+    for (int x = x0; x < x1; x++) {
+        acc += double(p[(long)x * nm]);
+        g += h2 * acc;
     }
-    ch.fold(m);
-}
-
-template <typename U>
-__device__ __forceinline__ void pchunk_put(U* __restrict__ red, int E, int LPB, int q, int s, const PChunk<U>& ch, int m)
-{
-    U la, lc, ld;
-    ch.last(m, la, lc, ld);
-    const int e0 = 2 * s;
-    red[e0 * LPB + q] = ch.A[0];
-    red[(E + e0) * LPB + q] = ch.C[0];
-    red[(2 * E + e0) * LPB + q] = ch.D[0];
-    red[(e0 + 1) * LPB + q] = la;
-    red[(E + e0 + 1) * LPB + q] = lc;
-    red[(2 * E + e0 + 1) * LPB + q] = ld;
+    double phi = -(scan(g, false) - g);   // phi of row x1
+    // the segment again from its last row: acc is the sum up to row x
+    for (int x = x1 - 1; x >= x0; x--) {
+        const double s = double(p[(long)x * nm]);
+        phi -= h2 * acc;
+        acc -= s;
+        p[(long)x * nm] = T(phi);
+    }
 }
 
 template <typename T>
-__device__ __forceinline__ PChunk<double>& pick_chunk(PChunk<T>& a, PChunk<double>& b)
-{
-    if constexpr (std::is_same<T, double>::value) return a;
-    else return b;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_pois_part(Dims d, const T* __restrict__ lam_y, const T* __restrict__ lam_z,
-                                                   T* __restrict__ P, const double* __restrict__ lam00, Bt bt)
+__global__ __launch_bounds__(POIS_THREADS, 4) void k_pois_part(Dims d, const T* __restrict__ lam_y, const T* __restrict__ lam_z,
+                                                      T* __restrict__ P, Bt bt)
 {
     extern __shared__ __align__(8) unsigned char pllc_smem[];
     // member: blockIdx.y
     P += blockIdx.y * bt.pk;
-    const int LPB = blockDim.x, PC = blockDim.y, E = 2 * PC;
-    double* red0 = reinterpret_cast<double*>(pllc_smem);          // [3][E] of the (0,0) line
-    T* red = reinterpret_cast<T*>(pllc_smem + sizeof(double) * 3 * E);   // [3][E][LPB]
+    const int LPB = blockDim.x, PC = blockDim.y;
     const int q = threadIdx.x, s = threadIdx.y;
     const long nm = (long)d.ny * d.nz;
+    if (blockIdx.x == gridDim.x - 1) {
+        pois_mean<T>(d, P, nm, reinterpret_cast<double*>(pllc_smem), s * LPB + q, LPB * PC);
+        return;
+    }
     const int n = d.nx;
     const int l = blockIdx.x * LPB + q;
-    const bool live = l < nm;
-    const bool mean = l == 0;
-    const int x0 = (s * n) / PC;
-    const int m = ((s + 1) * n) / PC - x0;
-    T* __restrict__ p = P + (live ? l : 0);
-    // the (0,0) line's FP64 chunk: in FP64 the same object as every other
-    // line's (one set of registers for the two branches)
+    const bool live = l < nm && l > 0;
+    const int x0 = s * PM, nv = min(PM, n - x0);
+    T* p = P + (live ? l : 0) + (long)x0 * nm;
     PChunk<T> ch;
-    PChunk<double> chd;
-    PChunk<double>& ch0 = pick_chunk(ch, chd);
     if (live) {
-        if (mean) {
-            const double dx2i = 1.0 / (d.dx * d.dx);
-            pois_chunk<double, T>(p, nm, x0, m, n, dx2i, -2.0 * dx2i + lam00[0] + lam00[1], true, ch0);
-            pchunk_put<double>(red0, E, 1, 0, s, ch0, m);
+        const int jy = l / d.nz, kz = l - jy * d.nz;
+        const T h = T(1.0) / (T(d.dx) * T(d.dx));
+        const T bm = T(-2.0) * h + lam_y[jy] + lam_z[kz];
+        const int tl = x0 + PM >= n ? nv - 1 : PM;
+        T sv[PM];
+        if (nv == PM) {
+#pragma unroll
+            for (int t = 0; t < PM; t++) sv[t] = p[(long)t * nm];
         } else {
-            const int jy = l / d.nz, kz = l % d.nz;
-            const T dx2i = T(1.0) / (T(d.dx) * T(d.dx));
-            pois_chunk<T, T>(p, nm, x0, m, n, dx2i, T(-2.0) * dx2i + lam_y[jy] + lam_z[kz], false, ch);
-            pchunk_put<T>(red, E, LPB, q, s, ch, m);
+            // past the line's end: its last row again, which no row reads
+            const unsigned mi = (unsigned)nm, lim = (nv - 1) * mi;
+#pragma unroll
+            for (int t = 0; t < PM; t++) sv[t] = p[min(t * mi, lim)];
         }
+        // row t: h x_{t-1} + bm x_t + h x_{t+1} = sv[t], Neumann ends
+#pragma unroll
+        for (int t = 0; t < PM; t++) {
+            const T b = t == 0 && s == 0 ? bm + h : bm;
+            ch.fwd(t, t == 0 && s == 0 ? T(0.0) : h, t == tl ? b + h : b, t == tl ? T(0.0) : h, sv[t]);
+            row_done();
+        }
+        ch.fold();
     }
-    __syncthreads();
-    if (live && s == 0) {
-        if (mean) pchunk_reduced<double>(red0, E, 1, 0);
-        else pchunk_reduced<T>(red, E, LPB, q);
-    }
-    __syncthreads();
+    chunk_couple<T>(reinterpret_cast<T*>(pllc_smem), PC, LPB, q, s, live, ch);
     if (!live) return;
-    if (mean) {
-        const double X0 = red0[2 * E + 2 * s], X1 = red0[2 * E + 2 * s + 1];
+    p = P + renew((long)l + (long)x0 * nm);
+    if (nv == PM) {
 #pragma unroll
-        for (int t = 0; t < PM; t++)
-            if (t < m)
-                p[(long)(x0 + t) * nm] = T(t == 0 ? X0 : t == m - 1 ? X1 : ch0.D[t] - ch0.A[t] * X0 - ch0.C[t] * X1);
+        for (int t = 0; t < PM; t++) p[(long)t * nm] = ch.D[t];
     } else {
-        const T X0 = red[(2 * E + 2 * s) * LPB + q], X1 = red[(2 * E + 2 * s + 1) * LPB + q];
 #pragma unroll
         for (int t = 0; t < PM; t++)
-            if (t < m) p[(long)(x0 + t) * nm] = t == 0 ? X0 : t == m - 1 ? X1 : ch.D[t] - ch.A[t] * X0 - ch.C[t] * X1;
+            if (t < nv) p[(long)t * nm] = ch.D[t];
     }
 }
 
@@ -3327,14 +3343,12 @@ static LineSet<T> line_set(Ctx<T>& c, int F, int DIR, T* S, T* CC, const Visc4<T
     return L;
 }
 
-// chunks per line of the partitioned solve for lines of nmin..nmax rows
-// (every chunk between 3 and PM rows), or 0 when the lines do not allow it
+// chunks per line of the partitioned solve for lines of nmin..nmax rows, or
+// 0 when the lines do not allow it
 static inline int part_chunks(int nmin, int nmax)
 {
-    if (nmin < 3) return 0;
     const int P = (nmax + PM - 1) / PM;
-    if (P > 64 || nmin / P < 3) return 0;
-    return P;
+    return nmin < 3 || P > 64 ? 0 : P;
 }
 
 template <typename T>
@@ -3373,9 +3387,13 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
         long lines = 0;
         for (int q = 0; q < nset; q++) {
             ls.s[q] = line_set<T>(c, F[q], DIR, S[q], CC[q], mu, qold[q], qnew[q], N[q], Nm1[q]);
-            if (vghost && DIR == 0 && F[q] != FC) ls.s[q].ghost_v = F[q];
-            const Rng& R = ls.s[q].R;
-            const long nl = DIR == 0 ? (long)(R.je - R.js + 1) * (R.ke - R.ks + 1)
+            LineSet<T>& L = ls.s[q];
+            if (vghost && DIR == 0 && F[q] != FC) L.ghost_v = F[q];
+            L.jg = L.ghost_c || L.ghost_v == FU || L.ghost_v == FW;
+            L.kg = L.ghost_c || L.ghost_v == FU || L.ghost_v == FV;
+            L.inlet = L.ghost_v == FV || L.ghost_v == FW;
+            const Rng& R = L.R;
+            const long nl = DIR == 0 ? (long)(R.je - R.js + 1 + 2 * L.jg) * (R.ke - R.ks + 1 + 2 * L.kg)
                           : DIR == 1 ? (long)(R.ie - R.is + 1) * (R.ke - R.ks + 1)
                                      : (long)(R.ie - R.is + 1) * (R.je - R.js + 1);
             lines = nl > lines ? nl : lines;
@@ -3389,10 +3407,14 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
         }
         const int P = c.line_solver == 0 ? part_chunks(nmin, nmax) : 0;
         if (P > 0 && DIR != 2) {
-            // wide rows per wavefront: rows start 8-byte aligned only, so
-            // longer contiguous runs fetch fewer partial cache lines
-            int LPB = std::min(sizeof(T) == 8 ? 32 : 64, std::max(1, 512 / P));
-            if (c.lpb[DIR] > 0) LPB = std::min(c.lpb[DIR], std::max(1, 512 / P));   // tuned
+            // lines per block: y-lines 256 bytes of a row (rows start 8-byte
+            // aligned only, so longer runs fetch fewer partial cache lines);
+            // x-lines, which couple more chunks, 16 lines (256x128x128, y at 16:
+            // 65 us instead of 57 FP64, 41 instead of 27 FP32; x at 32: 86
+            // instead of 83 FP64, 15.3 instead of 12.0 for c in FP32)
+            const int most = std::max(1, PART_THREADS / P);
+            int LPB = std::min(DIR == 0 ? 16 : 256 / (int)sizeof(T), most);
+            if (c.lpb[DIR] > 0) LPB = std::min(c.lpb[DIR], most);   // tuned
             // block count rounded up to a multiple of 8 (XCD order); the
             // blocks past the last line do nothing
             const dim3 blk(LPB, P, 1), grd((unsigned)(((lines + LPB - 1) / LPB + 7) / 8 * 8), nset, c.bt.nm);
@@ -3410,35 +3432,17 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
             ni = std::max(ni, R.ie - R.is + 1);
         }
         if (P > 0) {
-            // z-lines: LPB lines of an i-plane per block, tiles of pitch w
-            // (S, and mu when a set has variable coefficients)
-            const int w = (nmax + 1) | 1;
-            bool any_mu = false;
-            for (int q = 0; q < nset; q++) any_mu = any_mu || ls.s[q].mu != nullptr;
-            const size_t nt = any_mu ? 2 : 1;
-            int LPB = 32;
-            while (LPB > 1 && (nt * LPB * w + (size_t)6 * P * LPB) * sizeof(T) > 40960) LPB /= 2;
-            if (c.lpb[2] > 0) LPB = c.lpb[2];   // tuned
-            while (LPB > 1 && (nt * LPB * w + (size_t)6 * P * LPB) * sizeof(T) > 65536) LPB /= 2;
-            while (LPB > 1 && LPB * P > 256) LPB /= 2;
-            const size_t sm = (nt * LPB * w + (size_t)6 * P * LPB) * sizeof(T);
-            // FP64: persistent blocks, as many as fit on the device at once,
-            // each loading its next tile while it solves the current one.
-            // FP32 (half the bytes per tile, fewer registers without the
-            // prefetch, more blocks per CU): one block per tile measured
-            // faster.
-            const dim3 blk(LPB, P, 1);
-            const int nbx = (nj + LPB - 1) / LPB, ntiles = nbx * ni * nset;
-            const int mt = any_mu ? 1 : 0;
-            if (sizeof(T) == 8) {
-                if (!single(c, "sweep_z")) return;
-                const int G = std::max(1, std::min(ntiles, resident_blocks(k_sweep_part_z<T>, LPB * P, sm)));
-                PLLC_L(c, nm[2], (k_sweep_part_z<T><<<G, blk, sm, c.st>>>(c.d, ls, c.scal, g, r, w, mt, nbx, ni,
-                                                                          ntiles)));
-            } else {
-                const dim3 gz(nbx, ni, nset * c.bt.nm);
-                PLLC_L(c, nm[2], (k_sweep_part_zt<T><<<gz, blk, sm, c.st>>>(c.d, ls, c.scal, g, r, w, c.bt)));
-            }
+            // z-lines: a wave takes 64 / G lines of an i-plane, G lanes each
+            int G = 1;
+            while (G < P) G *= 2;
+            const int LW = 64 / G, nbx = (nj + LW - 1) / LW, ntiles = nbx * ni * nset;
+            int nw = Z_WAVES;
+            if (c.lpb[2] > 0) nw = std::max(1, std::min(Z_WAVES, c.lpb[2] / LW));   // tuned
+            const size_t sm = (size_t)nw * Z_TILE * sizeof(T);
+            // a multiple of 8 blocks (XCD order); the tiles past the last do nothing
+            const dim3 gz((unsigned)((ntiles + nw * 8 - 1) / (nw * 8) * 8), c.bt.nm, 1);
+            PLLC_L(c, nm[2], (k_sweep_wave_z<T><<<gz, 64 * nw, sm, c.st>>>(c.d, ls, c.scal, g, r, G, nbx, ni, ntiles,
+                                                                          c.bt)));
             continue;
         }
         if (!single(c, "sweep")) return;
@@ -3765,11 +3769,14 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts)
     dct2(c, c.P, sp, false);
     const int PC = c.line_solver == 0 ? part_chunks(c.d.nx, c.d.nx) : 0;
     if (PC > 0) {
-        const int LPB = std::min(64, std::max(1, 256 / PC));
-        const size_t sm = sizeof(double) * 3 * 2 * PC + sizeof(T) * 6 * PC * LPB;
-        const dim3 gp((unsigned)((nm + LPB - 1) / LPB), c.bt.nm, 1);
-        PLLC_L(c, "pois_x", (k_pois_part<T><<<gp, dim3(LPB, PC, 1), sm, c.st>>>(c.d, c.lam_y, c.lam_z, sp, c.lam00,
-                                                                               c.bt)));
+        // 128 bytes of a row per block, more where that is less than 256
+        // threads (512x256x256: 64 bytes 134 us FP64, 128 bytes 86; mixed 32
+        // bytes 138 us, 64 bytes 68, 128 bytes 57)
+        const int LPB = std::min(std::min(64, POIS_THREADS / PC), std::max((int)(128 / sizeof(T)), 256 / PC));
+        const size_t sm = sizeof(T) * 6 * PC * LPB;
+        // the last block is the mean line's
+        const dim3 gp((unsigned)((nm + LPB - 1) / LPB) + 1, c.bt.nm, 1);
+        PLLC_L(c, "pois_x", (k_pois_part<T><<<gp, dim3(LPB, PC, 1), sm, c.st>>>(c.d, c.lam_y, c.lam_z, sp, c.bt)));
     } else {
         if (!single(c, "poisson")) return;
         PLLC_L(c, "pois_x", (k_pois_x<T><<<line_grid(nm), 256, 0, c.st>>>(c.d, c.lam_y, c.lam_z, sp, c.QC, c.lam00)));
