@@ -43,15 +43,6 @@ __device__ __forceinline__ float divh<float>(float a, float, double rh)
     return a * float(rh);
 }
 
-// a / h in the explicit stencils.  Reference arithmetic (FAST false): divh,
-// the IEEE quotient.  FAST: a * (1/h), within an ulp, one operation.
-template <typename T, bool FAST>
-__device__ __forceinline__ T sdh(T a, T h, double rh)
-{
-    if (FAST) return a * T(rh);
-    return divh<T>(a, h, rh);
-}
-
 // 1/b and a/b on data: the IEEE quotient in FP64; in FP32 the hardware
 // reciprocal (v_rcp_f32, 1 ulp) and one multiply.  The FP32 callers' divisors
 // are normal numbers (line pivots near 1, WENO denominators >= 1e-36).
@@ -118,6 +109,7 @@ struct Phys {
     double edel[3][2];
     double fre[2];
     double rRe;   // 1/Re (divh)
+    double kap[4][3];   // cdel[F][D] / h (c: cdel), the A coefficients' factor of mu
 };
 
 // fills Phys::cdel/edel/fre from Re, Pe, Fx, Fy and the spacings
@@ -126,7 +118,11 @@ __host__ inline void pllc_phys_consts(Phys& ph, const Dims& d)
     const double h[3] = {d.dx, d.dy, d.dz};
     for (int D = 0; D < 3; D++) {
         ph.cdel[0][D] = 1.0 / (ph.Pe * h[D] * h[D]);
-        for (int F = 1; F <= 3; F++) ph.cdel[F][D] = (F - 1 == D ? 2.0 : 1.0) / (ph.Re * h[D]);
+        ph.kap[0][D] = ph.cdel[0][D];
+        for (int F = 1; F <= 3; F++) {
+            ph.cdel[F][D] = (F - 1 == D ? 2.0 : 1.0) / (ph.Re * h[D]);
+            ph.kap[F][D] = ph.cdel[F][D] / h[D];
+        }
     }
     ph.edel[0][0] = 1.0 / (ph.Re * d.dy * d.dx);
     ph.edel[0][1] = 1.0 / (ph.Re * d.dz * d.dx);
@@ -184,40 +180,11 @@ template <> struct Tr<float> { static constexpr float tiny = 1.0e-18f; };
 
 // ---------------------------------------------------------------- WENO
 
-// calculate_weno (pllcart3d.c:3455-3507) on five divided differences.
-// Reference arithmetic (FAST false): its operations in its order, the six
-// divisions as IEEE quotients.  FAST: the same expressions with fused
-// multiply-adds, and the weights from prcp reciprocals and one
-// normalisation, w1 c1 + w2 c2 + w3 c3 = (a1 c1 + a2 c2 + a3 c3) / (a1 + a2
-// + a3): the same value to a few ulps in 4 reciprocals instead of 6
-// divisions.  The denominators lie in [1e-198, 1e30] (epi >= 1e-99), normal
-// numbers.
-template <typename T, bool FAST = false>
+// calculate_weno (pllcart3d.c:3455-3507) on five divided differences, in the
+// reference's operations and order, the six divisions as IEEE quotients
+template <typename T>
 __device__ __forceinline__ T weno5(T v0, T v1, T v2, T v3, T v4)
 {
-    if (FAST) {
-        // the same expressions with fused multiply-adds and fmax
-        const T con1 = T(1.0) / T(6.0), con2 = T(13.0) / T(12.0), con3 = T(1.0) / T(4.0);
-        const T maxd = fmax(fmax(fmax(v0 * v0, v1 * v1), fmax(v2 * v2, v3 * v3)), v4 * v4);
-        const T c1 = con1 * fma(T(11.0), v2, fma(T(2.0), v0, T(-7.0) * v1));
-        const T c2 = con1 * fma(T(2.0), v3, fma(T(5.0), v2, -v1));
-        const T c3 = con1 * fma(T(5.0), v3, fma(T(2.0), v2, -v4));
-        T t1 = fma(T(-2.0), v1, v0) + v2;
-        T t2 = fma(T(3.0), v2, fma(T(-4.0), v1, v0));
-        const T s1 = fma(con2 * t1, t1, con3 * t2 * t2);
-        t1 = fma(T(-2.0), v2, v1) + v3;
-        t2 = v1 - v3;
-        const T s2 = fma(con2 * t1, t1, con3 * t2 * t2);
-        t1 = fma(T(-2.0), v3, v2) + v4;
-        t2 = fma(T(3.0), v2, fma(T(-4.0), v3, v4));
-        const T s3 = fma(con2 * t1, t1, con3 * t2 * t2);
-        const T epi = fma(T(1.0e-6), maxd, Tr<T>::tiny);
-        const T q1 = s1 + epi, q2 = s2 + epi, q3 = s3 + epi;
-        const T a1 = T(0.1) * prcp<T>(q1 * q1);
-        const T a2 = T(0.6) * prcp<T>(q2 * q2);
-        const T a3 = T(0.3) * prcp<T>(q3 * q3);
-        return fma(a1, c1, fma(a2, c2, a3 * c3)) * prcp<T>(a1 + a2 + a3);
-    }
     const T con1 = T(1.0) / T(6.0), con2 = T(13.0) / T(12.0), con3 = T(1.0) / T(4.0);
     T maxd = T(0.0), sq;
     sq = v0 * v0; maxd = (maxd > sq) ? maxd : sq;
@@ -282,23 +249,10 @@ __device__ __forceinline__ T upwind(const T* __restrict__ p, long st, int m, int
                  dd1(p, st, kk + 3 * sign, h, rh), dd1(p, st, kk + 4 * sign, h, rh));
 }
 
-// The six first differences of a line around point m: D[q] = D1 at face
-// m-3+q, q = 0..5, from the seven values pc[-3 st .. 3 st] (pc points at m).
-// Every stencil below reads them at fixed offsets, so each address is a
-// uniform offset from one per-field pointer.
-template <typename T, bool FAST = false>
-__device__ __forceinline__ void line_d1(const T* __restrict__ pc, long st, T h, double rh, T (&D)[6])
-{
-    T v[7];
-#pragma unroll
-    for (int q = 0; q < 7; q++) v[q] = pc[(long)(q - 3) * st];
-#pragma unroll
-    for (int q = 0; q < 6; q++) D[q] = sdh<T, FAST>(v[q + 1] - v[q], h, rh);
-}
-
-// upwind() on the differences of line_d1: the same ENO2 / HJ-WENO5 choice
-// and operands (1566-1574), with the faces picked by the upwind side
-template <typename T, bool FAST = false>
+// upwind() on the six first differences D[q] of a line around point m (D1 at
+// face m-3+q): the same ENO2 / HJ-WENO5 choice and operands (1566-1574), with
+// the faces picked by the upwind side
+template <typename T>
 __device__ __forceinline__ T upwind_d(const T (&D)[6], int m, int ms, int me, int sign, T h, double rh, T lo,
                                       T hi)
 {
@@ -308,13 +262,86 @@ __device__ __forceinline__ T upwind_d(const T (&D)[6], int m, int ms, int me, in
         const T d1k = up ? D[2] : D[3];
         const T d1m = up ? D[1] : D[2];
         const T d1p = up ? D[3] : D[4];
-        const T a = (kk < ms) ? lo : (kk > me) ? hi : sdh<T, FAST>(d1k - d1m, T(2.0) * h, 0.5 * rh);
-        const T b = (kk + 1 < ms) ? lo : (kk + 1 > me) ? hi : sdh<T, FAST>(d1p - d1k, T(2.0) * h, 0.5 * rh);
+        const T a = (kk < ms) ? lo : (kk > me) ? hi : divh<T>(d1k - d1m, T(2.0) * h, 0.5 * rh);
+        const T b = (kk + 1 < ms) ? lo : (kk + 1 > me) ? hi : divh<T>(d1p - d1k, T(2.0) * h, 0.5 * rh);
         const T d2 = (fabs(a) <= fabs(b)) ? a : b;
         return d1k + d2 * h * T(sign);
     }
-    return weno5<T, FAST>(up ? D[0] : D[5], up ? D[1] : D[4], up ? D[2] : D[3], up ? D[3] : D[2],
-                          up ? D[4] : D[1]);
+    return weno5<T>(up ? D[0] : D[5], up ? D[1] : D[4], up ? D[2] : D[3], up ? D[3] : D[2], up ? D[4] : D[1]);
+}
+
+// 2^-k for x in [2^k, 2^(k+1)), x > 0 normal
+__device__ __forceinline__ double inv_pow2(double x)
+{
+    return __hiloint2double(0x7fe00000 - (__double2hiint(x) & 0x7ff00000), 0);
+}
+__device__ __forceinline__ float inv_pow2(float x)
+{
+    return __int_as_float(0x7f000000 - (__float_as_int(x) & 0x7f800000));
+}
+
+// vel times the upwind derivative at point m of a line, the explicit
+// kernels' form: the expressions of upwind_d to rounding, on undivided
+// differences with one multiply by 1/h at the end, in 75 operations instead
+// of 110 (those kernels are bound by instruction issue in FP32 and near it in
+// FP64).  v: the values m-3 .. m+3; d2 and d3 receive v[3] - v[2] and
+// v[4] - v[3].
+//
+// With first differences D[q] and second differences E[q] the five upwind
+// differences of calculate_weno are D[2] (or D[3]) and steps f1 .. f4 from
+// it (up: E[0..3]; down: -E[4..1], whose sign s factors out), and
+//   w1 c1 + w2 c2 + w3 c3 = v2 + s/6 (a1 (5 f2 - 2 f1) + a2 (f2 + 2 f3)
+//                                     + a3 (4 f3 - f4)) / (a1 + a2 + a3).
+// The smoothness terms are taken 4 times (13/3 t1^2 + t2^2, epi likewise: a
+// common factor of the weights), and the weights 1/q^2 with the denominators
+// multiplied out, so one reciprocal serves instead of four: q >= 4 epi >= 4e-6
+// max|D|^2 and q <= 133 max|D|^2 + 4 epi, so that scaled by the power of two
+// of 4 epi each lies in [1, 7e7] and the products of the squares of two of
+// them below 3e31, inside both types' range.
+template <typename T>
+__device__ __forceinline__ T upwind_term(const T (&v)[7], int m, int ms, int me, T vel, T h, T rh, T lo, T hi, T& d2,
+                                         T& d3)
+{
+    T D[6], E[5];
+#pragma unroll
+    for (int q = 0; q < 6; q++) D[q] = v[q + 1] - v[q];
+#pragma unroll
+    for (int q = 0; q < 5; q++) E[q] = D[q + 1] - D[q];
+    d2 = D[2];
+    d3 = D[3];
+    const bool up = vel >= T(0.0);
+    const T c = up ? D[2] : D[3];
+    const T f2 = up ? E[1] : E[3], f3 = E[2];
+    T r;   // 6 s times the term added to c
+    if ((m <= ms + 1) || (m >= me - 1)) {
+        // ENO2: half the smaller of the second differences on either side,
+        // those outside the range read from the stale scratch (lo, hi)
+        T a = up ? f2 : f3, b = up ? f3 : f2;
+        if (m == ms && up) a = lo * (T(2.0) * h * h);
+        if (m == me && !up) b = hi * (T(2.0) * h * h);
+        r = T(3.0) * (fabs(a) <= fabs(b) ? a : b);
+    } else {
+        const T f1 = up ? E[0] : E[4], f4 = up ? E[3] : E[1], ve = up ? D[0] : D[5];
+        const T mx = fmax(fmax(fmax(fabs(D[1]), fabs(D[2])), fmax(fabs(D[3]), fabs(D[4]))), fabs(ve));
+        const T ep = fma(T(4.0e-6) * mx, mx, T(4.0) * Tr<T>::tiny * (h * h));
+        const T sc = inv_pow2(ep);
+        const T k = T(13.0) / T(3.0);
+        T t1 = f2 - f1, t2 = fma(T(3.0), f2, -f1);
+        const T q1 = fma(k * t1, t1, fma(t2, t2, ep)) * sc;
+        t1 = f3 - f2;
+        t2 = f2 + f3;
+        const T q2 = fma(k * t1, t1, fma(t2, t2, ep)) * sc;
+        t1 = f4 - f3;
+        t2 = fma(T(-3.0), f3, f4);
+        const T q3 = fma(k * t1, t1, fma(t2, t2, ep)) * sc;
+        T a1 = q2 * q3, a2 = q1 * q3, a3 = q1 * q2;
+        a1 = a1 * a1;
+        a2 = T(6.0) * a2 * a2;
+        a3 = T(3.0) * a3 * a3;
+        const T n1 = fma(T(5.0), f2, T(-2.0) * f1), n2 = fma(T(2.0), f3, f2), n3 = fma(T(4.0), f3, -f4);
+        r = fma(a1, n1, fma(a2, n2, a3 * n3)) * prcp<T>(a1 + a2 + a3);
+    }
+    return vel * rh * fma(up ? T(1.0) / T(6.0) : T(-1.0) / T(6.0), r, c);
 }
 
 // ------------------------------------------------ diffusion coefficients
@@ -326,7 +353,7 @@ __device__ __forceinline__ T upwind_d(const T (&D)[6], int m, int ms, int me, in
 template <typename T>
 struct Visc4 { const T* cell; const T* xy; const T* xz; const T* yz; };
 
-template <typename T, int F, int D, bool FAST = false>
+template <typename T, int F, int D>
 __device__ __forceinline__ void coefs(const Dims& d, const Phys& ph, const Visc4<T>& mu, long o, T& a, T& b, T& c)
 {
     const T h = D == 0 ? T(d.dx) : D == 1 ? T(d.dy) : T(d.dz);
@@ -339,22 +366,22 @@ __device__ __forceinline__ void coefs(const Dims& d, const Phys& ph, const Visc4
         return;
     }
     if (F == FU) {
-        if (D == 0) { a = sdh<T, FAST>(del * mu.cell[o - sx], h, rh); c = sdh<T, FAST>(del * mu.cell[o], h, rh); b = -(a + c); }
-        else if (D == 1) { a = sdh<T, FAST>(del * mu.xy[o], h, rh); c = sdh<T, FAST>(del * mu.xy[o + sy], h, rh); b = -(a + c); }
-        else { a = sdh<T, FAST>(del * mu.xz[o], h, rh); c = sdh<T, FAST>(del * mu.xz[o + 1], h, rh); b = -a - c; }
+        if (D == 0) { a = divh<T>(del * mu.cell[o - sx], h, rh); c = divh<T>(del * mu.cell[o], h, rh); b = -(a + c); }
+        else if (D == 1) { a = divh<T>(del * mu.xy[o], h, rh); c = divh<T>(del * mu.xy[o + sy], h, rh); b = -(a + c); }
+        else { a = divh<T>(del * mu.xz[o], h, rh); c = divh<T>(del * mu.xz[o + 1], h, rh); b = -a - c; }
         return;
     }
     if (F == FV) {
-        if (D == 0) { a = sdh<T, FAST>(del * mu.xy[o], h, rh); c = sdh<T, FAST>(del * mu.xy[o + sx], h, rh); }
-        else if (D == 1) { a = sdh<T, FAST>(del * mu.cell[o - sy], h, rh); c = sdh<T, FAST>(del * mu.cell[o], h, rh); }
-        else { a = sdh<T, FAST>(del * mu.yz[o], h, rh); c = sdh<T, FAST>(del * mu.yz[o + 1], h, rh); }
+        if (D == 0) { a = divh<T>(del * mu.xy[o], h, rh); c = divh<T>(del * mu.xy[o + sx], h, rh); }
+        else if (D == 1) { a = divh<T>(del * mu.cell[o - sy], h, rh); c = divh<T>(del * mu.cell[o], h, rh); }
+        else { a = divh<T>(del * mu.yz[o], h, rh); c = divh<T>(del * mu.yz[o + 1], h, rh); }
         b = -a - c;
         return;
     }
     // FW
-    if (D == 0) { a = sdh<T, FAST>(del * mu.xz[o], h, rh); c = sdh<T, FAST>(del * mu.xz[o + sx], h, rh); }
-    else if (D == 1) { a = sdh<T, FAST>(del * mu.yz[o], h, rh); c = sdh<T, FAST>(del * mu.yz[o + sy], h, rh); }
-    else { a = sdh<T, FAST>(del * mu.cell[o - 1], h, rh); c = sdh<T, FAST>(del * mu.cell[o], h, rh); }
+    if (D == 0) { a = divh<T>(del * mu.xz[o], h, rh); c = divh<T>(del * mu.xz[o + sx], h, rh); }
+    else if (D == 1) { a = divh<T>(del * mu.yz[o], h, rh); c = divh<T>(del * mu.yz[o + sy], h, rh); }
+    else { a = divh<T>(del * mu.cell[o - 1], h, rh); c = divh<T>(del * mu.cell[o], h, rh); }
     b = -a - c;
 }
 

@@ -160,38 +160,45 @@ __global__ __launch_bounds__(256) void k_rhs_c(Dims d, Phys ph0, const T* __rest
     // (the source keeps its value; at most the sign of a zero source differs)
     const T nm1 = r != T(0) ? Nm1[o] : T(0);
 
-    T D[6];
-    const T uval = T(0.5) * (u1 + u0);
+    const T uval = T(0.5) * (u1 + u0), vval = T(0.5) * (v1 + v0), wval = T(0.5) * (w1 + w0);
+    T nval, diff;
+    if constexpr (FAST) {
+        T xm, xp, ym, yp, zm, zp;
+        const T cx = upwind_term<T>(cx7, i, R.is, R.ie, uval, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
+        const T cy = upwind_term<T>(cy7, j, R.js, R.je, vval, T(d.dy), T(d.rdy), stale[0], stale[1], ym, yp);
+        const T cz = upwind_term<T>(cz7, k, R.ks, R.ke, wval, T(d.dz), T(d.rdz), stale[2], stale[3], zm, zp);
+        nval = -(cz + cx + cy);
+        diff = T(ph.kap[FC][0]) * (xp - xm);
+        diff = fma(T(ph.kap[FC][1]), yp - ym, diff);
+        diff = fma(T(ph.kap[FC][2]), zp - zm, diff);
+    } else {
+        T D[6];
 #pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(cx7[m + 1] - cx7[m], T(d.dx), d.rdx);
-    const T cxd = upwind_d<T, FAST>(D, i, R.is, R.ie, uval >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
-    const T convx = uval * cxd;
-    const T vval = T(0.5) * (v1 + v0);
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(cx7[m + 1] - cx7[m], T(d.dx), d.rdx);
+        const T convx = uval * upwind_d<T>(D, i, R.is, R.ie, uval >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
 #pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(cy7[m + 1] - cy7[m], T(d.dy), d.rdy);
-    const T cyd = upwind_d<T, FAST>(D, j, R.js, R.je, vval >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
-    const T convy = vval * cyd;
-    const T wval = T(0.5) * (w1 + w0);
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(cy7[m + 1] - cy7[m], T(d.dy), d.rdy);
+        const T convy = vval * upwind_d<T>(D, j, R.js, R.je, vval >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
 #pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(cz7[m + 1] - cz7[m], T(d.dz), d.rdz);
-    const T czd = upwind_d<T, FAST>(D, k, R.ks, R.ke, wval >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
-    T nval = -(wval * czd + convx + convy);
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(cz7[m + 1] - cz7[m], T(d.dz), d.rdz);
+        const T czd = upwind_d<T>(D, k, R.ks, R.ke, wval >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
+        nval = -(wval * czd + convx + convy);
+        T ax, bx, cx, ay, by, cy, az, bz, cz;
+        Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
+        coefs<T, FC, 0>(d, ph, none, o, ax, bx, cx);
+        coefs<T, FC, 1>(d, ph, none, o, ay, by, cy);
+        coefs<T, FC, 2>(d, ph, none, o, az, bz, cz);
+        const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
+        const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
+        const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
+        diff = axx + axy + axz;
+    }
     // the learned closure's correction of N (no counterpart in the
     // reference; ncorr is null without a closure)
     if (ncorr) nval += ncorr[o];
     N[o] = nval;
-
-    T ax, bx, cx, ay, by, cy, az, bz, cz;
-    Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
-    coefs<T, FC, 0, FAST>(d, ph, none, o, ax, bx, cx);
-    coefs<T, FC, 1, FAST>(d, ph, none, o, ay, by, cy);
-    coefs<T, FC, 2, FAST>(d, ph, none, o, az, bz, cz);
     const T conv = (g * nval + r * nm1);
-    const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
-    const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
-    const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
-    const T diff = (g + r) * (axx + axy + axz);
-    S[o] = dt * (conv + diff);
+    S[o] = dt * (conv + (g + r) * diff);
 }
 
 // xmom/ymom/zmom explicit part at one point of component F's range: H?_op
@@ -210,14 +217,14 @@ __global__ __launch_bounds__(256) void k_rhs_c(Dims d, Phys ph0, const T* __rest
 //   other component with the edge viscosities mA (first) and mB (second);
 //   A(mu_old) (A_umom/A_vmom/A_wmom, 1443-1536): mu.cell at o - s_F and o
 //   along F's own direction, mA and mB along the others.
-template <typename T, int F, bool FAST>
+template <typename T, int F>
 __device__ __forceinline__ void coef_vals(const Dims& d, const Phys& ph, int D, T m0, T m1, T& a, T& b, T& c)
 {
     const T h = D == 0 ? T(d.dx) : D == 1 ? T(d.dy) : T(d.dz);
     const double rh = D == 0 ? d.rdx : D == 1 ? d.rdy : d.rdz;
     const T del = T(ph.cdel[F][D]);
-    a = sdh<T, FAST>(del * m0, h, rh);
-    c = sdh<T, FAST>(del * m1, h, rh);
+    a = divh<T>(del * m0, h, rh);
+    c = divh<T>(del * m1, h, rh);
     // coefs(): -(a + c) for u along x and y, -a - c otherwise
     b = (F == FU && D != 2) ? -(a + c) : -a - c;
 }
@@ -273,77 +280,69 @@ __device__ __forceinline__ void rhs_mom_point(const Dims& d, const Phys& ph, con
     const T cn0 = force ? cn[o] : T(0), cn1 = force ? cn[o - sF] : T(0);
     const T pgv = pg[o], nm1 = r != T(0) ? Nm1[o] : T(0);   // as in k_rhs_c
 
-    // convec_term: upwind derivatives along x, y, z
     const T alpha = g + r;
-    T D[6];
     const T vx = F == FU ? qx[3] : T(0.25) * (av[0] + av[1] + av[2] + av[3]);
     const T vy = F == FV ? qy[3] : F == FU ? T(0.25) * (av[0] + av[1] + av[2] + av[3])
                                            : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
     const T vz = F == FW ? qz[3] : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
-#pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(qx[m + 1] - qx[m], T(d.dx), d.rdx);
-    const T dxd = upwind_d<T, FAST>(D, i, R.is, R.ie, vx >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
-    const T convx = vx * dxd;
-#pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(qy[m + 1] - qy[m], T(d.dy), d.rdy);
-    const T dyd = upwind_d<T, FAST>(D, j, R.js, R.je, vy >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
-    const T convy = vy * dyd;
-#pragma unroll
-    for (int m = 0; m < 6; m++) D[m] = sdh<T, FAST>(qz[m + 1] - qz[m], T(d.dz), d.rdz);
-    const T dzd = upwind_d<T, FAST>(D, k, R.ks, R.ke, vz >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
-    const T ct = vz * dzd + convx + convy;
-
-    // explicit_n: -convec_term + the cross-viscous terms, left to right
     const int fi = F - FU;
-    T del = T(ph.edel[fi][0]);
-    T p1, m1, p2, m2;
-    if (F == FU) {
-        p1 = del * ma1 * (av[2] - av[3]);
-        m1 = del * ma0 * (av[1] - av[0]);
-        del = T(ph.edel[fi][1]);
-        p2 = del * mb1 * (bv[2] - bv[3]);
-        m2 = del * mb0 * (bv[1] - bv[0]);
-    } else if (F == FV) {
-        p1 = del * ma1 * (av[3] - av[1]);
-        m1 = del * ma0 * (av[2] - av[0]);
-        del = T(ph.edel[fi][1]);
-        p2 = del * mb1 * (bv[3] - bv[1]);
-        m2 = del * mb0 * (bv[2] - bv[0]);
-    } else {
-        p1 = del * ma1 * (av[3] - av[1]);
-        m1 = del * ma0 * (av[2] - av[0]);
-        del = T(ph.edel[fi][1]);
-        p2 = del * mb1 * (bv[3] - bv[2]);
-        m2 = del * mb0 * (bv[1] - bv[0]);
-    }
-    const T nval = -ct + p1 - m1 + p2 - m2;
-    N[o] = nval;
-
-    // source: dt [g N + r N_nm1 + alpha A(mu_old) q + alpha (body force)]
-    T ax, bx, cx, ay, by, cy, az, bz, cz;
-    if (F == FU) {
-        coef_vals<T, F, FAST>(d, ph, 0, mc0, mc1, ax, bx, cx);
-        coef_vals<T, F, FAST>(d, ph, 1, ma0, ma1, ay, by, cy);
-        coef_vals<T, F, FAST>(d, ph, 2, mb0, mb1, az, bz, cz);
-    } else if (F == FV) {
-        coef_vals<T, F, FAST>(d, ph, 0, ma0, ma1, ax, bx, cx);
-        coef_vals<T, F, FAST>(d, ph, 1, mc0, mc1, ay, by, cy);
-        coef_vals<T, F, FAST>(d, ph, 2, mb0, mb1, az, bz, cz);
-    } else {
-        coef_vals<T, F, FAST>(d, ph, 0, ma0, ma1, ax, bx, cx);
-        coef_vals<T, F, FAST>(d, ph, 1, mb0, mb1, ay, by, cy);
-        coef_vals<T, F, FAST>(d, ph, 2, mc0, mc1, az, bz, cz);
-    }
-    const T conv = (g * nval + r * nm1);
-    const T axx = ax * qx[2] + bx * qx[3] + cx * qx[4];
-    const T axy = ay * qy[2] + by * qy[3] + cy * qy[4];
-    const T axz = az * qz[2] + bz * qz[3] + cz * qz[4];
-    const T visc = alpha * (axx + axy + axz);
+    // the cross-viscous differences at the upper and lower edges
+    const T a1 = F == FU ? av[2] - av[3] : av[3] - av[1];
+    const T a0 = F == FU ? av[1] - av[0] : av[2] - av[0];
+    const T b1 = F == FU ? bv[2] - bv[3] : F == FV ? bv[3] - bv[1] : bv[3] - bv[2];
+    const T b0 = F == FV ? bv[2] - bv[0] : bv[1] - bv[0];
+    // mu below and above the point along x, y and z
+    const T mx0 = F == FU ? mc0 : ma0, mx1 = F == FU ? mc1 : ma1;
+    const T my0 = F == FU ? ma0 : F == FV ? mc0 : mb0, my1 = F == FU ? ma1 : F == FV ? mc1 : mb1;
+    const T mz0 = F == FW ? mc0 : mb0, mz1 = F == FW ? mc1 : mb1;
     const T Re = T(ph.Re);
-    T bodyforce;
-    if (!force) bodyforce = alpha * (-sdh<T, FAST>(pgv, Re, ph.rRe));
-    else bodyforce = alpha * (-T(ph.fre[fi]) * (T(0.5) * (cn0 + cn1)) - sdh<T, FAST>(pgv, Re, ph.rRe));
-    S[o] = dt * (conv + visc + bodyforce);
+    if constexpr (FAST) {
+        T xm, xp, ym, yp, zm, zp;
+        const T cx = upwind_term<T>(qx, i, R.is, R.ie, vx, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
+        const T cy = upwind_term<T>(qy, j, R.js, R.je, vy, T(d.dy), T(d.rdy), stale[0], stale[1], ym, yp);
+        const T cz = upwind_term<T>(qz, k, R.ks, R.ke, vz, T(d.dz), T(d.rdz), stale[2], stale[3], zm, zp);
+        T nval = fma(T(ph.edel[fi][0]), fma(ma1, a1, -(ma0 * a0)), -(cz + cx + cy));
+        nval = fma(T(ph.edel[fi][1]), fma(mb1, b1, -(mb0 * b0)), nval);
+        N[o] = nval;
+        T visc = T(ph.kap[F][0]) * fma(mx1, xp, -(mx0 * xm));
+        visc = fma(T(ph.kap[F][1]), fma(my1, yp, -(my0 * ym)), visc);
+        visc = fma(T(ph.kap[F][2]), fma(mz1, zp, -(mz0 * zm)), visc);
+        visc = fma(-T(ph.rRe), pgv, visc);
+        if (force) visc = fma(-T(ph.fre[fi]), T(0.5) * (cn0 + cn1), visc);
+        S[o] = dt * fma(alpha, visc, fma(g, nval, r * nm1));
+    } else {
+        // convec_term: upwind derivatives along x, y, z
+        T D[6];
+#pragma unroll
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(qx[m + 1] - qx[m], T(d.dx), d.rdx);
+        const T convx = vx * upwind_d<T>(D, i, R.is, R.ie, vx >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
+#pragma unroll
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(qy[m + 1] - qy[m], T(d.dy), d.rdy);
+        const T convy = vy * upwind_d<T>(D, j, R.js, R.je, vy >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
+#pragma unroll
+        for (int m = 0; m < 6; m++) D[m] = divh<T>(qz[m + 1] - qz[m], T(d.dz), d.rdz);
+        const T dzd = upwind_d<T>(D, k, R.ks, R.ke, vz >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
+        const T ct = vz * dzd + convx + convy;
+        // explicit_n: -convec_term + the cross-viscous terms, left to right
+        const T p1 = T(ph.edel[fi][0]) * ma1 * a1, m1 = T(ph.edel[fi][0]) * ma0 * a0;
+        const T p2 = T(ph.edel[fi][1]) * mb1 * b1, m2 = T(ph.edel[fi][1]) * mb0 * b0;
+        const T nval = -ct + p1 - m1 + p2 - m2;
+        N[o] = nval;
+        // source: dt [g N + r N_nm1 + alpha A(mu_old) q + alpha (body force)]
+        T ax, bx, cx, ay, by, cy, az, bz, cz;
+        coef_vals<T, F>(d, ph, 0, mx0, mx1, ax, bx, cx);
+        coef_vals<T, F>(d, ph, 1, my0, my1, ay, by, cy);
+        coef_vals<T, F>(d, ph, 2, mz0, mz1, az, bz, cz);
+        const T conv = (g * nval + r * nm1);
+        const T axx = ax * qx[2] + bx * qx[3] + cx * qx[4];
+        const T axy = ay * qy[2] + by * qy[3] + cy * qy[4];
+        const T axz = az * qz[2] + bz * qz[3] + cz * qz[4];
+        const T visc = alpha * (axx + axy + axz);
+        T bodyforce;
+        if (!force) bodyforce = alpha * (-divh<T>(pgv, Re, ph.rRe));
+        else bodyforce = alpha * (-T(ph.fre[fi]) * (T(0.5) * (cn0 + cn1)) - divh<T>(pgv, Re, ph.rRe));
+        S[o] = dt * (conv + visc + bodyforce);
+    }
 }
 
 // one component over its range (one thread per point)
@@ -1032,9 +1031,9 @@ __device__ __forceinline__ T corr_pg_new(const Dims& d, const Phys& ph, const Co
 #pragma unroll
     for (int g = 0; g < 7; g++) gr[g] = corr_grad<T, F>(d, c, g);
     T ax, bx, cx, ay, by, cy, az, bz, cz;
-    coef_vals<T, F, false>(d, ph, 0, c.m[0], c.m[1], ax, bx, cx);
-    coef_vals<T, F, false>(d, ph, 1, c.m[2], c.m[3], ay, by, cy);
-    coef_vals<T, F, false>(d, ph, 2, c.m[4], c.m[5], az, bz, cz);
+    coef_vals<T, F>(d, ph, 0, c.m[0], c.m[1], ax, bx, cx);
+    coef_vals<T, F>(d, ph, 1, c.m[2], c.m[3], ay, by, cy);
+    coef_vals<T, F>(d, ph, 2, c.m[4], c.m[5], az, bz, cz);
     const T g0 = gr[0];
     const T pxx = (ax) * gr[1] + (bx) * g0 + (cx) * gr[2];
     const T pyy = (ay) * gr[3] + (by) * g0 + (cy) * gr[4];
