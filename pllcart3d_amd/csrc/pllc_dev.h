@@ -1,8 +1,9 @@
 // pllc_dev.h -- device-side definitions shared by the pllcart3d HIP kernels.
 //
-// Index space: every 3D field is one contiguous [i][j][k] block (k fastest)
-// of nx_max*ny_max*nz_max values with ghost widths (3,1,1), the same linear
-// index as the reference's double*** arrays (allocate_3d_calloc.h:46-64).
+// Index space: every 3D field is an [i][j][k] block (k fastest) with ghost
+// widths (3,1,1) and the strides of Dims: in the drop-in entry points the
+// contiguous nx_max*ny_max*nz_max values of the reference's double*** arrays
+// (allocate_3d_calloc.h:46-64), in simulations a pitched layout (pitch_dims).
 // Interior cells are i in [3, nx+2], j in [1, ny], k in [1, nz]
 // (grid_setup, pllcart3d.c:353-370).
 //
@@ -18,10 +19,30 @@ namespace pllc {
 struct Dims {
     int nx, ny, nz;   // interior cells
     int NX, NY, NZ;   // with ghosts
-    long sx, sy;      // strides of i and j (k stride is 1)
+    long sx, sy;      // strides of i and j (k stride is 1); sy >= NZ (pitch_dims)
     double dx, dy, dz;
     double rdx, rdy, rdz;   // 1/dx, 1/dy, 1/dz rounded once on the host (divh)
 };
+
+// The layout of a simulation's own fields (values of esize bytes): rows of a
+// whole number of 128-byte lines, and fields that start pitch_lead values
+// after an aligned address, so that the interior point k = 1 of every row
+// starts a line; the line after a row's points holds its ghost k = nz + 1 and
+// the next row's k = 0.  With rows at any 8-byte offset every 16 lanes of a
+// load or store touched two 64-byte blocks of the L1 instead of one.
+// Measured (packed rows -> this): 512x256x256 x-sweep 743 -> 693 us FP64, 419
+// -> 391 mixed, mixed momentum explicit part 392 -> 341, k_corr_pg 573 -> 540;
+// 256x128x128 x-sweep 83 -> 72 FP64.  k = 1 at 64 bytes into a line: slower
+// than packed rows (x-sweep 825, k_corr_pg mixed 598).
+__host__ inline long pitch_lead(int esize) { return 128 / esize - 1; }
+__host__ inline void pitch_dims(Dims& d, int esize)
+{
+    const long q = 128 / esize;
+    d.sy = (d.NZ + q - 1) / q * q;
+    d.sx = (long)d.NY * d.sy;
+}
+// values from one field's first point to the next field's
+__host__ inline long field_values(const Dims& d) { return (long)d.NX * d.sx; }
 
 // a / h for a divisor fixed on the host, with rh = 1/h correctly rounded
 // there.  FP64: q = a*rh and one fused correction r = a - q*h (exact),

@@ -129,7 +129,11 @@ struct Ops {
     // bulk() and stale() in one launch where the plane allows it
     static void bulk_stale(Ctx<T>& c, int slot, double alpha, bool advance_t, const T* qc, const T* qu, const T* qv,
                            const T* qw);
-    static void copy(Ctx<T>& c, const T* a, T* b, long n);
+    // b = a, every point of a field
+    static void copy(Ctx<T>& c, const T* a, T* b);
+    // rows of a field (pitched, T) to and from contiguous FP64 rows of NZ values
+    static void pack(Ctx<T>& c, const T* a, double* b, long rows);
+    static void unpack(Ctx<T>& c, const double* a, T* b, long rows);
     // velocity correction, outflow deficit and the pressure-gradient update
     // of all three components (mu_new) in one pass over the cells
     // ghosts: also update_veloghost_points' ghost copies of the corrected values

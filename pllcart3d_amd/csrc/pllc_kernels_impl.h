@@ -355,12 +355,12 @@ __global__ __launch_bounds__(256) void k_rhs_mom(Dims d, Phys ph0, const T* __re
 {
     const Rng R = field_rng(d, F);
     const int2 tl = xcd_tile();
-    const int k = tl.x * blockDim.x + threadIdx.x + R.ks;
+    const int k = tl.x * blockDim.x + threadIdx.x + 1;
     const int j = tl.y * blockDim.y + threadIdx.y + R.js;
     int il;
     const int m = bt_member(bt, blockIdx.z, gridDim.z, il);
     const int i = il + R.is;
-    if (k > R.ke || j > R.je) return;
+    if (k < R.ks || k > R.ke || j > R.je) return;
     const Phys& ph = bt_phys<B>(bt, ph0, m);
     rhs_mom_point<T, F, FAST>(d, ph, R, i, j, k, bt_f(bt, u, m), bt_f(bt, v, m), bt_f(bt, w, m), bt_mu(bt, mu, m),
                               bt_f(bt, cn, m), bt_f(bt, pg, m), bt_f(bt, Nm1, m), bt_f(bt, N, m), bt_f(bt, S, m),
@@ -746,9 +746,10 @@ __global__ __launch_bounds__(ZL) void k_sweep_z_lds(Dims d, LineSets<T> sets, co
 // centres on a one-cell ring, and edges from the 4-point mean of c (mean
 // first, then the law).
 //
-// The (j, k) plane of the index space (j 0 .. ny+1, k 0 .. nz+1) is
-// contiguous, so a plane is cut into chunks of 256 consecutive points, one
-// per block; gridDim.x (chunks per plane) is a multiple of 8 so that the
+// A (j, k) plane (j 0 .. ny+1, k 0 .. nz+1) is cut into chunks of 256 lanes,
+// one per block, of rows of nz + 2 lanes (k = 1 .. nz+1, then 0; no lane idle,
+// for the exponentials are half its time in FP64); gridDim.x (chunks per plane) is a
+// multiple of 8 so that the
 // XCD a block runs on (its linear id mod 8) depends only on blockIdx.x, and
 // XCD x takes chunks x nb/8 .. (x+1) nb/8 - 1 of every plane: the previous
 // plane's c (o - sx) was read into the same XCD's L2.
@@ -767,9 +768,10 @@ __global__ __launch_bounds__(256) void k_visc(Dims d, Phys ph0, const T* __restr
     const int nb8 = gridDim.x >> 3;
     const int chunk = (blockIdx.x & 7) * nb8 + (blockIdx.x >> 3);
     const int l = chunk * 256 + threadIdx.x;
-    const int pk = d.nz + 2;
-    if (l >= (d.ny + 2) * pk) return;
-    const int j = l / pk, k = l - j * pk;                      // 0 .. ny+1, 0 .. nz+1
+    const int w = d.nz + 2;
+    const int j = l / w, a = l - j * w;                        // 0 .. ny+1
+    if (j > d.ny + 1) return;
+    const int k = a <= d.nz ? a + 1 : 0;                       // 1 .. nz+1, 0
     const int i = blockIdx.y + 2;                              // 2 .. nx+3
     const long o = IX(d, i, j, k), sx = d.sx, sy = d.sy;
     // the seven values first (all inside the array: i >= 2 leaves a ghost
@@ -1225,34 +1227,62 @@ __global__ __launch_bounds__(256) void k_pg(Dims d, Phys ph, Visc4<T> mu, const 
 // ------------------------------------------------------------ reductions
 
 // find_cfl (3095-3118), pass 1: per-block max of
-// |u|/dx + |v|/dy + |w|/dz at cell centres.
+// |u|/dx + |v|/dy + |w|/dz at cell centres.  A block covers its tile of (j, k)
+// in CFL_PLANES planes, all their loads in flight together; the max within
+// a wave by lane exchange, over the waves through LDS (a max in any order is
+// the same value).
+constexpr int CFL_PLANES = 4;
 template <typename T>
 __global__ __launch_bounds__(256) void k_cfl_partial(Dims d, const T* __restrict__ u, const T* __restrict__ v,
                                                      const T* __restrict__ w, double* __restrict__ part, Bt bt)
 {
-    __shared__ double red[256];
+    __shared__ double red[4];
     const int2 tl = xcd_tile();
     const int k = tl.x * blockDim.x + threadIdx.x + 1;
     const int j = tl.y * blockDim.y + threadIdx.y + 1;
-    int il;
-    const int mb = bt_member(bt, blockIdx.z, gridDim.z, il);
-    const int i = il + 3;
+    int ib;
+    const int mb = bt_member(bt, blockIdx.z, gridDim.z, ib);
     const int t = threadIdx.y * blockDim.x + threadIdx.x;
     double m = 0.0;
     if (k <= d.nz && j <= d.ny) {
-        const long o = IX(d, i, j, k) + mb * bt.fs;
-        const double uv = 0.5 * ((double)u[o] + (double)u[o + d.sx]);
-        const double vv = 0.5 * ((double)v[o] + (double)v[o + d.sy]);
-        const double wv = 0.5 * ((double)w[o] + (double)w[o + 1]);
-        m = (fabs(uv) / d.dx) + (fabs(vv) / d.dy) + (fabs(wv) / d.dz);
+        const long o = IX(d, ib * CFL_PLANES + 3, j, k) + mb * bt.fs;
+        const int n = min(CFL_PLANES, d.nx - ib * CFL_PLANES);
+        T u0[CFL_PLANES + 1], v0[CFL_PLANES], v1[CFL_PLANES], w0[CFL_PLANES], w1[CFL_PLANES];
+        u0[0] = u[o];
+#pragma unroll
+        for (int p = 0; p < CFL_PLANES; p++) {
+            const long q = o + (long)min(p, n - 1) * d.sx;   // the last plane again past the end
+            u0[p + 1] = u[q + d.sx];
+            v0[p] = v[q];
+            v1[p] = v[q + d.sy];
+            w0[p] = w[q];
+            w1[p] = w[q + 1];
+        }
+#pragma unroll
+        for (int p = 0; p < CFL_PLANES; p++) {
+            if (p < n) {
+                const double uv = 0.5 * ((double)u0[p] + (double)u0[p + 1]);
+                const double vv = 0.5 * ((double)v0[p] + (double)v1[p]);
+                const double wv = 0.5 * ((double)w0[p] + (double)w1[p]);
+                const double x = (fabs(uv) / d.dx) + (fabs(vv) / d.dy) + (fabs(wv) / d.dz);
+                m = m > x ? m : x;
+            }
+        }
     }
-    red[t] = m;
+    // the last wave of a tile may have fewer than 64 lanes
+    const int lane = t & 63, nl = min(64, (int)(blockDim.x * blockDim.y) - (t - lane));
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        const double x = __shfl_xor(m, s);
+        m = (lane ^ s) < nl && x > m ? x : m;
+    }
+    if (lane == 0) red[t >> 6] = m;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (t < s) red[t] = red[t] > red[t + s] ? red[t] : red[t + s];
-        __syncthreads();
+    if (t == 0) {
+        const int nw = (blockDim.x * blockDim.y + 63) >> 6;
+        for (int s = 1; s < nw; s++) m = m > red[s] ? m : red[s];
+        part[mb * bt.np + ((long)ib * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
     }
-    if (t == 0) part[mb * bt.np + ((long)il * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = red[0];
 }
 
 // pass 2: max over the partials; dt = min(CFLmax/max, Timestep)
@@ -2200,10 +2230,28 @@ __global__ void k_set_scalar(double* __restrict__ p, int i, double v)
     if (threadIdx.x == 0) p[i] = v;
 }
 
-template <typename T>
-__global__ void k_copy(const T* __restrict__ a, T* __restrict__ b, long n)
+// rows of NZ values (grid.x blocks of (64, 4) threads over the rows): a field
+// onto another, out of and into the contiguous FP64 rows of the host's arrays
+template <typename T, typename F>
+__device__ __forceinline__ void field_rows(const Dims& d, long rows, F f)
 {
-    for (long l = (long)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (long)gridDim.x * blockDim.x) b[l] = a[l];
+    for (long r = (long)blockIdx.x * blockDim.y + threadIdx.y; r < rows; r += (long)gridDim.x * blockDim.y)
+        for (int k = threadIdx.x; k < d.NZ; k += 64) f(r * d.sy + k, r * d.NZ + k);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy(Dims d, const T* __restrict__ a, T* __restrict__ b, long rows)
+{
+    field_rows<T>(d, rows, [&](long o, long) { b[o] = a[o]; });
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_pack(Dims d, const T* __restrict__ a, double* __restrict__ b, long rows)
+{
+    field_rows<T>(d, rows, [&](long o, long l) { b[l] = double(a[o]); });
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_unpack(Dims d, const double* __restrict__ a, T* __restrict__ b, long rows)
+{
+    field_rows<T>(d, rows, [&](long o, long l) { b[o] = T(a[l]); });
 }
 
 template <typename T>
@@ -2463,7 +2511,9 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     template __global__ void k_dct_lines<T, false, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>); \
     template __global__ void k_dct_lines<T, true, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>);  \
     template __global__ void k_dct_lines<T, true, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>);  \
-    template __global__ void k_copy<T>(const T*, T*, long);                                                    \
+    template __global__ void k_copy<T>(Dims, const T*, T*, long);                                              \
+    template __global__ void k_pack<T>(Dims, const T*, double*, long);                                         \
+    template __global__ void k_unpack<T>(Dims, const double*, T*, long);                                       \
     template __global__ void k_fill<T>(T*, long, T);
 
 // ------------------------------------------------- wave perturbation
@@ -2759,6 +2809,9 @@ __device__ __forceinline__ void chunk_couple(T* __restrict__ buf, int P, int LPB
     }
 }
 
+// lanes per row of the x- and y-sweeps
+__host__ __device__ constexpr int line_row(int nz) { return (nz + 15) / 16 * 16; }
+
 // x- and y-lines (rows strided by sx / sy): block (LPB lines along k,
 // P chunks); a wavefront reads one row of consecutive k, coalesced.  At most
 // 128 registers (q_old is read after the coupling), so that in FP64 two
@@ -2778,27 +2831,29 @@ __global__ __launch_bounds__(PART_THREADS, 4) void k_sweep_part(Dims d, LineSets
     const LineSet<T> L = bt_lines<T, DIR>(bt, sets.s[blockIdx.y], blockIdx.z);
     scal += blockIdx.z * S_SIZE;
     const Rng R = L.R;
-    // x-lines: the y and z ghosts of the new values (kg, jg) are lanes of
-    // their own that solve the line next to the wall again and store at
-    // their own place, so a ghost costs no store of its own
-    const int kg = DIR == 0 && L.kg, jg = DIR == 0 && L.jg;
-    const int n0 = R.ke - R.ks + 1 + 2 * kg;
+    // Lanes cover k = 1 .. nz of a row, rounded up to 16 lanes (an aligned
+    // piece of it).  x-lines: the y ghosts of the new values (jg) are rows of
+    // lanes of their own that solve the line next to the wall again and store
+    // at their own place; the z ghosts (kg) are stored by the lanes at the
+    // row's ends
+    const int jg = DIR == 0 && L.jg;
+    const int n0 = line_row(d.nz);
     const int n1 = DIR == 0 ? R.je - R.js + 1 + 2 * jg : R.ie - R.is + 1;
     // blocks of one line set: grid x is a multiple of 8 (XCD order within the set)
     const int bx = (gridDim.x & 7) == 0 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const int l = bx * LPB + q;
     const int n = DIR == 0 ? R.ie - R.is + 1 : R.je - R.js + 1;
     const int x0 = s * PM;
+    const int a1 = l / n0, kl = l - a1 * n0 + 1;
     // a set with shorter lines than the launch's longest may need fewer chunks
-    const bool live = l < n0 * n1 && x0 < n;
-    const int a1 = live ? l / n0 : 0, a0 = live ? l - a1 * n0 : 0;
-    const int kl = R.ks - kg + a0, jl = R.js - jg + a1;   // the lane's place (x-lines)
-    const int k = min(max(kl, R.ks), R.ke);
+    const bool live = x0 < n && a1 < n1 && kl >= R.ks && kl <= R.ke;
+    const int k = live ? kl : R.ks;
+    const int jl = R.js - jg + a1;   // x-lines: the lane's place
     int i, j;
     long st;
-    if (DIR == 0) { j = min(max(jl, R.js), R.je); i = R.is; st = d.sx; }
-    else { i = R.is + a1; j = R.js; st = d.sy; }
-    const bool own = k == kl && (DIR != 0 || j == jl);   // not a ghost lane
+    if (DIR == 0) { j = live ? min(max(jl, R.js), R.je) : R.js; i = R.is; st = d.sx; }
+    else { i = live ? R.is + a1 : R.is; j = R.js; st = d.sy; }
+    const bool own = DIR != 0 || j == jl;   // not a ghost lane
     const bool last = x0 + PM >= n;
     const int nv = min(PM, n - x0);
     const long o0 = IX(d, i, j, k) + (long)(live ? x0 : 0) * st;
@@ -2875,11 +2930,10 @@ __global__ __launch_bounds__(PART_THREADS, 4) void k_sweep_part(Dims d, LineSets
     // c's ghosts are copies (700-712; the y-ghost rows' z ghosts too), the
     // velocities' z ghosts copies, their y ghosts negated, their corners
     // never written (velo_ghost_point)
-    const bool vel = L.F != FC, jgh = j != jl;
-    if (vel && jgh && k != kl) return;
-    const T sg = vel && jgh ? T(-1.0) : T(1.0);
+    const bool vel = L.F != FC;
+    const T sg = vel && !own ? T(-1.0) : T(1.0);
     const T* qo = L.qold + on;
-    T* qn = L.qnew + on + (long)(jl - j) * d.sy + (kl - k);
+    T* qn = L.qnew + on + (long)(jl - j) * d.sy;
     if (nv == PM) {
         T v[PM];
 #pragma unroll
@@ -2896,6 +2950,14 @@ __global__ __launch_bounds__(PART_THREADS, 4) void k_sweep_part(Dims d, LineSets
                 ch.D[t] = sg * (qo[(long)t * st] + ch.D[t]);
                 qn[(long)t * st] = ch.D[t];
             }
+    }
+    if (L.kg && (own || !vel) && (k == R.ks || k == R.ke)) {
+        for (int e = -1; e <= 1; e += 2) {
+            if (k != (e < 0 ? R.ks : R.ke)) continue;
+#pragma unroll
+            for (int t = 0; t < PM; t++)
+                if (t < nv) qn[(long)t * st + e] = ch.D[t];
+        }
     }
     // the inlet ghosts of v and w
     if (s == 0 && own && L.inlet) qn[-d.sx] = -ch.D[0];
@@ -3248,9 +3310,12 @@ static int resident_blocks(K f, int nthreads, size_t sm)
 template <typename T>
 static inline bool fast_stencils(const Ctx<T>& c) { return c.line_solver == 0; }
 
-// 256-thread tiles of one i-plane: 128 x 2 (k, j) when a k row has 96 or
-// more points (measured faster than 64 x 4, 32 x 8 and 256 x 1 for the
-// cell kernels at 128-point rows, mostly in FP32), 64 x 4 for shorter rows
+// Tiles of one i-plane of at most 256 threads (k, j), k from 1: a row is cut
+// into as few equal parts of at most 128 points as it needs, each rounded up
+// to 16 lanes (an aligned piece of a row), and a tile takes as many rows as
+// fit (128 x 2 measured faster than 64 x 4, 32 x 8 and 256 x 1 for the cell
+// kernels at 128-point rows; at 96 points 96 x 2 leaves no lane idle where
+// 128 x 2 left a quarter)
 // launchers without a batched form: false (and the error set) when the
 // context launches over a batch
 template <typename T>
@@ -3263,9 +3328,9 @@ static bool single(const Ctx<T>& c, const char* what)
 
 static inline dim3 cell_grid(const Rng& R, dim3& blk)
 {
-    const int nk = R.ke - R.ks + 1, bx = nk >= 96 ? 128 : 64, by = 256 / bx;
+    const int nk = R.ke, nt = (nk + 127) / 128, bx = ((nk + nt - 1) / nt + 15) / 16 * 16, by = 256 / bx;
     blk = dim3(bx, by, 1);
-    return dim3((nk + bx - 1) / bx, (R.je - R.js + 1 + by - 1) / by, R.ie - R.is + 1);
+    return dim3(nt, (R.je - R.js + 1 + by - 1) / by, R.ie - R.is + 1);
 }
 static inline dim3 line_grid(long n) { return dim3((unsigned)((n + 255) / 256)); }
 // a cell grid (planes along z) over the context's batch: nm times the planes
@@ -3383,7 +3448,7 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
     for (int t = 0; t < 3; t++) {
         const int DIR = order[t];
         LineSets<T> ls{};
-        long lines = 0;
+        long lines = 0, lanes = 0;
         for (int q = 0; q < nset; q++) {
             ls.s[q] = line_set<T>(c, F[q], DIR, S[q], CC[q], mu, qold[q], qnew[q], N[q], Nm1[q]);
             LineSet<T>& L = ls.s[q];
@@ -3392,10 +3457,10 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
             L.kg = L.ghost_c || L.ghost_v == FU || L.ghost_v == FV;
             L.inlet = L.ghost_v == FV || L.ghost_v == FW;
             const Rng& R = L.R;
-            const long nl = DIR == 0 ? (long)(R.je - R.js + 1 + 2 * L.jg) * (R.ke - R.ks + 1 + 2 * L.kg)
-                          : DIR == 1 ? (long)(R.ie - R.is + 1) * (R.ke - R.ks + 1)
-                                     : (long)(R.ie - R.is + 1) * (R.je - R.js + 1);
-            lines = nl > lines ? nl : lines;
+            const long ni = R.ie - R.is + 1, nj = R.je - R.js + 1, nk = R.ke - R.ks + 1;
+            lines = std::max(lines, DIR == 0 ? nj * nk : DIR == 1 ? ni * nk : ni * nj);
+            // the partitioned x- and y-sweeps' lanes
+            lanes = std::max(lanes, (DIR == 0 ? nj + 2 * L.jg : ni) * line_row(c.d.nz));
         }
         int nmax = 0, nmin = 1 << 30;
         for (int q = 0; q < nset; q++) {
@@ -3416,7 +3481,7 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
             if (c.lpb[DIR] > 0) LPB = std::min(c.lpb[DIR], most);   // tuned
             // block count rounded up to a multiple of 8 (XCD order); the
             // blocks past the last line do nothing
-            const dim3 blk(LPB, P, 1), grd((unsigned)(((lines + LPB - 1) / LPB + 7) / 8 * 8), nset, c.bt.nm);
+            const dim3 blk(LPB, P, 1), grd((unsigned)(((lanes + LPB - 1) / LPB + 7) / 8 * 8), nset, c.bt.nm);
             const size_t sm = (size_t)6 * P * LPB * sizeof(T);
             if (DIR == 0)
                 PLLC_L(c, nm[0], (k_sweep_part<T, 0><<<grd, blk, sm, c.st>>>(c.d, ls, c.scal, slot, g, r, c.bt)));
@@ -3489,7 +3554,7 @@ void Ops<T>::concentration(Ctx<T>& c, double g, double r, int slot, const T* un,
 template <typename T>
 void Ops<T>::viscosity(Ctx<T>& c, const T* cn, T* const mu[4])
 {
-    // chunks of 256 points per (j, k) plane, rounded up to a multiple of 8
+    // chunks of 256 lanes per (j, k) plane, rounded up to a multiple of 8
     const int nb = (int)(((long)(c.d.ny + 2) * (c.d.nz + 2) + 256 * 8 - 1) / (256 * 8)) * 8;
     const dim3 grd(nb, c.d.nx + 2, c.bt.nm);
     if (c.bt.nm > 1)
@@ -3837,8 +3902,9 @@ template <typename T>
 void Ops<T>::cfl(Ctx<T>& c)
 {
     dim3 blk;
-    const dim3 grd = cell_grid(field_rng(c.d, FC), blk);
-    // partials of member m at m * bt.np (one per block of its planes)
+    dim3 grd = cell_grid(field_rng(c.d, FC), blk);
+    grd.z = (c.d.nx + CFL_PLANES - 1) / CFL_PLANES;
+    // partials of member m at m * bt.np (one per block)
     PLLC_L(c, "cfl", (k_cfl_partial<T><<<bgrid(grd, c), blk, 0, c.st>>>(c.d, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD],
                                                                         c.part, c.bt)));
     PLLC_L(c, "cfl", (k_cfl_final<T><<<c.bt.nm, 1024, 0, c.st>>>(c.part, (long)grd.x * grd.y * grd.z, c.ph.CFLmax,
@@ -3878,10 +3944,25 @@ void Ops<T>::bulk_stale(Ctx<T>& c, int slot, double alpha, bool advance_t, const
                                                                           qw, c.stale, c.bt)));
 }
 
+static inline int row_grid(long rows) { return (int)std::min((rows + 3) / 4, 8192L); }
+
 template <typename T>
-void Ops<T>::copy(Ctx<T>& c, const T* a, T* b, long n)
+void Ops<T>::copy(Ctx<T>& c, const T* a, T* b)
 {
-    PLLC_L(c, "copy", (k_copy<T><<<bulk_grid(n), 256, 0, c.st>>>(a, b, n)));
+    const long rows = (long)c.d.NX * c.d.NY;
+    PLLC_L(c, "copy", (k_copy<T><<<row_grid(rows), dim3(64, 4), 0, c.st>>>(c.d, a, b, rows)));
+}
+
+template <typename T>
+void Ops<T>::pack(Ctx<T>& c, const T* a, double* b, long rows)
+{
+    k_pack<T><<<row_grid(rows), dim3(64, 4), 0, c.st>>>(c.d, a, b, rows);
+}
+
+template <typename T>
+void Ops<T>::unpack(Ctx<T>& c, const double* a, T* b, long rows)
+{
+    k_unpack<T><<<row_grid(rows), dim3(64, 4), 0, c.st>>>(c.d, a, b, rows);
 }
 
 template <typename T>

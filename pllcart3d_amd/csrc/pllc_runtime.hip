@@ -284,9 +284,8 @@ bool pllc_ctx_tables(Ctx<T>& c, std::vector<void*>& owned, const char* where)
         const char* ls = getenv("PLLC_LINE_SOLVER");
         c.line_solver = (ls && strcmp(ls, "thomas") == 0) ? 1 : 0;
     }
-    // one partial per block of the CFL pass: its cell tiles are 64 x 4 or
-    // 128 x 2 (k, j), so ceil(nz/64) ceil(ny/2) nx bounds both
-    c.npart = (long)((d.nz + 63) / 64) * ((d.ny + 1) / 2) * d.nx + 64;
+    // one partial per block of the CFL pass (fewer than a block per row)
+    c.npart = (long)((d.nz + 127) / 128) * d.ny * d.nx + 64;
     c.npart = std::max(c.npart, (long)(2 * 1056 + 2 * (((long)d.ny * d.nz + 255) / 256) + 64));
     if (!get((void**)&c.part, (size_t)c.npart * 8)) return false;
     if (!get((void**)&c.lam_y, d.ny * ts) || !get((void**)&c.lam_z, d.nz * ts) || !get((void**)&c.lam00, 2 * 8))
@@ -413,6 +412,7 @@ struct pllc_sim {
     // momentum sweeps (Ctx::mom_fork; PLLC_FORK=0: one stream)
     hipStream_t side = nullptr;
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;
+    double* xfer = nullptr;       // one field in FP64, contiguous: uploads and downloads (stage())
 };
 
 static void apply_tuned(pllc_sim* s);
@@ -437,7 +437,21 @@ template <typename T> static Ctx<T>& ctx(pllc_sim* s);
 template <> Ctx<double>& ctx<double>(pllc_sim* s) { return s->cd; }
 template <> Ctx<float>& ctx<float>(pllc_sim* s) { return s->cf; }
 
+// points of a field (host arrays; the device fields are pitched)
 static size_t npts(const pllc_sim* s) { return (size_t)s->cd.d.NX * s->cd.d.NY * s->cd.d.NZ; }
+
+// a zeroed device allocation of one pitched field; the pointer returned is
+// its first point
+template <typename T>
+static T* field_alloc(pllc_sim* s, const Dims& d, const char* W)
+{
+    void* p = nullptr;
+    const size_t bytes = (field_values(d) + pitch_lead(sizeof(T)) + 1) * sizeof(T);
+    if (!pllc_hip_ok(W, hipMalloc(&p, bytes))) return nullptr;
+    s->owned.push_back(p);
+    if (!pllc_hip_ok(W, hipMemset(p, 0, bytes))) return nullptr;
+    return (T*)p + pitch_lead(sizeof(T));
+}
 
 void pllc_fill_dims(const pllc_params* p, Dims& d, Phys& ph)
 {
@@ -462,15 +476,10 @@ static bool create_t(pllc_sim* s)
     const char* W = "pllc_sim_create";
     std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
     pllc_fill_dims(&s->p, c.d, c.ph);
+    pitch_dims(c.d, sizeof(T));
     c.st = s->st;
-    const size_t n = npts(s);
-    for (int f = 0; f < NFIELDS; f++) {
-        void* p = nullptr;
-        if (!pllc_hip_ok(W, hipMalloc(&p, n * sizeof(T)))) return false;
-        s->owned.push_back(p);
-        if (!pllc_hip_ok(W, hipMemset(p, 0, n * sizeof(T)))) return false;
-        c.f[f] = (T*)p;
-    }
+    for (int f = 0; f < NFIELDS; f++)
+        if (!(c.f[f] = field_alloc<T>(s, c.d, W))) return false;
     return pllc_ctx_tables<T>(c, s->owned, W);
 }
 
@@ -559,9 +568,9 @@ static const int kPairs[12][2] = {{C_NEW, C_OLD}, {C_N, C_NM1}, {U_NEW, U_OLD}, 
 
 // update_old_*: copy new -> old over every point (3402-3452)
 template <typename T>
-static void update_old_copy(pllc_sim* s, Ctx<T>& c)
+static void update_old_copy(Ctx<T>& c)
 {
-    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[0]], c.f[pr[1]], (long)npts(s));
+    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[0]], c.f[pr[1]]);
 }
 
 // after fused steps the pairs are swapped (old holds the latest state);
@@ -570,31 +579,50 @@ template <typename T>
 static void normalize(pllc_sim* s, Ctx<T>& c)
 {
     if (!s->new_stale) return;
-    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[1]], c.f[pr[0]], (long)npts(s));
+    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[1]], c.f[pr[0]]);
     s->new_stale = false;
 }
 
-template <typename T>
-static bool h2d(pllc_sim* s, T* dst, const double* src, size_t n, const char* W)
+// Fields cross the boundary through a contiguous FP64 block on the device,
+// kept with the simulation: a kernel lays rows out (or gathers them) and
+// converts, and the copy is one piece between it and the caller's memory
+// (the host's element-by-element conversion of mixed fields took 8 ms per
+// 256x128x128 field, the kernel and the copy 0.9).
+static double* stage(pllc_sim* s, const char* W)
 {
-    std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-    if (sizeof(T) == 8) return pllc_hip_ok(W, hipMemcpy(dst, src, n * 8, hipMemcpyHostToDevice));
-    std::vector<T> t(n);
-    for (size_t e = 0; e < n; e++) t[e] = T(src[e]);
-    (void)s;
-    return pllc_hip_ok(W, hipMemcpy(dst, t.data(), n * sizeof(T), hipMemcpyHostToDevice));
+    if (!s->xfer) {
+        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
+        void* p = nullptr;
+        if (!pllc_hip_ok(W, hipMalloc(&p, npts(s) * 8))) return nullptr;
+        s->owned.push_back(p);
+        s->xfer = (double*)p;
+    }
+    return s->xfer;
+}
+
+// dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ values
+template <typename T>
+static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W)
+{
+    double* t = stage(s, W);
+    if (!t) return false;
+    {
+        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
+        if (!pllc_hip_ok(W, hipMemcpy(t, src, (size_t)rows * c.d.NZ * 8, hipMemcpyHostToDevice))) return false;
+    }
+    Ops<T>::unpack(c, t, dst + r0 * c.d.sy, rows);
+    return pllc_hip_ok(W, hipStreamSynchronize(s->st));
 }
 
 template <typename T>
-static bool d2h(pllc_sim* s, double* dst, const T* src, size_t n, const char* W)
+static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W)
 {
+    double* t = stage(s, W);
+    if (!t) return false;
+    Ops<T>::pack(c, src, t, (long)c.d.NX * c.d.NY);
     if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
     std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-    if (sizeof(T) == 8) return pllc_hip_ok(W, hipMemcpy(dst, src, n * 8, hipMemcpyDeviceToHost));
-    std::vector<T> t(n);
-    if (!pllc_hip_ok(W, hipMemcpy(t.data(), src, n * sizeof(T), hipMemcpyDeviceToHost))) return false;
-    for (size_t e = 0; e < n; e++) dst[e] = double(t[e]);
-    return true;
+    return pllc_hip_ok(W, hipMemcpy(dst, t, npts(s) * 8, hipMemcpyDeviceToHost));
 }
 
 template <typename T>
@@ -604,14 +632,14 @@ static int init_t(pllc_sim* s, Ctx<T>& c, const double* c_full)
     const Dims& d = c.d;
     const size_t n = npts(s);
     for (int f = 0; f < NFIELDS; f++)
-        if (!pllc_hip_ok(W, hipMemsetAsync(c.f[f], 0, n * sizeof(T), s->st))) return -1;
+        if (!pllc_hip_ok(W, hipMemsetAsync(c.f[f], 0, field_values(d) * sizeof(T), s->st))) return -1;
     if (finish(s, W)) return -1;
     s->new_stale = false;
     // initial_condition (493-526): c on every cell, Poiseuille inlet face
     std::vector<double> h(n);
     if (c_full) memcpy(h.data(), c_full, n * 8);
     else if (pllc_ic_fill(&s->p, PLLC_IC_ERF, 0, 0.0, h.data())) return -1;
-    if (!h2d<T>(s, c.f[C_NEW], h.data(), n, W)) return -1;
+    if (!h2d<T>(s, c, c.f[C_NEW], 0, (long)d.NX * d.NY, h.data(), W)) return -1;
     const Geo g = make_geo(&s->p);
     std::vector<double> plane((size_t)d.NY * d.NZ, 0.0);
     auto pl = [&](int j, int k) -> double& { return plane[(size_t)j * d.NZ + k]; };
@@ -621,15 +649,15 @@ static int init_t(pllc_sim* s, Ctx<T>& c, const double* c_full)
         pl(j, d.nz + 1) = pl(j, d.nz);
     }
     for (int k = 0; k <= d.nz + 1; k++) { pl(0, k) = -pl(1, k); pl(d.ny + 1, k) = -pl(d.ny, k); }
-    if (!h2d<T>(s, c.f[U_NEW] + IX(d, 3, 0, 0), plane.data(), plane.size(), W)) return -1;
+    if (!h2d<T>(s, c, c.f[U_NEW], 3L * d.NY, d.NY, plane.data(), W)) return -1;
     Ops<T>::velo_ghost(c);   // update_ghost_points (81); phi is 0
-    update_old_copy<T>(s, c);  // (82-83)
+    update_old_copy<T>(c);  // (82-83)
     if (s->p.Nmvp == 1) {
         // slope_parameter on c->new after the initial condition (133)
         int jj, kk;
         pllc_centre_line(g.Yc.data(), 1, d.ny, g.Zc.data(), 1, d.nz, &jj, &kk);
         std::vector<double> line(d.nx);
-        for (int i = 0; i < d.nx; i++) line[i] = h[(size_t)IX(d, 3 + i, jj, kk)];
+        for (int i = 0; i < d.nx; i++) line[i] = h[((size_t)(3 + i) * d.NY + jj) * d.NZ + kk];
         const double cm = pllc_slope_parameter(line.data(), d.nx, s->p.Vratio, s->p.Mum, s->p.Lambda);
         if (cm < 0) { pllc_set_error(W, "slope parameter did not converge in 500 iterations"); return -1; }
         s->cm = cm;
@@ -659,7 +687,7 @@ static int upload_t(pllc_sim* s, Ctx<T>& c, int field, const double* host)
 {
     normalize<T>(s, c);
     if (finish(s, "pllc_sim_upload")) return -1;
-    if (!h2d<T>(s, c.f[field], host, npts(s), "pllc_sim_upload")) return -1;
+    if (!h2d<T>(s, c, c.f[field], 0, (long)c.d.NX * c.d.NY, host, "pllc_sim_upload")) return -1;
     // old and new may now differ where a step never writes: the next
     // substage copies (as update_old_* does) instead of swapping
     s->copy_next = true;
@@ -670,7 +698,7 @@ template <typename T>
 static int download_t(pllc_sim* s, Ctx<T>& c, int field, double* host)
 {
     normalize<T>(s, c);
-    return d2h<T>(s, host, c.f[field], npts(s), "pllc_sim_download") ? 0 : -1;
+    return d2h<T>(s, c, host, c.f[field], "pllc_sim_download") ? 0 : -1;
 }
 
 extern "C" int pllc_sim_upload(pllc_sim* s, int field, const double* host)
@@ -723,7 +751,7 @@ static double op_t(pllc_sim* s, Ctx<T>& c, int op, double dt, int rk, double vbu
     case PLLC_OP_PHI_GHOSTS: Ops<T>::phi_ghost(c); break;
     case PLLC_OP_VELO_CORRECTION: Ops<T>::velo_correction(c, g, r, rk); break;
     case PLLC_OP_PRESSURE_GRADIENT: Ops<T>::pressure_gradient(c, g, r, 7); break;
-    case PLLC_OP_UPDATE_OLD: update_old_copy<T>(s, c); break;
+    case PLLC_OP_UPDATE_OLD: update_old_copy<T>(c); break;
     case PLLC_OP_BULK_VELO:
         Ops<T>::bulk(c, rk, 0.0, false);
         return read_scalar(s, c.scal + S_RK + 4 * rk);
@@ -826,7 +854,7 @@ static void fused_step(pllc_sim* s, Ctx<T>& c)
         // velo_correction + pressure_gradient + update_veloghost_points
         Ops<T>::correction_and_gradient(c, g, r, rk, true);
         if (s->copy_next) {
-            update_old_copy<T>(s, c);
+            update_old_copy<T>(c);
             s->copy_next = false;
             s->new_stale = false;
         } else {
@@ -978,11 +1006,7 @@ static int set_closure_t(pllc_sim* s, Ctx<T>& c, pllc_cnn* m, int every)
         return -1;
     }
     if (!c.ncorr) {
-        void* p = nullptr;
-        if (!pllc_hip_ok(W, hipMalloc(&p, npts(s) * sizeof(T)))) return -1;
-        s->owned.push_back(p);
-        if (!pllc_hip_ok(W, hipMemset(p, 0, npts(s) * sizeof(T)))) return -1;
-        c.ncorr = (T*)p;
+        if (!(c.ncorr = field_alloc<T>(s, c.d, W))) return -1;
     }
     if (every < 0) {
         pllc_set_error(W, "negative refresh period");
@@ -1004,7 +1028,7 @@ static int run_guarded_t(pllc_sim* s, Ctx<T>& c, int nsteps, int check_every, do
                          int* fallbacks, double* worst)
 {
     const char* W = "pllc_sim_run_guarded";
-    const size_t n = npts(s);
+    const size_t n = field_values(c.d);
     if (s->snap.empty()) {
         for (int f = 0; f < NSTATE + 1; f++) {
             void* p = nullptr;
@@ -1212,7 +1236,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     b->m = ms;
     const int nm = (int)ms.size();
     const Ctx<float>& c0 = ms[0]->cf;
-    const long fs = (long)npts(ms[0]);
+    const long fs = field_values(c0.d), lead = pitch_lead(4);
     const long pk = (long)c0.d.nx * c0.d.ny * c0.d.nz;
     const long np = c0.npart;
     auto get = [&](size_t bytes) -> void* {
@@ -1225,7 +1249,11 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     b->c = c0;
     bool ok = pllc_hip_ok(W, hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking)) &&
               pllc_hip_ok(W, hipEventCreateWithFlags(&b->ev, hipEventDisableTiming));
-    for (int f = 0; ok && f < NFIELDS; f++) ok = (b->c.f[f] = (float*)get((size_t)nm * fs * 4)) != nullptr;
+    for (int f = 0; ok && f < NFIELDS; f++) {
+        float* q = (float*)get(((size_t)nm * fs + lead + 1) * 4);
+        ok = q != nullptr;
+        b->c.f[f] = q + (ok ? lead : 0);
+    }
     ok = ok && (b->c.P = (float*)get((size_t)nm * pk * 4)) && (b->c.Q = (float*)get((size_t)nm * pk * 4)) &&
          (b->c.scal = (double*)get((size_t)nm * S_SIZE * 8)) && (b->c.part = (double*)get((size_t)nm * np * 8)) &&
          (b->c.tval = (double*)get((size_t)nm * 8)) && (b->c.stale = (float*)get((size_t)nm * 16 * 4)) &&
