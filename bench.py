@@ -25,7 +25,7 @@ HBM_PEAK_GBS = 8000.0
 # and the A(mu) coefficients count as recomputed from c, scratch round trips
 # of the line solvers do not count).
 TOUCHES = {
-    "rhs_c": 7, "rhs_u": 8, "rhs_v": 8, "rhs_w": 8,
+    "rhs_c": 7, "rhs_u": 8, "rhs_v": 8, "rhs_w": 8, "rhs_uvw": 24, "rhs_cuvw": 31,   # the last two: joint launches
     "sweep_y": None, "sweep_z": None, "sweep_x": None,   # per-field, see below
     "div": 4, "velo_corr": 7, "pg": 8, "corr_pg": 14, "cfl": 1.5, "visc": 5,
 }
@@ -150,7 +150,8 @@ PEAK_TFLOPS = {8.0: 78.6, 4.0: 157.3}
 PROFILES = os.path.join(ROOT, "profiles")
 CLASS_KERNELS = {
     "sweep_x": ["k_sweep_part<{T}, 0>"], "sweep_y": ["k_sweep_part<{T}, 1>"],
-    "sweep_z": ["k_sweep_part_z<{T}>", "k_sweep_part_zt<{T}>"], "corr_pg": ["k_corr_pg<{T}, false>"],
+    "sweep_z": ["k_sweep_wave_z<{T}>", "k_sweep_part_z<{T}>", "k_sweep_part_zt<{T}>"], "corr_pg": ["k_corr_pg<{T}, false>"],
+    "rhs_cuvw": ["k_rhs<{T}, true, false>"],
     "rhs_c": ["k_rhs_c<{T}, true, false>"], "rhs_u": ["k_rhs_mom<{T}, 1, true, false>"],
     "rhs_v": ["k_rhs_mom<{T}, 2, true, false>"], "rhs_w": ["k_rhs_mom<{T}, 3, true, false>"],
     "div": ["k_div<{T}, false>"], "visc": ["k_visc<{T}, false>"],

@@ -121,92 +121,207 @@ __device__ __forceinline__ int2 xcd_tile()
     return make_int2(r % gx, r / gx);
 }
 
-// concentration's explicit part: Hc_op (1539-1644) and the source loop
-// (573-590).  One thread per interior cell.
-template <typename T, bool FAST, bool B = false>
-__global__ __launch_bounds__(256) void k_rhs_c(Dims d, Phys ph0, const T* __restrict__ cold, const T* __restrict__ un,
-                                               const T* __restrict__ vn, const T* __restrict__ wn,
-                                               const T* __restrict__ Nm1, T* __restrict__ N, T* __restrict__ S,
-                                               const T* __restrict__ stale0, const T* __restrict__ ncorr,
-                                               const double* __restrict__ scal0, T g, T r, Bt bt)
+// The field value uo values after p at the lane's byte offset v: p + uo is
+// uniform over the block and stays in scalar registers, v is the one vector
+// register all loads of a thread share.  (A plane of 2^32 bytes would need
+// fields larger than the device's memory.)
+template <typename T>
+__device__ __forceinline__ const T& lane_at(const T* __restrict__ p, long uo, unsigned v)
 {
-    const int2 tl = xcd_tile();
-    const int k = tl.x * blockDim.x + threadIdx.x + 1;
-    const int j = tl.y * blockDim.y + threadIdx.y + 1;
-    int il;
-    const int m = bt_member(bt, blockIdx.z, gridDim.z, il);
-    const int i = il + 3;
-    if (k > d.nz || j > d.ny) return;
-    const Phys& ph = bt_phys<B>(bt, ph0, m);
-    const double* __restrict__ scal = scal0 + m * S_SIZE;
-    const T* __restrict__ stale = stale0 + m * 16;
-    const Rng R = field_rng(d, FC);
-    // every field of member m at the same offset
-    const long o = IX(d, i, j, k) + m * bt.fs, sx = d.sx, sy = d.sy;
-    const T dt = T(scal[S_DT]);
-
-    // every operand first (one memory round trip), then the arithmetic
-    T cx7[7], cy7[7], cz7[7];
-#pragma unroll
-    for (int m = 0; m < 7; m++) {
-        cx7[m] = cold[o + (long)(m - 3) * sx];
-        cy7[m] = m == 3 ? T(0) : cold[o + (long)(m - 3) * sy];
-        cz7[m] = m == 3 ? T(0) : cold[o + m - 3];
-    }
-    cy7[3] = cx7[3];
-    cz7[3] = cx7[3];
-    const T u0 = un[o], u1 = un[o + sx], v0 = vn[o], v1 = vn[o + sy], w0 = wn[o], w1 = wn[o + 1];
-    // r = 0 (first substage): r N_nm1 is a signed zero, so N_nm1 is not read
-    // (the source keeps its value; at most the sign of a zero source differs)
-    const T nm1 = r != T(0) ? Nm1[o] : T(0);
-
-    const T uval = T(0.5) * (u1 + u0), vval = T(0.5) * (v1 + v0), wval = T(0.5) * (w1 + w0);
-    T nval, diff;
-    if constexpr (FAST) {
-        T xm, xp, ym, yp, zm, zp;
-        const T cx = upwind_term<T>(cx7, i, R.is, R.ie, uval, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
-        const T cy = upwind_term<T>(cy7, j, R.js, R.je, vval, T(d.dy), T(d.rdy), stale[0], stale[1], ym, yp);
-        const T cz = upwind_term<T>(cz7, k, R.ks, R.ke, wval, T(d.dz), T(d.rdz), stale[2], stale[3], zm, zp);
-        nval = -(cz + cx + cy);
-        diff = T(ph.kap[FC][0]) * (xp - xm);
-        diff = fma(T(ph.kap[FC][1]), yp - ym, diff);
-        diff = fma(T(ph.kap[FC][2]), zp - zm, diff);
-    } else {
-        T D[6];
-#pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(cx7[m + 1] - cx7[m], T(d.dx), d.rdx);
-        const T convx = uval * upwind_d<T>(D, i, R.is, R.ie, uval >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
-#pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(cy7[m + 1] - cy7[m], T(d.dy), d.rdy);
-        const T convy = vval * upwind_d<T>(D, j, R.js, R.je, vval >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
-#pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(cz7[m + 1] - cz7[m], T(d.dz), d.rdz);
-        const T czd = upwind_d<T>(D, k, R.ks, R.ke, wval >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
-        nval = -(wval * czd + convx + convy);
-        T ax, bx, cx, ay, by, cy, az, bz, cz;
-        Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
-        coefs<T, FC, 0>(d, ph, none, o, ax, bx, cx);
-        coefs<T, FC, 1>(d, ph, none, o, ay, by, cy);
-        coefs<T, FC, 2>(d, ph, none, o, az, bz, cz);
-        const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
-        const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
-        const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
-        diff = axx + axy + axz;
-    }
-    // the learned closure's correction of N (no counterpart in the
-    // reference; ncorr is null without a closure)
-    if (ncorr) nval += ncorr[o];
-    N[o] = nval;
-    const T conv = (g * nval + r * nm1);
-    S[o] = dt * (conv + (g + r) * diff);
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + uo) + v);
+}
+template <typename T>
+__device__ __forceinline__ T& lane_at(T* __restrict__ p, long uo, unsigned v)
+{
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(p + uo) + v);
 }
 
-// xmom/ymom/zmom explicit part at one point of component F's range: H?_op
-// with mu_old, then the source loop with A(mu_old) and the body force
-// (970-989, 1127-1146, 1280-1298).  u, v, w are the old velocities; q is the
-// component's own old field.  Every operand of the point is loaded first,
-// so the point's 37 loads are in flight together; the arithmetic below
-// then follows the reference's expressions in its order.
+// The lane offset anew in a loop's block: its widening to 64 bits then stays
+// beside the loads and stores, which take the 32-bit register as it is
+// (widened once before the loop it costs an addition per access).
+__device__ __forceinline__ void per_block(unsigned& v, long& o) { asm("" : "+v"(v), "+s"(o)); }
+
+// Consecutive points in k that a thread of the explicit kernels takes: an
+// 8-byte load of a wave occupies the L1's address unit for 17 cycles, a
+// 16-byte load (any 8-byte alignment) for the same 17, a 4-byte load for 5
+// (measured, all L1 hits), so FP64 threads take two points and FP32 threads
+// one.
+template <typename T> struct KP { static constexpr int value = sizeof(T) == 8 ? 2 : 1; };
+
+// n consecutive values at the lane's address, in 16-byte pieces in FP64
+typedef double dpair __attribute__((ext_vector_type(2), aligned(8)));
+template <int n>
+__device__ __forceinline__ void lane_run(const double* __restrict__ p, long uo, unsigned v, double (&a)[n])
+{
+#pragma unroll
+    for (int t = 0; t + 1 < n; t += 2) {
+        const dpair x = *reinterpret_cast<const dpair*>(&lane_at(p, uo + t, v));
+        a[t] = x.x;
+        a[t + 1] = x.y;
+    }
+    if (n & 1) a[n - 1] = lane_at(p, uo + n - 1, v);
+}
+template <int n>
+__device__ __forceinline__ void lane_run(const float* __restrict__ p, long uo, unsigned v, float (&a)[n])
+{
+#pragma unroll
+    for (int t = 0; t < n; t++) a[t] = lane_at(p, uo + t, v);
+}
+// the lane's values of k .. k + KP - 1 that lie in ks .. ke to the field
+__device__ __forceinline__ void lane_put(double* __restrict__ p, long uo, unsigned v, const double (&a)[2], int k,
+                                         int ks, int ke)
+{
+    if (k >= ks && k < ke) {
+        dpair x;
+        x.x = a[0];
+        x.y = a[1];
+        *reinterpret_cast<dpair*>(&lane_at(p, uo, v)) = x;
+    } else {
+        if (k >= ks && k <= ke) lane_at(p, uo, v) = a[0];
+        if (k + 1 >= ks && k + 1 <= ke) lane_at(p, uo + 1, v) = a[1];
+    }
+}
+__device__ __forceinline__ void lane_put(float* __restrict__ p, long uo, unsigned v, const float (&a)[1], int, int, int)
+{
+    lane_at(p, uo, v) = a[0];
+}
+
+// the seven values around each of a thread's points: along x from the planes
+// it carries, along y from the rows around it, along z from its own run of
+// KP + 6 values
+template <typename T>
+struct Cross {
+    static constexpr int K = KP<T>::value;
+    T x[7][K], y[7][K], lo[3], hi[3];
+    // the planes i - 3 .. i + 2 as if i - 1 had been done
+    __device__ __forceinline__ void start(const T* __restrict__ q, long o, unsigned v, long sx)
+    {
+#pragma unroll
+        for (int m = 1; m < 7; m++) lane_run(q, o + (long)(m - 4) * sx, v, x[m]);
+    }
+    // to plane i at o
+    __device__ __forceinline__ void next(const T* __restrict__ q, long o, unsigned v, long sx, long sy)
+    {
+#pragma unroll
+        for (int m = 0; m < 6; m++)
+#pragma unroll
+            for (int p = 0; p < K; p++) x[m][p] = x[m + 1][p];
+        lane_run(q, o + 3 * sx, v, x[6]);
+#pragma unroll
+        for (int m = 0; m < 7; m++)
+            if (m != 3) lane_run(q, o + (long)(m - 3) * sy, v, y[m]);
+        lane_run(q, o - 3, v, lo);
+        lane_run(q, o + K, v, hi);
+    }
+    // the stencils of point p
+    __device__ __forceinline__ void at(int p, T (&sx7)[7], T (&sy7)[7], T (&sz7)[7]) const
+    {
+#pragma unroll
+        for (int m = 0; m < 7; m++) {
+            sx7[m] = x[m][p];
+            sy7[m] = m == 3 ? x[3][p] : y[m][p];
+            const int t = p + m;   // of the run k - 3 .. k + K + 2
+            sz7[m] = t < 3 ? lo[t] : t < 3 + K ? x[3][t - 3] : hi[t - 3 - K];
+        }
+    }
+};
+
+// concentration's explicit part at the points i .. ie of one j and KP
+// consecutive k: Hc_op (1539-1644) and the source loop (573-590).  From plane
+// to plane the x stencil and the upper face's u stay in registers.
+template <typename T, bool FAST>
+__device__ __forceinline__ void rhs_conc_line(const Dims& d, const Phys& ph, const Rng& R, int i, int ie, int j, int k0,
+                                              long mo, const T* __restrict__ cold, const T* __restrict__ un,
+                                              const T* __restrict__ vn, const T* __restrict__ wn,
+                                              const T* __restrict__ Nm1, T* __restrict__ N, T* __restrict__ S,
+                                              const T* __restrict__ stale, const T* __restrict__ ncorr, T dt, T g, T r)
+{
+    constexpr int K = KP<T>::value;
+    const long sx = d.sx, sy = d.sy;
+    const T ylo = stale[0], yhi = stale[1], zlo = stale[2], zhi = stale[3];
+    const T kx = T(ph.kap[FC][0]), ky = T(ph.kap[FC][1]), kz = T(ph.kap[FC][2]);
+    unsigned l = (unsigned)((j * d.sy + k0) * sizeof(T));
+    long o = (long)i * sx + mo;   // uniform; the lane's own offset is l
+    Cross<T> st;
+    T u1[K];
+    st.start(cold, o, l, sx);
+    lane_run(un, o, l, u1);
+#pragma unroll 1
+    for (; i <= ie; i++, o += sx) {
+        per_block(l, o);
+        // every operand first (one memory round trip), then the arithmetic
+        T u0[K], v0[K], v1[K], w[K + 1], nm1[K], nc[K], nv[K], sv[K];
+        st.next(cold, o, l, sx, sy);
+#pragma unroll
+        for (int p = 0; p < K; p++) u0[p] = u1[p];
+        lane_run(un, o + sx, l, u1);
+        lane_run(vn, o, l, v0);
+        lane_run(vn, o + sy, l, v1);
+        lane_run(wn, o, l, w);
+        // r = 0 (first substage): r N_nm1 is a signed zero, so N_nm1 is not read
+        // (the source keeps its value; at most the sign of a zero source differs)
+        if (r != T(0)) lane_run(Nm1, o, l, nm1);
+        // the learned closure's correction of N (no counterpart in the
+        // reference; ncorr is null without a closure)
+        if (ncorr) lane_run(ncorr, o, l, nc);
+#pragma unroll
+        for (int p = 0; p < K; p++) {
+            const int k = k0 + p;
+            T cx7[7], cy7[7], cz7[7];
+            st.at(p, cx7, cy7, cz7);
+            const T uval = T(0.5) * (u1[p] + u0[p]), vval = T(0.5) * (v1[p] + v0[p]), wval = T(0.5) * (w[p + 1] + w[p]);
+            T nval, diff;
+            if constexpr (FAST) {
+                T xm, xp, ym, yp, zm, zp;
+                const T cx = upwind_term<T>(cx7, i, R.is, R.ie, uval, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
+                const T cy = upwind_term<T>(cy7, j, R.js, R.je, vval, T(d.dy), T(d.rdy), ylo, yhi, ym, yp);
+                const T cz = upwind_term<T>(cz7, k, R.ks, R.ke, wval, T(d.dz), T(d.rdz), zlo, zhi, zm, zp);
+                nval = -(cz + cx + cy);
+                diff = kx * (xp - xm);
+                diff = fma(ky, yp - ym, diff);
+                diff = fma(kz, zp - zm, diff);
+            } else {
+                T D[6];
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(cx7[m + 1] - cx7[m], T(d.dx), d.rdx);
+                const T convx =
+                    uval * upwind_d<T>(D, i, R.is, R.ie, uval >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(cy7[m + 1] - cy7[m], T(d.dy), d.rdy);
+                const T convy = vval * upwind_d<T>(D, j, R.js, R.je, vval >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, ylo, yhi);
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(cz7[m + 1] - cz7[m], T(d.dz), d.rdz);
+                const T czd = upwind_d<T>(D, k, R.ks, R.ke, wval >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, zlo, zhi);
+                nval = -(wval * czd + convx + convy);
+                T ax, bx, cx, ay, by, cy, az, bz, cz;
+                Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
+                coefs<T, FC, 0>(d, ph, none, 0, ax, bx, cx);
+                coefs<T, FC, 1>(d, ph, none, 0, ay, by, cy);
+                coefs<T, FC, 2>(d, ph, none, 0, az, bz, cz);
+                const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
+                const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
+                const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
+                diff = axx + axy + axz;
+            }
+            if (ncorr) nval += nc[p];
+            nv[p] = nval;
+            const T conv = (g * nval + r * (r != T(0) ? nm1[p] : T(0)));
+            sv[p] = dt * (conv + (g + r) * diff);
+        }
+        per_block(l, o);
+        lane_put(N, o, l, nv, k0, R.ks, R.ke);
+        lane_put(S, o, l, sv, k0, R.ks, R.ke);
+    }
+}
+
+// xmom/ymom/zmom explicit part at the points i .. ie of one (j, k) of
+// component F's range: H?_op with mu_old, then the source loop with A(mu_old)
+// and the body force (970-989, 1127-1146, 1280-1298).  u, v, w are the old
+// velocities; q is the component's own old field.  From plane to plane the x
+// stencil, the other components' values and the viscosities that the next
+// plane needs again stay in registers: 24 loads a point instead of 37.  Every
+// operand of the point is loaded first, so its loads are in flight together;
+// the arithmetic below then follows the reference's expressions in its order.
 //
 // Operands, by component (the "first" and "second" other components):
 //   advecting velocity in direction D (1669/1696/1722, 1780/1807/1834,
@@ -230,141 +345,257 @@ __device__ __forceinline__ void coef_vals(const Dims& d, const Phys& ph, int D, 
 }
 
 template <typename T, int F, bool FAST>
-__device__ __forceinline__ void rhs_mom_point(const Dims& d, const Phys& ph, const Rng& R, int i, int j, int k,
-                                              const T* __restrict__ u, const T* __restrict__ v,
-                                              const T* __restrict__ w, const Visc4<T>& mu, const T* __restrict__ cn,
-                                              const T* __restrict__ pg, const T* __restrict__ Nm1,
-                                              T* __restrict__ N, T* __restrict__ S, const T* __restrict__ stale,
-                                              T dt, T g, T r)
+__device__ __forceinline__ void rhs_mom_line(const Dims& d, const Phys& ph, const Rng& R, int i, int ie, int j, int k0,
+                                             long mo, const T* __restrict__ u, const T* __restrict__ v,
+                                             const T* __restrict__ w, const Visc4<T>& mu, const T* __restrict__ cn,
+                                             const T* __restrict__ pg, const T* __restrict__ Nm1,
+                                             T* __restrict__ N, T* __restrict__ S, const T* __restrict__ stale,
+                                             T dt, T g, T r)
 {
+    constexpr int K = KP<T>::value;
     const long sx = d.sx, sy = d.sy;
-    const long o = IX(d, i, j, k);
     const long sF = F == FU ? sx : F == FV ? sy : 1;
     const T* __restrict__ q = F == FU ? u : F == FV ? v : w;
     const T* __restrict__ pa = F == FU ? v : u;   // first other component
     const T* __restrict__ pb = F == FW ? v : w;   // second other component
-    const T* __restrict__ mA = F == FU ? mu.xy : F == FV ? mu.xy : mu.xz;
+    const T* __restrict__ mA = F == FW ? mu.xz : mu.xy;
     const T* __restrict__ mB = F == FU ? mu.xz : mu.yz;
-    const long sA = F == FU ? sy : sx;            // stride of mA's second value
-    const long sB = F == FW ? sy : 1;
-    // offsets of the 4-point averages, in the reference's summation order
-    long ao[4], bo[4];
-    if (F == FU) {
-        ao[0] = -sx; ao[1] = 0; ao[2] = sy; ao[3] = -sx + sy;
-        bo[0] = -sx; bo[1] = 0; bo[2] = 1; bo[3] = -sx + 1;
-    } else if (F == FV) {
-        ao[0] = -sy; ao[1] = sx - sy; ao[2] = 0; ao[3] = sx;
-        bo[0] = -sy; bo[1] = -sy + 1; bo[2] = 0; bo[3] = 1;
-    } else {
-        ao[0] = -1; ao[1] = sx - 1; ao[2] = 0; ao[3] = sx;
-        bo[0] = -1; bo[1] = 0; bo[2] = sy - 1; bo[3] = sy;
-    }
-
-    T qx[7], qy[7], qz[7], av[4], bv[4];
-#pragma unroll
-    for (int m = 0; m < 7; m++) {
-        qx[m] = q[o + (long)(m - 3) * sx];
-        qy[m] = m == 3 ? T(0) : q[o + (long)(m - 3) * sy];
-        qz[m] = m == 3 ? T(0) : q[o + m - 3];
-    }
-    qy[3] = qx[3];
-    qz[3] = qx[3];
-#pragma unroll
-    for (int m = 0; m < 4; m++) { av[m] = pa[o + ao[m]]; bv[m] = pb[o + bo[m]]; }
-    const T mc0 = mu.cell[o - sF], mc1 = mu.cell[o];
-    const T ma0 = mA[o], ma1 = mA[o + sA], mb0 = mB[o], mb1 = mB[o + sB];
+    unsigned l = (unsigned)((j * d.sy + k0) * sizeof(T));
+    const T ylo = stale[0], yhi = stale[1], zlo = stale[2], zhi = stale[3];
+    const T kx = T(ph.kap[F][0]), ky = T(ph.kap[F][1]), kz = T(ph.kap[F][2]);
+    const T e0 = T(ph.edel[F - FU][0]), e1 = T(ph.edel[F - FU][1]), rRe = T(ph.rRe);
     // c enters only the body force fre (c) of u and v; with fre = 0 that
     // term is a signed zero and the source the same bits without it, so c
     // is not read (the flag is uniform over the launch)
     const bool force = F != FW && ph.fre[F == FU ? 0 : 1] != 0.0;
-    const T cn0 = force ? cn[o] : T(0), cn1 = force ? cn[o - sF] : T(0);
-    const T pgv = pg[o], nm1 = r != T(0) ? Nm1[o] : T(0);   // as in k_rhs_c
+    const T fre = force ? T(ph.fre[F == FU ? 0 : 1]) : T(0);
 
-    const T alpha = g + r;
-    const T vx = F == FU ? qx[3] : T(0.25) * (av[0] + av[1] + av[2] + av[3]);
-    const T vy = F == FV ? qy[3] : F == FU ? T(0.25) * (av[0] + av[1] + av[2] + av[3])
-                                           : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
-    const T vz = F == FW ? qz[3] : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
-    const int fi = F - FU;
-    // the cross-viscous differences at the upper and lower edges
-    const T a1 = F == FU ? av[2] - av[3] : av[3] - av[1];
-    const T a0 = F == FU ? av[1] - av[0] : av[2] - av[0];
-    const T b1 = F == FU ? bv[2] - bv[3] : F == FV ? bv[3] - bv[1] : bv[3] - bv[2];
-    const T b0 = F == FV ? bv[2] - bv[0] : bv[1] - bv[0];
-    // mu below and above the point along x, y and z
-    const T mx0 = F == FU ? mc0 : ma0, mx1 = F == FU ? mc1 : ma1;
-    const T my0 = F == FU ? ma0 : F == FV ? mc0 : mb0, my1 = F == FU ? ma1 : F == FV ? mc1 : mb1;
-    const T mz0 = F == FW ? mc0 : mb0, mz1 = F == FW ? mc1 : mb1;
-    const T Re = T(ph.Re);
-    if constexpr (FAST) {
-        T xm, xp, ym, yp, zm, zp;
-        const T cx = upwind_term<T>(qx, i, R.is, R.ie, vx, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
-        const T cy = upwind_term<T>(qy, j, R.js, R.je, vy, T(d.dy), T(d.rdy), stale[0], stale[1], ym, yp);
-        const T cz = upwind_term<T>(qz, k, R.ks, R.ke, vz, T(d.dz), T(d.rdz), stale[2], stale[3], zm, zp);
-        T nval = fma(T(ph.edel[fi][0]), fma(ma1, a1, -(ma0 * a0)), -(cz + cx + cy));
-        nval = fma(T(ph.edel[fi][1]), fma(mb1, b1, -(mb0 * b0)), nval);
-        N[o] = nval;
-        T visc = T(ph.kap[F][0]) * fma(mx1, xp, -(mx0 * xm));
-        visc = fma(T(ph.kap[F][1]), fma(my1, yp, -(my0 * ym)), visc);
-        visc = fma(T(ph.kap[F][2]), fma(mz1, zp, -(mz0 * zm)), visc);
-        visc = fma(-T(ph.rRe), pgv, visc);
-        if (force) visc = fma(-T(ph.fre[fi]), T(0.5) * (cn0 + cn1), visc);
-        S[o] = dt * fma(alpha, visc, fma(g, nval, r * nm1));
+    long o = (long)i * sx + mo;   // uniform; the lane's own offset is l
+    // Carried along x (as the plane before i would leave them): the stencil;
+    // u: v at (j), (j + 1), w at k .. k + K and mu.cell of plane i - 1;
+    // v: u at (j - 1), (j) of plane i and mu.xy; w: u at k - 1 .. k + K - 1
+    // of plane i and mu.xz.
+    Cross<T> st;
+    T a1v[K], a2v[K], bw[K + 1], mc[K], ma[K], aw[K + 1];
+    st.start(q, o, l, sx);
+    if (F == FU) {
+        lane_run(pa, o - sx, l, a1v);
+        lane_run(pa, o - sx + sy, l, a2v);
+        lane_run(pb, o - sx, l, bw);
+        lane_run(mu.cell, o - sx, l, mc);
+    } else if (F == FV) {
+        lane_run(pa, o - sy, l, a1v);
+        lane_run(pa, o, l, a2v);
+        lane_run(mA, o, l, ma);
     } else {
-        // convec_term: upwind derivatives along x, y, z
-        T D[6];
+        lane_run(pa, o - 1, l, aw);
+        lane_run(mA, o, l, ma);
+    }
+#pragma unroll 1
+    for (; i <= ie; i++, o += sx) {
+        per_block(l, o);
+        st.next(q, o, l, sx, sy);
+        // the 4-point averages' values and the viscosities of every point, in
+        // the reference's order of summation
+        T av4[K][4], bv4[K][4], mcs[K][2], mas[K][2], mbs[K][2];
+        if (F == FU) {
+            // a: -sx, 0, sy, -sx + sy; b: -sx, 0, 1, -sx + 1
+            T n1[K], n2[K], nw[K + 1], nc[K], x1[K], x2[K], zw[K + 1];
+            lane_run(pa, o, l, n1);
+            lane_run(pa, o + sy, l, n2);
+            lane_run(pb, o, l, nw);
+            lane_run(mu.cell, o, l, nc);
+            lane_run(mA, o, l, x1);
+            lane_run(mA, o + sy, l, x2);
+            lane_run(mB, o, l, zw);
 #pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(qx[m + 1] - qx[m], T(d.dx), d.rdx);
-        const T convx = vx * upwind_d<T>(D, i, R.is, R.ie, vx >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
+            for (int p = 0; p < K; p++) {
+                av4[p][0] = a1v[p]; av4[p][1] = n1[p]; av4[p][2] = n2[p]; av4[p][3] = a2v[p];
+                bv4[p][0] = bw[p]; bv4[p][1] = nw[p]; bv4[p][2] = nw[p + 1]; bv4[p][3] = bw[p + 1];
+                mcs[p][0] = mc[p]; mcs[p][1] = nc[p];
+                mas[p][0] = x1[p]; mas[p][1] = x2[p];
+                mbs[p][0] = zw[p]; mbs[p][1] = zw[p + 1];
+            }
 #pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(qy[m + 1] - qy[m], T(d.dy), d.rdy);
-        const T convy = vy * upwind_d<T>(D, j, R.js, R.je, vy >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, stale[0], stale[1]);
+            for (int p = 0; p < K; p++) { a1v[p] = n1[p]; a2v[p] = n2[p]; mc[p] = nc[p]; }
 #pragma unroll
-        for (int m = 0; m < 6; m++) D[m] = divh<T>(qz[m + 1] - qz[m], T(d.dz), d.rdz);
-        const T dzd = upwind_d<T>(D, k, R.ks, R.ke, vz >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, stale[2], stale[3]);
-        const T ct = vz * dzd + convx + convy;
-        // explicit_n: -convec_term + the cross-viscous terms, left to right
-        const T p1 = T(ph.edel[fi][0]) * ma1 * a1, m1 = T(ph.edel[fi][0]) * ma0 * a0;
-        const T p2 = T(ph.edel[fi][1]) * mb1 * b1, m2 = T(ph.edel[fi][1]) * mb0 * b0;
-        const T nval = -ct + p1 - m1 + p2 - m2;
-        N[o] = nval;
-        // source: dt [g N + r N_nm1 + alpha A(mu_old) q + alpha (body force)]
-        T ax, bx, cx, ay, by, cy, az, bz, cz;
-        coef_vals<T, F>(d, ph, 0, mx0, mx1, ax, bx, cx);
-        coef_vals<T, F>(d, ph, 1, my0, my1, ay, by, cy);
-        coef_vals<T, F>(d, ph, 2, mz0, mz1, az, bz, cz);
-        const T conv = (g * nval + r * nm1);
-        const T axx = ax * qx[2] + bx * qx[3] + cx * qx[4];
-        const T axy = ay * qy[2] + by * qy[3] + cy * qy[4];
-        const T axz = az * qz[2] + bz * qz[3] + cz * qz[4];
-        const T visc = alpha * (axx + axy + axz);
-        T bodyforce;
-        if (!force) bodyforce = alpha * (-divh<T>(pgv, Re, ph.rRe));
-        else bodyforce = alpha * (-T(ph.fre[fi]) * (T(0.5) * (cn0 + cn1)) - divh<T>(pgv, Re, ph.rRe));
-        S[o] = dt * (conv + visc + bodyforce);
+            for (int p = 0; p <= K; p++) bw[p] = nw[p];
+        } else if (F == FV) {
+            // a: -sy, sx - sy, 0, sx; b: -sy, -sy + 1, 0, 1
+            T n1[K], n2[K], w0[K + 1], w1[K + 1], c0[K], c1[K], na[K], zw[K + 1];
+            lane_run(pa, o + sx - sy, l, n1);
+            lane_run(pa, o + sx, l, n2);
+            lane_run(pb, o - sy, l, w0);
+            lane_run(pb, o, l, w1);
+            lane_run(mu.cell, o - sy, l, c0);
+            lane_run(mu.cell, o, l, c1);
+            lane_run(mA, o + sx, l, na);
+            lane_run(mB, o, l, zw);
+#pragma unroll
+            for (int p = 0; p < K; p++) {
+                av4[p][0] = a1v[p]; av4[p][1] = n1[p]; av4[p][2] = a2v[p]; av4[p][3] = n2[p];
+                bv4[p][0] = w0[p]; bv4[p][1] = w0[p + 1]; bv4[p][2] = w1[p]; bv4[p][3] = w1[p + 1];
+                mcs[p][0] = c0[p]; mcs[p][1] = c1[p];
+                mas[p][0] = ma[p]; mas[p][1] = na[p];
+                mbs[p][0] = zw[p]; mbs[p][1] = zw[p + 1];
+            }
+#pragma unroll
+            for (int p = 0; p < K; p++) { a1v[p] = n1[p]; a2v[p] = n2[p]; ma[p] = na[p]; }
+        } else {
+            // a: -1, sx - 1, 0, sx; b: -1, 0, sy - 1, sy
+            T nw[K + 1], v0[K + 1], v1[K + 1], cw[K + 1], na[K], y0[K], y1[K];
+            lane_run(pa, o + sx - 1, l, nw);
+            lane_run(pb, o - 1, l, v0);
+            lane_run(pb, o + sy - 1, l, v1);
+            lane_run(mu.cell, o - 1, l, cw);
+            lane_run(mA, o + sx, l, na);
+            lane_run(mB, o, l, y0);
+            lane_run(mB, o + sy, l, y1);
+#pragma unroll
+            for (int p = 0; p < K; p++) {
+                av4[p][0] = aw[p]; av4[p][1] = nw[p]; av4[p][2] = aw[p + 1]; av4[p][3] = nw[p + 1];
+                bv4[p][0] = v0[p]; bv4[p][1] = v0[p + 1]; bv4[p][2] = v1[p]; bv4[p][3] = v1[p + 1];
+                mcs[p][0] = cw[p]; mcs[p][1] = cw[p + 1];
+                mas[p][0] = ma[p]; mas[p][1] = na[p];
+                mbs[p][0] = y0[p]; mbs[p][1] = y1[p];
+            }
+#pragma unroll
+            for (int p = 0; p <= K; p++) aw[p] = nw[p];
+#pragma unroll
+            for (int p = 0; p < K; p++) ma[p] = na[p];
+        }
+        T c0v[K], c1v[K], pgs[K], nms[K], nv[K], sv[K];
+        if (force) {
+            lane_run(cn, o, l, c0v);
+            lane_run(cn, o - sF, l, c1v);
+        }
+        lane_run(pg, o, l, pgs);
+        if (r != T(0)) lane_run(Nm1, o, l, nms);   // as in rhs_conc_line
+#pragma unroll
+        for (int p = 0; p < K; p++) {
+            const int k = k0 + p;
+            T qx[7], qy[7], qz[7];
+            st.at(p, qx, qy, qz);
+            const T (&av)[4] = av4[p];
+            const T (&bv)[4] = bv4[p];
+            const T mc0 = mcs[p][0], mc1 = mcs[p][1], ma0 = mas[p][0], ma1 = mas[p][1], mb0 = mbs[p][0], mb1 = mbs[p][1];
+            const T cn0 = force ? c0v[p] : T(0), cn1 = force ? c1v[p] : T(0);
+            const T pgv = pgs[p], nm1 = r != T(0) ? nms[p] : T(0);
+
+            const T alpha = g + r;
+            const T vx = F == FU ? qx[3] : T(0.25) * (av[0] + av[1] + av[2] + av[3]);
+            const T vy = F == FV ? qy[3] : F == FU ? T(0.25) * (av[0] + av[1] + av[2] + av[3])
+                                                   : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
+            const T vz = F == FW ? qz[3] : T(0.25) * (bv[0] + bv[1] + bv[2] + bv[3]);
+            // the cross-viscous differences at the upper and lower edges
+            const T a1 = F == FU ? av[2] - av[3] : av[3] - av[1];
+            const T a0 = F == FU ? av[1] - av[0] : av[2] - av[0];
+            const T b1 = F == FU ? bv[2] - bv[3] : F == FV ? bv[3] - bv[1] : bv[3] - bv[2];
+            const T b0 = F == FV ? bv[2] - bv[0] : bv[1] - bv[0];
+            // mu below and above the point along x, y and z
+            const T mx0 = F == FU ? mc0 : ma0, mx1 = F == FU ? mc1 : ma1;
+            const T my0 = F == FU ? ma0 : F == FV ? mc0 : mb0, my1 = F == FU ? ma1 : F == FV ? mc1 : mb1;
+            const T mz0 = F == FW ? mc0 : mb0, mz1 = F == FW ? mc1 : mb1;
+            const T Re = T(ph.Re);
+            if constexpr (FAST) {
+                T xm, xp, ym, yp, zm, zp;
+                const T cx = upwind_term<T>(qx, i, R.is, R.ie, vx, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
+                const T cy = upwind_term<T>(qy, j, R.js, R.je, vy, T(d.dy), T(d.rdy), ylo, yhi, ym, yp);
+                const T cz = upwind_term<T>(qz, k, R.ks, R.ke, vz, T(d.dz), T(d.rdz), zlo, zhi, zm, zp);
+                T nval = fma(e0, fma(ma1, a1, -(ma0 * a0)), -(cz + cx + cy));
+                nval = fma(e1, fma(mb1, b1, -(mb0 * b0)), nval);
+                nv[p] = nval;
+                T visc = kx * fma(mx1, xp, -(mx0 * xm));
+                visc = fma(ky, fma(my1, yp, -(my0 * ym)), visc);
+                visc = fma(kz, fma(mz1, zp, -(mz0 * zm)), visc);
+                visc = fma(-rRe, pgv, visc);
+                if (force) visc = fma(-fre, T(0.5) * (cn0 + cn1), visc);
+                sv[p] = dt * fma(alpha, visc, fma(g, nval, r * nm1));
+            } else {
+                // convec_term: upwind derivatives along x, y, z
+                T D[6];
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(qx[m + 1] - qx[m], T(d.dx), d.rdx);
+                const T convx = vx * upwind_d<T>(D, i, R.is, R.ie, vx >= T(0.0) ? 1 : -1, T(d.dx), d.rdx, T(0.0), T(0.0));
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(qy[m + 1] - qy[m], T(d.dy), d.rdy);
+                const T convy = vy * upwind_d<T>(D, j, R.js, R.je, vy >= T(0.0) ? 1 : -1, T(d.dy), d.rdy, ylo, yhi);
+#pragma unroll
+                for (int m = 0; m < 6; m++) D[m] = divh<T>(qz[m + 1] - qz[m], T(d.dz), d.rdz);
+                const T dzd = upwind_d<T>(D, k, R.ks, R.ke, vz >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, zlo, zhi);
+                const T ct = vz * dzd + convx + convy;
+                // explicit_n: -convec_term + the cross-viscous terms, left to right
+                const T p1 = e0 * ma1 * a1, m1 = e0 * ma0 * a0;
+                const T p2 = e1 * mb1 * b1, m2 = e1 * mb0 * b0;
+                const T nval = -ct + p1 - m1 + p2 - m2;
+                nv[p] = nval;
+                // source: dt [g N + r N_nm1 + alpha A(mu_old) q + alpha (body force)]
+                T ax, bx, cx, ay, by, cy, az, bz, cz;
+                coef_vals<T, F>(d, ph, 0, mx0, mx1, ax, bx, cx);
+                coef_vals<T, F>(d, ph, 1, my0, my1, ay, by, cy);
+                coef_vals<T, F>(d, ph, 2, mz0, mz1, az, bz, cz);
+                const T conv = (g * nval + r * nm1);
+                const T axx = ax * qx[2] + bx * qx[3] + cx * qx[4];
+                const T axy = ay * qy[2] + by * qy[3] + cy * qy[4];
+                const T axz = az * qz[2] + bz * qz[3] + cz * qz[4];
+                const T visc = alpha * (axx + axy + axz);
+                T bodyforce;
+                if (!force) bodyforce = alpha * (-divh<T>(pgv, Re, ph.rRe));
+                else bodyforce = alpha * (-fre * (T(0.5) * (cn0 + cn1)) - divh<T>(pgv, Re, ph.rRe));
+                sv[p] = dt * (conv + visc + bodyforce);
+            }
+        }
+        per_block(l, o);
+        lane_put(N, o, l, nv, k0, R.ks, R.ke);
+        lane_put(S, o, l, sv, k0, R.ks, R.ke);
     }
 }
 
-// one component over its range (one thread per point)
-template <typename T, int F, bool FAST, bool B = false>
-__global__ __launch_bounds__(256) void k_rhs_mom(Dims d, Phys ph0, const T* __restrict__ u, const T* __restrict__ v,
-                                                 const T* __restrict__ w, Visc4<T> mu, const T* __restrict__ cn,
-                                                 const T* __restrict__ pg, const T* __restrict__ Nm1, T* __restrict__ N,
-                                                 T* __restrict__ S, const T* __restrict__ stale,
-                                                 const double* __restrict__ scal, T g, T r, Bt bt)
+// the explicit parts of n fields (F: FC, FU, FV or FW) in one launch: np
+// planes a thread, the fields' blocks of the same planes next to each other in
+// dispatch order, so that the velocities and viscosities which they share
+// come from HBM once and a small grid pays for one launch: at 256x128x128
+// FP64 one launch per component moved 9.8 fields and the concentration's 6.9,
+// together 36, the joint one moves 18 (some of the 23 there are stay in the
+// last-level cache).  us, four launches -> one: 256x128x128 FP64 369 -> 263,
+// mixed 169 -> 134; 512x256x256 FP64 2740 -> 1920, mixed 1210 -> 1000;
+// 64x32x32 FP64 20 -> 9.  FP32 is bound by vector issue (92% of the cycles);
+// FP64 by latency with two waves per vector unit (54% issue, 36% waiting).
+template <typename T>
+struct RhsSets {
+    int n;
+    struct { int F; const T* pg; const T* Nm1; T* N; T* S; } s[4];
+};
+template <typename T, bool FAST, bool B = false>
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 2 : 6) void k_rhs(Dims d, Phys ph0, RhsSets<T> rs, const T* __restrict__ cold,
+                                             const T* __restrict__ u, const T* __restrict__ v, const T* __restrict__ w,
+                                             Visc4<T> mu, const T* __restrict__ cn, const T* __restrict__ ncorr,
+                                             const T* __restrict__ stale0, const double* __restrict__ scal, T g, T r,
+                                             int np, Bt bt)
 {
-    const Rng R = field_rng(d, F);
     const int2 tl = xcd_tile();
-    const int k = tl.x * blockDim.x + threadIdx.x + 1;
-    const int j = tl.y * blockDim.y + threadIdx.y + R.js;
+    const int k = (tl.x * blockDim.x + threadIdx.x) * KP<T>::value + 1;
+    const int j = tl.y * blockDim.y + threadIdx.y + 1;
     int il;
     const int m = bt_member(bt, blockIdx.z, gridDim.z, il);
-    const int i = il + R.is;
-    if (k < R.ks || k > R.ke || j > R.je) return;
+    const int grp = il / rs.n, q = il - grp * rs.n;
+    const auto& s = rs.s[q];
+    const int F = s.F;
+    const Rng R = field_rng(d, F);
+    const int i0 = 3 + grp * np, i = max(i0, R.is), ie = min(i0 + np - 1, R.ie);
+    if (k + KP<T>::value <= R.ks || k > R.ke || j < R.js || j > R.je) return;
     const Phys& ph = bt_phys<B>(bt, ph0, m);
-    rhs_mom_point<T, F, FAST>(d, ph, R, i, j, k, bt_f(bt, u, m), bt_f(bt, v, m), bt_f(bt, w, m), bt_mu(bt, mu, m),
-                              bt_f(bt, cn, m), bt_f(bt, pg, m), bt_f(bt, Nm1, m), bt_f(bt, N, m), bt_f(bt, S, m),
-                              stale + m * 16, T(scal[m * S_SIZE + S_DT]), g, r);
+    const T* stale = stale0 + m * 16 + 4 * F;
+    const T dt = T(scal[m * S_SIZE + S_DT]);
+    const long mo = m * bt.fs;
+    if (F == FC)
+        rhs_conc_line<T, FAST>(d, ph, R, i, ie, j, k, mo, cold, u, v, w, s.Nm1, s.N, s.S, stale, ncorr, dt, g, r);
+    else if (F == FU)
+        rhs_mom_line<T, FU, FAST>(d, ph, R, i, ie, j, k, mo, u, v, w, mu, cn, s.pg, s.Nm1, s.N, s.S, stale, dt, g, r);
+    else if (F == FV)
+        rhs_mom_line<T, FV, FAST>(d, ph, R, i, ie, j, k, mo, u, v, w, mu, cn, s.pg, s.Nm1, s.N, s.S, stale, dt, g, r);
+    else
+        rhs_mom_line<T, FW, FAST>(d, ph, R, i, ie, j, k, mo, u, v, w, mu, cn, s.pg, s.Nm1, s.N, s.S, stale, dt, g, r);
 }
 
 // --------------------------------------------------------- line solvers
@@ -2454,17 +2685,8 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
 // ------------------------------------------------------ instantiations
 
 #define PLLC_INST_RHS(T, FAST)                                                                                 \
-    template __global__ void k_rhs_c<T, FAST>(Dims, Phys, const T*, const T*, const T*, const T*, const T*, T*,  \
-                                              T*, const T*, const T*, const double*, T, T, Bt);                 \
-    template __global__ void k_rhs_mom<T, FU, FAST>(Dims, Phys, const T*, const T*, const T*, Visc4<T>,        \
-                                                    const T*, const T*, const T*, T*, T*, const T*,             \
-                                                    const double*, T, T, Bt);                                       \
-    template __global__ void k_rhs_mom<T, FV, FAST>(Dims, Phys, const T*, const T*, const T*, Visc4<T>,        \
-                                                    const T*, const T*, const T*, T*, T*, const T*,             \
-                                                    const double*, T, T, Bt);                                       \
-    template __global__ void k_rhs_mom<T, FW, FAST>(Dims, Phys, const T*, const T*, const T*, Visc4<T>,        \
-                                                    const T*, const T*, const T*, T*, T*, const T*,             \
-                                                    const double*, T, T, Bt);
+    template __global__ void k_rhs<T, FAST>(Dims, Phys, RhsSets<T>, const T*, const T*, const T*, const T*,        \
+                                            Visc4<T>, const T*, const T*, const T*, const double*, T, T, int, Bt);
 
 #define PLLC_INST_DCT_PLANES(T, N)                                                                             \
     template __global__ void k_dct_planes<T, false, N>(int, int, int, int, const T*, T*, const T*, const T*,   \
@@ -3268,7 +3490,7 @@ namespace pllc {
 
 #ifdef PLLC_F64_TU
 const char* kernel_class_names =
-    "stale;rhs_c;rhs_u;rhs_v;rhs_w;sweep_y;sweep_z;sweep_x;visc;velo_ghost;div;dct;pois_x;"
+    "stale;rhs_c;rhs_u;rhs_v;rhs_w;rhs_uvw;rhs_cuvw;sweep_y;sweep_z;sweep_x;visc;velo_ghost;div;dct;pois_x;"
     "phi_ghost;velo_corr;flux;pg;corr_pg;cfl;bulk;copy";
 #endif
 
@@ -3310,12 +3532,6 @@ static int resident_blocks(K f, int nthreads, size_t sm)
 template <typename T>
 static inline bool fast_stencils(const Ctx<T>& c) { return c.line_solver == 0; }
 
-// Tiles of one i-plane of at most 256 threads (k, j), k from 1: a row is cut
-// into as few equal parts of at most 128 points as it needs, each rounded up
-// to 16 lanes (an aligned piece of a row), and a tile takes as many rows as
-// fit (128 x 2 measured faster than 64 x 4, 32 x 8 and 256 x 1 for the cell
-// kernels at 128-point rows; at 96 points 96 x 2 leaves no lane idle where
-// 128 x 2 left a quarter)
 // launchers without a batched form: false (and the error set) when the
 // context launches over a batch
 template <typename T>
@@ -3326,9 +3542,15 @@ static bool single(const Ctx<T>& c, const char* what)
     return false;
 }
 
-static inline dim3 cell_grid(const Rng& R, dim3& blk)
+// Tiles of one i-plane of at most 256 threads (k, j), k from 1: a row is cut
+// into as few equal parts of at most 128 points as it needs, each rounded up
+// to 16 lanes (an aligned piece of a row), and a tile takes as many rows as
+// fit, kp points a lane (128 x 2 measured faster than 64 x 4, 32 x 8 and 256 x 1 for the cell
+// kernels at 128-point rows; at 96 points 96 x 2 leaves no lane idle where
+// 128 x 2 left a quarter)
+static inline dim3 cell_grid(const Rng& R, dim3& blk, int kp = 1)
 {
-    const int nk = R.ke, nt = (nk + 127) / 128, bx = ((nk + nt - 1) / nt + 15) / 16 * 16, by = 256 / bx;
+    const int nk = (R.ke + kp - 1) / kp, nt = (nk + 127) / 128, q = 16 / kp, bx = ((nk + nt - 1) / nt + q - 1) / q * q, by = 256 / bx;
     blk = dim3(bx, by, 1);
     return dim3(nt, (R.je - R.js + 1 + by - 1) / by, R.ie - R.is + 1);
 }
@@ -3339,6 +3561,34 @@ static inline dim3 bgrid(dim3 g, const Ctx<T>& c)
 {
     g.z *= (unsigned)c.bt.nm;
     return g;
+}
+// vector units of the device (4 in each CU)
+static int simds()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    return 4 * cus;
+}
+
+// A cell grid for n fields whose threads take np consecutive planes each.
+// More planes reuse more of the x neighbours in registers (24 loads a point
+// instead of 37) and share a thread's set-up, but leave fewer waves: np is the
+// largest power of two up to 8 that leaves 2.5 waves per vector unit.  us a
+// step at np = 1, 2, 4, 8: 64x32x32 mixed 221, 220, 224, -; 97x45x39 FP64 428,
+// 423, 426, -; 150x70x51 mixed 513, 490, 483, 492; 256x128x128 FP64 -, -, 2457,
+// 2416; 512x256x256 mixed 11785, 10640, 10424, 10177 (16: 10119, but 150x70x51
+// 508).
+template <typename T>
+static inline dim3 march_grid(const Rng& R, dim3& blk, const Ctx<T>& c, int n, int& np)
+{
+    dim3 g = cell_grid(R, blk, KP<T>::value);
+    const double waves = (double)n * c.bt.nm * g.x * g.y * g.z * 4 / simds();
+    np = 1;
+    while (np < 8 && waves >= 2 * np * 2.5) np *= 2;
+    g.z = (g.z + np - 1) / np * n;
+    return bgrid(g, c);
 }
 static inline int bulk_grid(long n) { long b = (n + 255) / 256; return (int)(b > 4096 ? 4096 : (b < 1 ? 1 : b)); }
 
@@ -3521,26 +3771,55 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
     }
 }
 
+// the field the explicit part of F leaves its source in.  With several
+// components u's, v's and w's are F_SRC, F_SRC2 and F_SRC3, u's F_SRC4 where
+// the concentration's (F_SRC) is still needed (split).
+template <typename T>
+static T* src_field(Ctx<T>& c, int F, bool several, bool split)
+{
+    if (!several || F == FC) return c.f[F_SRC];
+    T* s = c.f[F == FU ? (split ? F_SRC4 : F_SRC) : F == FV ? F_SRC2 : F_SRC3];
+    return s ? s : c.f[F_SRC];
+}
+
+// the explicit parts of the fields in the mask (bit 0 c, 1 u, 2 v, 3 w)
+template <typename T>
+static void rhs_set(Ctx<T>& c, int fields, double g, double r, const T* un, const T* vn, const T* wn, bool split)
+{
+    static const char* const names[16] = {"",        "rhs_c", "rhs_u", "", "rhs_v", "", "", "", "rhs_w", "",
+                                          "",        "",      "",      "", "rhs_uvw", "rhs_cuvw"};
+    const bool several = (fields & 14) == 14;
+    RhsSets<T> rs;
+    rs.n = 0;
+    for (int F = FC; F <= FW; F++) {
+        if (!(fields & (1 << F))) continue;
+        const int b = F == FC ? C_OLD : F == FU ? U_OLD : F == FV ? V_OLD : W_OLD;
+        const int n = F == FC ? C_N : b + 3;
+        rs.s[rs.n++] = {F, F == FC ? nullptr : c.f[b + 2], c.f[n + 1], c.f[n], src_field(c, F, several, split)};
+    }
+    dim3 blk;
+    int np;
+    const dim3 grd = march_grid(field_rng(c.d, FC), blk, c, rs.n, np);
+    auto go = [&](auto fast, auto bv) {
+        PLLC_L(c, names[fields], (k_rhs<T, decltype(fast)::value, decltype(bv)::value><<<grd, blk, 0, c.st>>>(
+                                     c.d, c.ph, rs, c.f[C_OLD], un, vn, wn, muo(c), c.f[C_NEW], c.ncorr, c.stale, c.scal,
+                                     T(g), T(r), np, c.bt)));
+    };
+    const bool fast = fast_stencils(c);
+    if (c.bt.nm > 1) fast ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    else fast ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
+}
+
 template <typename T>
 void Ops<T>::concentration(Ctx<T>& c, double g, double r, int slot, const T* un, const T* vn, const T* wn)
 {
-    dim3 blk;
-    const dim3 grd = bgrid(cell_grid(field_rng(c.d, FC), blk), c);
-    auto go = [&](auto bv) {
-        constexpr bool B = decltype(bv)::value;
-        if (fast_stencils(c))
-            PLLC_L(c, "rhs_c", (k_rhs_c<T, true, B><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[C_OLD], un, vn, wn,
-                                                                            c.f[C_NM1], c.f[C_N], c.f[F_SRC],
-                                                                            c.stale + 0, c.ncorr, c.scal, T(g), T(r),
-                                                                            c.bt)));
-        else
-            PLLC_L(c, "rhs_c", (k_rhs_c<T, false, B><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[C_OLD], un, vn, wn,
-                                                                             c.f[C_NM1], c.f[C_N], c.f[F_SRC],
-                                                                             c.stale + 0, c.ncorr, c.scal, T(g), T(r),
-                                                                             c.bt)));
-    };
-    if (c.bt.nm > 1) go(std::true_type{});
-    else go(std::false_type{});
+    rhs_set<T>(c, 1, g, r, un, vn, wn, false);
+    concentration_implicit(c, g, r, slot);
+}
+
+template <typename T>
+void Ops<T>::concentration_implicit(Ctx<T>& c, double g, double r, int slot)
+{
     const int F[1] = {FC};
     T* S[1] = {c.f[F_SRC]};
     T* CC[1] = {c.f[F_CC]};
@@ -3563,83 +3842,53 @@ void Ops<T>::viscosity(Ctx<T>& c, const T* cn, T* const mu[4])
         PLLC_L(c, "visc", (k_visc<T><<<grd, 256, 0, c.st>>>(c.d, c.ph, cn, mu[0], mu[1], mu[2], mu[3], c.bt)));
 }
 
-template <typename T, int F>
-static void rhs_mom(Ctx<T>& c, T g, T r, T* S)
-{
-    const int b = F == FU ? U_OLD : F == FV ? V_OLD : W_OLD;
-    const char* nm = F == FU ? "rhs_u" : F == FV ? "rhs_v" : "rhs_w";
-    dim3 blk;
-    const dim3 grd = bgrid(cell_grid(field_rng(c.d, F), blk), c);
-    auto go = [&](auto bv) {
-        constexpr bool B = decltype(bv)::value;
-        if (fast_stencils(c))
-            PLLC_L(c, nm, (k_rhs_mom<T, F, true, B><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[U_OLD], c.f[V_OLD],
-                                                                            c.f[W_OLD], muo(c), c.f[C_NEW],
-                                                                            c.f[b + 2], c.f[b + 4], c.f[b + 3], S,
-                                                                            c.stale + 4 * F, c.scal, g, r, c.bt)));
-        else
-            PLLC_L(c, nm, (k_rhs_mom<T, F, false, B><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[U_OLD], c.f[V_OLD],
-                                                                             c.f[W_OLD], muo(c), c.f[C_NEW],
-                                                                             c.f[b + 2], c.f[b + 4], c.f[b + 3], S,
-                                                                             c.stale + 4 * F, c.scal, g, r, c.bt)));
-    };
-    if (c.bt.nm > 1) go(std::true_type{});
-    else go(std::false_type{});
-}
-
-// comps: bit 0 u, bit 1 v, bit 2 w.  With several components their sources
-// go to F_SRC, F_SRC2, F_SRC3 (u's to F_SRC4 when split: F_SRC then holds
-// the concentration's) and the sweeps of all of them share launches; the
-// components are independent (each reads only old velocities, c_new and the
-// viscosities), so this equals xmom; ymom; zmom (179-181).  part: 1 the
-// explicit parts, 2 the sweeps, 3 both.
+// the sweeps of the components in the mask (bit 0 u, 1 v, 2 w) from the
+// sources of their explicit parts.  With several components the sweeps of
+// all of them share launches; the components are independent (each reads
+// only old velocities, c_new and the viscosities), so this equals xmom; ymom;
+// zmom (179-181).
 template <typename T>
-static void momentum_set(Ctx<T>& c, int comps, double gd, double rd, int slot, bool vghost = false, int part = 3,
-                         bool split = false)
+static void momentum_sweeps(Ctx<T>& c, int comps, double gd, double rd, int slot, bool vghost, bool split)
 {
-    const T g = T(gd), r = T(rd);
+    const bool several = comps == 7;
     int F[3], n = 0;
     T *S[3], *CC[3], *qo[3], *qn[3], *N[3], *Nm[3];
-    const int src[3] = {split ? F_SRC4 : F_SRC, F_SRC2, F_SRC3}, ccs[3] = {F_CC, F_CC2, F_CC3};
+    const int ccs[3] = {F_CC, F_CC2, F_CC3};
     for (int q = 0; q < 3; q++) {
         if (!(comps & (1 << q))) continue;
-        const int f = FU + q, b = q == 0 ? U_OLD : q == 1 ? V_OLD : W_OLD;
-        T* s = c.f[src[n]] ? c.f[src[n]] : c.f[F_SRC];
-        T* cc = c.f[ccs[n]] ? c.f[ccs[n]] : c.f[F_CC];
-        if (part & 1) {
-            if (f == FU) rhs_mom<T, FU>(c, g, r, s);
-            else if (f == FV) rhs_mom<T, FV>(c, g, r, s);
-            else rhs_mom<T, FW>(c, g, r, s);
-        }
-        F[n] = f; S[n] = s; CC[n] = cc;
+        const int b = q == 0 ? U_OLD : q == 1 ? V_OLD : W_OLD;
+        F[n] = FU + q; S[n] = src_field(c, FU + q, several, split);
+        CC[n] = c.f[ccs[n]] ? c.f[ccs[n]] : c.f[F_CC];
         qo[n] = c.f[b]; qn[n] = c.f[b + 1]; N[n] = c.f[b + 3]; Nm[n] = c.f[b + 4];
         n++;
     }
-    if (part & 2) adi_sets<T>(c, g, r, slot, F, n, S, CC, mun(c), qo, qn, N, Nm, vghost);
+    adi_sets<T>(c, T(gd), T(rd), slot, F, n, S, CC, mun(c), qo, qn, N, Nm, vghost);
 }
 
 template <typename T>
 void Ops<T>::momentum(Ctx<T>& c, int comp, double g, double r, int slot)
 {
-    momentum_set<T>(c, 1 << comp, g, r, slot);
+    rhs_set<T>(c, 2 << comp, g, r, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], false);
+    momentum_sweeps<T>(c, 1 << comp, g, r, slot, false, false);
 }
 
 template <typename T>
 void Ops<T>::momentum3(Ctx<T>& c, double g, double r, int slot, bool ghosts)
 {
-    momentum_set<T>(c, 7, g, r, slot, ghosts);
+    rhs_set<T>(c, 14, g, r, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], false);
+    momentum_sweeps<T>(c, 7, g, r, slot, ghosts, false);
 }
 
 template <typename T>
-void Ops<T>::momentum3_explicit(Ctx<T>& c, double g, double r)
+void Ops<T>::explicit_parts(Ctx<T>& c, double g, double r)
 {
-    momentum_set<T>(c, 7, g, r, 0, false, 1, true);
+    rhs_set<T>(c, 15, g, r, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], true);
 }
 
 template <typename T>
 void Ops<T>::momentum3_implicit(Ctx<T>& c, double g, double r, int slot, bool ghosts)
 {
-    momentum_set<T>(c, 7, g, r, slot, ghosts, 2, true);
+    momentum_sweeps<T>(c, 7, g, r, slot, ghosts, true);
 }
 
 template <typename T>

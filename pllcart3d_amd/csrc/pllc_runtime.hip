@@ -407,11 +407,6 @@ struct pllc_sim {
     long cnn_steps = 0;           // of every k-th step, held in between (steps counted here)
     std::vector<void*> snap;
     double* gscratch = nullptr;
-    // a side stream (default priority) for the momentum explicit parts,
-    // forked from st before the concentration update and joined before the
-    // momentum sweeps (Ctx::mom_fork; PLLC_FORK=0: one stream)
-    hipStream_t side = nullptr;
-    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     double* xfer = nullptr;       // one field in FP64, contiguous: uploads and downloads (stage())
 };
 
@@ -483,10 +478,6 @@ static bool create_t(pllc_sim* s)
     return pllc_ctx_tables<T>(c, s->owned, W);
 }
 
-// interior cells from which a simulation runs its momentum explicit parts
-// on the side stream
-constexpr long kForkMinCells = 600000;
-
 extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision)
 {
     if (!p || p->nx < 1 || p->ny < 1 || p->nz < 1) { pllc_set_error("pllc_sim_create", "bad dimensions"); return nullptr; }
@@ -503,19 +494,7 @@ extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision)
     ok = ok && (precision == PLLC_PREC_PLAIN ? create_t<double>(s) : create_t<float>(s));
     ok = ok && pllc_hip_ok("pllc_sim_create", hipEventCreate(&s->e0)) &&
          pllc_hip_ok("pllc_sim_create", hipEventCreate(&s->e1));
-    const char* fk = getenv("PLLC_FORK");
-    if (ok && !(fk && strcmp(fk, "0") == 0)) {
-        ok = pllc_hip_ok("pllc_sim_create", hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking)) &&
-             pllc_hip_ok("pllc_sim_create", hipEventCreateWithFlags(&s->fork_ev, hipEventDisableTiming)) &&
-             pllc_hip_ok("pllc_sim_create", hipEventCreateWithFlags(&s->join_ev, hipEventDisableTiming));
-        // the explicit parts read c_new only through the body force; the
-        // fork and join cost more than the overlap gains on small grids
-        // (measured: 64x32x32 mixed 0.35 -> 0.41 ms per step, 128x64x64
-        // even, 192x64x64 FP64 0.86 -> 0.82, 256x128x128 FP64 3.12 -> 3.03)
-        const long cells = (long)p->nx * p->ny * p->nz;
-        const int mf = (p->Fx == 0.0 && p->Fy == 0.0 && cells >= kForkMinCells) ? 1 : 0;
-        s->cd.mom_fork = s->cf.mom_fork = mf;
-    }
+    s->cd.joint = s->cf.joint = p->Fx == 0.0 && p->Fy == 0.0 ? 1 : 0;
     if (!ok) { pllc_sim_destroy(s); return nullptr; }
     s->Timestep = p->Timestep;
     const char* gr = getenv("PLLC_GRAPH");
@@ -530,16 +509,12 @@ extern "C" void pllc_sim_destroy(pllc_sim* s)
 {
     if (!s) return;
     if (s->st) (void)hipStreamSynchronize(s->st);
-    if (s->side) (void)hipStreamSynchronize(s->side);
     std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
     graph_drop(s);
     for (void* p : s->owned) (void)hipFree(p);
     for (hipEvent_t e : s->tev) (void)hipEventDestroy(e);
     if (s->e0) (void)hipEventDestroy(s->e0);
     if (s->e1) (void)hipEventDestroy(s->e1);
-    if (s->fork_ev) (void)hipEventDestroy(s->fork_ev);
-    if (s->join_ev) (void)hipEventDestroy(s->join_ev);
-    if (s->side) (void)hipStreamDestroy(s->side);
     if (s->st) (void)hipStreamDestroy(s->st);
     delete s;
 }
@@ -828,23 +803,18 @@ static void fused_step(pllc_sim* s, Ctx<T>& c)
         if (s->cnn && c.ncorr && (s->cnn_every == 0 || (rk == 0 && s->cnn_steps % s->cnn_every == 0)))
             pllc_cnn_correct<T>(s->cnn, c.d, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], c.f[MUO_CELL], c.ncorr,
                                 c.st);
-        // the momentum explicit parts beside the concentration update and
-        // the viscosity (they read old velocities, mu_old, pg and N_nm1;
-        // those write c_new, N_c, F_SRC and mu_new), joined before the sweeps
-        const bool fork = c.mom_fork && s->side && !c.hook && hipEventRecord(s->fork_ev, c.st) == hipSuccess &&
-                          hipStreamWaitEvent(s->side, s->fork_ev, 0) == hipSuccess;
-        if (fork) {
-            Ctx<T> cs = c;
-            cs.st = s->side;
-            Ops<T>::momentum3_explicit(cs, g, r);
-            if (!pllc_hip_ok("fused step", hipEventRecord(s->join_ev, s->side)))
-                (void)hipStreamSynchronize(s->side);   // no join event: the side stream's work is done first
+        // without a body force the momentum explicit parts read nothing that
+        // the concentration update and the viscosity write: they share its
+        // launch
+        if (c.joint) {
+            Ops<T>::explicit_parts(c, g, r);
+            Ops<T>::concentration_implicit(c, g, r, rk);
+        } else {
+            Ops<T>::concentration(c, g, r, rk, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
         }
-        Ops<T>::concentration(c, g, r, rk, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
         T* mun[4] = {c.f[MUN_CELL], c.f[MUN_XY], c.f[MUN_XZ], c.f[MUN_YZ]};
         Ops<T>::viscosity(c, c.f[C_NEW], mun);
-        if (fork) {
-            (void)pllc_hip_ok("fused step", hipStreamWaitEvent(c.st, s->join_ev, 0));
+        if (c.joint) {
             Ops<T>::momentum3_implicit(c, g, r, rk, true);
         } else {
             Ops<T>::momentum3(c, g, r, rk, true);   // with update_velo_boundary
@@ -1263,6 +1233,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
         return nullptr;
     }
     b->c.st = b->st;
+    for (pllc_sim* s : ms) b->c.joint = b->c.joint && s->cf.joint;
     b->c.QC = nullptr;
     b->c.bt.nm = nm;
     b->c.bt.fs = fs;
@@ -1432,11 +1403,6 @@ extern "C" pllc_ensemble* pllc_ensemble_create(const pllc_params* p, int n, int 
         if (v) e->done.push_back(v);
     }
     if (!ok) { pllc_ensemble_destroy(e); return nullptr; }
-    // the members' (and batches') steps overlap as the branches of one graph
-    // already; a side stream per step on top measured slower (10.2 -> 10.8
-    // ms per step of the 64-member ensemble), so an ensemble keeps one
-    // stream per step
-    for (pllc_sim* s : e->m) s->cd.mom_fork = s->cf.mom_fork = 0;
     // batches of the members with equal dims (mixed precision)
     const char* eb = getenv("PLLC_ENSEMBLE_BATCH");
     std::vector<bool> taken(n, false);
