@@ -407,7 +407,6 @@ struct pllc_sim {
     long cnn_steps = 0;           // of every k-th step, held in between (steps counted here)
     std::vector<void*> snap;
     double* gscratch = nullptr;
-    double* xfer = nullptr;       // one field in FP64, contiguous: uploads and downloads (stage())
 };
 
 static void apply_tuned(pllc_sim* s);
@@ -558,46 +557,53 @@ static void normalize(pllc_sim* s, Ctx<T>& c)
     s->new_stale = false;
 }
 
-// Fields cross the boundary through a contiguous FP64 block on the device,
-// kept with the simulation: a kernel lays rows out (or gathers them) and
-// converts, and the copy is one piece between it and the caller's memory
-// (the host's element-by-element conversion of mixed fields took 8 ms per
-// 256x128x128 field, the kernel and the copy 0.9).
-static double* stage(pllc_sim* s, const char* W)
+// Uploads and downloads pass through a scratch field of the sweeps as
+// contiguous FP64 rows of NZ values, as many rows at a time as it holds (a
+// row kernel packs and converts; converting a mixed field on the host cost
+// 8 ms at 256x128x128).  Its content lives only within an operator or a step.
+template <typename T>
+static double* stage(Ctx<T>& c, long& rows)
 {
-    if (!s->xfer) {
-        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-        void* p = nullptr;
-        if (!pllc_hip_ok(W, hipMalloc(&p, npts(s) * 8))) return nullptr;
-        s->owned.push_back(p);
-        s->xfer = (double*)p;
-    }
-    return s->xfer;
+    T* p = c.f[F_SRC2] + 1;   // a 128-byte line's start
+    rows = (long)((field_values(c.d) - 1) * sizeof(T) / (c.d.NZ * sizeof(double)));
+    return reinterpret_cast<double*>(p);
 }
 
 // dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ values
 template <typename T>
 static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W)
 {
-    double* t = stage(s, W);
-    if (!t) return false;
-    {
-        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-        if (!pllc_hip_ok(W, hipMemcpy(t, src, (size_t)rows * c.d.NZ * 8, hipMemcpyHostToDevice))) return false;
+    long most = 0;
+    double* t = stage(c, most);
+    if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
+    for (long q = 0; q < rows; q += most) {
+        const long n = std::min(most, rows - q);
+        {
+            std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
+            if (!pllc_hip_ok(W, hipMemcpy(t, src + q * c.d.NZ, (size_t)n * c.d.NZ * 8, hipMemcpyHostToDevice)))
+                return false;
+        }
+        Ops<T>::unpack(c, t, dst + (r0 + q) * c.d.sy, n);
+        if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
     }
-    Ops<T>::unpack(c, t, dst + r0 * c.d.sy, rows);
-    return pllc_hip_ok(W, hipStreamSynchronize(s->st));
+    return true;
 }
 
 template <typename T>
 static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W)
 {
-    double* t = stage(s, W);
-    if (!t) return false;
-    Ops<T>::pack(c, src, t, (long)c.d.NX * c.d.NY);
-    if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
-    std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-    return pllc_hip_ok(W, hipMemcpy(dst, t, npts(s) * 8, hipMemcpyDeviceToHost));
+    long most = 0;
+    double* t = stage(c, most);
+    const long rows = (long)c.d.NX * c.d.NY;
+    for (long q = 0; q < rows; q += most) {
+        const long n = std::min(most, rows - q);
+        Ops<T>::pack(c, src + q * c.d.sy, t, n);
+        if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
+        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
+        if (!pllc_hip_ok(W, hipMemcpy(dst + q * c.d.NZ, t, (size_t)n * c.d.NZ * 8, hipMemcpyDeviceToHost)))
+            return false;
+    }
+    return true;
 }
 
 template <typename T>
