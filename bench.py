@@ -150,7 +150,7 @@ PEAK_TFLOPS = {8.0: 78.6, 4.0: 157.3}
 PROFILES = os.path.join(ROOT, "profiles")
 CLASS_KERNELS = {
     "sweep_x": ["k_sweep_part<{T}, 0>"], "sweep_y": ["k_sweep_part<{T}, 1>"],
-    "sweep_z": ["k_sweep_wave_z<{T}>", "k_sweep_part_z<{T}>", "k_sweep_part_zt<{T}>"], "corr_pg": ["k_corr_pg<{T}, false>"],
+    "sweep_z": ["k_sweep_wave_z<{T}>", "k_sweep_part_z<{T}>", "k_sweep_part_zt<{T}>"], "corr_pg": ["k_corr_pg_run<{T}, false>", "k_corr_pg<{T}, false>"],
     "rhs_cuvw": ["k_rhs<{T}, true, false>"],
     "rhs_c": ["k_rhs_c<{T}, true, false>"], "rhs_u": ["k_rhs_mom<{T}, 1, true, false>"],
     "rhs_v": ["k_rhs_mom<{T}, 2, true, false>"], "rhs_w": ["k_rhs_mom<{T}, 3, true, false>"],

@@ -1433,6 +1433,183 @@ __global__ __launch_bounds__(256) void k_corr_pg(Dims d, Phys ph0, Visc4<T> mu, 
     }
 }
 
+// What k_corr_pg_run holds of phi and the viscosities around a thread's KP points
+// (k .. k + K - 1 of row j): names say the row (c: j, m: j - 1, p: j + 1,
+// mm: j - 2), the plane (1: i + 1, none: i, b: i - 1, bb: i - 2) and the runs'
+// first k.
+template <typename T>
+struct CorrRuns {
+    static constexpr int K = KP<T>::value;
+    T c[K + 3], m[K + 2], p[K + 1], mm[K];   // plane i: from k - 2, k - 1, k - 1, k
+    T c1[K + 1], m1[K];                      // plane i + 1: from k - 1, k
+    T cb[K + 2], mb[K], pb[K], cbb[K];       // plane i - 1: from k - 1, k, k; plane i - 2: k
+    T cell[K + 1], cellm[K], cellb[K];       // mu.cell: from k - 1; row j - 1; plane i - 1
+    T xy[K], xyp[K], xy1[K], xz[K + 1], xz1[K], yz[K + 1], yzp[K];
+
+    // component F's operands of point q (corr_load's)
+    template <int F>
+    __device__ __forceinline__ void ops(int q, CorrOps<T>& o) const
+    {
+        const T x0[7] = {c[q + 2], cb[q + 1], c1[q + 1], m[q + 1], p[q + 1], c[q + 1], c[q + 3]};
+        const T xu[7] = {cb[q + 1], cbb[q], c[q + 2], mb[q], pb[q], cb[q], cb[q + 2]};
+        const T xv[7] = {m[q + 1], mb[q], m1[q], mm[q], c[q + 2], m[q], m[q + 2]};
+        const T xw[7] = {c[q + 1], cb[q], c1[q], m[q], p[q], c[q], c[q + 2]};
+#pragma unroll
+        for (int g = 0; g < 7; g++) {
+            o.p0[g] = x0[g];
+            o.p1[g] = F == FU ? xu[g] : F == FV ? xv[g] : xw[g];
+        }
+        if (F == FU) {
+            o.m[0] = cellb[q]; o.m[1] = cell[q + 1]; o.m[2] = xy[q]; o.m[3] = xyp[q]; o.m[4] = xz[q]; o.m[5] = xz[q + 1];
+        } else if (F == FV) {
+            o.m[0] = xy[q]; o.m[1] = xy1[q]; o.m[2] = cellm[q]; o.m[3] = cell[q + 1]; o.m[4] = yz[q]; o.m[5] = yz[q + 1];
+        } else {
+            o.m[0] = xz[q]; o.m[1] = xz1[q]; o.m[2] = yz[q]; o.m[3] = yzp[q]; o.m[4] = cell[q]; o.m[5] = cell[q + 1];
+        }
+    }
+};
+
+// k_corr_pg on launches of many waves: a thread takes KP points in k and
+// CORR_PLANES consecutive planes, the two planes behind it, and of the plane
+// ahead what it shares with the next point, in registers (26 loads a point in
+// FP32 and half as many 16-byte ones in FP64 instead of 38).  us, k_corr_pg ->
+// this at 1, 2, 4, 8 planes: 256x128x128 FP64 134 -> 125, 126, 124, 128, mixed
+// 71 -> 71, 68, 70, 77; 512x256x256 FP64 1043 -> 985, 964, 973, 999, mixed 537
+// -> 536, 517, 509, 525; 256x96x96 mixed 39 -> 38, 37, 41, 44; 150x70x51 mixed
+// 12.9 -> 13.9, 12.0, 12.7, 17.7; 64x32x32 FP64 5.3 -> 6.9, 9.6, 15, 27: with
+// few waves the longer chain of a thread is what counts, hence the two forms
+// (correction_and_gradient).  Bound by HBM (16.8 fields, 4.6 TB/s at 256x128x128 FP64).
+constexpr int CORR_PLANES = 2;
+template <typename T, bool B = false>
+__global__ __launch_bounds__(256) void k_corr_pg_run(Dims d, Phys ph0, Visc4<T> mu, const T* __restrict__ phi,
+                                                 T* __restrict__ u, T* __restrict__ v, T* __restrict__ w,
+                                                 T* __restrict__ pgu, T* __restrict__ pgv, T* __restrict__ pgw,
+                                                 const double* __restrict__ scal0, T g, T r, int vghost, Bt bt)
+{
+    constexpr int K = KP<T>::value, np = CORR_PLANES;
+    const int2 tl = xcd_tile();
+    const int k0 = (tl.x * blockDim.x + threadIdx.x) * K + 1;
+    const int j = tl.y * blockDim.y + threadIdx.y + 1;
+    int il;
+    const int m = bt_member(bt, blockIdx.z, gridDim.z, il);
+    int i = il * np + 3;
+    const int ie = min(i + np - 1, d.nx + 2);
+    if (k0 > d.nz || j > d.ny) return;
+    const Phys& ph = bt_phys<B>(bt, ph0, m);
+    const double* __restrict__ scal = scal0 + m * S_SIZE;
+    const T fac = T(0.5) * T(scal[S_DT]) * (g + r);
+    const T facv = T(scal[S_DT]) * (g + r) / T(ph.Re);
+    const long sx = d.sx, sy = d.sy;
+    const T *cell = mu.cell, *xy = mu.xy, *xz = mu.xz, *yz = mu.yz;
+    unsigned l = (unsigned)((j * d.sy + k0) * sizeof(T));
+    long o = (long)i * sx + m * bt.fs;   // every field of member m at the same offset
+    // the operands of all three components are loaded for every point: a
+    // point whose component is no unknown reads at most two rows, planes or
+    // points below its own, inside the ghost ring or the previous plane, and
+    // stores nothing
+    CorrRuns<T> e;
+    lane_run(phi, o - 1, l, e.c1);
+    lane_run(phi, o - sy, l, e.m1);
+    {
+        T t[K + 2];
+        lane_run(phi, o - sx - 1, l, t);
+#pragma unroll
+        for (int q = 0; q < K + 2; q++) e.c[q + 1] = t[q];
+        T x[K], y[K], z[K];
+        lane_run(phi, o - sx - sy, l, x);
+        lane_run(phi, o - sx + sy, l, y);
+        lane_run(phi, o - 2 * sx, l, z);
+#pragma unroll
+        for (int q = 0; q < K; q++) { e.m[q + 1] = x[q]; e.p[q + 1] = y[q]; e.cb[q + 1] = z[q]; }
+        lane_run(cell, o - sx, l, x);
+#pragma unroll
+        for (int q = 0; q < K; q++) e.cell[q + 1] = x[q];
+    }
+    lane_run(xy, o, l, e.xy1);
+    lane_run(xz, o, l, e.xz1);
+#pragma unroll 1
+    for (; i <= ie; i++, o += sx) {
+        per_block(l, o);
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            e.cbb[q] = e.cb[q + 1];
+            e.mb[q] = e.m[q + 1];
+            e.pb[q] = e.p[q + 1];
+            e.cellb[q] = e.cell[q + 1];
+            e.xy[q] = e.xy1[q];
+            e.xz[q] = e.xz1[q];
+            e.m[q + 1] = e.m1[q];
+        }
+#pragma unroll
+        for (int q = 0; q < K + 2; q++) e.cb[q] = e.c[q + 1];
+#pragma unroll
+        for (int q = 0; q < K + 1; q++) e.c[q + 1] = e.c1[q];
+        lane_run(phi, o + sx - 1, l, e.c1);
+        lane_run(phi, o + sx - sy, l, e.m1);
+        e.c[0] = lane_at(phi, o - 2, l);
+        e.c[K + 2] = lane_at(phi, o + K, l);
+        e.m[0] = lane_at(phi, o - sy - 1, l);
+        e.m[K + 1] = lane_at(phi, o - sy + K, l);
+        lane_run(phi, o + sy - 1, l, e.p);
+        lane_run(phi, o - 2 * sy, l, e.mm);
+        lane_run(cell, o - 1, l, e.cell);
+        lane_run(cell, o - sy, l, e.cellm);
+        lane_run(xy, o + sy, l, e.xyp);
+        lane_run(xy, o + sx, l, e.xy1);
+        e.xz[K] = lane_at(xz, o + K, l);
+        lane_run(xz, o + sx, l, e.xz1);
+        lane_run(yz, o, l, e.yz);
+        lane_run(yz, o + sy, l, e.yzp);
+        T qv[K], qw[K], qu[K], gv[K], gw[K], gu[K];
+        lane_run(v, o, l, qv);
+        lane_run(w, o, l, qw);
+        lane_run(u, o, l, qu);
+        lane_run(pgv, o, l, gv);
+        lane_run(pgw, o, l, gw);
+        lane_run(pgu, o, l, gu);
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            CorrOps<T> co;
+            e.template ops<FV>(q, co);
+            co.q = qv[q]; co.pg = gv[q];
+            qv[q] = corr_q<T, FV>(d, co, facv);
+            gv[q] = corr_pg_new<T, FV>(d, ph, co, fac);
+            e.template ops<FW>(q, co);
+            co.q = qw[q]; co.pg = gw[q];
+            qw[q] = corr_q<T, FW>(d, co, facv);
+            gw[q] = corr_pg_new<T, FW>(d, ph, co, fac);
+            e.template ops<FU>(q, co);
+            co.q = qu[q]; co.pg = gu[q];
+            qu[q] = corr_q<T, FU>(d, co, facv);
+            gu[q] = corr_pg_new<T, FU>(d, ph, co, fac);
+        }
+        per_block(l, o);
+        if (j >= 2) {
+            lane_put(v, o, l, qv, k0, 1, d.nz);
+            lane_put(pgv, o, l, gv, k0, 1, d.nz);
+        }
+        if (k0 + K > 2) {
+            lane_put(w, o, l, qw, k0, 2, d.nz);
+            lane_put(pgw, o, l, gw, k0, 2, d.nz);
+        }
+        if (i >= 4) {
+            lane_put(u, o, l, qu, k0, 1, d.nz);
+            lane_put(pgu, o, l, gu, k0, 1, d.nz);
+        }
+        // with vghost, update_veloghost_points for the values just written
+        if (vghost) {
+#pragma unroll
+            for (int q = 0; q < K; q++) {
+                const int k = k0 + q;
+                if (k > d.nz) break;
+                if (j >= 2) velo_ghost_point<T>(d, FV, &lane_at(v, o + q, l), i, j, k, qv[q]);
+                if (k >= 2) velo_ghost_point<T>(d, FW, &lane_at(w, o + q, l), i, j, k, qw[q]);
+                if (i >= 4) velo_ghost_point<T>(d, FU, &lane_at(u, o + q, l), i, j, k, qu[q]);
+            }
+        }
+    }
+}
+
 // pressure_gradient alone (2964-3044): pg += grad(phi) - fac A(mu_new)
 // grad(phi) for the components in mask (bit 0 u, 1 v, 2 w) at their
 // unknowns; the gradients at the 7 stencil points are recomputed from phi.
@@ -3584,7 +3761,7 @@ template <typename T>
 static inline dim3 march_grid(const Rng& R, dim3& blk, const Ctx<T>& c, int n, int& np)
 {
     dim3 g = cell_grid(R, blk, KP<T>::value);
-    const double waves = (double)n * c.bt.nm * g.x * g.y * g.z * 4 / simds();
+    const double waves = (double)n * c.bt.nm * c.d.nx * c.d.ny * c.d.nz / (64 * KP<T>::value) / simds();
     np = 1;
     while (np < 8 && waves >= 2 * np * 2.5) np *= 2;
     g.z = (g.z + np - 1) / np * n;
@@ -4120,15 +4297,23 @@ void Ops<T>::velo_correction(Ctx<T>& c, double g, double r, int slot)
 template <typename T>
 void Ops<T>::correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bool ghosts)
 {
+    // the form with several points a thread from 4 of its one-plane waves per
+    // vector unit on (measured at k_corr_pg_run; 64x32x32 has 0.5 in FP64,
+    // 128x64x64 4, 600x20x20 3.7 (8.2 us, several points 9.4) and 150x70x51 8
+    // in FP32)
     dim3 blk;
-    const dim3 grd = bgrid(cell_grid(field_rng(c.d, FC), blk), c);
+    dim3 grd = cell_grid(field_rng(c.d, FC), blk, KP<T>::value);
+    const bool run = (double)c.bt.nm * c.d.nx * c.d.ny * c.d.nz / (64 * KP<T>::value) >= 4.0 * simds();
+    if (run) grd.z = (grd.z + CORR_PLANES - 1) / CORR_PLANES;
+    else grd = cell_grid(field_rng(c.d, FC), blk);
+    grd = bgrid(grd, c);
     const dim3 gf(c.d.ny, c.bt.nm, 1);
     auto go = [&](auto bv) {
         constexpr bool B = decltype(bv)::value;
-        PLLC_L(c, "corr_pg", (k_corr_pg<T, B><<<grd, blk, 0, c.st>>>(c.d, c.ph, mun(c), c.f[PHI], c.f[U_NEW],
-                                                                      c.f[V_NEW], c.f[W_NEW], c.f[U_PG], c.f[V_PG],
-                                                                      c.f[W_PG], c.scal, T(g), T(r), ghosts ? 1 : 0,
-                                                                      c.bt)));
+        auto* k = run ? k_corr_pg_run<T, B> : k_corr_pg<T, B>;
+        PLLC_L(c, "corr_pg", (k<<<grd, blk, 0, c.st>>>(c.d, c.ph, mun(c), c.f[PHI], c.f[U_NEW], c.f[V_NEW],
+                                                       c.f[W_NEW], c.f[U_PG], c.f[V_PG], c.f[W_PG], c.scal, T(g), T(r),
+                                                       ghosts ? 1 : 0, c.bt)));
         PLLC_L(c, "flux", (k_flux_rows<T><<<gf, 64, 0, c.st>>>(c.d, c.f[U_NEW], c.part, c.bt)));
         PLLC_L(c, "flux", (k_flux_apply<T, B><<<gf, 128, 0, c.st>>>(c.d, c.ph, c.f[U_NEW], c.scal, c.part, slot,
                                                                      c.bt)));
