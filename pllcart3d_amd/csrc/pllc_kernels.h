@@ -62,6 +62,9 @@ struct Ctx {
     T* Cfz = nullptr;
     T* Ciy = nullptr;    // REDFT01 matrices
     T* Ciz = nullptr;
+    // the same four matrices in matrix-operand order for k_dct_wide (planes of
+    // at most 128 x 128 without another transform); null when not used
+    T *Ofy = nullptr, *Ofz = nullptr, *Oiy = nullptr, *Oiz = nullptr;
     // twiddles of the fast transform (ny = nz = N, N = 128 or 256): 2N + 1
     // (cos, sin) pairs, see k_dct_plane / k_dct_lines; null when the dense
     // contractions are used
@@ -157,6 +160,9 @@ struct Ops {
     // whether planes of ny x nz (multiples of 16, at most 64) run both dense
     // contractions in one launch (k_dct_planes) with the kernels set up for it
     static bool dct_small_ready(int ny, int nz);
+    // whether planes of ny x nz (at most 128 x 128, any sizes) run both dense
+    // contractions in one launch (k_dct_wide) with the kernels set up for it
+    static bool dct_wide_ready(int ny, int nz);
     // {del, ca, cb, cc} of field F's lines in direction DIR (host, T)
     static void line_consts(const Phys& ph, const Dims& d, int F, int DIR, T* k);
     // whether the fused step of this context has a batched form (FP32,

@@ -2173,6 +2173,149 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
     }
 }
 
+// Dense (y, z) transforms of any plane up to DW_MAX x DW_MAX, both contractions
+// in one launch: one block per plane, which lies in LDS padded with zeros to
+// whole 16 x 16 tiles; the z contraction's tiles are held in registers until
+// every wave has read the plane and then take its place.  A wave makes R
+// tiles that share one operand of the DCT matrix, which it reads from the
+// matrix laid out in operand order (O[(tile row, k / 4)][lane], zero-padded:
+// one coalesced load per matrix instruction group, the same for every block,
+// from L2), the next four steps' loads in flight.  R is the smallest that
+// fits 16 waves (dw_share).  The MFMA sequence of every tile is k_gemm's, so
+// the result equals the two k_gemm launches bit for bit.  us, the two k_gemm
+// launches -> this, forward / inverse: 256x96x96 mixed 36 / 36 -> 19 / 21,
+// 150x70x51 mixed 23 / 23 -> 11 / 12, 97x45x39 FP64 20 / 20 -> 8.4 / 9.0,
+// 256x112x112 FP64 60 / 60 -> 46 / 49, 300x33x120 mixed 24 / 24 -> 24 / 25.
+// k_gemm's 64 x 128 tiles were padding or too few blocks there and Q made a
+// round trip; here a plane's load, its two contractions (6 us of matrix
+// instructions at 96 x 96 FP32) and its store follow each other in the one
+// block of a CU.  The whole plane's loads in flight at once instead of four a
+// thread: no faster.
+constexpr int DW_MAX = 128;
+__host__ __device__ constexpr int dw_tiles(int n) { return (n + 15) / 16; }
+__host__ __device__ constexpr int dw_pitch(int nz) { return 16 * dw_tiles(nz) + 4; }
+// tiles per wave along one direction (t tiles) with `other` tiles across
+__host__ __device__ constexpr int dw_share(int t, int other)
+{
+    int r = 1;
+    while (other * ((t + r - 1) / r) > 16) r++;
+    return r;
+}
+__host__ __device__ constexpr int dw_waves(int ny, int nz)
+{
+    const int ty = dw_tiles(ny), tz = dw_tiles(nz), ry = dw_share(ty, tz), rz = dw_share(tz, ty);
+    const int a = tz * ((ty + ry - 1) / ry), b = ty * ((tz + rz - 1) / rz);
+    return a > b ? a : b;
+}
+
+// R accumulators over kt steps of 4: op(u, k) the shared-memory operand of
+// tile u, O the other one; TA: O is the A operand
+template <typename T, int R, bool TA, typename F>
+__device__ __forceinline__ void dw_contract(typename Mma<T>::acc (&acc)[4], const T* __restrict__ O, int kt, F op)
+{
+    typedef typename Mma<T>::acc acc_t;
+#pragma unroll
+    for (int u = 0; u < R; u++) acc[u] = acc_t{T(0), T(0), T(0), T(0)};
+    T nx[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) nx[t] = O[64 * t];
+    for (int k = 0; k < kt; k += 4) {   // kt is a multiple of 4
+        T cu[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) cu[t] = nx[t];
+        if (k + 4 < kt) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) nx[t] = O[64 * (k + 4 + t)];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                const T x = op(u, 4 * (k + t));
+                acc[u] = TA ? Mma<T>::run(cu[t], x, acc[u]) : Mma<T>::run(x, cu[t], acc[u]);
+            }
+    }
+}
+
+template <typename T, bool INV>
+__global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* __restrict__ in, T* __restrict__ out,
+                                                   const T* __restrict__ Oz, const T* __restrict__ Oy, PhiOut<T> po)
+{
+    extern __shared__ unsigned char pllc_smem[];
+    typedef typename Mma<T>::acc acc_t;
+    T* P = reinterpret_cast<T*>(pllc_smem);   // [16 ty][pz]
+    const int ty = dw_tiles(ny), tz = dw_tiles(nz), pz = dw_pitch(nz);
+    const int ry = dw_share(ty, tz), rz = dw_share(tz, ty);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const long plane = (long)ny * nz;
+    const T* __restrict__ src = in + blockIdx.x * plane;
+    const int cells = 256 * ty * tz, nzp = 16 * tz;
+    for (int e0 = threadIdx.x; e0 < cells; e0 += 4 * blockDim.x) {
+        T v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int e = e0 + q * blockDim.x, y = e / nzp, z = e - y * nzp;
+            v[q] = y < ny && z < nz ? src[(long)y * nz + z] : T(0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int e = e0 + q * blockDim.x, y = e / nzp, z = e - y * nzp;
+            if (e < cells) P[y * pz + z] = v[q];
+        }
+    }
+    __syncthreads();
+    acc_t acc[4];
+    // z: Q[y][kz] = sum_m P[y][m] Cz[kz][m]; wave: column tile zt, row tiles
+    // y0 .. y0 + ry - 1 (past the last: the last again, not stored)
+    {
+        const int zt = wave % tz, y0 = wave / tz * ry;
+        const bool on = y0 < ty;
+        const T* a = P + li * pz + lk;
+        auto op = [&](int u, int k) { return a[16 * min(y0 + u, ty - 1) * pz + k]; };
+        const T* O = Oz + (long)zt * tz * 256 + lane;
+        if (on) {
+            if (ry == 1) dw_contract<T, 1, false>(acc, O, 4 * tz, op);
+            else if (ry == 2) dw_contract<T, 2, false>(acc, O, 4 * tz, op);
+            else if (ry == 3) dw_contract<T, 3, false>(acc, O, 4 * tz, op);
+            else dw_contract<T, 4, false>(acc, O, 4 * tz, op);
+        }
+        __syncthreads();   // the plane read by every wave
+        if (on) {
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (u < ry && y0 + u < ty) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) P[(16 * (y0 + u) + Mma<T>::row(lk, r)) * pz + 16 * zt + li] = acc[u][r];
+                }
+        }
+        __syncthreads();
+    }
+    // y: out[ky][kz] = sum_m Cy[ky][m] Q[m][kz]; wave: row tile yt, column
+    // tiles z0 .. z0 + rz - 1
+    const int yt = wave % ty, z0 = wave / ty * rz;
+    if (z0 >= tz) return;
+    const T* b = P + lk * pz + li;
+    auto op = [&](int u, int k) { return b[k * pz + 16 * min(z0 + u, tz - 1)]; };
+    const T* O = Oy + (long)yt * ty * 256 + lane;
+    if (rz == 1) dw_contract<T, 1, true>(acc, O, 4 * ty, op);
+    else if (rz == 2) dw_contract<T, 2, true>(acc, O, 4 * ty, op);
+    else if (rz == 3) dw_contract<T, 3, true>(acc, O, 4 * ty, op);
+    else dw_contract<T, 4, true>(acc, O, 4 * ty, op);
+    const T norm = T(4 * po.ny * po.nz);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        if (u >= rz || z0 + u >= tz) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int gm = 16 * yt + Mma<T>::row(lk, r), gn = 16 * (z0 + u) + li;
+            if (gm >= ny || gn >= nz) continue;
+            if (INV && po.phi) phi_store(po, (int)blockIdx.x, gm, gn, fdiv<T>(acc[u][r], norm));
+            else out[blockIdx.x * plane + (long)gm * nz + gn] = acc[u][r];
+        }
+    }
+}
+
 // ------------------------------------------------- fast DCT of planes
 //
 // The (y, z) transforms of phisolver_dct for ny = nz = N, N = 128 or 256
@@ -2900,6 +3043,8 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     PLLC_INST_DCT_PLANES(T, 32)                                                                                \
     PLLC_INST_DCT_PLANES(T, 48)                                                                                \
     PLLC_INST_DCT_PLANES(T, 64)                                                                                \
+    template __global__ void k_dct_wide<T, false>(int, int, const T*, T*, const T*, const T*, PhiOut<T>);      \
+    template __global__ void k_dct_wide<T, true>(int, int, const T*, T*, const T*, const T*, PhiOut<T>);       \
     template __global__ void k_gemm<T, true>(int, int, int, const T*, long, const T*, long, T*, long,          \
                                              PhiOut<T>);                                                        \
     template __global__ void k_gemm<T, false>(int, int, int, const T*, long, const T*, long, T*, long,         \
@@ -4150,6 +4295,20 @@ bool Ops<T>::dct_small_ready(int ny, int nz)
 }
 
 template <typename T>
+static int dct_wide_lds(int ny, int nz)
+{
+    return 16 * dw_tiles(ny) * dw_pitch(nz) * (int)sizeof(T);
+}
+
+template <typename T>
+bool Ops<T>::dct_wide_ready(int ny, int nz)
+{
+    if (ny > DW_MAX || nz > DW_MAX) return false;
+    const int sm = dct_wide_lds<T>(ny, nz);
+    return lds_optin((const void*)k_dct_wide<T, false>, sm) && lds_optin((const void*)k_dct_wide<T, true>, sm);
+}
+
+template <typename T>
 bool Ops<T>::dct_fast_ready(int n)
 {
     if (n == FD_N) {
@@ -4226,6 +4385,16 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         return;
     }
     if (!single(c, "dct2")) return;
+    if (c.Ofz) {
+        const size_t sm = (size_t)dct_wide_lds<T>(ny, nz);
+        const int nthr = 64 * dw_waves(ny, nz);
+        const PhiOut<T> po{inverse ? phi : nullptr, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
+        if (inverse)
+            PLLC_L(c, "dct", (k_dct_wide<T, true><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Oiz, c.Oiy, po)));
+        else
+            PLLC_L(c, "dct", (k_dct_wide<T, false><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Ofz, c.Ofy, po)));
+        return;
+    }
     const long R = (long)nx * ny, plane = (long)ny * nz;
     const dim3 gz((nz + 127) / 128, (unsigned)((R + 63) / 64), 1), gy((nz + 127) / 128, (ny + 63) / 64, nx);
     if (!inverse) {

@@ -364,6 +364,22 @@ bool pllc_ctx_tables(Ctx<T>& c, std::vector<void*>& owned, const char* where)
         for (size_t e = 0; e < w.size(); e++) wt[e] = T(w[e]);
         if (!pllc_hip_ok(where, hipMemcpy(c.tw, wt.data(), wt.size() * ts, hipMemcpyHostToDevice))) return false;
     }
+    // other planes of at most 128 x 128: both dense contractions in one launch
+    // (PLLC_DCT=gemm: two), the matrices in operand order: tile row t, step k
+    // of 4 columns, lane: C[16 t + lane % 16][4 k + lane / 16], zero past n
+    if (!c.tw && !c.cbf && !c.dsmall && !(dm && strcmp(dm, "gemm") == 0) && Ops<T>::dct_wide_ready(d.ny, d.nz)) {
+        T** dst[4] = {&c.Ofy, &c.Oiy, &c.Ofz, &c.Oiz};
+        for (int q = 0; q < 4; q++) {
+            const int m = q < 2 ? d.ny : d.nz, tiles = (m + 15) / 16;
+            pllc_dct_matrix(m, q & 1, h.data());
+            std::vector<T> o((size_t)tiles * tiles * 256, T(0));
+            for (int a = 0; a < m; a++)
+                for (int b = 0; b < m; b++)
+                    o[(((size_t)(a / 16) * tiles * 4 + b / 4) * 4 + b % 4) * 16 + a % 16] = T(h[(size_t)a * m + b]);
+            if (!get((void**)dst[q], o.size() * ts)) return false;
+            if (!pllc_hip_ok(where, hipMemcpy(*dst[q], o.data(), o.size() * ts, hipMemcpyHostToDevice))) return false;
+        }
+    }
     return true;
 }
 template bool pllc_ctx_tables<double>(Ctx<double>&, std::vector<void*>&, const char*);
