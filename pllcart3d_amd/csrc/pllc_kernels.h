@@ -127,7 +127,9 @@ struct Ops {
     static void velo_correction(Ctx<T>& c, double g, double r, int slot);
     // mask bit 0 u, bit 1 v, bit 2 w; coefficients A(mu) from c.f[MUN_*]
     static void pressure_gradient(Ctx<T>& c, double g, double r, int mask);
-    static void cfl(Ctx<T>& c);
+    // start: also what the first substage starts with (bulk_stale for slot 0
+    // with alpha, advancing tval), in the same launches where the plane allows it
+    static void cfl(Ctx<T>& c, bool start = false, double alpha = 0.0);
     static void bulk(Ctx<T>& c, int slot, double alpha, bool advance_t);
     // bulk() and stale() in one launch where the plane allows it
     static void bulk_stale(Ctx<T>& c, int slot, double alpha, bool advance_t, const T* qc, const T* qu, const T* qv,
@@ -140,7 +142,11 @@ struct Ops {
     // velocity correction, outflow deficit and the pressure-gradient update
     // of all three components (mu_new) in one pass over the cells
     // ghosts: also update_veloghost_points' ghost copies of the corrected values
-    static void correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bool ghosts = false);
+    // next >= 0: where the plane allows it (true returned) also what substage
+    // next starts with from the fields this one made: bulk_stale for slot next
+    // with alpha, advancing tval
+    static bool correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bool ghosts = false, int next = -1,
+                                        double alpha = 0.0);
     // shift_conc on field q: every (j,k) line re-sampled at Xc - shift[k]
     // (x: the NX cell centres, shift: NZ values, both on the device)
     static void shift_conc(Ctx<T>& c, T* q, const double* x, const double* shift);

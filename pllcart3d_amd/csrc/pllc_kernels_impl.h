@@ -1693,47 +1693,6 @@ __global__ __launch_bounds__(256) void k_cfl_partial(Dims d, const T* __restrict
     }
 }
 
-// pass 2: max over the partials; dt = min(CFLmax/max, Timestep)
-// (pllcart3d.c:159-160, 3115)
-// (one block of 1024 threads, eight loads per thread in flight per round;
-// a max in any order is the same value)
-template <typename T>
-__global__ __launch_bounds__(1024) void k_cfl_final(const double* __restrict__ part, long np, double CFLmax,
-                                                    double Timestep, double* __restrict__ scal, Bt bt)
-{
-    constexpr int NT = 1024, U = 8;
-    __shared__ double red[NT];
-    // member: blockIdx.x
-    if (bt.ph) {
-        CFLmax = bt.ph[blockIdx.x].CFLmax;
-        Timestep = bt.ph[blockIdx.x].Timestep;
-    }
-    part += blockIdx.x * bt.np;
-    scal += blockIdx.x * S_SIZE;
-    const int t = threadIdx.x;
-    double m = 0.0;
-    long l = t;
-    for (; l + (U - 1) * NT < np; l += U * NT) {
-        double a[U];
-#pragma unroll
-        for (int q = 0; q < U; q++) a[q] = part[l + q * NT];
-#pragma unroll
-        for (int q = 0; q < U; q++) m = m > a[q] ? m : a[q];
-    }
-    for (; l < np; l += NT) m = m > part[l] ? m : part[l];
-    red[t] = m;
-    __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if (t < s) red[t] = red[t] > red[t + s] ? red[t] : red[t + s];
-        __syncthreads();
-    }
-    if (t == 0) {
-        const double cfldt = CFLmax / red[0];
-        scal[S_CFL] = red[0];
-        scal[S_DT] = (cfldt < Timestep) ? cfldt : Timestep;
-    }
-}
-
 // bulk_velo (3381-3398): the signed u of largest |u| on the plane iend,
 // the first hit in (j,k) order winning ties.  Pass 1: per-block candidates
 // (value, scan index); pass 2: one block picks the winner, and advances the
@@ -1796,40 +1755,18 @@ __global__ __launch_bounds__(256) void k_bulk_final(const double* __restrict__ p
     }
 }
 
-// bulk_velo in one block over the whole plane (ny nz <= BULK1_MAX): each
-// thread scans its points in increasing index, then a tree over the block;
-// the winner (largest |u|, first index among ties) is the same in any order.
-// With q0 set, block 1 computes the 16 stale values (k_stale) meanwhile.
-constexpr int BULK1_MAX = 65536;
+// bulk_velo in one block of BULK_NT threads over the whole plane (ny nz <=
+// BULK1_MAX): each thread scans its points in increasing index, then a tree
+// over the block; the winner (largest |u|, first index among ties) is the
+// same in any order.
+constexpr int BULK1_MAX = 65536, BULK_NT = 1024;
 template <typename T>
-__global__ __launch_bounds__(1024) void k_bulk_stale(Dims d, const T* __restrict__ u, double* __restrict__ scal,
-                                                     int rk, double alpha, double* __restrict__ tval,
-                                                     const T* __restrict__ q0, const T* __restrict__ q1,
-                                                     const T* __restrict__ q2, const T* __restrict__ q3,
-                                                     T* __restrict__ stale, Bt bt)
+__device__ __forceinline__ void bulk_block(const Dims& d, const T* u, double* __restrict__ out, double* sv, long* si)
 {
-    constexpr int NT = 1024, U = 8;
+    constexpr int NT = BULK_NT, U = 8;
     const int t = threadIdx.x;
-    // member: blockIdx.y
-    {
-        const int mb = blockIdx.y;
-        u = bt_f(bt, u, mb);
-        q0 = bt_f(bt, q0, mb);
-        q1 = bt_f(bt, q1, mb);
-        q2 = bt_f(bt, q2, mb);
-        q3 = bt_f(bt, q3, mb);
-        scal += mb * S_SIZE;
-        if (tval) tval += mb;
-        if (stale) stale += mb * 16;
-    }
-    if (blockIdx.x == 1) {
-        if (t < 16) stale[t] = stale_value<T>(d, q0, q1, q2, q3, t);
-        return;
-    }
-    __shared__ double sv[NT];
-    __shared__ long si[NT];
     const int np = d.ny * d.nz;
-    const T* __restrict__ pl = u + IX(d, d.nx + 2, 1, 1);
+    const T* pl = u + IX(d, d.nx + 2, 1, 1);
     double v = 0.0;
     long id = -1;
     auto take = [&](double x, long l) {
@@ -1853,10 +1790,182 @@ __global__ __launch_bounds__(1024) void k_bulk_stale(Dims d, const T* __restrict
         if (t < s2 && bulk_better(sv[t + s2], si[t + s2], sv[t], si[t])) { sv[t] = sv[t + s2]; si[t] = si[t + s2]; }
         __syncthreads();
     }
-    if (t == 0) {
-        scal[S_RK + 4 * rk] = si[0] < 0 ? 0.0 : sv[0];
-        if (tval) tval[0] = tval[0] + alpha * scal[S_DT];
+    if (t == 0) *out = si[0] < 0 ? 0.0 : sv[0];
+}
+
+// pass 2: max over the partials; dt = min(CFLmax/max, Timestep)
+// (pllcart3d.c:159-160, 3115)
+// (one block of 1024 threads, eight loads per thread in flight per round;
+// a max in any order is the same value).  With tval the first substage's start
+// rides in the launch: block row 1 computes bulk_velo's value, row 2 the stale
+// values, and row 0 advances tval by alpha dt.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_cfl_final(const double* __restrict__ part, long np, double CFLmax,
+                                                    double Timestep, double* __restrict__ scal, Dims d, double alpha,
+                                                    double* __restrict__ tval, const T* __restrict__ q0,
+                                                    const T* __restrict__ q1, const T* __restrict__ q2,
+                                                    const T* __restrict__ q3, T* __restrict__ stale, Bt bt)
+{
+    constexpr int NT = 1024, U = 8;
+    static_assert(NT == BULK_NT, "a bulk_block");
+    __shared__ double red[NT];
+    __shared__ long si[NT];
+    if (blockIdx.y) {
+        const int m = blockIdx.x;
+        if (blockIdx.y == 1)
+            bulk_block<T>(d, bt_f(bt, q1, m), scal + m * S_SIZE + S_RK, red, si);
+        else if (threadIdx.x < 16)
+            stale[m * 16 + threadIdx.x] = stale_value<T>(d, bt_f(bt, q0, m), bt_f(bt, q1, m), bt_f(bt, q2, m),
+                                                         bt_f(bt, q3, m), threadIdx.x);
+        return;
     }
+    // member: blockIdx.x
+    if (bt.ph) {
+        CFLmax = bt.ph[blockIdx.x].CFLmax;
+        Timestep = bt.ph[blockIdx.x].Timestep;
+    }
+    part += blockIdx.x * bt.np;
+    scal += blockIdx.x * S_SIZE;
+    const int t = threadIdx.x;
+    double m = 0.0;
+    long l = t;
+    for (; l + (U - 1) * NT < np; l += U * NT) {
+        double a[U];
+#pragma unroll
+        for (int q = 0; q < U; q++) a[q] = part[l + q * NT];
+#pragma unroll
+        for (int q = 0; q < U; q++) m = m > a[q] ? m : a[q];
+    }
+    for (; l < np; l += NT) m = m > part[l] ? m : part[l];
+    red[t] = m;
+    __syncthreads();
+    for (int s = NT / 2; s > 0; s >>= 1) {
+        if (t < s) red[t] = red[t] > red[t + s] ? red[t] : red[t + s];
+        __syncthreads();
+    }
+    if (t == 0) {
+        const double cfldt = CFLmax / red[0];
+        scal[S_CFL] = red[0];
+        const double dt = (cfldt < Timestep) ? cfldt : Timestep;
+        scal[S_DT] = dt;
+        if (tval) tval[blockIdx.x] = tval[blockIdx.x] + alpha * dt;
+    }
+}
+
+// bulk_velo, and with q0 set the 16 stale values (k_stale) in block 1
+template <typename T>
+__global__ __launch_bounds__(1024) void k_bulk_stale(Dims d, const T* __restrict__ u, double* __restrict__ scal,
+                                                     int rk, double alpha, double* __restrict__ tval,
+                                                     const T* __restrict__ q0, const T* __restrict__ q1,
+                                                     const T* __restrict__ q2, const T* __restrict__ q3,
+                                                     T* __restrict__ stale, Bt bt)
+{
+    __shared__ double sv[BULK_NT];
+    __shared__ long si[BULK_NT];
+    // member: blockIdx.y
+    const int mb = blockIdx.y, t = threadIdx.x;
+    scal += mb * S_SIZE;
+    if (blockIdx.x == 1) {
+        if (t < 16)
+            stale[mb * 16 + t] = stale_value<T>(d, bt_f(bt, q0, mb), bt_f(bt, q1, mb), bt_f(bt, q2, mb),
+                                                bt_f(bt, q3, mb), t);
+        return;
+    }
+    bulk_block<T>(d, bt_f(bt, u, mb), scal + S_RK + 4 * rk, sv, si);
+    if (t == 0 && tval) tval[mb] = tval[mb] + alpha * scal[S_DT];
+}
+
+// What a substage ends with on planes of at most FE_MAX x FE_MAX, and what
+// the next one starts with, in one launch instead of three (k_flux_rows,
+// k_flux_apply, k_bulk_stale: 4.7 to 5.4 us each at 64x32x32, the floor of a
+// launch): block 0 sums both faces' rows as k_flux_rows does (FE_K columns of
+// every row at a time through LDS, the next ones in flight; a thread a row),
+// forms and adds the deficit as k_flux_apply does, and with next >= 0
+// computes the 16 stale values (they may read the outlet face) of the new
+// fields; block 1 then computes bulk_velo's value for substage next (its plane
+// is the one before the outlet face) and advances tval.  us, the three launches
+// -> this: 64x32x32 FP64 14 -> 5.4, 150x70x51 mixed 15 -> 8.2, 256x128x128 FP64
+// 22 -> 19, mixed 21 -> 15; the sums' serial chains are what is left, so larger
+// planes keep a block per row.
+constexpr int FE_MAX = 128, FE_K = 16;
+template <typename T, bool B = false>
+__global__ __launch_bounds__(1024) void k_step_end(Dims d, Phys ph0, T* u0, double* __restrict__ scal, int rk, int next,
+                                                   double alpha, double* __restrict__ tval, const T* __restrict__ q0,
+                                                   const T* __restrict__ q2, const T* __restrict__ q3,
+                                                   T* __restrict__ stale, Bt bt)
+{
+    __shared__ union {
+        struct { double x[2][FE_MAX][FE_K + 1], rows[2][FE_MAX + 1], sum[2]; } f;
+        struct { double sv[BULK_NT]; long si[BULK_NT]; } b;
+    } sh;
+    // member: blockIdx.y
+    const int m = blockIdx.y, t = threadIdx.x;
+    T* u = bt_f(bt, u0, m);
+    scal += m * S_SIZE;
+    if (blockIdx.x == 1) {
+        bulk_block<T>(d, u, scal + S_RK + 4 * next, sh.b.sv, sh.b.si);
+        if (t == 0) tval[m] = tval[m] + alpha * scal[S_DT];
+        return;
+    }
+    const Phys& ph = bt_phys<B>(bt, ph0, m);
+    const T* face[2] = {u + IX(d, 3, 1, 1), u + IX(d, d.nx + 3, 1, 1)};
+    constexpr int U = 2 * FE_MAX * FE_K / 1024;
+    T v[U];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            const int e = t + 1024 * q, k = k0 + (e & (FE_K - 1)), r = (e / FE_K) & (FE_MAX - 1), s = e / (FE_K * FE_MAX);
+            if (r < d.ny && k < d.nz) v[q] = face[s][(long)r * d.sy + k];
+        }
+    };
+    const int s = t >> 7, r = t & (FE_MAX - 1);   // the face and row of t < 256
+    const bool sums = t < 2 * FE_MAX && r < d.ny;
+    const double hz = d.dz, hy = d.dy;
+    double q = 0.0, last = 0.0;
+    fetch(0);
+    for (int k0 = 0; k0 < d.nz; k0 += FE_K) {
+        __syncthreads();   // the columns before read
+#pragma unroll
+        for (int p = 0; p < U; p++) {
+            const int e = t + 1024 * p;
+            sh.f.x[e / (FE_K * FE_MAX)][(e / FE_K) & (FE_MAX - 1)][e & (FE_K - 1)] = (double)v[p];
+        }
+        __syncthreads();
+        if (k0 + FE_K < d.nz) fetch(k0 + FE_K);
+        if (sums) {
+            const int n = min(FE_K, d.nz - k0);
+            for (int k = 0; k < n; k++) {
+                const double x = sh.f.x[s][r][k];
+                if (k0 + k > 0) q += 0.5 * hz * (x + last);
+                last = x;
+            }
+        }
+    }
+    if (sums) sh.f.rows[s][r + 1] = q;
+    __syncthreads();
+    if (t == 0 || t == 64) {   // a wave each
+        const double* qk = sh.f.rows[t >> 6];
+        double a = 0.0;
+        for (int j = 2; j <= d.ny; j++) a += 0.5 * hy * (qk[j - 1] + qk[j]);
+        sh.f.sum[t >> 6] = a;
+    }
+    __syncthreads();
+    const double qin = sh.f.sum[0], qout = sh.f.sum[1];
+    const double deficit = (qin - qout) / ((ph.Y2 - ph.Y1) * (ph.Z2 - ph.Z1));
+    if (t == 0) {
+        scal[S_RK + 4 * rk + 1] = qin;
+        scal[S_RK + 4 * rk + 2] = qout;
+        scal[S_RK + 4 * rk + 3] = deficit;
+    }
+    const T dv = T(deficit);
+    T* out = u + IX(d, d.nx + 3, 1, 1);
+    for (int e = t; e < d.ny * FE_MAX; e += 1024) {
+        const int j = e / FE_MAX, k = e & (FE_MAX - 1);
+        if (k < d.nz) out[(long)j * d.sy + k] += dv;
+    }
+    if (next < 0) return;
+    __syncthreads();
+    if (t < 16) stale[m * 16 + t] = stale_value<T>(d, bt_f(bt, q0, m), u, bt_f(bt, q2, m), bt_f(bt, q3, m), t);
 }
 
 // ---------------------------------------------------------------- DCT GEMM
@@ -4464,7 +4573,7 @@ void Ops<T>::velo_correction(Ctx<T>& c, double g, double r, int slot)
 }
 
 template <typename T>
-void Ops<T>::correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bool ghosts)
+bool Ops<T>::correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bool ghosts, int next, double alpha)
 {
     // the form with several points a thread from 4 of its one-plane waves per
     // vector unit on (measured at k_corr_pg_run; 64x32x32 has 0.5 in FP64,
@@ -4477,18 +4586,26 @@ void Ops<T>::correction_and_gradient(Ctx<T>& c, double g, double r, int slot, bo
     else grd = cell_grid(field_rng(c.d, FC), blk);
     grd = bgrid(grd, c);
     const dim3 gf(c.d.ny, c.bt.nm, 1);
+    const bool small = c.d.ny <= FE_MAX && c.d.nz <= FE_MAX;
     auto go = [&](auto bv) {
         constexpr bool B = decltype(bv)::value;
         auto* k = run ? k_corr_pg_run<T, B> : k_corr_pg<T, B>;
         PLLC_L(c, "corr_pg", (k<<<grd, blk, 0, c.st>>>(c.d, c.ph, mun(c), c.f[PHI], c.f[U_NEW], c.f[V_NEW],
                                                        c.f[W_NEW], c.f[U_PG], c.f[V_PG], c.f[W_PG], c.scal, T(g), T(r),
                                                        ghosts ? 1 : 0, c.bt)));
+        if (small) {
+            PLLC_L(c, "flux", (k_step_end<T, B><<<dim3(next < 0 ? 1 : 2, c.bt.nm), 1024, 0, c.st>>>(
+                                  c.d, c.ph, c.f[U_NEW], c.scal, slot, next, alpha, c.tval, c.f[C_NEW], c.f[V_NEW],
+                                  c.f[W_NEW], c.stale, c.bt)));
+            return;
+        }
         PLLC_L(c, "flux", (k_flux_rows<T><<<gf, 64, 0, c.st>>>(c.d, c.f[U_NEW], c.part, c.bt)));
         PLLC_L(c, "flux", (k_flux_apply<T, B><<<gf, 128, 0, c.st>>>(c.d, c.ph, c.f[U_NEW], c.scal, c.part, slot,
                                                                      c.bt)));
     };
     if (c.bt.nm > 1) go(std::true_type{});
     else go(std::false_type{});
+    return small;
 }
 
 template <typename T>
@@ -4502,16 +4619,19 @@ void Ops<T>::pressure_gradient(Ctx<T>& c, double g, double r, int mask)
 }
 
 template <typename T>
-void Ops<T>::cfl(Ctx<T>& c)
+void Ops<T>::cfl(Ctx<T>& c, bool start, double alpha)
 {
     dim3 blk;
     dim3 grd = cell_grid(field_rng(c.d, FC), blk);
     grd.z = (c.d.nx + CFL_PLANES - 1) / CFL_PLANES;
+    const bool with = start && (long)c.d.ny * c.d.nz <= BULK1_MAX;
     // partials of member m at m * bt.np (one per block)
     PLLC_L(c, "cfl", (k_cfl_partial<T><<<bgrid(grd, c), blk, 0, c.st>>>(c.d, c.f[U_OLD], c.f[V_OLD], c.f[W_OLD],
                                                                         c.part, c.bt)));
-    PLLC_L(c, "cfl", (k_cfl_final<T><<<c.bt.nm, 1024, 0, c.st>>>(c.part, (long)grd.x * grd.y * grd.z, c.ph.CFLmax,
-                                                                c.ph.Timestep, c.scal, c.bt)));
+    PLLC_L(c, "cfl", (k_cfl_final<T><<<dim3(c.bt.nm, with ? 3 : 1), 1024, 0, c.st>>>(
+                         c.part, (long)grd.x * grd.y * grd.z, c.ph.CFLmax, c.ph.Timestep, c.scal, c.d, alpha,
+                         with ? c.tval : nullptr, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], c.stale, c.bt)));
+    if (start && !with) bulk_stale(c, 0, alpha, true, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
 }
 
 template <typename T>

@@ -816,10 +816,13 @@ extern "C" double pllc_sim_op(pllc_sim* s, int op, double dt, int rk, double vbu
 template <typename T>
 static void fused_step(pllc_sim* s, Ctx<T>& c)
 {
-    Ops<T>::cfl(c);
+    // a substage starts with bulk_velo and the stale values of its old fields:
+    // in the launch that ends what came before where the plane allows it
+    Ops<T>::cfl(c, true, kRK1[0] + kRK2[0]);
+    bool started = true;
     for (int rk = 0; rk < 3; rk++) {
         const double g = kRK1[rk], r = kRK2[rk];
-        Ops<T>::bulk_stale(c, rk, g + r, true, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
+        if (!started) Ops<T>::bulk_stale(c, rk, g + r, true, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
         // the learned closure's correction of N from the substage's start
         // state (c, u, v, w and mu_old.cell)
         if (s->cnn && c.ncorr && (s->cnn_every == 0 || (rk == 0 && s->cnn_steps % s->cnn_every == 0)))
@@ -844,7 +847,8 @@ static void fused_step(pllc_sim* s, Ctx<T>& c)
         Ops<T>::divergence(c, g, r, false, true);
         Ops<T>::poisson(c, g, r, false, true);   // with update_phi_ghosts
         // velo_correction + pressure_gradient + update_veloghost_points
-        Ops<T>::correction_and_gradient(c, g, r, rk, true);
+        const int next = rk < 2 ? rk + 1 : -1;
+        started = Ops<T>::correction_and_gradient(c, g, r, rk, true, next, next < 0 ? 0.0 : kRK1[next] + kRK2[next]);
         if (s->copy_next) {
             update_old_copy<T>(c);
             s->copy_next = false;
