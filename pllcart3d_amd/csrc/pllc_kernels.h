@@ -100,6 +100,8 @@ struct Ctx {
     int joint = 0;
 };
 
+template <typename T> struct DivIn;
+
 // Operator launchers.  g, r are the RK coefficients (rk_gamma, rk_rho) the
 // reference passes by value; `slot` selects the device scalars of the
 // substage (vbulk, fluxes, deficit).  All launches go to c.st.
@@ -121,8 +123,10 @@ struct Ops {
     static void momentum3_implicit(Ctx<T>& c, double g, double r, int slot, bool ghosts);
     static void velo_ghost(Ctx<T>& c);
     static void divergence(Ctx<T>& c, double g, double r, bool write_div, bool pack);
-    // ghosts: phi's face ghosts too (update_phi_ghosts) in the same pass
-    static void poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts = false);
+    // ghosts: phi's face ghosts too (update_phi_ghosts) in the same pass;
+    // from_velo: the right-hand side from the new velocities (divergence and
+    // its packing in the forward transform), else from DIV or the packed block
+    static void poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts = false, bool from_velo = false);
     static void phi_ghost(Ctx<T>& c);
     static void velo_correction(Ctx<T>& c, double g, double r, int slot);
     // mask bit 0 u, bit 1 v, bit 2 w; coefficients A(mu) from c.f[MUN_*]
@@ -155,7 +159,8 @@ struct Ops {
     // dense 2D DCT of a packed block: REDFT10 (forward) or REDFT01
     // (inverse), z then y, `in` -> `out` through the temporary c.Q
     // phi (inverse only): the result goes to phi's interior instead of out
-    static void dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi = nullptr, bool ghosts = false);
+    static void dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi = nullptr, bool ghosts = false,
+                     const DivIn<T>* div = nullptr);
     // whether there is a fast transform for ny = nz = n and the device gives
     // its blocks the LDS it needs (n = 128: a whole plane of T; n = 256: 32
     // lines), with the kernels set up to use it

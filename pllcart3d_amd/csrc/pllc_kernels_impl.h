@@ -2001,6 +2001,38 @@ template <> struct Mma<float> {
     }
 };
 
+// Source of a forward transform's first contraction: the packed block `in`, or
+// with u set the Poisson right-hand side itself, Re / (dt (g + r)) times the
+// divergence of the new velocities (k_div's expressions), so that the packed
+// block is not made first (one launch and two passes over it less).  us, k_div
+// and the transform -> this: 256x128x128 FP64 58 -> 46, mixed 39 -> 27;
+// 512x256x256 FP64 395 -> 344, mixed 190 -> 121 (rows pass); 256x96x96 mixed 31
+// -> 25; 64x32x32 FP64 10 -> 6.8.
+template <typename T>
+struct DivIn {
+    const T *u, *v, *w;
+    const double* scal;
+    Dims d;
+    double Re;
+    T gr;
+    // member m's factor
+    __device__ __forceinline__ T fac(const Bt& bt, int m) const
+    {
+        const double re = bt.ph ? bt.ph[m].Re : Re;
+        return T(re) / (T(scal[m * S_SIZE + S_DT]) * gr);
+    }
+    // point (x, y, z) of the packed block, from the member's first value on
+    __device__ __forceinline__ T at(long mo, T fac, int x, int y, int z) const
+    {
+        const long o = IX(d, x + 3, y + 1, z + 1) + mo;
+        const T dvx = divh<T>(u[o + d.sx] - u[o], T(d.dx), d.rdx);
+        const T dvy = divh<T>(v[o + d.sy] - v[o], T(d.dy), d.rdy);
+        const T dvz = divh<T>(w[o + 1] - w[o], T(d.dz), d.rdz);
+        const T dv = (dvx + dvy + dvz);
+        return fac * dv;
+    }
+};
+
 // Epilogue of the last inverse contraction when phi is set: batch b, row
 // gm, column gn of the packed [x][y][z] block is phi's interior point
 // (3 + b, 1 + gm, 1 + gn), divided by the inverse transform's norm 4 ny nz
@@ -2164,7 +2196,7 @@ __host__ __device__ constexpr int dct_planes_threads(int N) { return N ? 4 * N :
 template <typename T, bool INV, int N>
 __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, int nplanes, const T* __restrict__ in,
                                                     T* __restrict__ out, const T* __restrict__ Cz,
-                                                    const T* __restrict__ Cy, PhiOut<T> po, Bt bt)
+                                                    const T* __restrict__ Cy, PhiOut<T> po, DivIn<T> dv, Bt bt)
 {
     static_assert(N % 16 == 0 && N <= DS_MAX, "square planes of 16 .. 64");
     extern __shared__ unsigned char pllc_smem[];
@@ -2200,6 +2232,16 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
     }
     T pf[PF];
     auto fetch = [&](int p) {
+        if (!INV && dv.u) {
+            const int m = p / nx, x = p - m * nx;
+            const T f = dv.fac(bt, m);
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                const int e = threadIdx.x + NT * u, y = e / nz;
+                if (N || e < plane) pf[u] = dv.at(m * bt.fs, f, x, y, e - y * nz);
+            }
+            return;
+        }
         const T* __restrict__ src = in + (long)p * plane;
 #pragma unroll
         for (int u = 0; u < PF; u++) {
@@ -2348,7 +2390,8 @@ __device__ __forceinline__ void dw_contract(typename Mma<T>::acc (&acc)[4], cons
 
 template <typename T, bool INV>
 __global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* __restrict__ in, T* __restrict__ out,
-                                                   const T* __restrict__ Oz, const T* __restrict__ Oy, PhiOut<T> po)
+                                                   const T* __restrict__ Oz, const T* __restrict__ Oy, PhiOut<T> po,
+                                                   DivIn<T> dv)
 {
     extern __shared__ unsigned char pllc_smem[];
     typedef typename Mma<T>::acc acc_t;
@@ -2360,12 +2403,15 @@ __global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* __re
     const long plane = (long)ny * nz;
     const T* __restrict__ src = in + blockIdx.x * plane;
     const int cells = 256 * ty * tz, nzp = 16 * tz;
+    const bool fused = !INV && dv.u;
+    const T f = fused ? dv.fac(Bt{}, 0) : T(0);
     for (int e0 = threadIdx.x; e0 < cells; e0 += 4 * blockDim.x) {
         T v[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const int e = e0 + q * blockDim.x, y = e / nzp, z = e - y * nzp;
-            v[q] = y < ny && z < nz ? src[(long)y * nz + z] : T(0);
+            v[q] = T(0);
+            if (y < ny && z < nz) v[q] = fused ? dv.at(0, f, blockIdx.x, y, z) : src[(long)y * nz + z];
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -2685,7 +2731,7 @@ template <typename T> struct FdCfg {
 
 template <typename T, bool INV>
 __global__ __launch_bounds__(FdCfg<T>::threads) void k_dct_plane(const T* in, T* out, const T* __restrict__ tw,
-                                                                 PhiOut<T> po)
+                                                                 PhiOut<T> po, DivIn<T> dv)
 {
     constexpr int FD_THREADS = FdCfg<T>::threads;
     constexpr bool SW = INV || FdCfg<T>::sw_fwd;
@@ -2696,8 +2742,15 @@ __global__ __launch_bounds__(FdCfg<T>::threads) void k_dct_plane(const T* in, T*
     const long base = (long)b * FD_N * FD_N;
     // point (y, z) of the plane sits at row lp(y), column lp(z) (lp the
     // identity without SW): every row and every column is a line in lp order
-    for (int e = tid; e < FD_N * FD_N; e += FD_THREADS)
-        pl[lp<SW>(e >> 7) * FD_P + lp<SW>(e & 127)] = in[base + e];
+    if (!INV && dv.u) {
+        const T f = dv.fac(Bt{}, 0);
+#pragma unroll 4
+        for (int e = tid; e < FD_N * FD_N; e += FD_THREADS)
+            pl[lp<SW>(e >> 7) * FD_P + lp<SW>(e & 127)] = dv.at(0, f, b, e >> 7, e & 127);
+    } else {
+        for (int e = tid; e < FD_N * FD_N; e += FD_THREADS)
+            pl[lp<SW>(e >> 7) * FD_P + lp<SW>(e & 127)] = in[base + e];
+    }
     __syncthreads();
     const int t = tid & 7;
     for (int l0 = 0; l0 < FD_N; l0 += LG) {
@@ -2842,7 +2895,8 @@ __global__ __launch_bounds__(512) void k_dct_bf16x3(const float* in, float* out,
 template <typename T>
 constexpr int fl_lines() { return sizeof(T) == 8 ? 16 : 32; }
 template <typename T, bool INV, int N, int AX, int FL>
-__global__ __launch_bounds__(8 * FL) void k_dct_lines(const T* in, T* out, const T* __restrict__ tw, PhiOut<T> po)
+__global__ __launch_bounds__(8 * FL) void k_dct_lines(const T* in, T* out, const T* __restrict__ tw, PhiOut<T> po,
+                                                     DivIn<T> dv)
 {
     extern __shared__ __align__(16) unsigned char pllc_smem[];
     T* ls = reinterpret_cast<T*>(pllc_smem);   // [FL][N + 1]
@@ -2857,8 +2911,18 @@ __global__ __launch_bounds__(8 * FL) void k_dct_lines(const T* in, T* out, const
     {
         // every load of the thread in flight before the first LDS write
         T v[R];
+        if (!INV && AX == 2 && dv.u) {
+            const T f = dv.fac(Bt{}, 0);
+            const int x = (int)(blk * FL / N), y0 = (int)(blk * FL % N);   // the block's rows lie in one plane
 #pragma unroll
-        for (int r = 0; r < R; r++) v[r] = in[base + goff(tid + NT * r)];
+            for (int r = 0; r < R; r++) {
+                const int e = tid + NT * r;
+                v[r] = dv.at(0, f, x, y0 + e / N, e % N);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) v[r] = in[base + goff(tid + NT * r)];
+        }
 #pragma unroll
         for (int r = 0; r < R; r++) ls[slot(tid + NT * r)] = v[r];
     }
@@ -3119,9 +3183,9 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
 
 #define PLLC_INST_DCT_PLANES(T, N)                                                                             \
     template __global__ void k_dct_planes<T, false, N>(int, int, int, int, const T*, T*, const T*, const T*,   \
-                                                       PhiOut<T>, Bt);                                         \
+                                                       PhiOut<T>, DivIn<T>, Bt);                               \
     template __global__ void k_dct_planes<T, true, N>(int, int, int, int, const T*, T*, const T*, const T*,    \
-                                                      PhiOut<T>, Bt);
+                                                      PhiOut<T>, DivIn<T>, Bt);
 
 #define PLLC_INST(T)                                                                                           \
     template __global__ void k_stale<T>(Dims, const T*, const T*, const T*, const T*, T*);                      \
@@ -3152,18 +3216,20 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     PLLC_INST_DCT_PLANES(T, 32)                                                                                \
     PLLC_INST_DCT_PLANES(T, 48)                                                                                \
     PLLC_INST_DCT_PLANES(T, 64)                                                                                \
-    template __global__ void k_dct_wide<T, false>(int, int, const T*, T*, const T*, const T*, PhiOut<T>);      \
-    template __global__ void k_dct_wide<T, true>(int, int, const T*, T*, const T*, const T*, PhiOut<T>);       \
+    template __global__ void k_dct_wide<T, false>(int, int, const T*, T*, const T*, const T*, PhiOut<T>,       \
+                                                  DivIn<T>);                                                   \
+    template __global__ void k_dct_wide<T, true>(int, int, const T*, T*, const T*, const T*, PhiOut<T>,        \
+                                                 DivIn<T>);                                                    \
     template __global__ void k_gemm<T, true>(int, int, int, const T*, long, const T*, long, T*, long,          \
                                              PhiOut<T>);                                                        \
     template __global__ void k_gemm<T, false>(int, int, int, const T*, long, const T*, long, T*, long,         \
                                               PhiOut<T>);                                                       \
-    template __global__ void k_dct_plane<T, false>(const T*, T*, const T*, PhiOut<T>);                        \
-    template __global__ void k_dct_plane<T, true>(const T*, T*, const T*, PhiOut<T>);                         \
-    template __global__ void k_dct_lines<T, false, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>); \
-    template __global__ void k_dct_lines<T, false, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>); \
-    template __global__ void k_dct_lines<T, true, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>);  \
-    template __global__ void k_dct_lines<T, true, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>);  \
+    template __global__ void k_dct_plane<T, false>(const T*, T*, const T*, PhiOut<T>, DivIn<T>);              \
+    template __global__ void k_dct_plane<T, true>(const T*, T*, const T*, PhiOut<T>, DivIn<T>);               \
+    template __global__ void k_dct_lines<T, false, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
+    template __global__ void k_dct_lines<T, false, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
+    template __global__ void k_dct_lines<T, true, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
+    template __global__ void k_dct_lines<T, true, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
     template __global__ void k_copy<T>(Dims, const T*, T*, long);                                              \
     template __global__ void k_pack<T>(Dims, const T*, double*, long);                                         \
     template __global__ void k_unpack<T>(Dims, const double*, T*, long);                                       \
@@ -4373,7 +4439,7 @@ bool Ops<T>::dct_mfma_ready(int n)
 
 // the k_dct_planes form for (ny, nz): unrolled for square planes
 template <typename T>
-using DctPlanesFn = void (*)(int, int, int, int, const T*, T*, const T*, const T*, PhiOut<T>, Bt);
+using DctPlanesFn = void (*)(int, int, int, int, const T*, T*, const T*, const T*, PhiOut<T>, DivIn<T>, Bt);
 template <typename T>
 static DctPlanesFn<T> dct_planes_fn(bool inv, int ny, int nz)
 {
@@ -4436,8 +4502,9 @@ bool Ops<T>::dct_fast_ready(int n)
 }
 
 template <typename T>
-void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool ghosts)
+void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool ghosts, const DivIn<T>* div)
 {
+    const DivIn<T> dv = div ? *div : DivIn<T>{};
     const int nx = c.d.nx, ny = c.d.ny, nz = c.d.nz;
     if constexpr (sizeof(T) == 4) {
         if (c.cbf && ny == DM_N && nz == DM_N) {
@@ -4457,10 +4524,10 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const size_t sm = (size_t)FD_N * FD_P * sizeof(T);
         const PhiOut<T> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
         if (inverse)
-            PLLC_L(c, "dct", (k_dct_plane<T, true><<<nx, FdCfg<T>::threads, sm, c.st>>>(in, out, c.tw, po)));
+            PLLC_L(c, "dct", (k_dct_plane<T, true><<<nx, FdCfg<T>::threads, sm, c.st>>>(in, out, c.tw, po, dv)));
         else
             PLLC_L(c, "dct", (k_dct_plane<T, false><<<nx, FdCfg<T>::threads, sm, c.st>>>(in, out, c.tw,
-                                                                                           PhiOut<T>{})));
+                                                                                           PhiOut<T>{}, dv)));
         return;
     }
     if (c.tw && ny == 256 && nz == 256) {
@@ -4470,12 +4537,14 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const size_t sm = (size_t)FL * (N + 1) * sizeof(T);
         const unsigned nb = (unsigned)((long)nx * N / FL);
         if (!inverse) {
-            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{})));
-            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, PhiOut<T>{})));
+            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{}, dv)));
+            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, PhiOut<T>{},
+                                                                                          DivIn<T>{})));
         } else {
             const PhiOut<T> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
-            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{})));
-            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, po)));
+            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{},
+                                                                                         DivIn<T>{})));
+            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, po, DivIn<T>{})));
         }
         return;
     }
@@ -4490,7 +4559,7 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const DctPlanesFn<T> kern = dct_planes_fn<T>(inverse, ny, nz);
         const int nthr = dct_planes_threads(ny == nz ? ny : 0);
         const int G = std::max(1, std::min(np, resident_blocks(kern, nthr, sm)));
-        PLLC_L(c, "dct", (kern<<<G, nthr, sm, c.st>>>(ny, nz, nx, np, in, out, tz, ty, po, c.bt)));
+        PLLC_L(c, "dct", (kern<<<G, nthr, sm, c.st>>>(ny, nz, nx, np, in, out, tz, ty, po, dv, c.bt)));
         return;
     }
     if (!single(c, "dct2")) return;
@@ -4499,9 +4568,9 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const int nthr = 64 * dw_waves(ny, nz);
         const PhiOut<T> po{inverse ? phi : nullptr, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
         if (inverse)
-            PLLC_L(c, "dct", (k_dct_wide<T, true><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Oiz, c.Oiy, po)));
+            PLLC_L(c, "dct", (k_dct_wide<T, true><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Oiz, c.Oiy, po, dv)));
         else
-            PLLC_L(c, "dct", (k_dct_wide<T, false><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Ofz, c.Ofy, po)));
+            PLLC_L(c, "dct", (k_dct_wide<T, false><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Ofz, c.Ofy, po, dv)));
         return;
     }
     const long R = (long)nx * ny, plane = (long)ny * nz;
@@ -4523,7 +4592,7 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
 }
 
 template <typename T>
-void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts)
+void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts, bool from_velo)
 {
     dim3 blk;
     const dim3 grd = cell_grid(field_rng(c.d, FC), blk);
@@ -4532,9 +4601,17 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts)
         if (!single(c, "poisson")) return;
         PLLC_L(c, "div", (k_pack_div<T><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[DIV], c.P, c.scal, T(g), T(r))));
     }
+    // the right-hand side made in the forward transform's load, or packed
+    // first for the transforms without one (k_gemm, k_dct_bf16x3)
+    DivIn<T> dv{};
+    if (from_velo) {
+        if (!c.cbf && (c.tw || c.dsmall || c.Ofz))
+            dv = {c.f[U_NEW], c.f[V_NEW], c.f[W_NEW], c.scal, c.d, c.ph.Re, T(T(g) + T(r))};
+        else divergence(c, g, r, false, true);
+    }
     // the spectrum, in place in P
     T* sp = c.P;
-    dct2(c, c.P, sp, false);
+    dct2(c, c.P, sp, false, nullptr, false, &dv);
     const int PC = c.line_solver == 0 ? part_chunks(c.d.nx, c.d.nx) : 0;
     if (PC > 0) {
         // 128 bytes of a row per block, more where that is less than 256

@@ -844,8 +844,7 @@ static void fused_step(pllc_sim* s, Ctx<T>& c)
         } else {
             Ops<T>::momentum3(c, g, r, rk, true);   // with update_velo_boundary
         }
-        Ops<T>::divergence(c, g, r, false, true);
-        Ops<T>::poisson(c, g, r, false, true);   // with update_phi_ghosts
+        Ops<T>::poisson(c, g, r, false, true, true);   // with the divergence and update_phi_ghosts
         // velo_correction + pressure_gradient + update_veloghost_points
         const int next = rk < 2 ? rk + 1 : -1;
         started = Ops<T>::correction_and_gradient(c, g, r, rk, true, next, next < 0 ? 0.0 : kRK1[next] + kRK2[next]);
