@@ -138,8 +138,8 @@ struct Ops {
     // bulk() and stale() in one launch where the plane allows it
     static void bulk_stale(Ctx<T>& c, int slot, double alpha, bool advance_t, const T* qc, const T* qu, const T* qv,
                            const T* qw);
-    // b = a, every point of a field
-    static void copy(Ctx<T>& c, const T* a, T* b);
+    // second = first of 12 pairs of fields (back: first = second), every point
+    static void copy_pairs(Ctx<T>& c, const int (&pairs)[12][2], bool back);
     // rows of a field (pitched, T) to and from contiguous FP64 rows of NZ values
     static void pack(Ctx<T>& c, const T* a, double* b, long rows);
     static void unpack(Ctx<T>& c, const double* a, T* b, long rows);
@@ -156,6 +156,8 @@ struct Ops {
     static void shift_conc(Ctx<T>& c, T* q, const double* x, const double* shift);
     static void fill(Ctx<T>& c, T* a, long n, T v);
     static void set_scalar(Ctx<T>& c, int idx, double v);
+    // two scalars, and with_stale stale() of the old fields, in one launch
+    static void op_start(Ctx<T>& c, int i0, double v0, int i1, double v1, bool with_stale);
     // dense 2D DCT of a packed block: REDFT10 (forward) or REDFT01
     // (inverse), z then y, `in` -> `out` through the temporary c.Q
     // phi (inverse only): the result goes to phi's interior instead of out

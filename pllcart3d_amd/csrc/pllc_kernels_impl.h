@@ -2947,11 +2947,16 @@ __global__ __launch_bounds__(8 * FL) void k_dct_lines(const T* in, T* out, const
 
 // ------------------------------------------------------------ utilities
 
-// stream-ordered store of one device scalar
+// stream-ordered store of two device scalars, and with stale set the 16 stale
+// values (k_stale) in the same launch
 template <typename T>
-__global__ void k_set_scalar(double* __restrict__ p, int i, double v)
+__global__ void k_set_scalars(double* __restrict__ p, int i0, double v0, int i1, double v1, Dims d,
+                              const T* __restrict__ q0, const T* __restrict__ q1, const T* __restrict__ q2,
+                              const T* __restrict__ q3, T* __restrict__ stale)
 {
-    if (threadIdx.x == 0) p[i] = v;
+    const int t = threadIdx.x;
+    if (t == 0) { p[i0] = v0; p[i1] = v1; }
+    if (stale && t < 16) stale[t] = stale_value<T>(d, q0, q1, q2, q3, t);
 }
 
 // rows of NZ values (grid.x blocks of (64, 4) threads over the rows): a field
@@ -2962,9 +2967,16 @@ __device__ __forceinline__ void field_rows(const Dims& d, long rows, F f)
     for (long r = (long)blockIdx.x * blockDim.y + threadIdx.y; r < rows; r += (long)gridDim.x * blockDim.y)
         for (int k = threadIdx.x; k < d.NZ; k += 64) f(r * d.sy + k, r * d.NZ + k);
 }
+// b = a for the 12 (new, old) pairs (block row: the pair) in one launch: 56 us
+// in 12 launches at 128x64x64 FP64, where a launch's floor is longer than a
+// field's 4 MB
 template <typename T>
-__global__ __launch_bounds__(256) void k_copy(Dims d, const T* __restrict__ a, T* __restrict__ b, long rows)
+struct CopyPairs { const T* a[12]; T* b[12]; };
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy_pairs(Dims d, CopyPairs<T> cp, long rows)
 {
+    const T* __restrict__ a = cp.a[blockIdx.y];
+    T* __restrict__ b = cp.b[blockIdx.y];
     field_rows<T>(d, rows, [&](long o, long) { b[o] = a[o]; });
 }
 template <typename T>
@@ -3230,7 +3242,7 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     template __global__ void k_dct_lines<T, false, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
     template __global__ void k_dct_lines<T, true, 256, 1, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
     template __global__ void k_dct_lines<T, true, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
-    template __global__ void k_copy<T>(Dims, const T*, T*, long);                                              \
+    template __global__ void k_copy_pairs<T>(Dims, CopyPairs<T>, long);                                        \
     template __global__ void k_pack<T>(Dims, const T*, double*, long);                                         \
     template __global__ void k_unpack<T>(Dims, const double*, T*, long);                                       \
     template __global__ void k_fill<T>(T*, long, T);
@@ -4747,10 +4759,12 @@ void Ops<T>::bulk_stale(Ctx<T>& c, int slot, double alpha, bool advance_t, const
 static inline int row_grid(long rows) { return (int)std::min((rows + 3) / 4, 8192L); }
 
 template <typename T>
-void Ops<T>::copy(Ctx<T>& c, const T* a, T* b)
+void Ops<T>::copy_pairs(Ctx<T>& c, const int (&pairs)[12][2], bool back)
 {
     const long rows = (long)c.d.NX * c.d.NY;
-    PLLC_L(c, "copy", (k_copy<T><<<row_grid(rows), dim3(64, 4), 0, c.st>>>(c.d, a, b, rows)));
+    CopyPairs<T> cp;
+    for (int q = 0; q < 12; q++) { cp.a[q] = c.f[pairs[q][back]]; cp.b[q] = c.f[pairs[q][!back]]; }
+    PLLC_L(c, "copy", (k_copy_pairs<T><<<dim3(row_grid(rows), 12), dim3(64, 4), 0, c.st>>>(c.d, cp, rows)));
 }
 
 template <typename T>
@@ -4774,7 +4788,14 @@ void Ops<T>::fill(Ctx<T>& c, T* a, long n, T v)
 template <typename T>
 void Ops<T>::set_scalar(Ctx<T>& c, int idx, double v)
 {
-    k_set_scalar<T><<<1, 64, 0, c.st>>>(c.scal, idx, v);
+    op_start(c, idx, v, idx, v, false);
+}
+
+template <typename T>
+void Ops<T>::op_start(Ctx<T>& c, int i0, double v0, int i1, double v1, bool with_stale)
+{
+    k_set_scalars<T><<<1, 64, 0, c.st>>>(c.scal, i0, v0, i1, v1, c.d, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD],
+                                         with_stale ? c.stale : nullptr);
 }
 
 template <typename T>

@@ -560,7 +560,7 @@ static const int kPairs[12][2] = {{C_NEW, C_OLD}, {C_N, C_NM1}, {U_NEW, U_OLD}, 
 template <typename T>
 static void update_old_copy(Ctx<T>& c)
 {
-    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[0]], c.f[pr[1]]);
+    Ops<T>::copy_pairs(c, kPairs, false);
 }
 
 // after fused steps the pairs are swapped (old holds the latest state);
@@ -569,7 +569,7 @@ template <typename T>
 static void normalize(pllc_sim* s, Ctx<T>& c)
 {
     if (!s->new_stale) return;
-    for (auto& pr : kPairs) Ops<T>::copy(c, c.f[pr[1]], c.f[pr[0]]);
+    Ops<T>::copy_pairs(c, kPairs, true);
     s->new_stale = false;
 }
 
@@ -723,22 +723,21 @@ static double op_t(pllc_sim* s, Ctx<T>& c, int op, double dt, int rk, double vbu
 {
     normalize<T>(s, c);
     const double g = kRK1[rk], r = kRK2[rk];
-    Ops<T>::set_scalar(c, S_DT, dt);
-    Ops<T>::set_scalar(c, S_RK + 4 * rk, vbulk);
+    const bool explicit_op =
+        op == PLLC_OP_CONCENTRATION || op == PLLC_OP_XMOM || op == PLLC_OP_YMOM || op == PLLC_OP_ZMOM;
+    Ops<T>::op_start(c, S_DT, dt, S_RK + 4 * rk, vbulk, explicit_op);
     T* mun[4] = {c.f[MUN_CELL], c.f[MUN_XY], c.f[MUN_XZ], c.f[MUN_YZ]};
     switch (op) {
     case PLLC_OP_CONCENTRATION:
         if (s->cnn && c.ncorr)
             pllc_cnn_correct<T>(s->cnn, c.d, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD], c.f[MUO_CELL], c.ncorr,
                                 c.st);
-        Ops<T>::stale(c, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
         Ops<T>::concentration(c, g, r, rk, c.f[U_NEW], c.f[V_NEW], c.f[W_NEW]);
         break;
     case PLLC_OP_VISCOSITY: Ops<T>::viscosity(c, c.f[C_NEW], mun); break;
     case PLLC_OP_XMOM:
     case PLLC_OP_YMOM:
     case PLLC_OP_ZMOM:
-        Ops<T>::stale(c, c.f[C_OLD], c.f[U_OLD], c.f[V_OLD], c.f[W_OLD]);
         Ops<T>::momentum(c, op - PLLC_OP_XMOM, g, r, rk);
         break;
     case PLLC_OP_VELO_BOUNDARY:

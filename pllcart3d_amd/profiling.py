@@ -1,7 +1,7 @@
 """Profiling workload and rocprofv3 summaries for the pllcart3d time step.
 
     python pllcart3d_amd/profiling.py run [--config front_256x128x128] [--steps 2] [--precision plain|mixed]
-        set-up, one UPDATE_OLD (12 whole-field copies of known size: the
+        set-up, one UPDATE_OLD (a copy of 12 whole fields of known size: the
         calibration of the HBM counters) and `steps` fused steps; run it
         under rocprofv3 --kernel-trace --stats or --pmc FETCH_SIZE / WRITE_SIZE.
 
@@ -14,13 +14,13 @@
     python pllcart3d_amd/profiling.py run --ensemble [--steps 4]
         the 64-member mixed-precision ensemble (three batches of equal grids,
         their step pairs the branches of one graph) after two warm-up steps;
-        a separate handle's UPDATE_OLD (12 copy kernels) marks where the
+        a separate handle's UPDATE_OLD (the copy kernel) marks where the
         summarised dispatches start.
 
     python pllcart3d_amd/profiling.py summary --trace T.db [--fetch F.db --write W.db]
         a markdown summary: per-kernel durations from the kernel trace and the
         HBM bytes per dispatch from the two counter passes, scaled by what the
-        same counters read for the copy kernel (one field read, one written).
+        same counters read for the copy kernel (as much read as written).
 """
 import argparse
 import collections
@@ -87,7 +87,7 @@ def run(args):
         t.close()
     sim = P.Sim(prm, precision=args.precision)
     sim.init(c0)
-    # the 12 copies of UPDATE_OLD calibrate the counters and mark where the
+    # the copies of UPDATE_OLD calibrate the counters and mark where the
     # summarised dispatches start
     sim.op("UPDATE_OLD")
     sim.run(args.steps)
@@ -195,14 +195,17 @@ def summary(args):
         if not copy:
             raise SystemExit("no copy kernel in the counter passes")
         ck = copy[0]
+        # UPDATE_OLD copies its 12 fields in one dispatch of k_copy_pairs
         field_kib = args.points * args.bytes / 1024.0
+        per = 12 if ck.startswith("k_copy_pairs") else 1
         cf = sum(f[ck]) / len(f[ck])
         cw = sum(w[ck]) / len(w[ck])
-        sf, sw = field_kib / cf, field_kib / cw
+        sf, sw = per * field_kib / cf, per * field_kib / cw
         out.append("")
-        out.append("Calibration: `%s` copies one field of %d points x %d B = %.0f KiB; per dispatch "
+        out.append("Calibration: `%s` copies %s of %d points x %d B = %.0f KiB; per dispatch "
                    "FETCH_SIZE reads %.0f KiB and WRITE_SIZE %.0f KiB, so the factors are %.3f (fetch) "
-                   "and %.3f (write)." % (ck, args.points, args.bytes, field_kib, cf, cw, sf, sw))
+                   "and %.3f (write)." % (ck, "one field" if per == 1 else "%d fields" % per, args.points,
+                                                    args.bytes, per * field_kib, cf, cw, sf, sw))
         out.append("")
         out.append("| kernel | dispatches | HBM read MB | HBM write MB | read+write fields |")
         out.append("|---|---:|---:|---:|---:|")
