@@ -171,7 +171,9 @@ __global__ __launch_bounds__(256) void k_conv(G3 g, const unsigned short* __rest
 // shifted by o), B[p][co] (lane l: cells 4 (l / 16) + q, channel l % 16),
 // accumulator D[ci][co] (lane l: ci = 4 (l / 16) + q, co = l % 16).  The
 // waves of the grid take 16-cell segments in turn; a block's four waves
-// add their sums in LDS, one wave after the other.
+// add their sums in LDS, one wave after the other.  Bound by the latency of
+// the 2-byte loads at one block per CU: 37 us at 64x32x32 with the 12 loads a
+// row's three offsets make, 27 with the 6 distinct cells of them.
 __global__ __launch_bounds__(256) void k_conv_wgrad(G3 g, const unsigned short* __restrict__ a,
                                                     const unsigned short* __restrict__ dz, float* __restrict__ part)
 {
@@ -199,18 +201,25 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(G3 g, const unsigned short* 
             b[q] = (short)h;
             db += bf2f(h);
         }
+        // a lane's cells k0 + 4 kq - 1 .. + 4 of each neighbouring row serve the
+        // row's three offsets along k
 #pragma unroll
-        for (int o = 0; o < NOFF; o++) {
-            const int ii = i + o / 9 - 1, jj = j + (o / 3) % 3 - 1, dk = o % 3 - 1;
+        for (int rw = 0; rw < 9; rw++) {
+            const int ii = i + rw / 3 - 1, jj = j + rw % 3 - 1;
             const bool rowok = ii >= 0 && ii < g.nx && jj >= 0 && jj < g.ny;
-            bf16x4 av;
+            unsigned short h[6];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int kc = k0 + 4 * kq + q, kk = kc + dk;
-                const bool ok = rowok && kc < g.nz && kk >= 0 && kk < g.nz;
-                av[q] = (short)(ok ? a[vox(g, ii, jj, kk) * CH + m] : (unsigned short)0);
+            for (int q = 0; q < 6; q++) {
+                const int kk = k0 + 4 * kq + q - 1;
+                h[q] = rowok && kk >= 0 && kk < g.nz ? a[vox(g, ii, jj, kk) * CH + m] : (unsigned short)0;
             }
-            acc[o] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b, acc[o], 0, 0, 0);
+#pragma unroll
+            for (int dk = 0; dk < 3; dk++) {
+                bf16x4 av;
+#pragma unroll
+                for (int q = 0; q < 4; q++) av[q] = (short)(k0 + 4 * kq + q < g.nz ? h[q + dk] : (unsigned short)0);
+                acc[3 * rw + dk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b, acc[3 * rw + dk], 0, 0, 0);
+            }
         }
     }
     // the four waves add their sums in turn (a fixed order: the result does
@@ -235,14 +244,40 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(G3 g, const unsigned short* 
     for (int x = threadIdx.x; x < NOFF * 256 + CH; x += 256) dst[x] = red[x];
 }
 
-// out[x] = sum over nb blocks of part[b][x] (fixed order)
-__global__ void k_sum_parts(const float* __restrict__ part, int nb, int n, float* __restrict__ out)
+// out[x] = sum over nb blocks of part[b][x], b ascending (a fixed order).  A
+// block takes 64 x: its 16 rows of threads have 256 of the parts' values in
+// flight together and hand them over through LDS, 64 parts at a time, to its
+// first wave, which adds them in order.  The parts are 7 MB; one
+// thread per x over all parts, 28 blocks on 256 CUs, waited for its loads: 58 us
+// for 256 parts of 6928 values, this 7.3.
+constexpr int SP_X = 64, SP_R = 16, SP_N = 16, SP_T = 4;   // x, thread rows, values a thread, of them a time
+__global__ __launch_bounds__(SP_X * SP_R) void k_sum_parts(const float* __restrict__ part, int nb, int n,
+                                                           float* __restrict__ out)
 {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n) return;
+    __shared__ float sh[2][SP_T * SP_R][SP_X];
+    const int t = threadIdx.x, r = threadIdx.y, x = blockIdx.x * SP_X + t;
     float s = 0.f;
-    for (int b = 0; b < nb; b++) s += part[(long)b * n + x];
-    out[x] = s;
+    for (int b0 = 0; b0 < nb; b0 += SP_N * SP_R) {
+        float v[SP_N];
+#pragma unroll
+        for (int q = 0; q < SP_N; q++) {
+            const int b = b0 + q * SP_R + r;
+            v[q] = x < n && b < nb ? part[(long)b * n + x] : 0.f;
+        }
+#pragma unroll
+        for (int q0 = 0; q0 < SP_N; q0 += SP_T) {
+            float (&buf)[SP_T * SP_R][SP_X] = sh[(q0 / SP_T) & 1];
+#pragma unroll
+            for (int q = 0; q < SP_T; q++) buf[q * SP_R + r][t] = v[q0 + q];
+            // the other buffer is read until the next round's barrier
+            __syncthreads();
+            if (r == 0) {
+                const int m = min(SP_T * SP_R, nb - b0 - q0 * SP_R);
+                for (int q = 0; q < m; q++) s += buf[q][t];
+            }
+        }
+    }
+    if (r == 0 && x < n) out[x] = s;
 }
 
 // Loss of one sample: masked mean of (y - t)^2.  dy[p][0] = 2 (y - t) / nm on
@@ -531,18 +566,18 @@ void backward(pllc_cnn* m, const unsigned short* x)
 {
     const int nb = conv_blocks(m->g);
     const int n = NOFF * 256 + CH;
-    const int rb = (n + 255) / 256;
+    const int rb = (n + SP_X - 1) / SP_X;
     // layer 3: dW3, db3 from (a2, dy); dz2 = (dy * W3^T) (1 - a2^2)
     k_conv_wgrad<<<WG_BLOCKS, 256, 0, m->st>>>(m->g, m->a2, m->dz, m->part);
-    k_sum_parts<<<rb, 256, 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W3);
+    k_sum_parts<<<rb, dim3(SP_X, SP_R), 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W3);
     k_conv<<<nb, 256, 0, m->st>>>(m->g, m->dz, m->Wb[2], nullptr, EPI_DTANH, m->a2, m->dz2, nullptr);
     // layer 2: dW2, db2 from (a1, dz2); dz1 = (dz2 * W2^T) (1 - a1^2) into m->dz
     k_conv_wgrad<<<WG_BLOCKS, 256, 0, m->st>>>(m->g, m->a1, m->dz2, m->part);
-    k_sum_parts<<<rb, 256, 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W2);
+    k_sum_parts<<<rb, dim3(SP_X, SP_R), 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W2);
     k_conv<<<nb, 256, 0, m->st>>>(m->g, m->dz2, m->Wb[1], nullptr, EPI_DTANH, m->a1, m->dz, nullptr);
     // layer 1: dW1, db1 from (x, dz1)
     k_conv_wgrad<<<WG_BLOCKS, 256, 0, m->st>>>(m->g, x, m->dz, m->part);
-    k_sum_parts<<<rb, 256, 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W1);
+    k_sum_parts<<<rb, dim3(SP_X, SP_R), 0, m->st>>>(m->part, WG_BLOCKS, n, m->grad + OFF_W1);
 }
 
 // loss of the current y against sample s; dy into m->dz; returns the sum
