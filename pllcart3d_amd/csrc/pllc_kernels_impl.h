@@ -556,10 +556,9 @@ __device__ __forceinline__ void rhs_mom_line(const Dims& d, const Phys& ph, cons
 // dispatch order, so that the velocities and viscosities which they share
 // come from HBM once and a small grid pays for one launch: at 256x128x128
 // FP64 one launch per component moved 9.8 fields and the concentration's 6.9,
-// together 36, the joint one moves 18 (some of the 23 there are stay in the
-// last-level cache).  us, four launches -> one: 256x128x128 FP64 369 -> 263,
-// mixed 169 -> 134; 512x256x256 FP64 2740 -> 1920, mixed 1210 -> 1000;
-// 64x32x32 FP64 20 -> 9.  FP32 is bound by vector issue (92% of the cycles);
+// together 36, the joint one moves 25 (there are 23).  us, four launches ->
+// one: 256x128x128 FP64 369 -> 263, mixed 169 -> 134; 512x256x256 FP64 2740 ->
+// 1920, mixed 1210 -> 1000; 64x32x32 FP64 20 -> 9.  FP32 is bound by vector issue (92% of the cycles);
 // FP64 by latency with two waves per vector unit (54% issue, 36% waiting).
 template <typename T>
 struct RhsSets {
@@ -1478,7 +1477,8 @@ struct CorrRuns {
 // -> 536, 517, 509, 525; 256x96x96 mixed 39 -> 38, 37, 41, 44; 150x70x51 mixed
 // 12.9 -> 13.9, 12.0, 12.7, 17.7; 64x32x32 FP64 5.3 -> 6.9, 9.6, 15, 27: with
 // few waves the longer chain of a thread is what counts, hence the two forms
-// (correction_and_gradient).  Bound by HBM (16.8 fields, 4.6 TB/s at 256x128x128 FP64).
+// (correction_and_gradient).  Bound by the
+// memory: 20 fields at 256x128x128 FP64, 5.6 TB/s (one plane a thread: 16.8 at 4.4).
 constexpr int CORR_PLANES = 2;
 template <typename T, bool B = false>
 __global__ __launch_bounds__(256) void k_corr_pg_run(Dims d, Phys ph0, Visc4<T> mu, const T* __restrict__ phi,
@@ -4614,7 +4614,9 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts, 
         PLLC_L(c, "div", (k_pack_div<T><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[DIV], c.P, c.scal, T(g), T(r))));
     }
     // the right-hand side made in the forward transform's load, or packed
-    // first for the transforms without one (k_gemm, k_dct_bf16x3)
+    // first for the transforms without one (k_gemm, k_dct_bf16x3).  (A batch's
+    // blocks take many planes in turn; packed first its 64 members measured
+    // 8.94 ms a step, this 8.91.)
     DivIn<T> dv{};
     if (from_velo) {
         if (!c.cbf && (c.tw || c.dsmall || c.Ofz))

@@ -195,17 +195,26 @@ def summary(args):
         if not copy:
             raise SystemExit("no copy kernel in the counter passes")
         ck = copy[0]
-        # UPDATE_OLD copies its 12 fields in one dispatch of k_copy_pairs
         field_kib = args.points * args.bytes / 1024.0
-        per = 12 if ck.startswith("k_copy_pairs") else 1
+        exp_f = exp_w = field_kib
+        per = 1
+        if ck.startswith("k_copy_pairs"):
+            # UPDATE_OLD copies its 12 fields in one dispatch; a pitched row of
+            # `row` points (k = 1 on a 128-byte line) is fetched in whole lines
+            # (k = 0 lies in the line that holds the row before's last point) and
+            # written in 32-byte pieces
+            per, b = 12, args.bytes
+            rows = args.points / args.row
+            exp_f = per * rows * -(-args.row * b // 128) * 128 / 1024.0
+            exp_w = per * rows * (2 + (args.row - 2) * b // 32) * 32 / 1024.0
         cf = sum(f[ck]) / len(f[ck])
         cw = sum(w[ck]) / len(w[ck])
-        sf, sw = per * field_kib / cf, per * field_kib / cw
+        sf, sw = exp_f / cf, exp_w / cw
         out.append("")
         out.append("Calibration: `%s` copies %s of %d points x %d B = %.0f KiB; per dispatch "
                    "FETCH_SIZE reads %.0f KiB and WRITE_SIZE %.0f KiB, so the factors are %.3f (fetch) "
                    "and %.3f (write)." % (ck, "one field" if per == 1 else "%d fields" % per, args.points,
-                                                    args.bytes, per * field_kib, cf, cw, sf, sw))
+                                         args.bytes, per * field_kib, cf, cw, sf, sw))
         out.append("")
         out.append("| kernel | dispatches | HBM read MB | HBM write MB | read+write fields |")
         out.append("|---|---:|---:|---:|---:|")
@@ -233,6 +242,7 @@ def main():
     s.add_argument("--fetch")
     s.add_argument("--write")
     s.add_argument("--points", type=int, default=262 * 130 * 130, help="points of one field (with ghosts)")
+    s.add_argument("--row", type=int, default=130, help="points of one row (with ghosts)")
     s.add_argument("--bytes", type=int, default=8, help="bytes per value")
     s.add_argument("--ensemble", action="store_true", help="an ensemble run's trace (every stream, per grid)")
     s.add_argument("--steps", type=int, default=4, help="the ensemble run's profiled steps")
