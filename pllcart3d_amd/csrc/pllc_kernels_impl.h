@@ -4166,32 +4166,36 @@ static LineSet<T> line_set(Ctx<T>& c, int F, int DIR, T* S, T* CC, const Visc4<T
     return L;
 }
 
-// chunks per line of the partitioned solve for lines of nmin..nmax rows, or
-// 0 when the lines do not allow it
-static inline int part_chunks(int nmin, int nmax)
+// chunks per line of the partitioned solve for lines of nmin..nmax rows along
+// DIR, or 0 when the lines do not allow it.  z: a chunk is a lane of a wave.  x
+// (y-lines have at most 1024 rows): at least two lines of 256 chunks in a
+// block; the lines' pieces of a row get short (8 bytes a chunk's lane, 7 lines
+// at 1030 rows), yet 1030x33x20 FP64 takes 9.6 ms a step with one thread per
+// line and 0.94 so, 4096x16x16 mixed 33.8 and 0.82.
+static inline int part_chunks(int nmin, int nmax, int DIR)
 {
     const int P = (nmax + PM - 1) / PM;
-    return nmin < 3 || P > 64 ? 0 : P;
+    return nmin < 3 || P > (DIR == 2 ? 64 : 256) ? 0 : P;
 }
 
 template <typename T>
 bool Ops<T>::batchable(const Ctx<T>& c)
 {
     if (sizeof(T) != 4 || c.line_solver != 0 || !c.dsmall || c.cbf || c.ncorr) return false;
-    if ((long)c.d.ny * c.d.nz > BULK1_MAX || part_chunks(c.d.nx, c.d.nx) == 0) return false;
+    if ((long)c.d.ny * c.d.nz > BULK1_MAX || part_chunks(c.d.nx, c.d.nx, 0) == 0) return false;
     for (int DIR = 0; DIR < 3; DIR++) {
         int nmin = 1 << 30, nmax = 0;
         for (int F = FC; F <= FW; F++) {
             const Rng R = field_rng(c.d, F);
             const int n = DIR == 0 ? R.ie - R.is + 1 : DIR == 1 ? R.je - R.js + 1 : R.ke - R.ks + 1;
             if (F == FC) {
-                if (part_chunks(n, n) == 0) return false;
+                if (part_chunks(n, n, DIR) == 0) return false;
                 continue;
             }
             nmin = std::min(nmin, n);
             nmax = std::max(nmax, n);
         }
-        if (part_chunks(nmin, nmax) == 0) return false;
+        if (part_chunks(nmin, nmax, DIR) == 0) return false;
     }
     return true;
 }
@@ -4228,7 +4232,7 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
             nmax = std::max(nmax, n);
             nmin = std::min(nmin, n);
         }
-        const int P = c.line_solver == 0 ? part_chunks(nmin, nmax) : 0;
+        const int P = c.line_solver == 0 ? part_chunks(nmin, nmax, DIR) : 0;
         if (P > 0 && DIR != 2) {
             // lines per block: y-lines 256 bytes of a row (rows start 8-byte
             // aligned only, so longer runs fetch fewer partial cache lines);
@@ -4626,7 +4630,7 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts, 
     // the spectrum, in place in P
     T* sp = c.P;
     dct2(c, c.P, sp, false, nullptr, false, &dv);
-    const int PC = c.line_solver == 0 ? part_chunks(c.d.nx, c.d.nx) : 0;
+    const int PC = c.line_solver == 0 ? part_chunks(c.d.nx, c.d.nx, 0) : 0;
     if (PC > 0) {
         // 128 bytes of a row per block, more where that is less than 256
         // threads (512x256x256: 64 bytes 134 us FP64, 128 bytes 86; mixed 32
