@@ -4427,15 +4427,18 @@ void Ops<T>::divergence(Ctx<T>& c, double g, double r, bool write_div, bool pack
 }
 
 // opts kernel f in to sm bytes of dynamic LDS per block; false when the
-// device cannot give them
-static bool lds_optin(const void* f, int sm)
+// device cannot give them.  The limit belongs to the kernel, not to a handle,
+// so it is set to what the largest of the kernel's planes takes (most; the
+// device's own limit where that is less): set to sm, a handle of small planes
+// lowered it under a living one of larger planes (135168 to 5120 bytes).
+static bool lds_optin(const void* f, int sm, int most)
 {
     int dev = 0, lim = 0;
     if (hipGetDevice(&dev) != hipSuccess) return false;
     if (hipDeviceGetAttribute(&lim, hipDeviceAttributeSharedMemPerBlockOptin, dev) != hipSuccess || lim <= 0)
         if (hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) return false;
     if (sm > lim) return false;
-    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, sm) != hipSuccess) {
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, std::min(most, lim)) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
@@ -4448,7 +4451,7 @@ bool Ops<T>::dct_mfma_ready(int n)
     if constexpr (sizeof(T) == 4) {
         if (n != DM_N) return false;
         const int sm = DM_N * DM_P * (int)sizeof(float);
-        return lds_optin((const void*)k_dct_bf16x3<false>, sm) && lds_optin((const void*)k_dct_bf16x3<true>, sm);
+        return lds_optin((const void*)k_dct_bf16x3<false>, sm, sm) && lds_optin((const void*)k_dct_bf16x3<true>, sm, sm);
     }
     return false;
 }
@@ -4481,8 +4484,11 @@ bool Ops<T>::dct_small_ready(int ny, int nz)
 {
     if (ny % 16 || nz % 16 || ny > DS_MAX || nz > DS_MAX) return false;
     const int smp = dct_planes_lds<T>(ny, nz);
-    return lds_optin((const void*)dct_planes_fn<T>(false, ny, nz), smp) &&
-           lds_optin((const void*)dct_planes_fn<T>(true, ny, nz), smp);
+    // the unrolled forms have one size each; the other one's planes take
+    // less than four tables of the largest side
+    const int most = ny == nz ? smp : 4 * DS_MAX * ds_pitch(DS_MAX) * (int)sizeof(T);
+    return lds_optin((const void*)dct_planes_fn<T>(false, ny, nz), smp, most) &&
+           lds_optin((const void*)dct_planes_fn<T>(true, ny, nz), smp, most);
 }
 
 template <typename T>
@@ -4495,8 +4501,9 @@ template <typename T>
 bool Ops<T>::dct_wide_ready(int ny, int nz)
 {
     if (ny > DW_MAX || nz > DW_MAX) return false;
-    const int sm = dct_wide_lds<T>(ny, nz);
-    return lds_optin((const void*)k_dct_wide<T, false>, sm) && lds_optin((const void*)k_dct_wide<T, true>, sm);
+    const int sm = dct_wide_lds<T>(ny, nz), most = dct_wide_lds<T>(DW_MAX, DW_MAX);
+    return lds_optin((const void*)k_dct_wide<T, false>, sm, most) &&
+           lds_optin((const void*)k_dct_wide<T, true>, sm, most);
 }
 
 template <typename T>
@@ -4504,15 +4511,16 @@ bool Ops<T>::dct_fast_ready(int n)
 {
     if (n == FD_N) {
         const int sm = FD_N * FD_P * (int)sizeof(T);
-        return lds_optin((const void*)k_dct_plane<T, false>, sm) && lds_optin((const void*)k_dct_plane<T, true>, sm);
+        return lds_optin((const void*)k_dct_plane<T, false>, sm, sm) &&
+               lds_optin((const void*)k_dct_plane<T, true>, sm, sm);
     }
     if (n == 256) {
         constexpr int FL = fl_lines<T>();
         const int sm = FL * (256 + 1) * (int)sizeof(T);
-        return lds_optin((const void*)k_dct_lines<T, false, 256, 1, FL>, sm) &&
-               lds_optin((const void*)k_dct_lines<T, false, 256, 2, FL>, sm) &&
-               lds_optin((const void*)k_dct_lines<T, true, 256, 1, FL>, sm) &&
-               lds_optin((const void*)k_dct_lines<T, true, 256, 2, FL>, sm);
+        return lds_optin((const void*)k_dct_lines<T, false, 256, 1, FL>, sm, sm) &&
+               lds_optin((const void*)k_dct_lines<T, false, 256, 2, FL>, sm, sm) &&
+               lds_optin((const void*)k_dct_lines<T, true, 256, 1, FL>, sm, sm) &&
+               lds_optin((const void*)k_dct_lines<T, true, 256, 2, FL>, sm, sm);
     }
     return false;
 }
