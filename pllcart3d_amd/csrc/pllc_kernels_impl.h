@@ -2190,13 +2190,14 @@ __host__ __device__ constexpr int ds_pitch(int nz) { return nz + 4; }
 // tile's MFMA sequence is k_gemm's (a zero accumulator, k ascending in
 // steps of 4), so the result equals the two k_gemm launches bit for bit,
 // without Q's round trip through HBM.  A plane is read whole before any of
-// it is written, by its one block, so in may equal out.
+// it is written, by its one block, so in may equal out (neither is
+// __restrict__).
 __host__ __device__ constexpr int dct_planes_threads(int N) { return N ? 4 * N : 256; }
 
 template <typename T, bool INV, int N>
-__global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, int nplanes, const T* __restrict__ in,
-                                                    T* __restrict__ out, const T* __restrict__ Cz,
-                                                    const T* __restrict__ Cy, PhiOut<T> po, DivIn<T> dv, Bt bt)
+__global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, int nplanes, const T* in, T* out,
+                                                    const T* __restrict__ Cz, const T* __restrict__ Cy, PhiOut<T> po,
+                                                    DivIn<T> dv, Bt bt)
 {
     static_assert(N % 16 == 0 && N <= DS_MAX, "square planes of 16 .. 64");
     extern __shared__ unsigned char pllc_smem[];
@@ -2242,7 +2243,7 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
             }
             return;
         }
-        const T* __restrict__ src = in + (long)p * plane;
+        const T* src = in + (long)p * plane;
 #pragma unroll
         for (int u = 0; u < PF; u++) {
             const int e = threadIdx.x + NT * u;
@@ -2341,7 +2342,8 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
 // round trip; here a plane's load, its two contractions (6 us of matrix
 // instructions at 96 x 96 FP32) and its store follow each other in the one
 // block of a CU.  The whole plane's loads in flight at once instead of four a
-// thread: no faster.
+// thread: no faster.  A plane is read whole before any of it is written, so
+// in may equal out (neither is __restrict__).
 constexpr int DW_MAX = 128;
 __host__ __device__ constexpr int dw_tiles(int n) { return (n + 15) / 16; }
 __host__ __device__ constexpr int dw_pitch(int nz) { return 16 * dw_tiles(nz) + 4; }
@@ -2389,9 +2391,8 @@ __device__ __forceinline__ void dw_contract(typename Mma<T>::acc (&acc)[4], cons
 }
 
 template <typename T, bool INV>
-__global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* __restrict__ in, T* __restrict__ out,
-                                                   const T* __restrict__ Oz, const T* __restrict__ Oy, PhiOut<T> po,
-                                                   DivIn<T> dv)
+__global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* in, T* out, const T* __restrict__ Oz,
+                                                   const T* __restrict__ Oy, PhiOut<T> po, DivIn<T> dv)
 {
     extern __shared__ unsigned char pllc_smem[];
     typedef typename Mma<T>::acc acc_t;
@@ -2401,7 +2402,7 @@ __global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* __re
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, lk = lane >> 4;
     const long plane = (long)ny * nz;
-    const T* __restrict__ src = in + blockIdx.x * plane;
+    const T* src = in + blockIdx.x * plane;
     const int cells = 256 * ty * tz, nzp = 16 * tz;
     const bool fused = !INV && dv.u;
     const T f = fused ? dv.fac(Bt{}, 0) : T(0);
