@@ -16,6 +16,7 @@
 #include <utility>
 
 #include "pllc_dev.h"
+#include "pllc_grid.h"
 #include "pllc_host.h"
 #include "pllc_kernels.h"
 
@@ -4082,21 +4083,13 @@ static int simds()
     return 4 * cus;
 }
 
-// A cell grid for n fields whose threads take np consecutive planes each.
-// More planes reuse more of the x neighbours in registers (24 loads a point
-// instead of 37) and share a thread's set-up, but leave fewer waves: np is the
-// largest power of two up to 8 that leaves 2.5 waves per vector unit.  us a
-// step at np = 1, 2, 4, 8: 64x32x32 mixed 221, 220, 224, -; 97x45x39 FP64 428,
-// 423, 426, -; 150x70x51 mixed 513, 490, 483, 492; 256x128x128 FP64 -, -, 2457,
-// 2416; 512x256x256 mixed 11785, 10640, 10424, 10177 (16: 10119, but 150x70x51
-// 508).
+// a cell grid for n fields whose threads take np consecutive planes each
 template <typename T>
 static inline dim3 march_grid(const Rng& R, dim3& blk, const Ctx<T>& c, int n, int& np)
 {
     dim3 g = cell_grid(R, blk, KP<T>::value);
     const double waves = (double)n * c.bt.nm * c.d.nx * c.d.ny * c.d.nz / (64 * KP<T>::value) / simds();
-    np = 1;
-    while (np < 8 && waves >= 2 * np * 2.5) np *= 2;
+    np = march_planes(waves, (int)g.z, n * c.bt.nm);
     g.z = (g.z + np - 1) / np * n;
     return bgrid(g, c);
 }
