@@ -34,15 +34,30 @@ struct Dims {
 // -> 391 mixed, mixed momentum explicit part 392 -> 341, k_corr_pg 573 -> 540;
 // 256x128x128 x-sweep 83 -> 72 FP64.  k = 1 at 64 bytes into a line: slower
 // than packed rows (x-sweep 825, k_corr_pg mixed 598).
+// Short rows stay packed (sy = NZ): where the lines would add more than half to
+// a row, what is moved and held grows faster than the accesses gain.  us a
+// step, pitched -> packed: 512x128x32 mixed (88% more) 857 -> 788, 400x160x40
+// mixed (52%) 1442 -> 1283, 512x128x16 860 -> 812 and mixed 584 -> 502, 400x400x4
+// mixed 2490 -> 1875 with 770 -> 168 MB; below the line 512x256x64 mixed (45%)
+// 3187 -> 3266, 512x128x32 FP64 (41%) 1427 -> 1411, 256x128x128 mixed (23%) 1303
+// -> 1349.
 __host__ inline long pitch_lead(int esize) { return 128 / esize - 1; }
 __host__ inline void pitch_dims(Dims& d, int esize)
 {
     const long q = 128 / esize;
     d.sy = (d.NZ + q - 1) / q * q;
+    if (2 * (d.sy - d.NZ) > d.NZ) d.sy = d.NZ;
     d.sx = (long)d.NY * d.sy;
 }
-// values from one field's first point to the next field's
+// values of one field
 __host__ inline long field_values(const Dims& d) { return (long)d.NX * d.sx; }
+// values from one field's first point to the next one's in a slab of several:
+// whole 128-byte lines
+__host__ inline long field_stride(const Dims& d, int esize)
+{
+    const long q = 128 / esize;
+    return (field_values(d) + q - 1) / q * q;
+}
 
 // a / h for a divisor fixed on the host, with rh = 1/h correctly rounded
 // there.  FP64: q = a*rh and one fused correction r = a - q*h (exact),

@@ -1230,7 +1230,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     b->m = ms;
     const int nm = (int)ms.size();
     const Ctx<float>& c0 = ms[0]->cf;
-    const long fs = field_values(c0.d), lead = pitch_lead(4);
+    const long fs = field_stride(c0.d, 4), lead = pitch_lead(4);
     const long pk = (long)c0.d.nx * c0.d.ny * c0.d.nz;
     const long np = c0.npart;
     auto get = [&](size_t bytes) -> void* {
