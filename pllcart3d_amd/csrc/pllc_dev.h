@@ -3,7 +3,7 @@
 // Index space: every 3D field is an [i][j][k] block (k fastest) with ghost
 // widths (3,1,1) and the strides of Dims: in the drop-in entry points the
 // contiguous nx_max*ny_max*nz_max values of the reference's double*** arrays
-// (allocate_3d_calloc.h:46-64), in simulations a pitched layout (pitch_dims).
+// (allocate_3d_calloc.h:46-64), in large simulations a pitched layout (pitch_dims).
 // Interior cells are i in [3, nx+2], j in [1, ny], k in [1, nz]
 // (grid_setup, pllcart3d.c:353-370).
 //
@@ -24,29 +24,38 @@ struct Dims {
     double rdx, rdy, rdz;   // 1/dx, 1/dy, 1/dz rounded once on the host (divh)
 };
 
-// The layout of a simulation's own fields (values of esize bytes): rows of a
-// whole number of 128-byte lines, and fields that start pitch_lead values
-// after an aligned address, so that the interior point k = 1 of every row
-// starts a line; the line after a row's points holds its ghost k = nz + 1 and
-// the next row's k = 0.  With rows at any 8-byte offset every 16 lanes of a
-// load or store touched two 64-byte blocks of the L1 instead of one.
-// Measured (packed rows -> this): 512x256x256 x-sweep 743 -> 693 us FP64, 419
-// -> 391 mixed, mixed momentum explicit part 392 -> 341, k_corr_pg 573 -> 540;
-// 256x128x128 x-sweep 83 -> 72 FP64.  k = 1 at 64 bytes into a line: slower
-// than packed rows (x-sweep 825, k_corr_pg mixed 598).
-// Short rows stay packed (sy = NZ): where the lines would add more than half to
-// a row, what is moved and held grows faster than the accesses gain.  us a
-// step, pitched -> packed: 512x128x32 mixed (88% more) 857 -> 788, 400x160x40
-// mixed (52%) 1442 -> 1283, 512x128x16 860 -> 812 and mixed 584 -> 502, 400x400x4
-// mixed 2490 -> 1875 with 770 -> 168 MB; below the line 512x256x64 mixed (45%)
-// 3187 -> 3266, 512x128x32 FP64 (41%) 1427 -> 1411, 256x128x128 mixed (23%) 1303
-// -> 1349.
-__host__ inline long pitch_lead(int esize) { return 128 / esize - 1; }
-__host__ inline void pitch_dims(Dims& d, int esize)
+// The layout of a simulation's own fields (values of esize bytes).  Large
+// fields are pitched: rows of a whole number of 128-byte lines, and fields that
+// start pitch_lead values after an aligned address, so that the interior point
+// k = 1 of every row starts a line; the line after a row's points holds its
+// ghost k = nz + 1 and the next row's k = 0.  With rows at any 8-byte offset
+// every 16 lanes of a load or store touched two 64-byte blocks of the L1
+// instead of one.  Measured (packed rows -> this): 512x256x256 x-sweep 743 ->
+// 693 us FP64, 419 -> 391 mixed, mixed momentum explicit part 392 -> 341,
+// k_corr_pg 573 -> 540; 256x128x128 x-sweep 83 -> 72 FP64.  k = 1 at 64 bytes
+// into a line: slower than packed rows (x-sweep 825, k_corr_pg mixed 598).
+//
+// Smaller fields, which the caches hold in part, and fields whose rows the lines
+// would lengthen by more than half are packed (sy = NZ): nothing is gained there
+// and a packed FP64 field is also the host's layout.  us a step, pitched ->
+// packed: 256x96x96 mixed 862 -> 851, 300x120x80 mixed 1220 -> 1190, 400x50x50
+// FP64 978 -> 900, 192x64x64 FP64 625 -> 627, 512x128x32 mixed 857 -> 788,
+// 400x400x4 mixed 2490 -> 1875 (770 -> 168 MB); above the line 256x128x112 FP64
+// 2260 -> 2304, 256x128x128 mixed 1303 -> 1349, 512x256x64 mixed 3187 -> 3266.
+constexpr long PITCH_POINTS = 3500000;
+__host__ inline long pitched_row(const Dims& d, int esize)
 {
     const long q = 128 / esize;
-    d.sy = (d.NZ + q - 1) / q * q;
-    if (2 * (d.sy - d.NZ) > d.NZ) d.sy = d.NZ;
+    return (d.NZ + q - 1) / q * q;
+}
+__host__ inline bool pitched(const Dims& d, int esize)
+{
+    return (long)d.NX * d.NY * d.NZ >= PITCH_POINTS && 2 * (pitched_row(d, esize) - d.NZ) <= d.NZ;
+}
+__host__ inline long pitch_lead(const Dims& d, int esize) { return pitched(d, esize) ? 128 / esize - 1 : 0; }
+__host__ inline void pitch_dims(Dims& d, int esize)
+{
+    d.sy = pitched(d, esize) ? pitched_row(d, esize) : d.NZ;
     d.sx = (long)d.NY * d.sy;
 }
 // values of one field

@@ -447,20 +447,21 @@ template <typename T> static Ctx<T>& ctx(pllc_sim* s);
 template <> Ctx<double>& ctx<double>(pllc_sim* s) { return s->cd; }
 template <> Ctx<float>& ctx<float>(pllc_sim* s) { return s->cf; }
 
-// points of a field (host arrays; the device fields are pitched)
+// points of a field (host arrays; a device field may be pitched)
 static size_t npts(const pllc_sim* s) { return (size_t)s->cd.d.NX * s->cd.d.NY * s->cd.d.NZ; }
 
-// a zeroed device allocation of one pitched field; the pointer returned is
-// its first point
+// a zeroed device allocation of one field; the pointer returned is its first
+// point
 template <typename T>
 static T* field_alloc(pllc_sim* s, const Dims& d, const char* W)
 {
     void* p = nullptr;
-    const size_t bytes = (field_values(d) + pitch_lead(sizeof(T)) + 1) * sizeof(T);
+    const long lead = pitch_lead(d, sizeof(T));
+    const size_t bytes = (field_values(d) + lead + (lead ? 1 : 0)) * sizeof(T);
     if (!pllc_hip_ok(W, hipMalloc(&p, bytes))) return nullptr;
     s->owned.push_back(p);
     if (!pllc_hip_ok(W, hipMemset(p, 0, bytes))) return nullptr;
-    return (T*)p + pitch_lead(sizeof(T));
+    return (T*)p + lead;
 }
 
 void pllc_fill_dims(const pllc_params* p, Dims& d, Phys& ph)
@@ -580,8 +581,9 @@ static void normalize(pllc_sim* s, Ctx<T>& c)
 template <typename T>
 static double* stage(Ctx<T>& c, long& rows)
 {
-    T* p = c.f[F_SRC2] + 1;   // a 128-byte line's start
-    rows = (long)((field_values(c.d) - 1) * sizeof(T) / (c.d.NZ * sizeof(double)));
+    const int skip = pitched(c.d, sizeof(T)) ? 1 : 0;   // to a 128-byte line's start
+    T* p = c.f[F_SRC2] + skip;
+    rows = (long)((field_values(c.d) - skip) * sizeof(T) / (c.d.NZ * sizeof(double)));
     return reinterpret_cast<double*>(p);
 }
 
@@ -1230,7 +1232,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     b->m = ms;
     const int nm = (int)ms.size();
     const Ctx<float>& c0 = ms[0]->cf;
-    const long fs = field_stride(c0.d, 4), lead = pitch_lead(4);
+    const long fs = field_stride(c0.d, 4), lead = pitch_lead(c0.d, 4);
     const long pk = (long)c0.d.nx * c0.d.ny * c0.d.nz;
     const long np = c0.npart;
     auto get = [&](size_t bytes) -> void* {
