@@ -574,10 +574,39 @@ static void normalize(pllc_sim* s, Ctx<T>& c)
     s->new_stale = false;
 }
 
-// Uploads and downloads pass through a scratch field of the sweeps as
-// contiguous FP64 rows of NZ values, as many rows at a time as it holds (a
-// row kernel packs and converts; converting a mixed field on the host cost
-// 8 ms at 256x128x128).  Its content lives only within an operator or a step.
+// How a field's values and the host's FP64 rows of NZ values get to each other.
+// DIRECT: a packed FP64 field is the host's layout.  HOST: a packed FP32 field
+// is copied as it is and converted on the host.  STAGED: through a scratch field
+// of the sweeps (its content lives only within an operator or a step) as FP64
+// rows, as many at a time as it holds, which a row kernel packs and converts.
+// us a download, STAGED against the other two: FP64 64x32x32 31 : 20 (page-
+// locked host memory), 150x70x51 110 : 91; FP32 64x32x32 51 : 29 and 97x45x39 68 :
+// 61, but 128x64x64 122 : 218 and 256x128x128 682 : 2104.  Pageable host memory
+// takes twice the bytes worse: 64x32x32 67 : 29, 128x64x64 278 : 221, 300x120x24
+// 449 : 344, 256x128x128 (pitched) 1976 : 2154.  Hence FP32 fields convert on the
+// host if packed, unless the host memory is page-locked and the field has 250000
+// points or more.
+enum class Route { DIRECT, HOST, STAGED };
+constexpr long STAGE_POINTS = 250000;
+
+static bool page_locked(const void* p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeHost;
+}
+
+template <typename T>
+static Route route(const Dims& d, const void* host)
+{
+    if (pitched(d, sizeof(T))) return Route::STAGED;
+    if (sizeof(T) == sizeof(double)) return Route::DIRECT;
+    return field_values(d) >= STAGE_POINTS && page_locked(host) ? Route::STAGED : Route::HOST;
+}
+
 template <typename T>
 static double* stage(Ctx<T>& c, long& rows)
 {
@@ -587,41 +616,67 @@ static double* stage(Ctx<T>& c, long& rows)
     return reinterpret_cast<double*>(p);
 }
 
-// dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ values
+// dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ
+// values.  Copies and kernels are queued on the handle's stream and waited for
+// once, also after a failure: what is queued uses the host's memory.
 template <typename T>
 static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W)
 {
-    long most = 0;
-    double* t = stage(c, most);
-    if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
-    for (long q = 0; q < rows; q += most) {
-        const long n = std::min(most, rows - q);
-        {
-            std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-            if (!pllc_hip_ok(W, hipMemcpy(t, src + q * c.d.NZ, (size_t)n * c.d.NZ * 8, hipMemcpyHostToDevice)))
-                return false;
+    const long n = rows * c.d.NZ;
+    bool ok = true;
+    std::vector<T> t;
+    switch (route<T>(c.d, src)) {
+    case Route::DIRECT:
+        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * c.d.sy, src, n * 8, hipMemcpyHostToDevice, s->st));
+        break;
+    case Route::HOST:
+        t.resize(n);
+        for (long e = 0; e < n; e++) t[e] = T(src[e]);
+        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * c.d.sy, t.data(), n * sizeof(T), hipMemcpyHostToDevice, s->st));
+        break;
+    case Route::STAGED: {
+        long most = 0;
+        double* b = stage(c, most);
+        for (long q = 0; ok && q < rows; q += most) {
+            const long m = std::min(most, rows - q);
+            ok = pllc_hip_ok(W, hipMemcpyAsync(b, src + q * c.d.NZ, m * c.d.NZ * 8, hipMemcpyHostToDevice, s->st));
+            if (ok) Ops<T>::unpack(c, b, dst + (r0 + q) * c.d.sy, m);
         }
-        Ops<T>::unpack(c, t, dst + (r0 + q) * c.d.sy, n);
-        if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
+        break;
     }
-    return true;
+    }
+    return pllc_hip_ok(W, hipStreamSynchronize(s->st)) && ok;
 }
 
 template <typename T>
 static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W)
 {
-    long most = 0;
-    double* t = stage(c, most);
-    const long rows = (long)c.d.NX * c.d.NY;
-    for (long q = 0; q < rows; q += most) {
-        const long n = std::min(most, rows - q);
-        Ops<T>::pack(c, src + q * c.d.sy, t, n);
+    const long rows = (long)c.d.NX * c.d.NY, n = rows * c.d.NZ;
+    bool ok = true;
+    std::vector<T> t;
+    switch (route<T>(c.d, dst)) {
+    case Route::DIRECT: ok = pllc_hip_ok(W, hipMemcpyAsync(dst, src, n * 8, hipMemcpyDeviceToHost, s->st)); break;
+    case Route::HOST: {
+        // (a synchronous copy: 16x8x8 15 us, a queued one 20)
+        t.resize(n);
         if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
         std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-        if (!pllc_hip_ok(W, hipMemcpy(dst + q * c.d.NZ, t, (size_t)n * c.d.NZ * 8, hipMemcpyDeviceToHost)))
-            return false;
+        if (!pllc_hip_ok(W, hipMemcpy(t.data(), src, n * sizeof(T), hipMemcpyDeviceToHost))) return false;
+        for (long e = 0; e < n; e++) dst[e] = double(t[e]);
+        return true;
     }
-    return true;
+    case Route::STAGED: {
+        long most = 0;
+        double* b = stage(c, most);
+        for (long q = 0; ok && q < rows; q += most) {
+            const long m = std::min(most, rows - q);
+            Ops<T>::pack(c, src + q * c.d.sy, b, m);
+            ok = pllc_hip_ok(W, hipMemcpyAsync(dst + q * c.d.NZ, b, m * c.d.NZ * 8, hipMemcpyDeviceToHost, s->st));
+        }
+        break;
+    }
+    }
+    return pllc_hip_ok(W, hipStreamSynchronize(s->st)) && ok;
 }
 
 template <typename T>
@@ -685,12 +740,11 @@ template <typename T>
 static int upload_t(pllc_sim* s, Ctx<T>& c, int field, const double* host)
 {
     normalize<T>(s, c);
-    if (finish(s, "pllc_sim_upload")) return -1;
     if (!h2d<T>(s, c, c.f[field], 0, (long)c.d.NX * c.d.NY, host, "pllc_sim_upload")) return -1;
     // old and new may now differ where a step never writes: the next
     // substage copies (as update_old_* does) instead of swapping
     s->copy_next = true;
-    return finish(s, "pllc_sim_upload");
+    return pllc_hip_ok("pllc_sim_upload", hipGetLastError()) ? 0 : -1;
 }
 
 template <typename T>
