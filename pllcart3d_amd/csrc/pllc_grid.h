@@ -22,4 +22,35 @@ inline int march_planes(double waves, int planes, int groups)
     return np;
 }
 
+// z-lines of n rows that a wave takes (k_sweep_wave_z): 64 / G, G the power of
+// two of at least the line's chunks of 16 rows
+inline int z_lines_per_wave(int n)
+{
+    int G = 1;
+    while (16 * G < n) G *= 2;
+    return G > 64 ? 1 : 64 / G;
+}
+// waves in a block of the z-sweep, `most` of them unless tuned to `lines` per block
+inline int z_block_waves(int lines, int n, int most)
+{
+    if (lines <= 0) return most;
+    const int w = lines / z_lines_per_wave(n);
+    return w < 1 ? 1 : w > most ? most : w;
+}
+
+// the lines per block that the autotuner times for lines of n rows along
+// direction dir (0 x, 1 y, 2 z): for z those of 1, 2 and 4 waves (8 to 64 lines
+// are one and the same launch for n <= 16, and for n <= 32 none of them the
+// default's 4 waves)
+inline int tune_lines(int dir, int n, int (&c)[4])
+{
+    if (dir == 2) {
+        for (int q = 0; q < 3; q++) c[q] = z_lines_per_wave(n) << q;
+        return 3;
+    }
+    const int all[4] = {8, 16, 32, 64};
+    for (int q = 0; q < 4; q++) c[q] = all[q];
+    return 4;
+}
+
 }  // namespace pllc

@@ -4254,11 +4254,8 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
         }
         if (P > 0) {
             // z-lines: a wave takes 64 / G lines of an i-plane, G lanes each
-            int G = 1;
-            while (G < P) G *= 2;
-            const int LW = 64 / G, nbx = (nj + LW - 1) / LW, ntiles = nbx * ni * nset;
-            int nw = Z_WAVES;
-            if (c.lpb[2] > 0) nw = std::max(1, std::min(Z_WAVES, c.lpb[2] / LW));   // tuned
+            const int LW = z_lines_per_wave(nmax), G = 64 / LW, nbx = (nj + LW - 1) / LW, ntiles = nbx * ni * nset;
+            const int nw = z_block_waves(c.lpb[2], nmax, Z_WAVES);
             const size_t sm = (size_t)nw * Z_TILE * sizeof(T);
             // a multiple of 8 blocks (XCD order); the tiles past the last do nothing
             const dim3 gz((unsigned)((ntiles + nw * 8 - 1) / (nw * 8) * 8), c.bt.nm, 1);

@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "pllc_grid.h"
 #include "pllc_kernels.h"
 #include "pllc_host.h"
 #include "pllcart3d.h"
@@ -1203,13 +1204,16 @@ static void apply_tuned(pllc_sim* s)
 
 extern "C" int pllc_sim_autotune(pllc_sim* s, int nsteps, int* lpb_out)
 {
-    static const int cand[] = {8, 16, 32, 64};
+    const int rows[3] = {s->p.nx, s->p.ny, s->p.nz};
     int best[3] = {0, 0, 0};
     set_lpb(s, best);
     for (int d = 0; d < 3; d++) {
         double tbest = 1e30;
         int lbest = 0;
-        for (int L : cand) {
+        int cand[4];
+        const int m = tune_lines(d, rows[d], cand);
+        for (int q = 0; q < m; q++) {
+            const int L = cand[q];
             int trial[3] = {best[0], best[1], best[2]};
             trial[d] = L;
             set_lpb(s, trial);

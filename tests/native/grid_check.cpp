@@ -1,7 +1,9 @@
 /* Checks the explicit kernels' planes per thread (march_planes in
  * pllc_grid.h): prints the number of cases in which the launch has more than
  * 65535 blocks along z, takes more planes a thread than it must for that, or
- * departs from the rule on waves where the blocks are few. */
+ * departs from the rule on waves where the blocks are few.  Then the number of
+ * z-line lengths for which the autotuner does not time each block shape of the
+ * z-sweep (1, 2 and 4 waves) exactly once. */
 #include <cstdio>
 #include <initializer_list>
 
@@ -24,6 +26,13 @@ int main()
                     while (rule < 8 && waves >= 5.0 * rule) rule *= 2;
                     if (blocks(np) > 65535 || np < rule || (np > rule && blocks(np / 2) <= 65535)) bad++;
                 }
-    printf("%ld\n", bad);
+    long untuned = 0;
+    for (int n = 1; n <= 1024; n++) {
+        int c[4], seen[5] = {0, 0, 0, 0, 0};
+        const int m = pllc::tune_lines(2, n, c);
+        for (int q = 0; q < m; q++) seen[pllc::z_block_waves(c[q], n, 4)]++;
+        if (seen[1] != 1 || seen[2] != 1 || seen[3] || seen[4] != 1 || pllc::z_block_waves(0, n, 4) != 4) untuned++;
+    }
+    printf("%ld %ld\n", bad, untuned);
     return 0;
 }

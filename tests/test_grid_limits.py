@@ -1,6 +1,7 @@
-"""Launches of long thin grids stay within 65535 blocks along z: the rule on
-the host, over its range, and on the GPU the first sizes at which the joint
-explicit launch reaches the limit."""
+"""Launch shapes that follow from sizes alone.  Launches of long thin grids stay
+within 65535 blocks along z: the rule on the host, over its range, and on the
+GPU the first sizes at which the joint explicit launch reaches the limit.  The
+autotuner's candidates."""
 import os
 import subprocess
 
@@ -16,12 +17,13 @@ SEQ = ["CONCENTRATION", "VISCOSITY", "XMOM", "YMOM", "ZMOM", "VELO_BOUNDARY", "D
        "PHI_GHOSTS", "VELO_CORRECTION", "VELOGHOST", "PRESSURE_GRADIENT", "UPDATE_OLD"]
 
 
-def test_planes_per_thread_keep_the_block_limit(tmp_path):
+@pytest.mark.parametrize("what", ["blocks along z", "z-sweep block shapes tuned"])
+def test_rules_on_the_host(tmp_path, what):
     exe = tmp_path / "grid_check"
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", CSRC, "-o", str(exe),
                     os.path.join(HERE, "native", "grid_check.cpp")], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
-    assert int(out) == 0
+    assert int(out.split()[["blocks along z", "z-sweep block shapes tuned"].index(what)]) == 0
 
 
 @pytest.mark.gpu
@@ -69,3 +71,22 @@ def test_long_thin_grid_tracks_oracle(oracle_mod):
     print("[long thin grid]", {k: "%.2e" % v for k, v in err.items()}, flush=True)
     assert err["c"] <= 1e-11
     assert max(err["velocity"], err["phi"]) <= 16 * 16389 ** 2 / np.pi ** 2 * np.finfo(float).eps
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nz", [12, 24, 40])
+def test_tuned_shapes_leave_the_bits(nz):
+    """A handle with the shapes that the autotuner kept for its grid gives the
+    bits of one created before; the z-lines are those of 1, 2 or 4 waves."""
+    prm = P.make_params(40, 20, nz, Vratio=3.0, Pe=300.0, Inf_thick=0.1)
+    c0 = P.ic_fill(prm, P.IC_NOISE, 3, 0.05)
+    a = P.Sim(prm, "mixed")
+    lines = P.Sim(prm, "mixed").autotune(2)
+    print("[autotune] nz %d lines per block x/y/z %s" % (nz, lines), flush=True)
+    assert lines[2] in [w * {12: 64, 24: 32, 40: 16}[nz] for w in (1, 2, 4)]
+    b = P.Sim(prm, "mixed")
+    for s in (a, b):
+        s.init(c0)
+        s.run(3)
+    for f in ("C_OLD", "U_OLD", "V_OLD", "W_OLD", "PHI"):
+        assert np.array_equal(a.download(f), b.download(f)), f
