@@ -176,6 +176,31 @@ def issue_summary(args):
     sys.stdout.write("\n".join(out) + "\n")
 
 
+DEFAULT_POINTS, DEFAULT_ROW = 262 * 130 * 130, 130   # front_256x128x128
+
+
+def _row(args):
+    """Points of a row, which no other grid shares with the default one."""
+    row = args.row or (DEFAULT_ROW if args.points == DEFAULT_POINTS else 0)
+    if not row or args.points % row:
+        raise SystemExit("--row (points of one row, with ghosts) has to go with --points")
+    return row
+
+
+def _field_kib(points, row, b):
+    """KiB that a copy of one field fetches and writes.  Packed fields: their
+    own bytes.  Pitched ones (pitch_dims in pllc_dev.h; k = 1 on a 128-byte
+    line) are fetched in whole lines (k = 0 lies in the line that holds the row
+    before's last point) and written in 32-byte pieces (one for k = 0, and
+    those of the interior and of k = nz + 1, which ends in the interior's last
+    piece or starts one)."""
+    q = 128 // b
+    if points < 3500000 or 2 * (-(-row // q) * q - row) > row:
+        return points * b / 1024.0, points * b / 1024.0
+    rows = points / row
+    return rows * -(-row * b // 128) * 128 / 1024.0, rows * (2 + (row - 2) * b // 32) * 32 / 1024.0
+
+
 def summary(args):
     if getattr(args, "issue", False):
         return issue_summary(args)
@@ -199,14 +224,9 @@ def summary(args):
         exp_f = exp_w = field_kib
         per = 1
         if ck.startswith("k_copy_pairs"):
-            # UPDATE_OLD copies its 12 fields in one dispatch; a pitched row of
-            # `row` points (k = 1 on a 128-byte line) is fetched in whole lines
-            # (k = 0 lies in the line that holds the row before's last point) and
-            # written in 32-byte pieces
-            per, b = 12, args.bytes
-            rows = args.points / args.row
-            exp_f = per * rows * -(-args.row * b // 128) * 128 / 1024.0
-            exp_w = per * rows * (2 + (args.row - 2) * b // 32) * 32 / 1024.0
+            # UPDATE_OLD copies its 12 fields in one dispatch
+            per = 12
+            exp_f, exp_w = (per * e for e in _field_kib(args.points, _row(args), args.bytes))
         cf = sum(f[ck]) / len(f[ck])
         cw = sum(w[ck]) / len(w[ck])
         sf, sw = exp_f / cf, exp_w / cw
@@ -241,8 +261,8 @@ def main():
     s.add_argument("--trace", required=True)
     s.add_argument("--fetch")
     s.add_argument("--write")
-    s.add_argument("--points", type=int, default=262 * 130 * 130, help="points of one field (with ghosts)")
-    s.add_argument("--row", type=int, default=130, help="points of one row (with ghosts)")
+    s.add_argument("--points", type=int, default=DEFAULT_POINTS, help="points of one field (with ghosts)")
+    s.add_argument("--row", type=int, help="points of one row (with ghosts), with --points")
     s.add_argument("--bytes", type=int, default=8, help="bytes per value")
     s.add_argument("--ensemble", action="store_true", help="an ensemble run's trace (every stream, per grid)")
     s.add_argument("--steps", type=int, default=4, help="the ensemble run's profiled steps")
