@@ -140,7 +140,7 @@ struct Ops {
                            const T* qw);
     // second = first of 12 pairs of fields (back: first = second), every point
     static void copy_pairs(Ctx<T>& c, const int (&pairs)[12][2], bool back);
-    // rows of a field (pitched, T) to and from contiguous FP64 rows of NZ values
+    // rows of a field (T, pitched or packed) to and from contiguous FP64 rows of NZ values
     static void pack(Ctx<T>& c, const T* a, double* b, long rows);
     static void unpack(Ctx<T>& c, const double* a, T* b, long rows);
     // velocity correction, outflow deficit and the pressure-gradient update
@@ -154,7 +154,6 @@ struct Ops {
     // shift_conc on field q: every (j,k) line re-sampled at Xc - shift[k]
     // (x: the NX cell centres, shift: NZ values, both on the device)
     static void shift_conc(Ctx<T>& c, T* q, const double* x, const double* shift);
-    static void fill(Ctx<T>& c, T* a, long n, T v);
     static void set_scalar(Ctx<T>& c, int idx, double v);
     // two scalars, and with_stale stale() of the old fields, in one launch
     static void op_start(Ctx<T>& c, int i0, double v0, int i1, double v1, bool with_stale);

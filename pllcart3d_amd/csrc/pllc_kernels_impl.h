@@ -1081,22 +1081,17 @@ __global__ void k_phi_ghost(Dims d, T* __restrict__ phi)
 
 // divergence (1983-1999).  Writes div (if non-null) and/or the scaled
 // Poisson source Re/(dt*alpha)*div packed as [x][y][z] (2018-2024).
-template <typename T, bool B = false>
-__global__ __launch_bounds__(256) void k_div(Dims d, Phys ph0, const T* __restrict__ u, const T* __restrict__ v,
+template <typename T>
+__global__ __launch_bounds__(256) void k_div(Dims d, Phys ph, const T* __restrict__ u, const T* __restrict__ v,
                                              const T* __restrict__ w, T* __restrict__ div, T* __restrict__ P,
-                                             const double* __restrict__ scal0, T g, T r, Bt bt)
+                                             const double* __restrict__ scal, T g, T r)
 {
     const int2 tl = xcd_tile();
     const int k = tl.x * blockDim.x + threadIdx.x + 1;
     const int j = tl.y * blockDim.y + threadIdx.y + 1;
-    int il;
-    const int m = bt_member(bt, blockIdx.z, gridDim.z, il);
-    const int i = il + 3;
+    const int i = blockIdx.z + 3;
     if (k > d.nz || j > d.ny) return;
-    const Phys& ph = bt_phys<B>(bt, ph0, m);
-    const double* __restrict__ scal = scal0 + m * S_SIZE;
-    if (P) P += m * bt.pk;
-    const long o = IX(d, i, j, k) + m * bt.fs;
+    const long o = IX(d, i, j, k);
     const T dvx = divh<T>(u[o + d.sx] - u[o], T(d.dx), d.rdx);
     const T dvy = divh<T>(v[o + d.sy] - v[o], T(d.dy), d.rdy);
     const T dvz = divh<T>(w[o + 1] - w[o], T(d.dz), d.rdz);
@@ -2992,12 +2987,6 @@ __global__ __launch_bounds__(256) void k_unpack(Dims d, const double* __restrict
     field_rows<T>(d, rows, [&](long o, long l) { b[o] = T(a[l]); });
 }
 
-template <typename T>
-__global__ void k_fill(T* __restrict__ a, long n, T v)
-{
-    for (long l = (long)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (long)gridDim.x * blockDim.x) a[l] = v;
-}
-
 #ifdef PLLC_F64_TU
 // ------------------------------------------------------------ diagnostics
 
@@ -3215,8 +3204,7 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     template __global__ void k_visc<T>(Dims, Phys, const T*, T*, T*, T*, T*, Bt);                              \
     template __global__ void k_velo_ghost<T>(Dims, T*, T*, T*);                                                \
     template __global__ void k_phi_ghost<T>(Dims, T*);                                                         \
-    template __global__ void k_div<T>(Dims, Phys, const T*, const T*, const T*, T*, T*, const double*, T, T,   \
-                                     Bt);                                                                   \
+    template __global__ void k_div<T>(Dims, Phys, const T*, const T*, const T*, T*, T*, const double*, T, T);   \
     template __global__ void k_pack_div<T>(Dims, Phys, const T*, T*, const double*, T, T);                     \
     template __global__ void k_pois_x<T>(Dims, const T*, const T*, T*, T*, const double*);                     \
     template __global__ void k_velo_corr<T>(Dims, Phys, const T*, T*, T*, T*, const double*, T, T);            \
@@ -3246,8 +3234,7 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     template __global__ void k_dct_lines<T, true, 256, 2, fl_lines<T>()>(const T*, T*, const T*, PhiOut<T>, DivIn<T>); \
     template __global__ void k_copy_pairs<T>(Dims, CopyPairs<T>, long);                                        \
     template __global__ void k_pack<T>(Dims, const T*, double*, long);                                         \
-    template __global__ void k_unpack<T>(Dims, const double*, T*, long);                                       \
-    template __global__ void k_fill<T>(T*, long, T);
+    template __global__ void k_unpack<T>(Dims, const double*, T*, long);
 
 // ------------------------------------------------- wave perturbation
 //
@@ -3326,18 +3313,6 @@ __global__ void k_spline_lines(int N, long nlines, int nk, long sj, long sk, lon
     for (int ii = 0; ii < N; ii++) Y[(long)ii * rs] = C[(long)ii * rs];
 }
 
-// XCD-aware order of the line blocks: with the block count of the (x, y)
-// grid a multiple of 8, XCD x takes the x-th eighth of the blocks in (x, y)
-// order instead of every eighth block, so blocks whose rows share a cache
-// line at their edges (rows start at any 8-byte offset) run in one L2.
-__device__ __forceinline__ int2 xcd_block_xy()
-{
-    const int gx = gridDim.x, nt = gx * gridDim.y;
-    int r = blockIdx.x + gx * blockIdx.y;
-    if ((nt & 7) == 0) r = (r & 7) * (nt >> 3) + (r >> 3);
-    return make_int2(r % gx, r / gx);
-}
-
 // ------------------------------------------------ partitioned line solve
 //
 // The same systems as k_sweep, each line cut into P chunks of PM rows, one
@@ -3354,7 +3329,9 @@ __device__ __forceinline__ int2 xcd_block_xy()
 //
 // The kernels are bound by the latency of one chunk's instructions, so a
 // chunk is straight code: all chunks have PM rows, a line's last chunk filled
-// up with rows x = 0 that couple to nothing, and boundary rows differ by
+// up with its last row again (they read the line's last row, whose upper
+// coefficient is zero, so no row of the line reads them, and the coupling takes
+// a zero first row after the last chunk), and boundary rows differ by
 // numbers instead of branches.  (Chunks of varying length with their rows
 // under conditions took 711 branches and 1700 integer instructions for the
 // 650 FP64 operations of an x chunk, and one thread per line solving the
@@ -3565,7 +3542,7 @@ __global__ __launch_bounds__(PART_THREADS, 4) void k_sweep_part(Dims d, LineSets
     scal += blockIdx.z * S_SIZE;
     const Rng R = L.R;
     // Lanes cover k = 1 .. nz of a row, rounded up to 16 lanes (an aligned
-    // piece of it).  x-lines: the y ghosts of the new values (jg) are rows of
+    // piece of a pitched one).  x-lines: the y ghosts of the new values (jg) are rows of
     // lanes of their own that solve the line next to the wall again and store
     // at their own place; the z ghosts (kg) are stored by the lanes at the
     // row's ends
@@ -4055,7 +4032,7 @@ static bool single(const Ctx<T>& c, const char* what)
 
 // Tiles of one i-plane of at most 256 threads (k, j), k from 1: a row is cut
 // into as few equal parts of at most 128 points as it needs, each rounded up
-// to 16 lanes (an aligned piece of a row), and a tile takes as many rows as
+// to 16 lanes (an aligned piece of a pitched row), and a tile takes as many rows as
 // fit, kp points a lane (128 x 2 measured faster than 64 x 4, 32 x 8 and 256 x 1 for the cell
 // kernels at 128-point rows; at 96 points 96 x 2 leaves no lane idle where
 // 128 x 2 left a quarter)
@@ -4228,8 +4205,8 @@ static void adi_sets(Ctx<T>& c, T g, T r, int slot, const int* F, int nset, T* c
         }
         const int P = c.line_solver == 0 ? part_chunks(nmin, nmax, DIR) : 0;
         if (P > 0 && DIR != 2) {
-            // lines per block: y-lines 256 bytes of a row (rows start 8-byte
-            // aligned only, so longer runs fetch fewer partial cache lines);
+            // lines per block: y-lines 256 bytes of a row (short pieces of it
+            // fetch more lines than they use);
             // x-lines, which couple more chunks, 16 lines (256x128x128, y at 16:
             // 65 us instead of 57 FP64, 41 instead of 27 FP32; x at 32: 86
             // instead of 83 FP64, 15.3 instead of 12.0 for c in FP32)
@@ -4405,16 +4382,12 @@ void Ops<T>::velo_ghost(Ctx<T>& c)
 template <typename T>
 void Ops<T>::divergence(Ctx<T>& c, double g, double r, bool write_div, bool pack)
 {
+    if (!single(c, "divergence")) return;
     dim3 blk;
-    const dim3 grd = bgrid(cell_grid(field_rng(c.d, FC), blk), c);
-    if (c.bt.nm > 1)
-        PLLC_L(c, "div", (k_div<T, true><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[U_NEW], c.f[V_NEW], c.f[W_NEW],
-                                                                 write_div ? c.f[DIV] : nullptr, pack ? c.P : nullptr,
-                                                                 c.scal, T(g), T(r), c.bt)));
-    else
-        PLLC_L(c, "div", (k_div<T><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[U_NEW], c.f[V_NEW], c.f[W_NEW],
-                                                           write_div ? c.f[DIV] : nullptr, pack ? c.P : nullptr, c.scal,
-                                                           T(g), T(r), c.bt)));
+    const dim3 grd = cell_grid(field_rng(c.d, FC), blk);
+    PLLC_L(c, "div", (k_div<T><<<grd, blk, 0, c.st>>>(c.d, c.ph, c.f[U_NEW], c.f[V_NEW], c.f[W_NEW],
+                                                       write_div ? c.f[DIV] : nullptr, pack ? c.P : nullptr, c.scal,
+                                                       T(g), T(r))));
 }
 
 // opts kernel f in to sm bytes of dynamic LDS per block; false when the
@@ -4782,12 +4755,6 @@ template <typename T>
 void Ops<T>::unpack(Ctx<T>& c, const double* a, T* b, long rows)
 {
     k_unpack<T><<<row_grid(rows), dim3(64, 4), 0, c.st>>>(c.d, a, b, rows);
-}
-
-template <typename T>
-void Ops<T>::fill(Ctx<T>& c, T* a, long n, T v)
-{
-    k_fill<T><<<bulk_grid(n), 256, 0, c.st>>>(a, n, v);
 }
 
 template <typename T>
