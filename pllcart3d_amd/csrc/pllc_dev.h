@@ -26,7 +26,7 @@ struct Dims {
 
 // The layout of a simulation's own fields (values of esize bytes).  Large
 // fields are pitched: rows of a whole number of 128-byte lines, and fields that
-// start pitch_lead values after an aligned address, so that the interior point
+// start a line less one value after an aligned address, so that the interior point
 // k = 1 of every row starts a line; the line after a row's points holds its
 // ghost k = nz + 1 and the next row's k = 0.  With rows at any 8-byte offset
 // every 16 lanes of a load or store touched two 64-byte blocks of the L1
@@ -35,37 +35,38 @@ struct Dims {
 // k_corr_pg 573 -> 540; 256x128x128 x-sweep 83 -> 72 FP64.  k = 1 at 64 bytes
 // into a line: slower than packed rows (x-sweep 825, k_corr_pg mixed 598).
 //
-// Smaller fields, which the caches hold in part, and fields whose rows the lines
-// would lengthen by more than half are packed (sy = NZ): nothing is gained there
-// and a packed FP64 field is also the host's layout.  us a step, pitched ->
-// packed: 256x96x96 mixed 862 -> 851, 300x120x80 mixed 1220 -> 1190, 400x50x50
-// FP64 978 -> 900, 192x64x64 FP64 625 -> 627, 512x128x32 mixed 857 -> 788,
-// 400x400x4 mixed 2490 -> 1875 (770 -> 168 MB); above the line 256x128x112 FP64
-// 2260 -> 2304, 256x128x128 mixed 1303 -> 1349, 512x256x64 mixed 3187 -> 3266.
-constexpr long PITCH_POINTS = 3500000;
-__host__ inline long pitched_row(const Dims& d, int esize)
+// Fields of fewer points (all members of a batch together: what a launch covers)
+// are packed (sy = NZ), and so are rows shorter than a wave, several of which a
+// wave covers at any offset: nothing is gained there, short rows grow by up to a
+// multiple, and a packed FP64 field is also the host's layout.  us a step,
+// pitched -> packed: 400x400x4 mixed 2490 -> 1875 (770 -> 168 MB), 512x128x32
+// mixed 857 -> 788, 400x50x50 FP64 978 -> 900, 16 members of 128x48x48 1830 ->
+// 1767, 200x64x100 mixed 600 -> 571, 60x128x128 FP64 839 -> 826, 192x64x64 mixed
+// 418 -> 417; on the pitched side of the line 200x60x128 mixed 632 -> 651, 8
+// members of 192x64x64 2021 -> 2105, 256x96x96 FP64 1516 -> 1525 (mixed 862 ->
+// 851), 200x128x128 FP64 1955 -> 2000, 100x256x256 mixed 2083 -> 2257.
+constexpr long PITCH_POINTS = 1500000;
+constexpr int PITCH_ROW = 64;
+// sets the strides of fields of `members` handles stepped together; returns the
+// values between an aligned address and a field's first point
+__host__ inline long pitch_dims(Dims& d, int esize, long members)
 {
     const long q = 128 / esize;
-    return (d.NZ + q - 1) / q * q;
-}
-__host__ inline bool pitched(const Dims& d, int esize)
-{
-    return (long)d.NX * d.NY * d.NZ >= PITCH_POINTS && 2 * (pitched_row(d, esize) - d.NZ) <= d.NZ;
-}
-__host__ inline long pitch_lead(const Dims& d, int esize) { return pitched(d, esize) ? 128 / esize - 1 : 0; }
-__host__ inline void pitch_dims(Dims& d, int esize)
-{
-    d.sy = pitched(d, esize) ? pitched_row(d, esize) : d.NZ;
+    const bool pitch = d.nz >= PITCH_ROW && (long)d.NX * d.NY * d.NZ * members >= PITCH_POINTS;
+    d.sy = pitch ? (d.NZ + q - 1) / q * q : d.NZ;
     d.sx = (long)d.NY * d.sy;
+    return pitch ? q - 1 : 0;
 }
-// values of one field
+// values of one field, and with the room of two rows behind it, so that as a
+// buffer of FP64 rows an FP32 field holds half its rows whatever their number
 __host__ inline long field_values(const Dims& d) { return (long)d.NX * d.sx; }
+__host__ inline long field_room(const Dims& d) { return field_values(d) + 2 * d.NZ; }
 // values from one field's first point to the next one's in a slab of several:
 // whole 128-byte lines
 __host__ inline long field_stride(const Dims& d, int esize)
 {
     const long q = 128 / esize;
-    return (field_values(d) + q - 1) / q * q;
+    return (field_room(d) + q - 1) / q * q;
 }
 
 // a / h for a divisor fixed on the host, with rh = 1/h correctly rounded

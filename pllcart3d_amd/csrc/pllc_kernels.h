@@ -51,6 +51,7 @@ struct Ctx {
     Phys ph;
     hipStream_t st = nullptr;
     T* f[NFIELDS] = {};
+    long lead = 0;       // values between an aligned address and a field (pitch_dims)
     T* P = nullptr;      // packed [nx][ny][nz] Poisson block
     T* Q = nullptr;      // second packed block
     T* QC = nullptr;     // Thomas factors of the Poisson x-lines

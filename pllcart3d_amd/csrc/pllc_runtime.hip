@@ -8,6 +8,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -423,6 +424,7 @@ struct pllc_sim {
     int cnn_every = 0;            // 0: a new correction every substage; k: at the first substage
     long cnn_steps = 0;           // of every k-th step, held in between (steps counted here)
     std::vector<void*> snap;
+    std::vector<float> host;      // the last conversions' host side (HOST transfers)
     double* gscratch = nullptr;
 };
 
@@ -454,15 +456,14 @@ static size_t npts(const pllc_sim* s) { return (size_t)s->cd.d.NX * s->cd.d.NY *
 // a zeroed device allocation of one field; the pointer returned is its first
 // point
 template <typename T>
-static T* field_alloc(pllc_sim* s, const Dims& d, const char* W)
+static T* field_alloc(pllc_sim* s, const Ctx<T>& c, const char* W)
 {
     void* p = nullptr;
-    const long lead = pitch_lead(d, sizeof(T));
-    const size_t bytes = (field_values(d) + lead + (lead ? 1 : 0)) * sizeof(T);
+    const size_t bytes = (field_room(c.d) + c.lead) * sizeof(T);
     if (!pllc_hip_ok(W, hipMalloc(&p, bytes))) return nullptr;
     s->owned.push_back(p);
     if (!pllc_hip_ok(W, hipMemset(p, 0, bytes))) return nullptr;
-    return (T*)p + lead;
+    return (T*)p + c.lead;
 }
 
 void pllc_fill_dims(const pllc_params* p, Dims& d, Phys& ph)
@@ -482,20 +483,21 @@ void pllc_fill_dims(const pllc_params* p, Dims& d, Phys& ph)
 }
 
 template <typename T>
-static bool create_t(pllc_sim* s)
+static bool create_t(pllc_sim* s, long members)
 {
     Ctx<T>& c = ctx<T>(s);
     const char* W = "pllc_sim_create";
     std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
     pllc_fill_dims(&s->p, c.d, c.ph);
-    pitch_dims(c.d, sizeof(T));
+    c.lead = pitch_dims(c.d, sizeof(T), members);
     c.st = s->st;
     for (int f = 0; f < NFIELDS; f++)
-        if (!(c.f[f] = field_alloc<T>(s, c.d, W))) return false;
+        if (!(c.f[f] = field_alloc<T>(s, c, W))) return false;
     return pllc_ctx_tables<T>(c, s->owned, W);
 }
 
-extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision)
+// members: how many handles of this grid an ensemble steps together
+static pllc_sim* sim_create(const pllc_params* p, int precision, long members)
 {
     if (!p || p->nx < 1 || p->ny < 1 || p->nz < 1) { pllc_set_error("pllc_sim_create", "bad dimensions"); return nullptr; }
     if (p->ny > 1024 || p->nz > 1024) { pllc_set_error("pllc_sim_create", "ny or nz > 1024 not supported"); return nullptr; }
@@ -508,7 +510,7 @@ extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision)
     s->prec = precision;
     pllc_fill_dims(p, s->cd.d, s->cd.ph);   // dims are read from cd in both precisions
     bool ok = pllc_hip_ok("pllc_sim_create", hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking));
-    ok = ok && (precision == PLLC_PREC_PLAIN ? create_t<double>(s) : create_t<float>(s));
+    ok = ok && (precision == PLLC_PREC_PLAIN ? create_t<double>(s, members) : create_t<float>(s, members));
     ok = ok && pllc_hip_ok("pllc_sim_create", hipEventCreate(&s->e0)) &&
          pllc_hip_ok("pllc_sim_create", hipEventCreate(&s->e1));
     s->cd.joint = s->cf.joint = p->Fx == 0.0 && p->Fy == 0.0 ? 1 : 0;
@@ -519,6 +521,8 @@ extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision)
     apply_tuned(s);
     return s;
 }
+
+extern "C" pllc_sim* pllc_sim_create2(const pllc_params* p, int precision) { return sim_create(p, precision, 1); }
 
 extern "C" pllc_sim* pllc_sim_create(const pllc_params* p) { return pllc_sim_create2(p, PLLC_PREC_PLAIN); }
 
@@ -576,19 +580,20 @@ static void normalize(pllc_sim* s, Ctx<T>& c)
 }
 
 // How a field's values and the host's FP64 rows of NZ values get to each other.
-// DIRECT: a packed FP64 field is the host's layout.  HOST: a packed FP32 field
-// is copied as it is and converted on the host.  STAGED: through a scratch field
+// DIRECT: a packed FP64 field is the host's layout.  HOST: an FP32 field is
+// copied as it is and converted on the host.  STAGED: through a scratch field
 // of the sweeps (its content lives only within an operator or a step) as FP64
 // rows, as many at a time as it holds, which a row kernel packs and converts.
-// us a download, STAGED against the other two: FP64 64x32x32 31 : 20 (page-
-// locked host memory), 150x70x51 110 : 91; FP32 64x32x32 51 : 29 and 97x45x39 68 :
-// 61, but 128x64x64 122 : 218 and 256x128x128 682 : 2104.  Pageable host memory
-// takes twice the bytes worse: 64x32x32 67 : 29, 128x64x64 278 : 221, 300x120x24
-// 449 : 344, 256x128x128 (pitched) 1976 : 2154.  Hence FP32 fields convert on the
-// host if packed, unless the host memory is page-locked and the field has 250000
-// points or more.
+// us a download, STAGED : DIRECT, FP64 in page-locked host memory: 64x32x32 31 :
+// 20, 150x70x51 110 : 91.  FP32, STAGED : HOST, page-locked: 24x16x16 41 : 29,
+// 64x32x32 54 : 40 (95 where the program's other threads read the array between
+// two downloads, which takes its lines to their caches), 170x32x32 70 : 66 (190),
+// 128x64x64 126 : 236, 256x128x128 714 : 2437; pageable (a copy of its own on the
+// host for either): 64x32x32 73 : 39, 128x64x64 306 : 220, 150x90x100 701 : 714,
+// 256x96x96 1186 : 1427.  Hence the line for FP32: 50000 points where the host
+// memory is page-locked, 1.5 million where not.
 enum class Route { DIRECT, HOST, STAGED };
-constexpr long STAGE_POINTS = 250000;
+constexpr long STAGE_LOCKED = 50000, STAGE_PAGED = 1500000;
 
 static bool page_locked(const void* p)
 {
@@ -603,18 +608,31 @@ static bool page_locked(const void* p)
 template <typename T>
 static Route route(const Dims& d, const void* host)
 {
-    if (pitched(d, sizeof(T))) return Route::STAGED;
-    if (sizeof(T) == sizeof(double)) return Route::DIRECT;
-    return field_values(d) >= STAGE_POINTS && page_locked(host) ? Route::STAGED : Route::HOST;
+    if (sizeof(T) == sizeof(double)) return d.sy == d.NZ ? Route::DIRECT : Route::STAGED;
+    const long n = (long)d.NX * d.NY * d.NZ;
+    return n >= STAGE_PAGED || (n >= STAGE_LOCKED && page_locked(host)) ? Route::STAGED : Route::HOST;
 }
 
 template <typename T>
 static double* stage(Ctx<T>& c, long& rows)
 {
-    const int skip = pitched(c.d, sizeof(T)) ? 1 : 0;   // to a 128-byte line's start
+    const int skip = c.lead ? 1 : 0;   // to a 128-byte line's start
     T* p = c.f[F_SRC2] + skip;
-    rows = (long)((field_values(c.d) - skip) * sizeof(T) / (c.d.NZ * sizeof(double)));
+    rows = (long)((field_room(c.d) - skip) * sizeof(T) / (c.d.NZ * sizeof(double)));
     return reinterpret_cast<double*>(p);
+}
+
+// the host's side of a HOST transfer, kept with the handle (allocated anew for
+// every transfer, its page faults took twice the conversion's time)
+template <typename T>
+static T* host_side(pllc_sim* s, size_t n)
+{
+    if constexpr (std::is_same<T, float>::value) {
+        if (s->host.size() < n) s->host.resize(n);
+        return s->host.data();
+    } else {
+        return nullptr;   // FP64 fields have no such transfers
+    }
 }
 
 // dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ
@@ -623,25 +641,26 @@ static double* stage(Ctx<T>& c, long& rows)
 template <typename T>
 static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W)
 {
-    const long n = rows * c.d.NZ;
+    const long nz = c.d.NZ, sy = c.d.sy, n = rows * sy - (sy - nz);   // up to the last row's last point
     bool ok = true;
-    std::vector<T> t;
     switch (route<T>(c.d, src)) {
     case Route::DIRECT:
-        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * c.d.sy, src, n * 8, hipMemcpyHostToDevice, s->st));
+        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * sy, src, rows * nz * 8, hipMemcpyHostToDevice, s->st));
         break;
-    case Route::HOST:
-        t.resize(n);
-        for (long e = 0; e < n; e++) t[e] = T(src[e]);
-        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * c.d.sy, t.data(), n * sizeof(T), hipMemcpyHostToDevice, s->st));
+    case Route::HOST: {
+        T* t = host_side<T>(s, n);
+        for (long r = 0; r < rows; r++)
+            for (long k = 0; k < nz; k++) t[r * sy + k] = T(src[r * nz + k]);
+        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * sy, t, n * sizeof(T), hipMemcpyHostToDevice, s->st));
         break;
+    }
     case Route::STAGED: {
         long most = 0;
         double* b = stage(c, most);
         for (long q = 0; ok && q < rows; q += most) {
             const long m = std::min(most, rows - q);
-            ok = pllc_hip_ok(W, hipMemcpyAsync(b, src + q * c.d.NZ, m * c.d.NZ * 8, hipMemcpyHostToDevice, s->st));
-            if (ok) Ops<T>::unpack(c, b, dst + (r0 + q) * c.d.sy, m);
+            ok = pllc_hip_ok(W, hipMemcpyAsync(b, src + q * nz, m * nz * 8, hipMemcpyHostToDevice, s->st));
+            if (ok) Ops<T>::unpack(c, b, dst + (r0 + q) * sy, m);
         }
         break;
     }
@@ -652,18 +671,18 @@ static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double
 template <typename T>
 static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W)
 {
-    const long rows = (long)c.d.NX * c.d.NY, n = rows * c.d.NZ;
+    const long rows = (long)c.d.NX * c.d.NY, nz = c.d.NZ, sy = c.d.sy, n = rows * sy - (sy - nz);
     bool ok = true;
-    std::vector<T> t;
     switch (route<T>(c.d, dst)) {
-    case Route::DIRECT: ok = pllc_hip_ok(W, hipMemcpyAsync(dst, src, n * 8, hipMemcpyDeviceToHost, s->st)); break;
+    case Route::DIRECT: ok = pllc_hip_ok(W, hipMemcpyAsync(dst, src, rows * nz * 8, hipMemcpyDeviceToHost, s->st)); break;
     case Route::HOST: {
         // (a synchronous copy: 16x8x8 15 us, a queued one 20)
-        t.resize(n);
+        T* t = host_side<T>(s, n);
         if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
         std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-        if (!pllc_hip_ok(W, hipMemcpy(t.data(), src, n * sizeof(T), hipMemcpyDeviceToHost))) return false;
-        for (long e = 0; e < n; e++) dst[e] = double(t[e]);
+        if (!pllc_hip_ok(W, hipMemcpy(t, src, n * sizeof(T), hipMemcpyDeviceToHost))) return false;
+        for (long r = 0; r < rows; r++)
+            for (long k = 0; k < nz; k++) dst[r * nz + k] = double(t[r * sy + k]);
         return true;
     }
     case Route::STAGED: {
@@ -671,8 +690,8 @@ static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W
         double* b = stage(c, most);
         for (long q = 0; ok && q < rows; q += most) {
             const long m = std::min(most, rows - q);
-            Ops<T>::pack(c, src + q * c.d.sy, b, m);
-            ok = pllc_hip_ok(W, hipMemcpyAsync(dst + q * c.d.NZ, b, m * c.d.NZ * 8, hipMemcpyDeviceToHost, s->st));
+            Ops<T>::pack(c, src + q * sy, b, m);
+            ok = pllc_hip_ok(W, hipMemcpyAsync(dst + q * nz, b, m * nz * 8, hipMemcpyDeviceToHost, s->st));
         }
         break;
     }
@@ -1057,7 +1076,7 @@ static int set_closure_t(pllc_sim* s, Ctx<T>& c, pllc_cnn* m, int every)
         return -1;
     }
     if (!c.ncorr) {
-        if (!(c.ncorr = field_alloc<T>(s, c.d, W))) return -1;
+        if (!(c.ncorr = field_alloc<T>(s, c, W))) return -1;
     }
     if (every < 0) {
         pllc_set_error(W, "negative refresh period");
@@ -1290,7 +1309,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     b->m = ms;
     const int nm = (int)ms.size();
     const Ctx<float>& c0 = ms[0]->cf;
-    const long fs = field_stride(c0.d, 4), lead = pitch_lead(c0.d, 4);
+    const long fs = field_stride(c0.d, 4), lead = c0.lead;
     const long pk = (long)c0.d.nx * c0.d.ny * c0.d.nz;
     const long np = c0.npart;
     auto get = [&](size_t bytes) -> void* {
@@ -1304,7 +1323,7 @@ static ens_batch* batch_create(const std::vector<pllc_sim*>& ms)
     bool ok = pllc_hip_ok(W, hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking)) &&
               pllc_hip_ok(W, hipEventCreateWithFlags(&b->ev, hipEventDisableTiming));
     for (int f = 0; ok && f < NFIELDS; f++) {
-        float* q = (float*)get(((size_t)nm * fs + lead + 1) * 4);
+        float* q = (float*)get(((size_t)nm * fs + lead) * 4);
         ok = q != nullptr;
         b->c.f[f] = q + (ok ? lead : 0);
     }
@@ -1480,7 +1499,11 @@ extern "C" pllc_ensemble* pllc_ensemble_create(const pllc_params* p, int n, int 
     const char* og = getenv("PLLC_ENSEMBLE_GRAPH");
     e->one_graph = !(og && strcmp(og, "0") == 0);
     for (int i = 0; ok && i < n; i++) {
-        pllc_sim* s = pllc_sim_create2(&p[i], precision);
+        // (the members of a batch are those of equal grids, in mixed precision)
+        const long alike = precision != PLLC_PREC_MIXED ? 1 : std::count_if(p, p + n, [&](const pllc_params& q) {
+            return q.nx == p[i].nx && q.ny == p[i].ny && q.nz == p[i].nz;
+        });
+        pllc_sim* s = sim_create(&p[i], precision, alike);
         hipEvent_t v = nullptr;
         ok = s != nullptr && pllc_hip_ok(W, hipEventCreateWithFlags(&v, hipEventDisableTiming));
         if (s) e->m.push_back(s);

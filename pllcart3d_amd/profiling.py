@@ -194,8 +194,7 @@ def _field_kib(points, row, b):
     before's last point) and written in 32-byte pieces (one for k = 0, and
     those of the interior and of k = nz + 1, which ends in the interior's last
     piece or starts one)."""
-    q = 128 // b
-    if points < 3500000 or 2 * (-(-row // q) * q - row) > row:
+    if points < 1500000 or row < 66:
         return points * b / 1024.0, points * b / 1024.0
     rows = points / row
     return rows * -(-row * b // 128) * 128 / 1024.0, rows * (2 + (row - 2) * b // 32) * 32 / 1024.0

@@ -1,6 +1,6 @@
-"""Fields of at least 3.5 million points, whose rows are pitched to whole
-128-byte lines: rows one value longer than a line, one shorter than two and
-of whole lines, through uploads, downloads and a step."""
+"""Large fields (from 1.5 million points and 64 points a row on), whose rows are
+pitched to whole 128-byte lines: rows one value longer than a line, one shorter
+than two and of whole lines, through uploads, downloads and a step."""
 import os
 
 import numpy as np
@@ -75,3 +75,26 @@ def test_fused_step_equals_operators(precision):
     for f in ("C_OLD", "U_OLD", "V_OLD", "W_OLD", "PHI", "U_PG", "W_PG", "MUO_CELL"):
         x, y = a.download(f), b.download(f)
         assert np.array_equal(x, y), (precision, f, np.abs(x - y).max())
+
+
+def test_batched_members_equal_standalone_runs():
+    """Two members of 200x64x64, pitched as the batch has 1.8 million points,
+    keep the bits of the same simulations run alone, whose rows are packed."""
+    prm = [P.make_params(200, 64, 64, Vratio=3.0 - i, Pe=300.0 + 100 * i, Inf_thick=0.1) for i in range(2)]
+    c0 = [P.ic_fill(p, P.IC_NOISE, 3 + i, 0.05) for i, p in enumerate(prm)]
+    ens = P.Ensemble(prm, "mixed")
+    assert ens.batches() == 1
+    alone = [P.Sim(p, "mixed") for p in prm]
+    for m, s, c in zip(ens.members, alone, c0):
+        m.init(c)
+        s.init(c)
+    w = np.random.default_rng(1).standard_normal(alone[0].shape)
+    for steps in (2, 3):
+        ens.run(steps)
+        for m, s in zip(ens.members, alone):
+            s.run(steps)
+            for f in ("C_OLD", "U_OLD", "V_OLD", "W_OLD", "PHI", "U_PG"):
+                assert np.array_equal(m.download(f), s.download(f)), (steps, f)
+            m.upload("DIV", w)
+            assert np.array_equal(m.download("DIV"), w.astype(np.float32).astype(float))
+    ens.close()

@@ -1,6 +1,7 @@
 """Uploads and downloads by every route: packed FP64 fields as they are, FP32
-ones converted on the host or (from 250000 points on, page-locked host memory)
-on the device in several pieces, pitched ones through the device."""
+ones converted on the host or (from 50000 points on where the host memory is
+page-locked, from 1.5 million on where not) on the device in several pieces,
+pitched FP64 ones through the device."""
 import ctypes
 
 import numpy as np
@@ -23,7 +24,7 @@ def _call(fn, sim, field, a):
 
 @pytest.mark.parametrize("locked", [False, True])
 @pytest.mark.parametrize("precision", ["plain", "mixed"])
-@pytest.mark.parametrize("shape", [(7, 6, 4), (129, 40, 39), (130, 41, 43), (520, 82, 81)])
+@pytest.mark.parametrize("shape", [(7, 6, 4), (30, 38, 32), (31, 40, 32), (129, 40, 39), (130, 41, 43), (250, 90, 78), (520, 82, 81)])
 def test_round_trip(shape, precision, locked):
     """Every value comes back as uploaded (mixed: rounded to FP32 once), from
     and to host memory of either kind, before and after fused steps (whose

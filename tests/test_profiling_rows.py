@@ -47,7 +47,7 @@ def test_pitched_rows(tmp_path, capsys, nx, ny, row, b):
 
 
 def test_packed_fields(tmp_path, capsys):
-    """Fewer than 3.5 million points: the fields' own bytes, whatever the row."""
+    """Fewer than 1.5 million points: the fields' own bytes, whatever the row."""
     kib = 12 * 134 * 66 * 66 * 8 / 1024
     out = _summary(tmp_path, capsys, kib, kib, points=134 * 66 * 66, row=66)
     assert "factors are 1.000 (fetch) and 1.000 (write)" in out
