@@ -158,10 +158,10 @@ struct Ops {
     static void set_scalar(Ctx<T>& c, int idx, double v);
     // two scalars, and with_stale stale() of the old fields, in one launch
     static void op_start(Ctx<T>& c, int i0, double v0, int i1, double v1, bool with_stale);
-    // dense 2D DCT of a packed block: REDFT10 (forward) or REDFT01
-    // (inverse), z then y, `in` -> `out` through the temporary c.Q
-    // phi (inverse only): the result goes to phi's interior instead of out
-    static void dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi = nullptr, bool ghosts = false,
+    // 2D DCT of a packed block in place: REDFT10 (forward) or REDFT01
+    // (inverse), z then y (k_gemm: through the temporary c.Q)
+    // phi (inverse only): the result goes to phi's interior instead of io
+    static void dct2(Ctx<T>& c, T* io, bool inverse, T* phi = nullptr, bool ghosts = false,
                      const DivIn<T>* div = nullptr);
     // whether there is a fast transform for ny = nz = n and the device gives
     // its blocks the LDS it needs (n = 128: a whole plane of T; n = 256: 32

@@ -2186,12 +2186,11 @@ __host__ __device__ constexpr int ds_pitch(int nz) { return nz + 4; }
 // tile's MFMA sequence is k_gemm's (a zero accumulator, k ascending in
 // steps of 4), so the result equals the two k_gemm launches bit for bit,
 // without Q's round trip through HBM.  A plane is read whole before any of
-// it is written, by its one block, so in may equal out (neither is
-// __restrict__).
+// it is written, by its one block: the transform is in place (io).
 __host__ __device__ constexpr int dct_planes_threads(int N) { return N ? 4 * N : 256; }
 
 template <typename T, bool INV, int N>
-__global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, int nplanes, const T* in, T* out,
+__global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, int nplanes, T* __restrict__ io,
                                                     const T* __restrict__ Cz, const T* __restrict__ Cy, PhiOut<T> po,
                                                     DivIn<T> dv, Bt bt)
 {
@@ -2239,7 +2238,7 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
             }
             return;
         }
-        const T* src = in + (long)p * plane;
+        const T* src = io + (long)p * plane;
 #pragma unroll
         for (int u = 0; u < PF; u++) {
             const int e = threadIdx.x + NT * u;
@@ -2314,7 +2313,7 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
             for (int r = 0; r < 4; r++) {
                 const int gm = ty0[u] + Mma<T>::row(lk, r), gn = tz0[u] + li;
                 if (INV && po.phi) phi_store(pm, x, gm, gn, fdiv<T>(acc[u][r], norm));
-                else out[(long)p * plane + (long)gm * nz + gn] = acc[u][r];
+                else io[(long)p * plane + (long)gm * nz + gn] = acc[u][r];
             }
         }
         __syncthreads();   // Q read by every wave, P holds plane p + G
@@ -2338,8 +2337,8 @@ __global__ __launch_bounds__(256) void k_dct_planes(int ny_, int nz_, int nx, in
 // round trip; here a plane's load, its two contractions (6 us of matrix
 // instructions at 96 x 96 FP32) and its store follow each other in the one
 // block of a CU.  The whole plane's loads in flight at once instead of four a
-// thread: no faster.  A plane is read whole before any of it is written, so
-// in may equal out (neither is __restrict__).
+// thread: no faster.  A plane is read whole before any of it is written: the
+// transform is in place (io).
 constexpr int DW_MAX = 128;
 __host__ __device__ constexpr int dw_tiles(int n) { return (n + 15) / 16; }
 __host__ __device__ constexpr int dw_pitch(int nz) { return 16 * dw_tiles(nz) + 4; }
@@ -2387,7 +2386,7 @@ __device__ __forceinline__ void dw_contract(typename Mma<T>::acc (&acc)[4], cons
 }
 
 template <typename T, bool INV>
-__global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* in, T* out, const T* __restrict__ Oz,
+__global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, T* __restrict__ io, const T* __restrict__ Oz,
                                                    const T* __restrict__ Oy, PhiOut<T> po, DivIn<T> dv)
 {
     extern __shared__ unsigned char pllc_smem[];
@@ -2398,7 +2397,7 @@ __global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* in, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, lk = lane >> 4;
     const long plane = (long)ny * nz;
-    const T* src = in + blockIdx.x * plane;
+    const T* src = io + blockIdx.x * plane;
     const int cells = 256 * ty * tz, nzp = 16 * tz;
     const bool fused = !INV && dv.u;
     const T f = fused ? dv.fac(Bt{}, 0) : T(0);
@@ -2463,7 +2462,7 @@ __global__ __launch_bounds__(1024) void k_dct_wide(int ny, int nz, const T* in, 
             const int gm = 16 * yt + Mma<T>::row(lk, r), gn = 16 * (z0 + u) + li;
             if (gm >= ny || gn >= nz) continue;
             if (INV && po.phi) phi_store(po, (int)blockIdx.x, gm, gn, fdiv<T>(acc[u][r], norm));
-            else out[blockIdx.x * plane + (long)gm * nz + gn] = acc[u][r];
+            else io[blockIdx.x * plane + (long)gm * nz + gn] = acc[u][r];
         }
     }
 }
@@ -3185,10 +3184,10 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
                                             Visc4<T>, const T*, const T*, const T*, const double*, T, T, int, Bt);
 
 #define PLLC_INST_DCT_PLANES(T, N)                                                                             \
-    template __global__ void k_dct_planes<T, false, N>(int, int, int, int, const T*, T*, const T*, const T*,   \
-                                                       PhiOut<T>, DivIn<T>, Bt);                               \
-    template __global__ void k_dct_planes<T, true, N>(int, int, int, int, const T*, T*, const T*, const T*,    \
-                                                      PhiOut<T>, DivIn<T>, Bt);
+    template __global__ void k_dct_planes<T, false, N>(int, int, int, int, T*, const T*, const T*, PhiOut<T>,  \
+                                                       DivIn<T>, Bt);                                          \
+    template __global__ void k_dct_planes<T, true, N>(int, int, int, int, T*, const T*, const T*, PhiOut<T>,   \
+                                                      DivIn<T>, Bt);
 
 #define PLLC_INST(T)                                                                                           \
     template __global__ void k_stale<T>(Dims, const T*, const T*, const T*, const T*, T*);                      \
@@ -3218,10 +3217,8 @@ __global__ void k_weno_batch(const double* __restrict__ d1, const int* __restric
     PLLC_INST_DCT_PLANES(T, 32)                                                                                \
     PLLC_INST_DCT_PLANES(T, 48)                                                                                \
     PLLC_INST_DCT_PLANES(T, 64)                                                                                \
-    template __global__ void k_dct_wide<T, false>(int, int, const T*, T*, const T*, const T*, PhiOut<T>,       \
-                                                  DivIn<T>);                                                   \
-    template __global__ void k_dct_wide<T, true>(int, int, const T*, T*, const T*, const T*, PhiOut<T>,        \
-                                                 DivIn<T>);                                                    \
+    template __global__ void k_dct_wide<T, false>(int, int, T*, const T*, const T*, PhiOut<T>, DivIn<T>);      \
+    template __global__ void k_dct_wide<T, true>(int, int, T*, const T*, const T*, PhiOut<T>, DivIn<T>);       \
     template __global__ void k_gemm<T, true>(int, int, int, const T*, long, const T*, long, T*, long,          \
                                              PhiOut<T>);                                                        \
     template __global__ void k_gemm<T, false>(int, int, int, const T*, long, const T*, long, T*, long,         \
@@ -4422,7 +4419,7 @@ bool Ops<T>::dct_mfma_ready(int n)
 
 // the k_dct_planes form for (ny, nz): unrolled for square planes
 template <typename T>
-using DctPlanesFn = void (*)(int, int, int, int, const T*, T*, const T*, const T*, PhiOut<T>, DivIn<T>, Bt);
+using DctPlanesFn = void (*)(int, int, int, int, T*, const T*, const T*, PhiOut<T>, DivIn<T>, Bt);
 template <typename T>
 static DctPlanesFn<T> dct_planes_fn(bool inv, int ny, int nz)
 {
@@ -4490,7 +4487,7 @@ bool Ops<T>::dct_fast_ready(int n)
 }
 
 template <typename T>
-void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool ghosts, const DivIn<T>* div)
+void Ops<T>::dct2(Ctx<T>& c, T* io, bool inverse, T* phi, bool ghosts, const DivIn<T>* div)
 {
     const DivIn<T> dv = div ? *div : DivIn<T>{};
     const int nx = c.d.nx, ny = c.d.ny, nz = c.d.nz;
@@ -4500,9 +4497,9 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
             const size_t sm = (size_t)DM_N * DM_P * sizeof(float);
             if (inverse) {
                 const PhiOut<float> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
-                PLLC_L(c, "dct", (k_dct_bf16x3<true><<<nx, 512, sm, c.st>>>(in, out, c.cbf, po)));
+                PLLC_L(c, "dct", (k_dct_bf16x3<true><<<nx, 512, sm, c.st>>>(io, io, c.cbf, po)));
             } else {
-                PLLC_L(c, "dct", (k_dct_bf16x3<false><<<nx, 512, sm, c.st>>>(in, out, c.cbf, PhiOut<float>{})));
+                PLLC_L(c, "dct", (k_dct_bf16x3<false><<<nx, 512, sm, c.st>>>(io, io, c.cbf, PhiOut<float>{})));
             }
             return;
         }
@@ -4512,9 +4509,9 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const size_t sm = (size_t)FD_N * FD_P * sizeof(T);
         const PhiOut<T> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
         if (inverse)
-            PLLC_L(c, "dct", (k_dct_plane<T, true><<<nx, FdCfg<T>::threads, sm, c.st>>>(in, out, c.tw, po, dv)));
+            PLLC_L(c, "dct", (k_dct_plane<T, true><<<nx, FdCfg<T>::threads, sm, c.st>>>(io, io, c.tw, po, dv)));
         else
-            PLLC_L(c, "dct", (k_dct_plane<T, false><<<nx, FdCfg<T>::threads, sm, c.st>>>(in, out, c.tw,
+            PLLC_L(c, "dct", (k_dct_plane<T, false><<<nx, FdCfg<T>::threads, sm, c.st>>>(io, io, c.tw,
                                                                                            PhiOut<T>{}, dv)));
         return;
     }
@@ -4525,14 +4522,14 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const size_t sm = (size_t)FL * (N + 1) * sizeof(T);
         const unsigned nb = (unsigned)((long)nx * N / FL);
         if (!inverse) {
-            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{}, dv)));
-            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, PhiOut<T>{},
+            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(io, io, c.tw, PhiOut<T>{}, dv)));
+            PLLC_L(c, "dct", (k_dct_lines<T, false, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(io, io, c.tw, PhiOut<T>{},
                                                                                           DivIn<T>{})));
         } else {
             const PhiOut<T> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
-            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(in, out, c.tw, PhiOut<T>{},
+            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 1, FL><<<nb, 8 * FL, sm, c.st>>>(io, io, c.tw, PhiOut<T>{},
                                                                                          DivIn<T>{})));
-            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(out, out, c.tw, po, DivIn<T>{})));
+            PLLC_L(c, "dct", (k_dct_lines<T, true, N, 2, FL><<<nb, 8 * FL, sm, c.st>>>(io, io, c.tw, po, DivIn<T>{})));
         }
         return;
     }
@@ -4547,7 +4544,7 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const DctPlanesFn<T> kern = dct_planes_fn<T>(inverse, ny, nz);
         const int nthr = dct_planes_threads(ny == nz ? ny : 0);
         const int G = std::max(1, std::min(np, resident_blocks(kern, nthr, sm)));
-        PLLC_L(c, "dct", (kern<<<G, nthr, sm, c.st>>>(ny, nz, nx, np, in, out, tz, ty, po, dv, c.bt)));
+        PLLC_L(c, "dct", (kern<<<G, nthr, sm, c.st>>>(ny, nz, nx, np, io, tz, ty, po, dv, c.bt)));
         return;
     }
     if (!single(c, "dct2")) return;
@@ -4556,26 +4553,26 @@ void Ops<T>::dct2(Ctx<T>& c, const T* in, T* out, bool inverse, T* phi, bool gho
         const int nthr = 64 * dw_waves(ny, nz);
         const PhiOut<T> po{inverse ? phi : nullptr, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
         if (inverse)
-            PLLC_L(c, "dct", (k_dct_wide<T, true><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Oiz, c.Oiy, po, dv)));
+            PLLC_L(c, "dct", (k_dct_wide<T, true><<<nx, nthr, sm, c.st>>>(ny, nz, io, c.Oiz, c.Oiy, po, dv)));
         else
-            PLLC_L(c, "dct", (k_dct_wide<T, false><<<nx, nthr, sm, c.st>>>(ny, nz, in, out, c.Ofz, c.Ofy, po, dv)));
+            PLLC_L(c, "dct", (k_dct_wide<T, false><<<nx, nthr, sm, c.st>>>(ny, nz, io, c.Ofz, c.Ofy, po, dv)));
         return;
     }
     const long R = (long)nx * ny, plane = (long)ny * nz;
     const dim3 gz((nz + 127) / 128, (unsigned)((R + 63) / 64), 1), gy((nz + 127) / 128, (ny + 63) / 64, nx);
     if (!inverse) {
-        // z: Q[r][kz] = sum_m in[r][m] Cfz[kz][m]; then y: out[x] = Cfy Q[x]
-        PLLC_L(c, "dct", (k_gemm<T, true><<<gz, 256, 0, c.st>>>((int)R, nz, nz, in, 0, c.Cfz, 0, c.Q, 0,
+        // z: Q[r][kz] = sum_m io[r][m] Cfz[kz][m]; then y: io[x] = Cfy Q[x]
+        PLLC_L(c, "dct", (k_gemm<T, true><<<gz, 256, 0, c.st>>>((int)R, nz, nz, io, 0, c.Cfz, 0, c.Q, 0,
                                                                   PhiOut<T>{})));
-        PLLC_L(c, "dct", (k_gemm<T, false><<<gy, 256, 0, c.st>>>(ny, nz, ny, c.Cfy, 0, c.Q, plane, out, plane,
+        PLLC_L(c, "dct", (k_gemm<T, false><<<gy, 256, 0, c.st>>>(ny, nz, ny, c.Cfy, 0, c.Q, plane, io, plane,
                                                                    PhiOut<T>{})));
     } else {
         // z then y, as the forward transform; with phi set the y pass writes
-        // phi (and with ghosts its face ghosts) instead of out
-        PLLC_L(c, "dct", (k_gemm<T, true><<<gz, 256, 0, c.st>>>((int)R, nz, nz, in, 0, c.Ciz, 0, c.Q, 0,
+        // phi (and with ghosts its face ghosts) instead of io
+        PLLC_L(c, "dct", (k_gemm<T, true><<<gz, 256, 0, c.st>>>((int)R, nz, nz, io, 0, c.Ciz, 0, c.Q, 0,
                                                                   PhiOut<T>{})));
         const PhiOut<T> po{phi, c.d.sx, c.d.sy, nx, ny, nz, ghosts ? 1 : 0};
-        PLLC_L(c, "dct", (k_gemm<T, false><<<gy, 256, 0, c.st>>>(ny, nz, ny, c.Ciy, 0, c.Q, plane, out, plane, po)));
+        PLLC_L(c, "dct", (k_gemm<T, false><<<gy, 256, 0, c.st>>>(ny, nz, ny, c.Ciy, 0, c.Q, plane, io, plane, po)));
     }
 }
 
@@ -4601,7 +4598,7 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts, 
     }
     // the spectrum, in place in P
     T* sp = c.P;
-    dct2(c, c.P, sp, false, nullptr, false, &dv);
+    dct2(c, sp, false, nullptr, false, &dv);
     const int PC = c.line_solver == 0 ? part_chunks(c.d.nx, c.d.nx, 0) : 0;
     if (PC > 0) {
         // 128 bytes of a row per block, more where that is less than 256
@@ -4617,7 +4614,7 @@ void Ops<T>::poisson(Ctx<T>& c, double g, double r, bool from_div, bool ghosts, 
         PLLC_L(c, "pois_x", (k_pois_x<T><<<line_grid(nm), 256, 0, c.st>>>(c.d, c.lam_y, c.lam_z, sp, c.QC, c.lam00)));
     }
     // the inverse transform's last pass writes phi, normalised
-    dct2(c, sp, sp, true, c.f[PHI], ghosts);
+    dct2(c, sp, true, c.f[PHI], ghosts);
 }
 
 template <typename T>

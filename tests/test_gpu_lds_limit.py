@@ -11,8 +11,8 @@ from pllcart3d_amd._lib import load
 
 pytestmark = pytest.mark.gpu
 
-WIDE = "_ZN4pllc10k_dct_wideI%sLb%dEEEviiPKT_PS1_S3_S3_NS_6PhiOutIS1_EENS_5DivInIS1_EE"
-PLANES = "_ZN4pllc12k_dct_planesI%sLb%dELi0EEEviiiiPKT_PS1_S3_S3_NS_6PhiOutIS1_EENS_5DivInIS1_EENS_2BtE"
+WIDE = "_ZN4pllc10k_dct_wideI%sLb%dEEEviiPT_PKS1_S4_NS_6PhiOutIS1_EENS_5DivInIS1_EE"
+PLANES = "_ZN4pllc12k_dct_planesI%sLb%dELi0EEEviiiiPT_PKS1_S4_NS_6PhiOutIS1_EENS_5DivInIS1_EENS_2BtE"
 
 
 class _Attributes(C.Structure):   # hipFuncAttributes
