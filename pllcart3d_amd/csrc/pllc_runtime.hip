@@ -605,12 +605,26 @@ static bool page_locked(const void* p)
     return a.type == hipMemoryTypeHost;
 }
 
+// once: a handle's first transfer, for which HOST would allocate its buffer
 template <typename T>
-static Route route(const Dims& d, const void* host)
+static Route route(const Dims& d, bool locked, bool once = false)
 {
     if (sizeof(T) == sizeof(double)) return d.sy == d.NZ ? Route::DIRECT : Route::STAGED;
     const long n = (long)d.NX * d.NY * d.NZ;
-    return n >= STAGE_PAGED || (n >= STAGE_LOCKED && page_locked(host)) ? Route::STAGED : Route::HOST;
+    return n >= STAGE_PAGED || (n >= STAGE_LOCKED && (once || locked)) ? Route::STAGED : Route::HOST;
+}
+
+// A copy after the handle's queued work: queued itself where the host memory is
+// page-locked; else synchronous, as the runtime would give the handle's stream
+// pinned buffers of its own to pass it through (0.6 ms for its first copy, 15 ms
+// for an ensemble of 24 members).
+static bool host_copy(pllc_sim* s, void* dst, const void* src, size_t bytes, hipMemcpyKind kind, bool locked,
+                      const char* W)
+{
+    if (locked) return pllc_hip_ok(W, hipMemcpyAsync(dst, src, bytes, kind, s->st));
+    if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
+    std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
+    return pllc_hip_ok(W, hipMemcpy(dst, src, bytes, kind));
 }
 
 template <typename T>
@@ -636,22 +650,21 @@ static T* host_side(pllc_sim* s, size_t n)
 }
 
 // dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ
-// values.  Copies and kernels are queued on the handle's stream and waited for
-// once, also after a failure: what is queued uses the host's memory.
+// values.  What is queued uses the host's memory, so the end waits for it, also
+// after a failure.
 template <typename T>
-static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W)
+static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double* src, const char* W, bool once = false)
 {
     const long nz = c.d.NZ, sy = c.d.sy, n = rows * sy - (sy - nz);   // up to the last row's last point
+    const bool locked = page_locked(src);
     bool ok = true;
-    switch (route<T>(c.d, src)) {
-    case Route::DIRECT:
-        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * sy, src, rows * nz * 8, hipMemcpyHostToDevice, s->st));
-        break;
+    switch (route<T>(c.d, locked, once)) {
+    case Route::DIRECT: ok = host_copy(s, dst + r0 * sy, src, rows * nz * 8, hipMemcpyHostToDevice, locked, W); break;
     case Route::HOST: {
         T* t = host_side<T>(s, n);
         for (long r = 0; r < rows; r++)
             for (long k = 0; k < nz; k++) t[r * sy + k] = T(src[r * nz + k]);
-        ok = pllc_hip_ok(W, hipMemcpyAsync(dst + r0 * sy, t, n * sizeof(T), hipMemcpyHostToDevice, s->st));
+        ok = host_copy(s, dst + r0 * sy, t, n * sizeof(T), hipMemcpyHostToDevice, false, W);
         break;
     }
     case Route::STAGED: {
@@ -659,7 +672,7 @@ static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double
         double* b = stage(c, most);
         for (long q = 0; ok && q < rows; q += most) {
             const long m = std::min(most, rows - q);
-            ok = pllc_hip_ok(W, hipMemcpyAsync(b, src + q * nz, m * nz * 8, hipMemcpyHostToDevice, s->st));
+            ok = host_copy(s, b, src + q * nz, m * nz * 8, hipMemcpyHostToDevice, locked, W);
             if (ok) Ops<T>::unpack(c, b, dst + (r0 + q) * sy, m);
         }
         break;
@@ -672,15 +685,13 @@ template <typename T>
 static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W)
 {
     const long rows = (long)c.d.NX * c.d.NY, nz = c.d.NZ, sy = c.d.sy, n = rows * sy - (sy - nz);
+    const bool locked = page_locked(dst);
     bool ok = true;
-    switch (route<T>(c.d, dst)) {
-    case Route::DIRECT: ok = pllc_hip_ok(W, hipMemcpyAsync(dst, src, rows * nz * 8, hipMemcpyDeviceToHost, s->st)); break;
+    switch (route<T>(c.d, locked)) {
+    case Route::DIRECT: ok = host_copy(s, dst, src, rows * nz * 8, hipMemcpyDeviceToHost, locked, W); break;
     case Route::HOST: {
-        // (a synchronous copy: 16x8x8 15 us, a queued one 20)
         T* t = host_side<T>(s, n);
-        if (!pllc_hip_ok(W, hipStreamSynchronize(s->st))) return false;
-        std::lock_guard<std::recursive_mutex> lk(pllc_api_mutex());
-        if (!pllc_hip_ok(W, hipMemcpy(t, src, n * sizeof(T), hipMemcpyDeviceToHost))) return false;
+        if (!host_copy(s, t, src, n * sizeof(T), hipMemcpyDeviceToHost, false, W)) return false;
         for (long r = 0; r < rows; r++)
             for (long k = 0; k < nz; k++) dst[r * nz + k] = double(t[r * sy + k]);
         return true;
@@ -691,7 +702,7 @@ static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W
         for (long q = 0; ok && q < rows; q += most) {
             const long m = std::min(most, rows - q);
             Ops<T>::pack(c, src + q * sy, b, m);
-            ok = pllc_hip_ok(W, hipMemcpyAsync(dst + q * nz, b, m * nz * 8, hipMemcpyDeviceToHost, s->st));
+            ok = host_copy(s, dst + q * nz, b, m * nz * 8, hipMemcpyDeviceToHost, locked, W);
         }
         break;
     }
@@ -713,7 +724,7 @@ static int init_t(pllc_sim* s, Ctx<T>& c, const double* c_full)
     std::vector<double> h(n);
     if (c_full) memcpy(h.data(), c_full, n * 8);
     else if (pllc_ic_fill(&s->p, PLLC_IC_ERF, 0, 0.0, h.data())) return -1;
-    if (!h2d<T>(s, c, c.f[C_NEW], 0, (long)d.NX * d.NY, h.data(), W)) return -1;
+    if (!h2d<T>(s, c, c.f[C_NEW], 0, (long)d.NX * d.NY, h.data(), W, true)) return -1;
     const Geo g = make_geo(&s->p);
     std::vector<double> plane((size_t)d.NY * d.NZ, 0.0);
     auto pl = [&](int j, int k) -> double& { return plane[(size_t)j * d.NZ + k]; };
@@ -723,7 +734,7 @@ static int init_t(pllc_sim* s, Ctx<T>& c, const double* c_full)
         pl(j, d.nz + 1) = pl(j, d.nz);
     }
     for (int k = 0; k <= d.nz + 1; k++) { pl(0, k) = -pl(1, k); pl(d.ny + 1, k) = -pl(d.ny, k); }
-    if (!h2d<T>(s, c, c.f[U_NEW], 3L * d.NY, d.NY, plane.data(), W)) return -1;
+    if (!h2d<T>(s, c, c.f[U_NEW], 3L * d.NY, d.NY, plane.data(), W, true)) return -1;
     Ops<T>::velo_ghost(c);   // update_ghost_points (81); phi is 0
     update_old_copy<T>(c);  // (82-83)
     if (s->p.Nmvp == 1) {
