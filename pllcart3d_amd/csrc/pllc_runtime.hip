@@ -7,6 +7,7 @@
 #include <array>
 #include <map>
 #include <mutex>
+#include <new>
 #include <tuple>
 #include <type_traits>
 #include <cmath>
@@ -637,16 +638,20 @@ static double* stage(Ctx<T>& c, long& rows)
 }
 
 // the host's side of a HOST transfer, kept with the handle (allocated anew for
-// every transfer, its page faults took twice the conversion's time)
+// every transfer, its page faults took twice the conversion's time); null (error
+// set) when there is no memory for it
 template <typename T>
-static T* host_side(pllc_sim* s, size_t n)
+static T* host_side(pllc_sim* s, size_t n, const char* W)
 {
-    if constexpr (std::is_same<T, float>::value) {
-        if (s->host.size() < n) s->host.resize(n);
-        return s->host.data();
-    } else {
-        return nullptr;   // FP64 fields have no such transfers
+    if constexpr (std::is_same<T, float>::value) {   // FP64 fields have no such transfers
+        try {
+            if (s->host.size() < n) s->host.resize(n);
+            return s->host.data();
+        } catch (const std::bad_alloc&) {
+            pllc_set_error(W, "no host memory for the conversion");
+        }
     }
+    return nullptr;
 }
 
 // dst (a field, or rows of it from row r0 on) from `rows` host rows of NZ
@@ -661,7 +666,8 @@ static bool h2d(pllc_sim* s, Ctx<T>& c, T* dst, long r0, long rows, const double
     switch (route<T>(c.d, locked, once)) {
     case Route::DIRECT: ok = host_copy(s, dst + r0 * sy, src, rows * nz * 8, hipMemcpyHostToDevice, locked, W); break;
     case Route::HOST: {
-        T* t = host_side<T>(s, n);
+        T* t = host_side<T>(s, n, W);
+        if (!t) return false;
         for (long r = 0; r < rows; r++)
             for (long k = 0; k < nz; k++) t[r * sy + k] = T(src[r * nz + k]);
         ok = host_copy(s, dst + r0 * sy, t, n * sizeof(T), hipMemcpyHostToDevice, false, W);
@@ -690,8 +696,8 @@ static bool d2h(pllc_sim* s, Ctx<T>& c, double* dst, const T* src, const char* W
     switch (route<T>(c.d, locked)) {
     case Route::DIRECT: ok = host_copy(s, dst, src, rows * nz * 8, hipMemcpyDeviceToHost, locked, W); break;
     case Route::HOST: {
-        T* t = host_side<T>(s, n);
-        if (!host_copy(s, t, src, n * sizeof(T), hipMemcpyDeviceToHost, false, W)) return false;
+        T* t = host_side<T>(s, n, W);
+        if (!t || !host_copy(s, t, src, n * sizeof(T), hipMemcpyDeviceToHost, false, W)) return false;
         for (long r = 0; r < rows; r++)
             for (long k = 0; k < nz; k++) dst[r * nz + k] = double(t[r * sy + k]);
         return true;
