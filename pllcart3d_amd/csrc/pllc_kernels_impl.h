@@ -272,15 +272,38 @@ __device__ __forceinline__ void rhs_conc_line(const Dims& d, const Phys& ph, con
             st.at(p, cx7, cy7, cz7);
             const T uval = T(0.5) * (u1[p] + u0[p]), vval = T(0.5) * (v1[p] + v0[p]), wval = T(0.5) * (w[p + 1] + w[p]);
             T nval, diff;
+            // A c by the reference's sums (1411-1440, 573-590)
+            auto diffusion = [&]() {
+                T ax, bx, cx, ay, by, cy, az, bz, cz;
+                Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
+                coefs<T, FC, 0>(d, ph, none, 0, ax, bx, cx);
+                coefs<T, FC, 1>(d, ph, none, 0, ay, by, cy);
+                coefs<T, FC, 2>(d, ph, none, 0, az, bz, cz);
+                const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
+                const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
+                const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
+                return axx + axy + axz;
+            };
             if constexpr (FAST) {
                 T xm, xp, ym, yp, zm, zp;
                 const T cx = upwind_term<T>(cx7, i, R.is, R.ie, uval, T(d.dx), T(d.rdx), T(0.0), T(0.0), xm, xp);
                 const T cy = upwind_term<T>(cy7, j, R.js, R.je, vval, T(d.dy), T(d.rdy), ylo, yhi, ym, yp);
                 const T cz = upwind_term<T>(cz7, k, R.ks, R.ke, wval, T(d.dz), T(d.rdz), zlo, zhi, zm, zp);
                 nval = -(cz + cx + cy);
-                diff = kx * (xp - xm);
-                diff = fma(ky, yp - ym, diff);
-                diff = fma(kz, zp - zm, diff);
+                // FP64: in the reference's roundings.  Where c is 1 up to its last
+                // bits the sums leave those bits to rounding, and the front amplifies
+                // whatever differs there: with the differences xp - xm, which round
+                // less, c departs from the reference by 1.7e-12 in 200 steps at
+                // 256x128x128 and 4e-11 in 730 (as the reference does from itself when
+                // its initial state changes in the last bit), so by 7e-16.  263.1 ->
+                // 263.8 us a launch.
+                if constexpr (sizeof(T) == 8) {
+                    diff = diffusion();
+                } else {
+                    diff = kx * (xp - xm);
+                    diff = fma(ky, yp - ym, diff);
+                    diff = fma(kz, zp - zm, diff);
+                }
             } else {
                 T D[6];
 #pragma unroll
@@ -294,15 +317,7 @@ __device__ __forceinline__ void rhs_conc_line(const Dims& d, const Phys& ph, con
                 for (int m = 0; m < 6; m++) D[m] = divh<T>(cz7[m + 1] - cz7[m], T(d.dz), d.rdz);
                 const T czd = upwind_d<T>(D, k, R.ks, R.ke, wval >= T(0.0) ? 1 : -1, T(d.dz), d.rdz, zlo, zhi);
                 nval = -(wval * czd + convx + convy);
-                T ax, bx, cx, ay, by, cy, az, bz, cz;
-                Visc4<T> none{nullptr, nullptr, nullptr, nullptr};
-                coefs<T, FC, 0>(d, ph, none, 0, ax, bx, cx);
-                coefs<T, FC, 1>(d, ph, none, 0, ay, by, cy);
-                coefs<T, FC, 2>(d, ph, none, 0, az, bz, cz);
-                const T axx = ax * cx7[2] + bx * cx7[3] + cx * cx7[4];
-                const T axy = ay * cy7[2] + by * cy7[3] + cy * cy7[4];
-                const T axz = az * cz7[2] + bz * cz7[3] + cz * cz7[4];
-                diff = axx + axy + axz;
+                diff = diffusion();
             }
             if (ncorr) nval += nc[p];
             nv[p] = nval;
